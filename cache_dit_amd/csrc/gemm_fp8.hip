@@ -427,10 +427,19 @@ struct NoGroup {};
 // clock (100 MHz) at its start and after its last store has been issued and its DMA has
 // drained, the id of the XCD it ran on and the number of tiles it took -- so that the spread
 // of the finish times over the XCDs can be read off a real launch.
+// KTAIL: K is any multiple of 16 (the conversion policy asks no more of a Linear), not of a
+// step's 128 bytes. The 16-byte chunks of a panel row beyond K are sent to an offset beyond
+// the DMA descriptor, for which zeros land in the LDS: both operands are zero there, and so
+// is what the last step adds. K shorter than the prefetch depth is walked as `depth` steps of
+// which the last ones are all zeros. The chunk a lane fetches is the same for every DMA
+// instruction of a panel (swz_a / swz_b take the row bits that the lane and the parity of the
+// wave give), so a step costs one comparison per panel and one OR per DMA instruction.
+// Without it such a K ran one scalar FMA per element: 1357 x 2224 x 4464 16.8 ms (1.6
+// TFLOP/s); with it 25 us.
 struct StampArgs {
   unsigned long long* stamps;
 };
-template <class C, int OUT = CDIT_DT_BF16, bool GROUPED = false, bool STAMPS = false>
+template <class C, int OUT = CDIT_DT_BF16, bool GROUPED = false, bool STAMPS = false, bool KTAIL = false>
 __global__ __launch_bounds__(C::THREADS) __attribute__((amdgpu_waves_per_eu(1, 1))) void
 gemm_fp8_wide(GemmArgs g, int tiles_m, int tiles_n,
               std::conditional_t<GROUPED, GemmGroup, std::conditional_t<STAMPS, StampArgs, NoGroup>> grp) {
@@ -448,7 +457,8 @@ gemm_fp8_wide(GemmArgs g, int tiles_m, int tiles_n,
   // output stores per wave and tile (16 bytes per lane each); every wave issues all of them
   constexpr int NST = TM * (TN / 2) * (OUT == CDIT_DT_F32 ? 2 : 1);
   static_assert((D - 2) * C::ND + C::NDA + NST <= 63, "vmcnt is a 6-bit counter");
-  const int KT = g.K / BKW;  // >= D (checked by the launcher)
+  // >= max(D, 3) (checked by the launcher, or padded here)
+  const int KT = KTAIL ? max((g.K + BKW - 1) / BKW, D > 3 ? D : 3) : g.K / BKW;
   int ntiles = tiles_m * tiles_n;
   if constexpr (GROUPED) ntiles = grp.tile_begin[grp.acts];
 
@@ -566,6 +576,13 @@ gemm_fp8_wide(GemmArgs g, int tiles_m, int tiles_n,
     }
   };
   set_source(m0, n0, cur, cur_act);
+  // KTAIL: first K byte of the chunk this lane fetches of every A (B) panel row
+  const int chunk_a = ((lane & 7) ^ swz_a(wave * 8 + (lane >> 3))) * 16;
+  const int chunk_b = ((lane & 7) ^ swz_b(wave * 8 + (lane >> 3))) * 16;
+  auto beyond_k = [&](int kt, int chunk) -> uint32_t {
+    if constexpr (KTAIL) return kt * BKW + chunk < g.K ? 0u : 0x80000000u;
+    return 0u;
+  };
   // buffer_load ... lds (MUBUF form: the compiler tracks it with vmcnt only, while
   // the global_load form makes it wait for all LDS reads at every use). With a
   // descriptor of zero records every lane is out of range: nothing is fetched and
@@ -575,14 +592,14 @@ gemm_fp8_wide(GemmArgs g, int tiles_m, int tiles_n,
         __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(A), 0, nrec, 0x00020000);
     __builtin_amdgcn_raw_ptr_buffer_load_lds(
         rsrc, (__attribute__((address_space(3))) void*)(smem + a_lds + (wave + 4 * p) * 1024), 16,
-        (int)off[p], kt * BKW, 0, 0);
+        (int)(off[p] | beyond_k(kt, chunk_a)), kt * BKW, 0, 0);
   };
   auto dma_b = [&](int kt, int b_lds, int p) {
     const __amdgpu_buffer_rsrc_t rsrc =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(B), 0, nrec, 0x00020000);
     __builtin_amdgcn_raw_ptr_buffer_load_lds(
         rsrc, (__attribute__((address_space(3))) void*)(smem + b_lds + (wave + 4 * p) * 1024), 16,
-        (int)off[C::NDA + p], kt * BKW, 0, 0);
+        (int)(off[C::NDA + p] | beyond_k(kt, chunk_b)), kt * BKW, 0, 0);
   };
 
   // operand read map
@@ -1012,11 +1029,11 @@ gemm_fp8_wide(GemmArgs g, int tiles_m, int tiles_n,
   }
 }
 
-template <class C, int OUT = CDIT_DT_BF16>
+template <class C, int OUT = CDIT_DT_BF16, bool KTAIL = false>
 int launch_wide(const GemmArgs& g, hipStream_t stream) {
   static bool lds_allowed[64];
-  if (int rc = allow_dynamic_lds(reinterpret_cast<const void*>(&gemm_fp8_wide<C, OUT>), C::LDS_BYTES,
-                                 lds_allowed))
+  if (int rc = allow_dynamic_lds(reinterpret_cast<const void*>(&gemm_fp8_wide<C, OUT, false, false, KTAIL>),
+                                 C::LDS_BYTES, lds_allowed))
     return rc;
   const int cus = cu_count();
   if (cus <= 0) {
@@ -1026,8 +1043,8 @@ int launch_wide(const GemmArgs& g, hipStream_t stream) {
   const int tiles_m = (g.M + C::BM - 1) / C::BM, tiles_n = (g.N + C::BN - 1) / C::BN;
   const int ntiles = tiles_m * tiles_n;
   // one persistent workgroup per CU (its LDS and registers fill the CU)
-  hipLaunchKernelGGL((gemm_fp8_wide<C, OUT>), dim3(ntiles < cus ? ntiles : cus), dim3(C::THREADS),
-                     C::LDS_BYTES, stream, g, tiles_m, tiles_n, NoGroup{});
+  hipLaunchKernelGGL((gemm_fp8_wide<C, OUT, false, false, KTAIL>), dim3(ntiles < cus ? ntiles : cus),
+                     dim3(C::THREADS), C::LDS_BYTES, stream, g, tiles_m, tiles_n, NoGroup{});
   return 0;
 }
 
@@ -1102,7 +1119,7 @@ __global__ __launch_bounds__(256) void gemm_fp8_skinny(GemmArgs g) {
   const int r = lane & 15, kg = lane >> 4;
   const int n0 = blockIdx.x * 16;
   const int nrow = min(n0 + r, g.N - 1);
-  const int KT = g.K / 128;           // 128-byte steps in total
+  const int KT = (g.K + 127) / 128;   // 128-byte steps in total, the last one maybe partial
   const int per = (KT + 3) / 4;       // steps per wave
   const int k_begin = wave * per, k_end = min(KT, k_begin + per);
   const uint8_t* __restrict__ wp = g.b + (int64_t)nrow * g.ldb + kg * 32;
@@ -1116,12 +1133,13 @@ __global__ __launch_bounds__(256) void gemm_fp8_skinny(GemmArgs g) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int kt = min(k0 + u, k_end - 1);  // clamped duplicates are not accumulated
-      const v4i* wq = reinterpret_cast<const v4i*>(wp + (int64_t)kt * 128);
-      w[u][0] = wq[0];
-      w[u][1] = wq[1];
-      const v4i* aq = reinterpret_cast<const v4i*>(ap + (int64_t)kt * 128);
-      a[u][0] = aq[0];
-      a[u][1] = aq[1];
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {  // (16 bytes beyond K are zeros on both sides)
+        const int k = kt * 128 + e * 16;
+        const bool in = k + kg * 32 < g.K;
+        w[u][e] = in ? *reinterpret_cast<const v4i*>(wp + k) : v4i{0, 0, 0, 0};
+        a[u][e] = in ? *reinterpret_cast<const v4i*>(ap + k) : v4i{0, 0, 0, 0};
+      }
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -1184,7 +1202,7 @@ __global__ __launch_bounds__(256) void linear_fp8_skinny_fused(GemmArgs g, uint8
   const int r = lane & 15, kg = lane >> 4;
   const int n0 = blockIdx.x * 16;
   const int nrow = min(n0 + r, g.N - 1);
-  const int KT = g.K / 128;
+  const int KT = (g.K + 127) / 128;
   const int per = (KT + 3) / 4;
   const int k_begin = wave * per, k_end = min(KT, k_begin + per);
   const int pitch = g.K + kFusedPad;
@@ -1195,9 +1213,11 @@ __global__ __launch_bounds__(256) void linear_fp8_skinny_fused(GemmArgs g, uint8
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int kt = min(k0 + u, max(k_end, 1) - 1);  // clamped duplicates are not accumulated
-      const v4i* wq = reinterpret_cast<const v4i*>(wp + (int64_t)kt * 128);
-      w[u][0] = wq[0];
-      w[u][1] = wq[1];
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {  // (16 bytes beyond K are zeros on both sides)
+        const int k = kt * 128 + e * 16;
+        w[u][e] = k + kg * 32 < g.K ? *reinterpret_cast<const v4i*>(wp + k) : v4i{0, 0, 0, 0};
+      }
     }
   };
   load_w(k_begin);
@@ -1251,8 +1271,13 @@ __global__ __launch_bounds__(256) void linear_fp8_skinny_fused(GemmArgs g, uint8
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       if (k0 + u < k_end) {
-        const v4i* aq = reinterpret_cast<const v4i*>(ap + (k0 + u) * 128);
-        v8i af = __builtin_shufflevector(aq[0], aq[1], 0, 1, 2, 3, 4, 5, 6, 7);
+        v4i a[2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          const int k = (k0 + u) * 128 + e * 16;
+          a[e] = k + kg * 32 < g.K ? *reinterpret_cast<const v4i*>(ap + k) : v4i{0, 0, 0, 0};
+        }
+        v8i af = __builtin_shufflevector(a[0], a[1], 0, 1, 2, 3, 4, 5, 6, 7);
         if (!a_valid) af = v8i{0, 0, 0, 0, 0, 0, 0, 0};
         const v8i wf = __builtin_shufflevector(w[u][0], w[u][1], 0, 1, 2, 3, 4, 5, 6, 7);
         acc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf, af, acc, 0, 0, 0, 0, 0, 0);
@@ -1411,8 +1436,8 @@ __global__ __launch_bounds__(64 * kRow1Waves) void linear_fp8_row1(GemmArgs g, u
 }
 
 // Any shape, any alignment: a 16x16 output tile per workgroup, one output
-// element per thread, scalar decode + FMA. Only for shapes the tiled kernel
-// cannot take (K not a multiple of 128, N not a multiple of 8, odd strides).
+// element per thread, scalar decode + FMA. Only for what the other kernels cannot take
+// (N not a multiple of 8, odd strides, misaligned operands).
 __global__ __launch_bounds__(256) void gemm_fp8_generic(GemmArgs g) {
   const int n = blockIdx.x * 16 + (threadIdx.x & 15);
   const int m = blockIdx.y * 16 + (threadIdx.x >> 4);
@@ -1443,8 +1468,9 @@ int launch_tiled(const GemmArgs& g, hipStream_t stream) {
   return 0;
 }
 
-bool tiled_ok(const GemmArgs& g) {
-  return g.K >= BK && g.K % BK == 0 && g.N % 8 == 0 && g.lda % 16 == 0 && g.ldb % 16 == 0 && g.ldo % 8 == 0 &&
+// What every kernel but the generic one asks of its operands; K is any multiple of 16 here.
+bool aligned_ok(const GemmArgs& g) {
+  return g.K >= 16 && g.K % 16 == 0 && g.N % 8 == 0 && g.lda % 16 == 0 && g.ldb % 16 == 0 && g.ldo % 8 == 0 &&
          reinterpret_cast<uintptr_t>(g.a) % 16 == 0 && reinterpret_cast<uintptr_t>(g.b) % 16 == 0 &&
          reinterpret_cast<uintptr_t>(g.out) % 16 == 0 &&
          // the epilogues fetch scales and bias in 16-byte pieces
@@ -1455,6 +1481,8 @@ bool tiled_ok(const GemmArgs& g) {
          (int64_t)512 * g.lda < (int64_t)1 << 31 && (int64_t)512 * g.ldb < (int64_t)1 << 31 &&
          (int64_t)512 * g.ldo < (int64_t)1 << 29;
 }
+
+bool tiled_ok(const GemmArgs& g) { return g.K >= BK && g.K % BK == 0 && aligned_ok(g); }
 
 }  // namespace
 
@@ -1483,7 +1511,7 @@ typedef CfgWide<288, 192, 4, 2, false> V14H;
 template <bool FUSED>
 int launch_row1(const GemmArgs& g, uint8_t* q_ws, float* scale_ws, int scale_mode, int variant,
                 hipStream_t stream) {
-  const bool ok = g.M == 1 && g.K >= 128 && g.K % 128 == 0 && g.K <= 4096 && g.ldb % 16 == 0 &&
+  const bool ok = g.M == 1 && g.K >= 16 && g.K % 16 == 0 && g.K <= 4096 && g.ldb % 16 == 0 &&
                   reinterpret_cast<uintptr_t>(g.a) % 16 == 0 && reinterpret_cast<uintptr_t>(g.b) % 16 == 0 &&
                   (!FUSED || reinterpret_cast<uintptr_t>(q_ws) % 8 == 0) &&
                   (variant < 0 || variant == 51);
@@ -1512,11 +1540,11 @@ int launch_linear_fp8_skinny_fused(const GemmArgs& g, void* q_ws, float* scale_w
   two_step.a = q_ws;
   two_step.a_scale = scale_ws;
   two_step.lda = g.K;
-  if (!tiled_ok(two_step)) return 1;
+  if (!aligned_ok(two_step)) return 1;
   if (launch_row1<true>(g, static_cast<uint8_t*>(q_ws), scale_ws, scale_mode, variant, stream) == 0) return 0;
   const int64_t lds = (int64_t)g.M * (g.K + kFusedPad);
-  const bool ok = g.M >= 1 && g.M <= 16 && (variant < 0 || variant == 50) && g.K >= 128 &&
-                  g.K % 128 == 0 && g.N % 8 == 0 && lds <= 48 * 1024 && g.lda % 8 == 0 &&
+  const bool ok = g.M >= 1 && g.M <= 16 && (variant < 0 || variant == 50) && g.K >= 16 &&
+                  g.K % 16 == 0 && g.N % 8 == 0 && lds <= 48 * 1024 && g.lda % 8 == 0 &&
                   g.ldb % 16 == 0 && g.ldo % 8 == 0 &&
                   reinterpret_cast<uintptr_t>(g.a) % 16 == 0 &&
                   reinterpret_cast<uintptr_t>(g.b) % 16 == 0 &&
@@ -1534,6 +1562,7 @@ struct TileChoice {
 };
 template <class Tiles, class WideOk>
 TileChoice choose_bf16_variant(Tiles tiles, WideOk wide_ok);
+int launch_gemm_fp8_ktail(const GemmArgs& g, int variant, hipStream_t stream);
 template <class WideOk>
 int launch_bf16_variant(const GemmArgs& g, int variant, WideOk wide_ok, hipStream_t stream);
 
@@ -1548,7 +1577,7 @@ int launch_gemm_fp8_stamps(const GemmArgs& g, unsigned long long* stamps, int* w
 }
 
 int launch_gemm_fp8(const GemmArgs& g, int variant, hipStream_t stream) {
-  if (!tiled_ok(g) || variant == 100) {
+  if (!aligned_ok(g) || variant == 100) {
     dim3 grid((g.N + 15) / 16, (g.M + 15) / 16);
     hipLaunchKernelGGL(gemm_fp8_generic, grid, dim3(256), 0, stream, g);
     return 0;
@@ -1564,6 +1593,7 @@ int launch_gemm_fp8(const GemmArgs& g, int variant, hipStream_t stream) {
     hipLaunchKernelGGL(gemm_fp8_skinny, dim3((g.N + 15) / 16), dim3(256), 0, stream, g);
     return 0;
   }
+  if (!tiled_ok(g)) return launch_gemm_fp8_ktail(g, variant, stream);
   // the wide kernels stream K two or more steps ahead: shorter K runs the 128x128 kernel
   // at least `depth` K steps to prefetch, and at least 3: the epilogue operands of a tile are
   // staged in LDS two steps before its end, which must be behind the first barrier of the
@@ -1598,6 +1628,31 @@ int launch_gemm_fp8(const GemmArgs& g, int variant, hipStream_t stream) {
         wide_ok).variant;
   }
   return launch_bf16_variant(g, variant, wide_ok, stream);
+}
+
+// K a multiple of 16 but not of 128, or shorter than a step: the KTAIL instances of the wide
+// kernel (they take any K, so the choice of the tile is the one for a long K; fp16 and fp32
+// outputs have one large and one small tile, as below).
+int launch_gemm_fp8_ktail(const GemmArgs& g, int variant, hipStream_t stream) {
+  auto tiles = [&](int bm, int bn) { return (int64_t)((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn); };
+  if (g.out_dtype != CDIT_DT_BF16) {
+    const int64_t ncu = cu_count() > 0 ? cu_count() : 256;
+    const bool large = variant == 15 || (variant != 17 && (tiles(256, 192) + ncu - 1) / ncu * 256 * 192 * 1000 <=
+                                                              (tiles(64, 128) + ncu - 1) / ncu * 64 * 128 * 1493);
+    if (g.out_dtype == CDIT_DT_F16)
+      return large ? launch_wide<V15, CDIT_DT_F16, true>(g, stream) : launch_wide<V17, CDIT_DT_F16, true>(g, stream);
+    return large ? launch_wide<V15, CDIT_DT_F32, true>(g, stream) : launch_wide<V17, CDIT_DT_F32, true>(g, stream);
+  }
+  const bool forced = variant == 12 || (variant >= 14 && variant <= 18);
+  if (!forced) variant = choose_bf16_variant(tiles, [](int) { return true; }).variant;
+  switch (variant) {
+    case 12: return launch_wide<V12, CDIT_DT_BF16, true>(g, stream);
+    case 14: return launch_wide<V14, CDIT_DT_BF16, true>(g, stream);
+    case 15: return launch_wide<V15, CDIT_DT_BF16, true>(g, stream);
+    case 16: return launch_wide<V16, CDIT_DT_BF16, true>(g, stream);
+    case 17: return launch_wide<V17, CDIT_DT_BF16, true>(g, stream);
+    default: return launch_wide<V18, CDIT_DT_BF16, true>(g, stream);
+  }
 }
 
 // Tile choice for a bf16-output problem whose tile count for a bm x bn tile is tiles(bm, bn)

@@ -376,7 +376,11 @@ struct NoGroup {};
 // has its own weight, scale, bias, output and epilogue flag, K and the row strides are
 // common (the B-side fields of `g` and grp.a_scale are unused). The instances without it are
 // unchanged by its existence.
-template <class C, bool GROUPED = false>
+// KTAIL: K is any multiple of 16, as in the w8a8 kernel: the 16-byte chunks of a panel row
+// beyond K go to an offset beyond the DMA descriptor, for which zeros land in the LDS, and a
+// K shorter than the prefetch depth is padded with steps of zeros. The chunk a lane fetches
+// is the same for every DMA instruction of a panel.
+template <class C, bool GROUPED = false, bool KTAIL = false>
 __global__ __launch_bounds__(C::THREADS) __attribute__((amdgpu_waves_per_eu(1, 1))) void
 gemm_w8a16_wide(GemmArgs g, int tiles_m, int tiles_n,
                 std::conditional_t<GROUPED, GemmGroup, NoGroup> grp) {
@@ -389,7 +393,8 @@ gemm_w8a16_wide(GemmArgs g, int tiles_m, int tiles_n,
   // lambda makes the host pass drop the kernel stub without a diagnostic
   constexpr int TM = C::TM, TN = C::TN, H = C::H, A_ROW = C::A_ROW, B_ROW = C::B_ROW;
   constexpr int D = C::DEPTH;
-  const int KT = g.K / BKE;  // >= D (checked by the launcher)
+  // >= max(D, 3) (checked by the launcher, or padded here)
+  const int KT = KTAIL ? max((g.K + BKE - 1) / BKE, D > 3 ? D : 3) : g.K / BKE;
   int ntiles = tiles_m * tiles_n;
   if constexpr (GROUPED) ntiles = grp.tile_begin[grp.acts];
 
@@ -487,19 +492,26 @@ gemm_w8a16_wide(GemmArgs g, int tiles_m, int tiles_n,
     }
   };
   set_source(m0, n0, cur, cur_act);
+  // KTAIL: first K element of the chunk this lane fetches of every A (B) panel row
+  const int chunk_a = ((lane & 7) ^ (((wave * 8 + (lane >> 3)) >> 1) & 7)) * 8;
+  const int chunk_b = ((lane & 3) ^ ((lane >> 4) & 3)) * 16;
+  auto beyond_k = [&](int kt, int chunk) -> uint32_t {
+    if constexpr (KTAIL) return kt * BKE + chunk < g.K ? 0u : 0x80000000u;
+    return 0u;
+  };
   auto dma_a = [&](int kt, int a_lds, int p) {
     const __amdgpu_buffer_rsrc_t rsrc =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(A), 0, nrec, 0x00020000);
     __builtin_amdgcn_raw_ptr_buffer_load_lds(
         rsrc, (__attribute__((address_space(3))) void*)(smem + a_lds + (wave + 4 * p) * 1024), 16,
-        (int)off[p], kt * A_ROW, 0, 0);
+        (int)(off[p] | beyond_k(kt, chunk_a)), kt * A_ROW, 0, 0);
   };
   auto dma_b = [&](int kt, int b_lds, int p) {
     const __amdgpu_buffer_rsrc_t rsrc =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(B), 0, nrec, 0x00020000);
     __builtin_amdgcn_raw_ptr_buffer_load_lds(
         rsrc, (__attribute__((address_space(3))) void*)(smem + b_lds + (wave + 4 * p) * 1024), 16,
-        (int)off[C::NDA + p], kt * B_ROW, 0, 0);
+        (int)(off[C::NDA + p] | beyond_k(kt, chunk_b)), kt * B_ROW, 0, 0);
   };
 
   // operand read map: A row lane&31 of its block, chunks 4t+2h+s; W operand row
@@ -863,11 +875,11 @@ gemm_w8a16_wide(GemmArgs g, int tiles_m, int tiles_n,
   wait_vm<0>();
 }
 
-template <class C>
+template <class C, bool KTAIL = false>
 int launch_wide(const GemmArgs& g, hipStream_t stream) {
   static bool lds_allowed[64];
-  if (int rc = allow_dynamic_lds(reinterpret_cast<const void*>(&gemm_w8a16_wide<C>), C::LDS_BYTES,
-                                 lds_allowed))
+  if (int rc = allow_dynamic_lds(reinterpret_cast<const void*>(&gemm_w8a16_wide<C, false, KTAIL>),
+                                 C::LDS_BYTES, lds_allowed))
     return rc;
   const int cus = cu_count();
   if (cus <= 0) {
@@ -877,8 +889,8 @@ int launch_wide(const GemmArgs& g, hipStream_t stream) {
   const int tiles_m = (g.M + C::BM - 1) / C::BM, tiles_n = (g.N + C::BN - 1) / C::BN;
   const int ntiles = tiles_m * tiles_n;
   // one persistent workgroup per CU (its LDS and registers fill the CU)
-  hipLaunchKernelGGL(gemm_w8a16_wide<C>, dim3(ntiles < cus ? ntiles : cus), dim3(C::THREADS),
-                     C::LDS_BYTES, stream, g, tiles_m, tiles_n, NoGroup{});
+  hipLaunchKernelGGL((gemm_w8a16_wide<C, false, KTAIL>), dim3(ntiles < cus ? ntiles : cus),
+                     dim3(C::THREADS), C::LDS_BYTES, stream, g, tiles_m, tiles_n, NoGroup{});
   return 0;
 }
 
@@ -928,7 +940,7 @@ __global__ __launch_bounds__(256) void gemm_w8a16_skinny(GemmArgs g) {
   const int r = lane & 15, kg = lane >> 4;
   const int n0 = blockIdx.x * 16;
   const int nrow = min(n0 + r, g.N - 1);
-  const int KT = g.K / 128;
+  const int KT = (g.K + 127) / 128;  // the last 128-element chunk may be partial
   const int per = (KT + 3) / 4;
   const int k_begin = wave * per, k_end = min(KT, k_begin + per);
   const uint8_t* __restrict__ wp = g.b + (int64_t)nrow * g.ldb + kg * 32;
@@ -943,12 +955,14 @@ __global__ __launch_bounds__(256) void gemm_w8a16_skinny(GemmArgs g) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int kt = min(k0 + u, k_end - 1);
-      const uint4* wq = reinterpret_cast<const uint4*>(wp + (int64_t)kt * 128);
-      w[u][0] = wq[0];
-      w[u][1] = wq[1];
       const v8bf* aq = reinterpret_cast<const v8bf*>(ap + (int64_t)kt * 128);
 #pragma unroll
-      for (int t = 0; t < 4; ++t) a[u][t] = aq[t];
+      for (int e = 0; e < 2; ++e) {  // (16 elements beyond K are zeros on both sides)
+        const bool in = kt * 128 + kg * 32 + e * 16 < g.K;
+        w[u][e] = in ? *reinterpret_cast<const uint4*>(wp + kt * 128 + e * 16) : uint4{0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int t = 2 * e; t < 2 * e + 2; ++t) a[u][t] = in ? aq[t] : v8bf{0, 0, 0, 0, 0, 0, 0, 0};
+      }
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -1099,8 +1113,9 @@ int launch_tiled(const GemmArgs& g, hipStream_t stream) {
   return 0;
 }
 
-bool tiled_ok(const GemmArgs& g) {
-  return g.K >= BKE && g.K % BKE == 0 && g.N % 8 == 0 && g.lda % 8 == 0 && g.ldb % 16 == 0 &&
+// What every kernel but the generic one asks of its operands; K is any multiple of 16 here.
+bool aligned_ok(const GemmArgs& g) {
+  return g.K >= 16 && g.K % 16 == 0 && g.N % 8 == 0 && g.lda % 8 == 0 && g.ldb % 16 == 0 &&
          g.ldo % 8 == 0 && reinterpret_cast<uintptr_t>(g.a) % 16 == 0 &&
          reinterpret_cast<uintptr_t>(g.b) % 16 == 0 &&
          reinterpret_cast<uintptr_t>(g.out) % 16 == 0 &&
@@ -1110,6 +1125,8 @@ bool tiled_ok(const GemmArgs& g) {
          (int64_t)1024 * g.lda < (int64_t)1 << 31 && (int64_t)512 * g.ldb < (int64_t)1 << 31 &&
          (int64_t)512 * g.ldo < (int64_t)1 << 29;  // 32-bit byte offsets within a block of rows
 }
+
+bool tiled_ok(const GemmArgs& g) { return g.K >= BKE && g.K % BKE == 0 && aligned_ok(g); }
 
 }  // namespace
 
@@ -1163,13 +1180,14 @@ TileChoice choose_variant(Tiles tiles, WideOk wide_ok) {
 }  // namespace
 
 int launch_gemm_w8a16(const GemmArgs& g, int variant, hipStream_t stream) {
-  if (!tiled_ok(g) || variant == 100) {
+  const bool k_tail = !tiled_ok(g);  // K not a whole number of steps
+  if (!aligned_ok(g) || (k_tail && g.M > 16 && g.N % 16 != 0) || variant == 100) {
     dim3 grid((g.N + 15) / 16, (g.M + 15) / 16);
     hipLaunchKernelGGL(gemm_w8a16_generic, grid, dim3(256), 0, stream, g);
     return 0;
   }
-  if ((variant < 0 || variant == 51) && g.M == 1 && g.K % 128 == 0 && g.K <= 4096) {
-    // (tiled_ok has checked the alignment of the operands and of ldb)
+  if ((variant < 0 || variant == 51) && g.M == 1 && g.K <= 4096) {
+    // (aligned_ok has checked the alignment of the operands and of ldb)
     constexpr int rows_wg = kRow1Rows * kRow1Waves;
     const dim3 grid((g.N + rows_wg - 1) / rows_wg), block(64 * kRow1Waves);
     switch ((g.K + 1023) / 1024) {
@@ -1180,9 +1198,9 @@ int launch_gemm_w8a16(const GemmArgs& g, int variant, hipStream_t stream) {
     }
     return 0;
   }
-  if ((variant < 0 && g.M <= 16 && g.K % 128 == 0) || variant == 50) {
-    if (g.M > 16 || g.K % 128 != 0) {
-      set_error("cdit_w8a16_gemm: the skinny kernel takes M <= 16 and K %% 128 == 0");
+  if ((variant < 0 && g.M <= 16) || variant == 50) {
+    if (g.M > 16) {
+      set_error("cdit_w8a16_gemm: the skinny kernel takes M <= 16");
       return CDIT_EINVAL;
     }
     hipLaunchKernelGGL(gemm_w8a16_skinny, dim3((g.N + 15) / 16), dim3(256), 0, stream, g);
@@ -1192,11 +1210,23 @@ int launch_gemm_w8a16(const GemmArgs& g, int variant, hipStream_t stream) {
   // at least `depth` K steps to prefetch, and at least 3: the epilogue operands of a tile are
   // staged in LDS two steps before its end, which must be behind the first barrier of the
   // tile (before it, slower waves may still be reading the previous tile's)
-  auto wide_ok = [&](int depth) { return g.K >= (depth > 3 ? depth : 3) * BKE && g.N % 16 == 0; };
-  if (variant < 0) {
+  auto wide_ok = [&](int depth) {
+    return (k_tail || g.K >= (depth > 3 ? depth : 3) * BKE) && g.N % 16 == 0;
+  };
+  if (variant < 0 || (k_tail && (variant < 7 || variant > 12))) {
     variant = choose_variant(
         [&](int bm, int bn) { return (int64_t)((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn); },
         wide_ok).variant;
+  }
+  if (k_tail) {  // the KTAIL instances of the wide kernel take any K
+    switch (variant) {
+      case 7: return launch_wide<W7, true>(g, stream);
+      case 8: return launch_wide<W8, true>(g, stream);
+      case 9: return launch_wide<W9, true>(g, stream);
+      case 10: return launch_wide<W10, true>(g, stream);
+      case 11: return launch_wide<W11, true>(g, stream);
+      default: return launch_wide<W12, true>(g, stream);
+    }
   }
   switch (variant) {
     case 0: return launch_tiled<W0>(g, stream);

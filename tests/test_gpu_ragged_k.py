@@ -1,0 +1,112 @@
+"""K that is a multiple of 16 and of nothing more, through every kernel that takes it: exact
+integers (every partial sum is below 2^24, so each order of summation gives the same fp32
+value and the comparison is bit for bit), operands that are views of wider rows whose
+remaining bytes are NaN (a read beyond K that counted would show), outputs framed by
+sentinels."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+FP8 = torch.float8_e4m3fn
+DEV = "cuda"
+
+# below one step of 128 (64) elements, on both sides of its multiples, below the prefetch depth,
+# and long
+KS = [16, 48, 112, 144, 240, 272, 336, 656, 1040, 2224]
+SHAPES = [(17, 72), (65, 136), (300, 528), (577, 400)]  # edges of the tiles, ragged rows and columns
+
+
+@pytest.fixture(autouse=True)
+def _auto_variant():
+  from cache_dit_amd import _native
+  _native.set_gemm_variant(-1)
+  yield
+  _native.set_gemm_variant(-1)
+
+
+def _ints(low, high, shape, g):
+  return torch.randint(low, high, shape, generator=g, device=DEV).float()
+
+
+def _framed(values, pad, dtype):
+  """`values` [R, K] as a view of rows of K + pad elements, the rest NaN."""
+  full = torch.full((values.shape[0], values.shape[1] + pad), float("nan"), device=DEV).to(dtype)
+  full[:, :values.shape[1]] = values.to(dtype)
+  return full[:, :values.shape[1]]
+
+
+def _problem(M, N, K, seed, act_dtype):
+  g = torch.Generator(device=DEV).manual_seed(seed)
+  a, w = _ints(-3, 4, (M, K), g), _ints(-3, 4, (N, K), g)
+  sa = torch.pow(2.0, torch.randint(-3, 3, (M, ), generator=g, device=DEV).float())
+  sw = torch.pow(2.0, torch.randint(-3, 3, (N, ), generator=g, device=DEV).float())
+  b = torch.randint(-8, 9, (N, ), generator=g, device=DEV).to(torch.bfloat16)
+  # fp64: the reference itself must not round
+  exact = (a.double() @ w.double().t()) * sw.double()[None, :]
+  return (_framed(a, 32, act_dtype), _framed(w, 48, FP8), sa, sw, b, exact)
+
+
+def _check(run, exact, M, N, what):
+  full = torch.full((M + 2, N + 8), 777.0, dtype=torch.bfloat16, device=DEV)
+  run(full[1:M + 1, :N])
+  torch.cuda.synchronize()
+  assert torch.equal(full[1:M + 1, :N], exact.float().to(torch.bfloat16)), what
+  full[1:M + 1, :N] = 777.0
+  assert bool((full == 777.0).all()), ("wrote outside the output", what)
+
+
+@pytest.mark.parametrize("variant", [-1, 12, 14, 15, 16, 17, 18])
+def test_w8a8_tiles(variant):
+  from cache_dit_amd import _native, ops
+  _native.set_gemm_variant(variant)
+  for i, K in enumerate(KS):
+    for M, N in SHAPES:
+      a, w, sa, sw, b, exact = _problem(M, N, K, 7 * i + M, FP8)
+      exact = exact * sa.double()[:, None] + b.double()[None, :]
+      _check(lambda out: ops.gemm_rowwise_into(a, sa, w, sw, b, out, 0), exact, M, N, (variant, M, N, K))
+
+
+@pytest.mark.parametrize("variant", [-1, 7, 8, 9, 10, 11, 12])
+def test_w8a16_tiles(variant):
+  from cache_dit_amd import _native, ops
+  _native.set_gemm_variant(variant)
+  for i, K in enumerate(KS):
+    for M, N in SHAPES:
+      # (72 and 136 columns are multiples of 8 and not of 16: the kernel for any shape)
+      a, w, _, sw, b, exact = _problem(M, N, K, 11 * i + M, torch.bfloat16)
+      exact = exact + b.double()[None, :]
+      _check(lambda out: ops.w8a16_into(a, w, sw, b, out, 0), exact, M, N, (variant, M, N, K))
+
+
+@pytest.mark.parametrize("M", [1, 2, 16])
+def test_few_rows(M):
+  from cache_dit_amd import ops
+  N = 264
+  for i, K in enumerate(KS + [4096 - 16, 4096 + 16]):
+    a, w, sa, sw, b, exact = _problem(M, N, K, 13 * i + M, FP8)
+    want = exact * sa.double()[:, None] + b.double()[None, :]
+    _check(lambda out: ops.gemm_rowwise_into(a, sa, w, sw, b, out, 0), want, M, N, ("w8a8", M, K))
+    x, w, _, sw, b, exact = _problem(M, N, K, 13 * i + M, torch.bfloat16)
+    _check(lambda out: ops.w8a16_into(x, w, sw, b, out, 0), exact + b.double()[None, :], M, N, ("w8a16", M, K))
+    # the whole Linear: rows whose maximum is 7 * 64, so that the scale is 1 and the codes are
+    # the integers themselves
+    x[:, 0] = 448.0
+    exact = (x.double() @ w.float().double().t()) * sw.double()[None, :] + b.double()[None, :]
+    q = torch.empty((M, K), dtype=FP8, device=DEV)
+    s = torch.empty((M, ), dtype=torch.float32, device=DEV)
+    _check(lambda out: ops.linear_w8a8_into(x, w, sw, b, out, q, s, 0, 0), exact, M, N, ("linear", M, K))
+    assert torch.equal(q.float(), x.float()) and bool((s == 1.0).all())
+
+
+@pytest.mark.parametrize("out_dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("variant", [15, 17])
+def test_other_output_types(out_dtype, variant):
+  from cache_dit_amd import _native, ops
+  _native.set_gemm_variant(variant)
+  for K in KS:
+    M, N = 300, 528
+    a, w, sa, sw, _, exact = _problem(M, N, K, K, FP8)
+    out = torch.empty((M, N), dtype=out_dtype, device=DEV)
+    ops.gemm_rowwise_into(a, sa, w, sw, None, out, 0)
+    torch.cuda.synchronize()
+    assert torch.equal(out, (exact * sa.double()[:, None]).float().to(out_dtype)), (out_dtype, variant, K)
