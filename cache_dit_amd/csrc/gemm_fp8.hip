@@ -576,30 +576,40 @@ gemm_fp8_wide(GemmArgs g, int tiles_m, int tiles_n,
     }
   };
   set_source(m0, n0, cur, cur_act);
-  // KTAIL: first K byte of the chunk this lane fetches of every A (B) panel row
-  const int chunk_a = ((lane & 7) ^ swz_a(wave * 8 + (lane >> 3))) * 16;
-  const int chunk_b = ((lane & 7) ^ swz_b(wave * 8 + (lane >> 3))) * 16;
-  auto beyond_k = [&](int kt, int chunk) -> uint32_t {
-    if constexpr (KTAIL) return kt * BKW + chunk < g.K ? 0u : 0x80000000u;
-    return 0u;
-  };
   // buffer_load ... lds (MUBUF form: the compiler tracks it with vmcnt only, while
   // the global_load form makes it wait for all LDS reads at every use). With a
   // descriptor of zero records every lane is out of range: nothing is fetched and
   // zeros land in the (free) stage, so the loop body has no special cases.
+  // KTAIL: a chunk of a panel row beyond K goes to an offset beyond the descriptor. (Kept out of
+  // the other instances altogether: an `| 0` that the optimiser folds still changed their
+  // register allocation.)
   auto dma_a = [&](int kt, int a_lds, int p) {
     const __amdgpu_buffer_rsrc_t rsrc =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(A), 0, nrec, 0x00020000);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(
-        rsrc, (__attribute__((address_space(3))) void*)(smem + a_lds + (wave + 4 * p) * 1024), 16,
-        (int)(off[p] | beyond_k(kt, chunk_a)), kt * BKW, 0, 0);
+    if constexpr (KTAIL) {
+      const int chunk = (lane & 7) ^ swz_a(wave * 8 + (lane >> 3));  // of every row it fetches
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          rsrc, (__attribute__((address_space(3))) void*)(smem + a_lds + (wave + 4 * p) * 1024), 16,
+          (int)(off[p] | (kt * BKW + chunk * 16 < g.K ? 0u : 0x80000000u)), kt * BKW, 0, 0);
+    } else {
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          rsrc, (__attribute__((address_space(3))) void*)(smem + a_lds + (wave + 4 * p) * 1024), 16,
+          (int)off[p], kt * BKW, 0, 0);
+    }
   };
   auto dma_b = [&](int kt, int b_lds, int p) {
     const __amdgpu_buffer_rsrc_t rsrc =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(B), 0, nrec, 0x00020000);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(
-        rsrc, (__attribute__((address_space(3))) void*)(smem + b_lds + (wave + 4 * p) * 1024), 16,
-        (int)(off[C::NDA + p] | beyond_k(kt, chunk_b)), kt * BKW, 0, 0);
+    if constexpr (KTAIL) {
+      const int chunk = (lane & 7) ^ swz_b(wave * 8 + (lane >> 3));
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          rsrc, (__attribute__((address_space(3))) void*)(smem + b_lds + (wave + 4 * p) * 1024), 16,
+          (int)(off[C::NDA + p] | (kt * BKW + chunk * 16 < g.K ? 0u : 0x80000000u)), kt * BKW, 0, 0);
+    } else {
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          rsrc, (__attribute__((address_space(3))) void*)(smem + b_lds + (wave + 4 * p) * 1024), 16,
+          (int)off[C::NDA + p], kt * BKW, 0, 0);
+    }
   };
 
   // operand read map
