@@ -936,8 +936,17 @@ int launch_wide_grouped(const GemmArgs& g, GemmGroup grp, hipStream_t stream) {
   return 0;
 }
 
+// Eight e4m3 values (two words) as bf16, exact. Not for operands of inline-assembly MFMAs.
+__device__ __forceinline__ v8bf e4m3x8_to_bf16(uint32_t lo, uint32_t hi) {
+  const v2bf c0 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 1.0f, false);
+  const v2bf c1 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 1.0f, true);
+  const v2bf c2 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 1.0f, false);
+  const v2bf c3 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 1.0f, true);
+  return v8bf{c0[0], c0[1], c1[0], c1[1], c2[0], c2[1], c3[0], c3[1]};
+}
+
 // ---------------------------------------------------------------------------
-// Skinny kernel for M <= 16 (M = 1 modulation Linears): weight streaming. A
+// Skinny kernel for 4 < M <= 16, and for fewer rows at K > 4096: weight streaming. A
 // workgroup of 4 waves owns 16 output channels, each wave a quarter of K. Per
 // 128-element chunk a lane (weight row l&15, K group l>>4) loads 32 e4m3 bytes
 // straight from HBM and the matching 32 bf16 activations (zero for rows >= M),
@@ -981,14 +990,10 @@ __global__ __launch_bounds__(256) void gemm_w8a16_skinny(GemmArgs g) {
                                    w[u][1].x, w[u][1].y, w[u][1].z, w[u][1].w};
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
-          const v2bf c0 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(words[2 * t], 1.0f, false);
-          const v2bf c1 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(words[2 * t], 1.0f, true);
-          const v2bf c2 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(words[2 * t + 1], 1.0f, false);
-          const v2bf c3 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(words[2 * t + 1], 1.0f, true);
-          const v8bf wf = {c0[0], c0[1], c1[0], c1[1], c2[0], c2[1], c3[0], c3[1]};
           v8bf af = a[u][t];
           if (!a_valid) af = v8bf{0, 0, 0, 0, 0, 0, 0, 0};
-          acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf, af, acc, 0, 0, 0);
+          acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(e4m3x8_to_bf16(words[2 * t], words[2 * t + 1]), af,
+                                                        acc, 0, 0, 0);
         }
       }
     }
@@ -1019,16 +1024,24 @@ __global__ __launch_bounds__(256) void gemm_w8a16_skinny(GemmArgs g) {
   }
 }
 
-// One activation row (M = 1: the modulation Linears), K <= 4096, with the access pattern of
-// the w8a8 path's linear_fp8_row1: a load instruction of the wavefront reads 1 KiB of one
-// weight row (lane l bytes 16 l .. 16 l + 15) where the 16-row arrangement above makes every
-// lane a memory request of its own; the MFMA's 16 "rows" are 16 interleaved K subsets of that
-// row, the activation is fetched at the same positions lane for lane (32 bytes of bf16 per
-// 16 weight bytes), D[i][i] is the partial dot product over subset i and the diagonal sums
-// to the whole one. A wavefront owns three whole rows, all of their loads in flight at once.
+// One to four activation rows (the modulation Linears: one embedding per image, with guidance
+// and a batch a few), K <= 4096, with the access pattern of the w8a8 path's linear_fp8_row1: a
+// load instruction of the wavefront reads 1 KiB of one weight row (lane l bytes 16 l ..
+// 16 l + 15) where the 16-row arrangement above makes every lane a memory request of its own;
+// the MFMA's 16 "rows" are 16 interleaved K subsets of that row, the activation is fetched at
+// the same positions lane for lane (32 bytes of bf16 per 16 weight bytes), D[i][i] is the partial
+// dot product over subset i and the diagonal sums to the whole one. A wavefront owns three whole
+// weight rows, all of their loads in flight at once; each further activation row costs its
+// MFMAs and a diagonal sum per weight row and no memory traffic to speak of.
+// With a different weight matrix per launch, against the 16-row kernel below 5 rows: 2 rows
+// 16.4 -> 14.2 us at N = 18432, K = 3072 (4.0 TB/s of weights), 8.2 -> 4.4 at 4096 x 1088;
+// 4 rows 18.3 -> 17.6 and, at N = 9216, 12.3 -> 9.9; one row is as before (12.0 and 7.5).
+// The activations are fetched inside the K loop: held across it they took the registers of
+// the wavefronts that keep the weight loads in flight.
 constexpr int kRow1Rows = 3, kRow1Waves = 4;
-template <int CHK>
-__global__ __launch_bounds__(64 * kRow1Waves) void gemm_w8a16_row1(GemmArgs g) {
+template <int CHK, int MA>
+__global__ __launch_bounds__(64 * kRow1Waves, MA == 1 ? 1 : (MA == 2 ? 6 : 4) - (CHK == 4 ? MA / 2 : 0)) void
+gemm_w8a16_rows(GemmArgs g) {
   constexpr int R = kRow1Rows;
   typedef float v4f_ __attribute__((ext_vector_type(4)));
   typedef unsigned int u4v __attribute__((ext_vector_type(4)));
@@ -1048,47 +1061,67 @@ __global__ __launch_bounds__(64 * kRow1Waves) void gemm_w8a16_row1(GemmArgs g) {
       }
     }
   }
-  const uint16_t* __restrict__ ap = static_cast<const uint16_t*>(g.a) + lane * 16;
   const v8bf zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
-  v8bf xa[CHK][2];
+  v4f_ acc[R][MA];
+#pragma unroll
+  for (int q = 0; q < R; ++q) {
+#pragma unroll
+    for (int m = 0; m < MA; ++m) acc[q][m] = v4f_{0.0f, 0.0f, 0.0f, 0.0f};
+  }
 #pragma unroll
   for (int c = 0; c < CHK; ++c) {
+    v8bf xa[MA][2];
     const bool in = c * 1024 + lane * 16 < g.K;
-    const v8bf* src = reinterpret_cast<const v8bf*>(ap + c * 1024);
-    xa[c][0] = in ? src[0] : zero8;
-    xa[c][1] = in ? src[1] : zero8;
+#pragma unroll
+    for (int m = 0; m < MA; ++m) {
+      const v8bf* src = reinterpret_cast<const v8bf*>(static_cast<const uint16_t*>(g.a) + m * g.lda +
+                                                      c * 1024 + lane * 16);
+      xa[m][0] = in ? src[0] : zero8;
+      xa[m][1] = in ? src[1] : zero8;
+    }
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const v8bf wf = e4m3x8_to_bf16(w[q][c][2 * t], w[q][c][2 * t + 1]);
+#pragma unroll
+        for (int m = 0; m < MA; ++m)
+          acc[q][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf, xa[m][t], acc[q][m], 0, 0, 0);
+      }
+    }
   }
   // lane l holds D[4 (l >> 4) + e][l & 15]: the diagonal entry of lanes 0-3, 20-23, 40-43, 60-63
   const int diag = (lane & 15) - 4 * (lane >> 4);
-  float mine = 0.0f;  // lane q keeps the dot product of row row0 + q
+  float mine = 0.0f;  // lane q * MA + m keeps the dot product of weight row row0 + q, row m
 #pragma unroll
   for (int q = 0; q < R; ++q) {
-    v4f_ acc = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int c = 0; c < CHK; ++c) {
-      const uint32_t words[4] = {w[q][c][0], w[q][c][1], w[q][c][2], w[q][c][3]};
+    for (int m = 0; m < MA; ++m) {
+      float d = 0.0f;
 #pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        const v2bf c0 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(words[2 * t], 1.0f, false);
-        const v2bf c1 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(words[2 * t], 1.0f, true);
-        const v2bf c2 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(words[2 * t + 1], 1.0f, false);
-        const v2bf c3 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(words[2 * t + 1], 1.0f, true);
-        const v8bf wf = {c0[0], c0[1], c1[0], c1[1], c2[0], c2[1], c3[0], c3[1]};
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf, xa[c][t], acc, 0, 0, 0);
-      }
+      for (int e = 0; e < 4; ++e) d = diag == e ? acc[q][m][e] : d;
+      const float sum = wave_sum_f32(d);
+      mine = lane == q * MA + m ? sum : mine;
     }
-    float d = 0.0f;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) d = diag == e ? acc[e] : d;
-    const float sum = wave_sum_f32(d);
-    mine = lane == q ? sum : mine;
   }
-  const int n = row0 + lane;
-  if (lane < R && n < g.N) {
+  const int n = row0 + lane / MA, m = lane % MA;
+  if (lane < R * MA && n < g.N) {
     float t = mine * g.b_scale[n];
     if (g.bias) t += __uint_as_float((uint32_t)g.bias[n] << 16);
     if (g.epilogue & CDIT_EPI_GELU_TANH) t = gelu_tanh(t);
-    g.out[n] = (uint16_t)(pack_bf16x2(t, 0.0f) & 0xffffu);
+    g.out[m * g.ldo + n] = (uint16_t)(pack_bf16x2(t, 0.0f) & 0xffffu);
+  }
+}
+
+template <int CHK>
+void launch_rows_chk(const GemmArgs& g, hipStream_t stream) {
+  constexpr int rows_wg = kRow1Rows * kRow1Waves;
+  const dim3 grid((g.N + rows_wg - 1) / rows_wg), block(64 * kRow1Waves);
+  switch (g.M) {
+    case 1: hipLaunchKernelGGL((gemm_w8a16_rows<CHK, 1>), grid, block, 0, stream, g); break;
+    case 2: hipLaunchKernelGGL((gemm_w8a16_rows<CHK, 2>), grid, block, 0, stream, g); break;
+    case 3: hipLaunchKernelGGL((gemm_w8a16_rows<CHK, 3>), grid, block, 0, stream, g); break;
+    default: hipLaunchKernelGGL((gemm_w8a16_rows<CHK, 4>), grid, block, 0, stream, g); break;
   }
 }
 
@@ -1196,15 +1229,13 @@ int launch_gemm_w8a16(const GemmArgs& g, int variant, hipStream_t stream) {
     hipLaunchKernelGGL(gemm_w8a16_generic, grid, dim3(256), 0, stream, g);
     return 0;
   }
-  if ((variant < 0 || variant == 51) && g.M == 1 && g.K <= 4096) {
-    // (aligned_ok has checked the alignment of the operands and of ldb)
-    constexpr int rows_wg = kRow1Rows * kRow1Waves;
-    const dim3 grid((g.N + rows_wg - 1) / rows_wg), block(64 * kRow1Waves);
+  if ((variant < 0 || variant == 51) && g.M <= 4 && g.K <= 4096) {
+    // (aligned_ok has checked the alignment of the operands and of lda and ldb)
     switch ((g.K + 1023) / 1024) {
-      case 1: hipLaunchKernelGGL(gemm_w8a16_row1<1>, grid, block, 0, stream, g); break;
-      case 2: hipLaunchKernelGGL(gemm_w8a16_row1<2>, grid, block, 0, stream, g); break;
-      case 3: hipLaunchKernelGGL(gemm_w8a16_row1<3>, grid, block, 0, stream, g); break;
-      default: hipLaunchKernelGGL(gemm_w8a16_row1<4>, grid, block, 0, stream, g); break;
+      case 1: launch_rows_chk<1>(g, stream); break;
+      case 2: launch_rows_chk<2>(g, stream); break;
+      case 3: launch_rows_chk<3>(g, stream); break;
+      default: launch_rows_chk<4>(g, stream); break;
     }
     return 0;
   }

@@ -125,6 +125,26 @@ def test_one_row_kernel_exact_and_k_positions(N, K):
     assert torch.equal(out.cpu(), to.w8a16_linear(x.to(torch.bfloat16), w, ones, fused=True)), pos
 
 
+@pytest.mark.parametrize("M", [2, 3, 4])
+@pytest.mark.parametrize("N,K", [(18432, 3072), (1008, 2048), (24, 16), (6160, 4096), (528, 1152), (272, 3968)])
+def test_few_rows_kernel(M, N, K):
+  """M = 2 to 4 with K <= 4096 runs the whole-row kernel too: integer operands bit-equal to the
+  oracle (every sum is exact in any order), random ones with GELU within the tolerance."""
+  from cache_dit_amd import _native
+  g = torch.Generator().manual_seed(M + N + K)
+  x = torch.randint(-4, 5, (M, K), generator=g).to(torch.bfloat16)
+  w = torch.randint(-4, 5, (N, K), generator=g).float().to(FP8)
+  ws = torch.full((N, 1), 0.25)
+  auto = _run(x, w, ws, None).cpu()
+  assert torch.equal(auto, to.w8a16_linear(x, w, ws, fused=True))
+  _native.set_gemm_variant(50)
+  assert torch.equal(_run(x, w, ws, None).cpu(), auto)
+  _native.set_gemm_variant(-1)
+  x, wq, ws, b = _problem(M, N, K, seed=M * 7 + N + K)
+  ref = to.w8a16_linear(x, wq, ws * 8, b, gelu="fused", fused=True)
+  _assert_close(_run(x, wq, ws * 8, b, epilogue=1), ref)
+
+
 def test_one_row_kernel_writes_only_its_row():
   from cache_dit_amd import _native
   N, K = 1040, 3072
