@@ -1586,6 +1586,40 @@ int launch_gemm_fp8_stamps(const GemmArgs& g, unsigned long long* stamps, int* w
   return launch_wide_stamps<V14>(g, stamps, workgroups, stream);
 }
 
+// The tile for fp16 and fp32 outputs: one large, one middle and one small tile are built for
+// them, with the cost model of the small bf16-output problems (choose_bf16_variant: whole
+// rounds over the CUs times tile area, the small tile penalised by its lower MFMA rate; ties go
+// to the larger tile). The middle one is for a few hundred to a thousand rows, where the large
+// tile leaves CUs idle and the small one needs a second round.
+// fp16 at 1021 x 3072 x 3072: 25.1 us (64 x 128) -> 17.8 (128 x 128), 28.2 with 256 x 192;
+// 700 x 4096 x 3072 26.0 -> 17.2; fp32 at 256 x 12288 x 3072 31.0 -> 21.9; 4608 x 3072 x 3072,
+// fp16, 60.7 -> 51.0.
+// -1: K is too short for any of them.
+template <class WideOk>
+int choose_other_out_variant(const GemmArgs& g, int variant, WideOk wide_ok) {
+  const int64_t cus = cu_count() > 0 ? cu_count() : 256;
+  const struct { int v, bm, bn, pen, depth; } cand[] = {
+      {15, 256, 192, 1000, V15::DEPTH}, {18, 128, 128, 1000, V18::DEPTH}, {17, 64, 128, 1493, V17::DEPTH}};
+  int best = -1;
+  int64_t cost = INT64_MAX;
+  for (const auto& c : cand) {
+    if (!wide_ok(c.depth)) continue;
+    if (variant == c.v) return variant;
+    const int64_t tiles = (int64_t)((g.M + c.bm - 1) / c.bm) * ((g.N + c.bn - 1) / c.bn);
+    const int64_t t = (tiles + cus - 1) / cus * c.bm * c.bn * c.pen;
+    if (t < cost) best = c.v, cost = t;
+  }
+  return best;
+}
+template <int OUT, bool KTAIL>
+int launch_other_out(const GemmArgs& g, int variant, hipStream_t stream) {
+  switch (variant) {
+    case 15: return launch_wide<V15, OUT, KTAIL>(g, stream);
+    case 17: return launch_wide<V17, OUT, KTAIL>(g, stream);
+    default: return launch_wide<V18, OUT, KTAIL>(g, stream);
+  }
+}
+
 int launch_gemm_fp8(const GemmArgs& g, int variant, hipStream_t stream) {
   if (!aligned_ok(g) || variant == 100) {
     dim3 grid((g.N + 15) / 16, (g.M + 15) / 16);
@@ -1610,24 +1644,12 @@ int launch_gemm_fp8(const GemmArgs& g, int variant, hipStream_t stream) {
   // tile (before it, slower waves may still be reading the previous tile's)
   auto wide_ok = [&](int depth) { return g.K >= 128 * (depth > 3 ? depth : 3); };
   if (g.out_dtype != CDIT_DT_BF16) {
-    // fp16 / fp32 outputs (the op's other two out_dtype ids): one large and one small
-    // wide tile are built for them, chosen like the small-problem case below; what
-    // those cannot take runs the generic kernel.
-    const int64_t t_large = (int64_t)((g.M + 255) / 256) * ((g.N + 191) / 192);
-    const int64_t t_small = (int64_t)((g.M + 63) / 64) * ((g.N + 127) / 128);
-    const int64_t ncu = cu_count() > 0 ? cu_count() : 256;
-    const bool large = variant == 15 ||
-                       (variant != 17 && (!wide_ok(V17::DEPTH) ||
-                                          (t_large + ncu - 1) / ncu * 256 * 192 * 1000 <=
-                                              (t_small + ncu - 1) / ncu * 64 * 128 * 1493));
-    if (large && wide_ok(V15::DEPTH)) {
-      return g.out_dtype == CDIT_DT_F16 ? launch_wide<V15, CDIT_DT_F16>(g, stream)
-                                        : launch_wide<V15, CDIT_DT_F32>(g, stream);
-    }
-    if (!large && wide_ok(V17::DEPTH)) {
-      return g.out_dtype == CDIT_DT_F16 ? launch_wide<V17, CDIT_DT_F16>(g, stream)
-                                        : launch_wide<V17, CDIT_DT_F32>(g, stream);
-    }
+    // fp16 / fp32 outputs (the op's other two out_dtype ids); what no wide tile can take
+    // runs the generic kernel.
+    const int v = choose_other_out_variant(g, variant, wide_ok);
+    if (v >= 0)
+      return g.out_dtype == CDIT_DT_F16 ? launch_other_out<CDIT_DT_F16, false>(g, v, stream)
+                                        : launch_other_out<CDIT_DT_F32, false>(g, v, stream);
     dim3 grid((g.N + 15) / 16, (g.M + 15) / 16);
     hipLaunchKernelGGL(gemm_fp8_generic, grid, dim3(256), 0, stream, g);
     return 0;
@@ -1642,16 +1664,13 @@ int launch_gemm_fp8(const GemmArgs& g, int variant, hipStream_t stream) {
 
 // K a multiple of 16 but not of 128, or shorter than a step: the KTAIL instances of the wide
 // kernel (they take any K, so the choice of the tile is the one for a long K; fp16 and fp32
-// outputs have one large and one small tile, as below).
+// outputs have three tiles, as above).
 int launch_gemm_fp8_ktail(const GemmArgs& g, int variant, hipStream_t stream) {
   auto tiles = [&](int bm, int bn) { return (int64_t)((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn); };
   if (g.out_dtype != CDIT_DT_BF16) {
-    const int64_t ncu = cu_count() > 0 ? cu_count() : 256;
-    const bool large = variant == 15 || (variant != 17 && (tiles(256, 192) + ncu - 1) / ncu * 256 * 192 * 1000 <=
-                                                              (tiles(64, 128) + ncu - 1) / ncu * 64 * 128 * 1493);
-    if (g.out_dtype == CDIT_DT_F16)
-      return large ? launch_wide<V15, CDIT_DT_F16, true>(g, stream) : launch_wide<V17, CDIT_DT_F16, true>(g, stream);
-    return large ? launch_wide<V15, CDIT_DT_F32, true>(g, stream) : launch_wide<V17, CDIT_DT_F32, true>(g, stream);
+    const int v = choose_other_out_variant(g, variant, [](int) { return true; });
+    return g.out_dtype == CDIT_DT_F16 ? launch_other_out<CDIT_DT_F16, true>(g, v, stream)
+                                      : launch_other_out<CDIT_DT_F32, true>(g, v, stream);
   }
   const bool forced = variant == 12 || (variant >= 14 && variant <= 18);
   if (!forced) variant = choose_bf16_variant(tiles, [](int) { return true; }).variant;

@@ -184,6 +184,24 @@ def test_one_row_kernel_writes_only_its_row(out_dtype):
   assert (buf[0, N:] == 7.0).all() and (buf[1] == 7.0).all()
 
 
+@pytest.mark.parametrize("out_dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("variant", [-1, 15, 17, 18])
+@pytest.mark.parametrize("M,N,K", [(128, 128, 512), (129, 136, 640), (257, 392, 528), (17, 8, 1024), (385, 2048, 112)])
+def test_other_output_types_every_tile(variant, out_dtype, M, N, K):
+  """fp16 and fp32 outputs at the edges of their three tiles, whole K steps and a partial last
+  one: integer operands, so every sum is exact and the output bit-equal to the oracle's."""
+  from cache_dit_amd import _native, ops
+  if variant == 17 and K == 512:
+    pytest.skip("too few K steps for the small tile's prefetch depth")
+  g = torch.Generator().manual_seed(M + N + K)
+  x = torch.randint(-4, 5, (M, K), generator=g).float().to(FP8)
+  w = torch.randint(-4, 5, (N, K), generator=g).float().to(FP8)
+  xs, ws = torch.full((M, 1), 0.5), torch.full((N, 1), 0.25)
+  _native.set_gemm_variant(variant)
+  out = ops.float8_inference_scaled_mm(x.cuda(), xs.cuda(), w.cuda().t(), ws.cuda().t(), out_dtype)
+  assert torch.equal(out.cpu(), to.scaled_mm_rowwise(x, xs, w, ws, None, out_dtype=out_dtype))
+
+
 @pytest.mark.parametrize("scale_mode", [0, 1])
 @pytest.mark.parametrize("kind", ["normal", "zero", "tiny", "huge", "nan", "inf"])
 def test_one_row_fused_linear_matches_the_two_calls(kind, scale_mode):
