@@ -248,9 +248,8 @@ class Fp8DynamicLinear(_Fp8LinearBase):
         if self.sibling_group is not None:
           return self.sibling_group.forward_member(self, x)
     share = self.share_input_quant and not stateless
-    return torch.ops.cdit.linear_w8a8(x, self.weight, self.weight_scale, self.bias,
-                                      self._scale_mode_id, self.epilogue,
-                                      ops.GRANULARITY_PER_ROW, share)
+    return ops.linear_w8a8_op(x, self.weight, self.weight_scale, self.bias, self._scale_mode_id,
+                              self.epilogue, ops.GRANULARITY_PER_ROW, share)
 
 
 class Fp8DynamicLinearPerTensor(_Fp8LinearBase):
@@ -261,9 +260,8 @@ class Fp8DynamicLinearPerTensor(_Fp8LinearBase):
 
   def forward(self, x: torch.Tensor) -> torch.Tensor:
     self._check_input(x)
-    return torch.ops.cdit.linear_w8a8(x, self.weight, self.weight_scale, self.bias,
-                                      self._scale_mode_id, self.epilogue,
-                                      ops.GRANULARITY_PER_TENSOR, False)
+    return ops.linear_w8a8_op(x, self.weight, self.weight_scale, self.bias, self._scale_mode_id,
+                              self.epilogue, ops.GRANULARITY_PER_TENSOR, False)
 
 
 class Fp8WeightOnlyLinear(_Fp8LinearBase):
@@ -292,8 +290,8 @@ class Fp8WeightOnlyLinear(_Fp8LinearBase):
           _recorder.note(self, x)
         if self.sibling_group is not None:
           return self.sibling_group.forward_member(self, x)
-    return torch.ops.cdit.w8a16_mm(x, self.weight.t(), self.weight_scale, self.bias,
-                                   _native.DT_BF16, self.epilogue)
+    return ops.w8a16_mm_op(x, self.weight.t(), self.weight_scale, self.bias, _native.DT_BF16,
+                           self.epilogue)
 
 
 _CLASS_OF = {

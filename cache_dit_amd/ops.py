@@ -44,22 +44,27 @@ def _stream_ptr(t: torch.Tensor) -> int:
   return torch._C._cuda_getCurrentRawStream(t.device.index)
 
 
-class _DeviceOf:
-  """Makes `t`'s device current for the launch when it is not already (the kernels
-  run on the current HIP device); free when it is."""
-  __slots__ = ("guard", )
-
-  def __init__(self, t: torch.Tensor):
-    self.guard = None if t.device.index == torch.cuda.current_device() else torch.cuda.device(
-        t.device)
+class _CurrentDevice:
+  """What _DeviceOf gives for a tensor on the current device: nothing to do."""
+  __slots__ = ()
 
   def __enter__(self):
-    if self.guard is not None:
-      self.guard.__enter__()
+    pass
 
   def __exit__(self, *exc):
-    if self.guard is not None:
-      self.guard.__exit__(*exc)
+    pass
+
+
+_CURRENT_DEVICE = _CurrentDevice()
+
+
+def _DeviceOf(t: torch.Tensor):
+  """Makes `t`'s device current for the launch when it is not already (the kernels
+  run on the current HIP device); free when it is."""
+  # (a tensor on the GPU exists, so torch.cuda.current_device()'s lazy initialisation is done)
+  if t.device.index == torch._C._cuda_getDevice():
+    return _CURRENT_DEVICE
+  return torch.cuda.device(t.device)
 
 
 def activation_workspace(M: int, K: int, device: torch.device):
@@ -145,7 +150,8 @@ def quant_rowwise_into(x2: torch.Tensor, q: torch.Tensor, scale: torch.Tensor,
                        scale_mode_id: int, gemm_follows: bool = False) -> None:
   """gemm_follows: the codes are read by a GEMM launched next on this stream (a cache
   hint for the quantizer; the results are the same)."""
-  _reject_codes_only("quant_rowwise_into", x2)
+  if _codes_only:
+    _reject_codes_only("quant_rowwise_into", x2)
   M, K = x2.shape
   mode = scale_mode_id | (_native.QUANT_GEMM_FOLLOWS if gemm_follows else 0)
   with _DeviceOf(x2):
@@ -305,7 +311,8 @@ def w8a16_batched_into(acts) -> None:
 
 def w8a16_into(x2: torch.Tensor, w: torch.Tensor, w_scale: torch.Tensor,
                bias: Optional[torch.Tensor], out: torch.Tensor, epilogue: int) -> None:
-  _reject_codes_only("w8a16_into", x2)
+  if _codes_only:
+    _reject_codes_only("w8a16_into", x2)
   M, K = x2.shape
   N = w.shape[0]
   with _DeviceOf(x2):
@@ -439,7 +446,8 @@ def linear_w8a8_into(x2: torch.Tensor, w: torch.Tensor, w_scale: torch.Tensor,
                      bias: Optional[torch.Tensor], out: torch.Tensor, q_ws: torch.Tensor,
                      s_ws: torch.Tensor, scale_mode_id: int, epilogue: int) -> None:
   """Quantizer + GEMM of one Linear forward in a single library call."""
-  _reject_codes_only("linear_w8a8_into", x2)
+  if _codes_only:
+    _reject_codes_only("linear_w8a8_into", x2)
   M, K = x2.shape
   N = w.shape[0]
   with _DeviceOf(x2):
@@ -491,10 +499,23 @@ torch.library.define(
 
 
 def _as_rows(x: torch.Tensor) -> torch.Tensor:
-  x2 = x.reshape(-1, x.shape[-1])
+  x2 = x if x.dim() == 2 and x.shape[1] > 0 else x.reshape(-1, x.shape[-1])
   if x2.stride(-1) != 1:
     x2 = x2.contiguous()
   return x2
+
+
+def _vector(t: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
+  """The elements of t as contiguous memory of `dtype`; the launchers only take its address,
+  so a tensor that is that already (any shape) is handed on as it is."""
+  if t.dtype == dtype and t.is_contiguous():
+    return t
+  return t.reshape(-1).to(dtype).contiguous()
+
+
+def _shaped(t: torch.Tensor, *shape) -> torch.Tensor:
+  """t.reshape(shape), without the call for a tensor of that shape."""
+  return t if t.shape == shape else t.reshape(shape)
 
 
 @torch.library.impl("cdit::fp8_rowwise_quant", "CUDA")
@@ -510,7 +531,7 @@ def _fp8_rowwise_quant(x: torch.Tensor, scale_mode: int = 0) -> Tuple[torch.Tens
   scale = torch.empty((x2.shape[0], ), dtype=torch.float32, device=x.device)
   if x2.numel() > 0 or x2.shape[0] > 0:
     quant_rowwise_into(x2, q, scale, scale_mode)
-  return q.reshape(x.shape), scale.reshape(*x.shape[:-1], 1)
+  return _shaped(q, *x.shape), scale.view(*x.shape[:-1], 1)
 
 
 @torch.library.register_fake("cdit::fp8_rowwise_quant")
@@ -537,10 +558,9 @@ def _aligned16(t: torch.Tensor) -> torch.Tensor:
 
 
 def _scale_vector(scale: torch.Tensor, n: int) -> torch.Tensor:
-  s = scale.reshape(-1).to(torch.float32)
-  if s.numel() == 1 and n != 1:
-    s = s.expand(n)
-  return _aligned16(s.contiguous())
+  if scale.numel() == 1 and n != 1:
+    scale = scale.reshape(-1).to(torch.float32).expand(n)
+  return _aligned16(_vector(scale, torch.float32))
 
 
 @torch.library.impl("cdit::float8_inference_scaled_mm", "CUDA")
@@ -577,9 +597,9 @@ def _float8_inference_scaled_mm(a_data, a_scale, b_data, b_scale, bias, out_dtyp
     out = out + bias.reshape(-1)
   else:
     if bias is not None:
-      bias = _aligned16(bias.reshape(-1).to(out_dtype).contiguous())
+      bias = _aligned16(_vector(bias, out_dtype))
     gemm_rowwise_into(a2, a_s, w, b_s, bias, out, int(epilogue))
-  return out.reshape(*a_data.shape[:-1], N)
+  return _shaped(out, *a_data.shape[:-1], N)
 
 
 @torch.library.register_fake("cdit::float8_inference_scaled_mm")
@@ -714,7 +734,7 @@ def _linear_w8a8(x, weight, weight_scale, bias, scale_mode=0, epilogue=0, granul
     else:
       q, s = activation_workspace(M, K, x2.device)
       linear_w8a8_into(x2, w, w_s, bias, out, q, s, int(scale_mode), int(epilogue))
-  return out.view(*x.shape[:-1], N)
+  return _shaped(out, *x.shape[:-1], N)
 
 
 @torch.library.impl("cdit::linear_w8a8_cat2", "CUDA")
@@ -888,18 +908,24 @@ def _w8a16_mm(x, b_data, b_scale, bias, out_dtype_id, epilogue=0):
     raise ValueError(f"{name}: shape mismatch x {tuple(x.shape)} x b {tuple(b_data.shape)}")
   if b_scale.numel() != N:
     raise ValueError(f"{name}: b_scale must have {N} elements")
-  b_s = b_scale.reshape(-1).to(torch.float32).contiguous()
+  b_s = _vector(b_scale, torch.float32)
   if bias is not None:
-    bias = bias.reshape(-1).to(torch.bfloat16).contiguous()
+    bias = _vector(bias, torch.bfloat16)
   out = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
   w8a16_into(x2, w, b_s, bias, out, int(epilogue))
-  return out.reshape(*x.shape[:-1], N)
+  return _shaped(out, *x.shape[:-1], N)
 
 
 @torch.library.register_fake("cdit::w8a16_mm")
 def _fake_w8a16_mm(x, b_data, b_scale, bias, out_dtype_id, epilogue=0):
   return x.new_empty((*x.shape[:-1], b_data.shape[-1]), dtype=decode_output_dtype(out_dtype_id))
 
+
+# The overloads, looked up once: a call through the packet resolves them again each time.
+linear_w8a8_op = torch.ops.cdit.linear_w8a8.default
+w8a16_mm_op = torch.ops.cdit.w8a16_mm.default
+_fp8_rowwise_quant_op = torch.ops.cdit.fp8_rowwise_quant.default
+_scaled_mm_op = torch.ops.cdit.float8_inference_scaled_mm.default
 
 # --------------------------------------------------------------------------- python-level API
 
@@ -927,7 +953,7 @@ def fp8_rowwise_quant(x: torch.Tensor,
                       scale_mode: str = "bf16div") -> Tuple[torch.Tensor, torch.Tensor]:
   """Per-row dynamic e4m3 quantization of a bf16 tensor -> (codes, scale[...,1])."""
   _require_cuda("fp8_rowwise_quant", x)
-  return torch.ops.cdit.fp8_rowwise_quant(x, _native.SCALE_MODE_IDS[scale_mode])
+  return _fp8_rowwise_quant_op(x, _native.SCALE_MODE_IDS[scale_mode])
 
 
 def float8_inference_scaled_mm(
@@ -947,9 +973,8 @@ def float8_inference_scaled_mm(
   if output_scale is not None:
     raise NotImplementedError("float8 scaled_mm wrapper does not support scale_result yet.")
   _require_cuda("float8_inference_scaled_mm", a_data, b_data)
-  return torch.ops.cdit.float8_inference_scaled_mm(a_data, a_scale, b_data, b_scale, bias,
-                                                   encode_output_dtype(output_dtype),
-                                                   use_fast_accum, epilogue)
+  return _scaled_mm_op(a_data, a_scale, b_data, b_scale, bias, encode_output_dtype(output_dtype),
+                       use_fast_accum, epilogue)
 
 
 def w8a16_mm(x: torch.Tensor,
@@ -959,5 +984,4 @@ def w8a16_mm(x: torch.Tensor,
              output_dtype: torch.dtype = torch.bfloat16,
              epilogue: int = 0) -> torch.Tensor:
   _require_cuda("w8a16_mm", x, b_data)
-  return torch.ops.cdit.w8a16_mm(x, b_data, b_scale, bias, encode_output_dtype(output_dtype),
-                                 epilogue)
+  return w8a16_mm_op(x, b_data, b_scale, bias, encode_output_dtype(output_dtype), epilogue)
