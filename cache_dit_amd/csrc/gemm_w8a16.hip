@@ -946,6 +946,167 @@ __device__ __forceinline__ v8bf e4m3x8_to_bf16(uint32_t lo, uint32_t hi) {
 }
 
 // ---------------------------------------------------------------------------
+// A few dozen rows (the prompt's projections: M = 17 to 128 or so): one wavefront, alone in
+// its workgroup, per 32 x 32 tile. A 128 x 64 tile of the wide kernel gives such a problem to a
+// few dozen CUs, whose prefetch cannot keep the weight stream in flight; 32 x 32 tiles put it on
+// all of them. The wavefront has a ring of D stages (A 32 rows x 128 B, B 32 rows x 64 B, the
+// swizzles of the wide kernel) that LDS-DMA fills D steps ahead; nobody else touches them, so
+// there are no barriers, only waits on its own loads and LDS reads. Operands are read one step
+// ahead of their MFMAs, and a stage is refilled as soon as they are in registers, between the
+// second and the third MFMA of the step. MFMA, K order and epilogue arithmetic are those of the
+// wide kernel, so the results are bit-identical to it (a member of a batch may run there).
+// What bounds it: a chain of four dependent MFMAs (128 clocks) and six DMA instructions per step.
+// One wavefront issues all of it in order: about 500 clocks per step.
+// Another weight matrix per launch, against 128 x 64 tiles: 77 x 4096 x 3072 22.1 -> 16.1 us,
+// 17 x 3072 x 3072 15.3 -> 12.1, 128 x 3072 x 3072 20.4 -> 13.2, 256 x 3072 x 1536 19.8 -> 12.9,
+// 512 x 4096 x 1024 20.4 -> 15.6, 32 x 3072 x 12288 18.3 -> 17.3; with 672 tiles
+// (200 x 4096 x 3072) 21.5 -> 22.2 and with 864 (77 x 3072 x 9216) 19.6 -> 29.9: not taken.
+constexpr int kTileDepth = 8, kTileLds = kTileDepth * 32 * 3 * BKE;
+template <bool GELU>
+__global__ __launch_bounds__(64) void gemm_w8a16_wavetile(GemmArgs g, int tiles_m, int tiles_n) {
+  constexpr int D = kTileDepth, A_BYTES = 32 * 2 * BKE, STAGE = kTileLds / D, NDMA = 6;
+  static_assert((D - 1) * NDMA < 63 && D * STAGE <= 64 * 1024, "vmcnt has 6 bits; LDS without opt-in");
+  extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+  // the row tiles of one column tile on one XCD (workgroups go to the 8 XCDs in turn): its
+  // weights come from HBM once
+  const int id = blockIdx.x;
+  const int tn = id / 8 / tiles_m * 8 + id % 8, tm = id / 8 % tiles_m;
+  if (tn >= tiles_n) return;
+  const int lane = threadIdx.x, m0 = tm * 32, n0 = tn * 32;
+  const int h = lane >> 5, r32 = lane & 31;
+  const int KT = (g.K + BKE - 1) / BKE;
+
+  // scale and bias of the lane's 16 columns n0 + 16 h .. (N % 16 == 0: all in or all out)
+  const int nw = n0 + 16 * h;
+  const bool n_in = nw < g.N;
+  v4f bs[4];
+  uint4 bi[2] = {{0u, 0u, 0u, 0u}, {0u, 0u, 0u, 0u}};
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+    bs[q] = n_in ? reinterpret_cast<const v4f*>(g.b_scale + nw)[q] : v4f{0.0f, 0.0f, 0.0f, 0.0f};
+  if (n_in && g.bias) {
+    bi[0] = reinterpret_cast<const uint4*>(g.bias + nw)[0];
+    bi[1] = reinterpret_cast<const uint4*>(g.bias + nw)[1];
+  }
+
+  // DMA maps: an instruction fills 8 A rows (chunk (lane & 7) ^ swizzle, which differs between
+  // even and odd instructions by 4) or 16 B rows
+  const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint8_t*>(static_cast<const uint8_t*>(g.a)) + (int64_t)m0 * g.lda * 2, 0, 0x7fffffff, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint8_t*>(g.b) + (int64_t)n0 * g.ldb, 0, 0x7fffffff, 0x00020000);
+  const int ca = (lane & 7) ^ (lane >> 4), cb = (lane & 3) ^ ((lane >> 4) & 3);
+  uint32_t off[NDMA];
+#pragma unroll
+  for (int p = 0; p < 4; ++p)
+    off[p] = (uint32_t)min(8 * p + (lane >> 3), g.M - 1 - m0) * (uint32_t)(g.lda * 2) + (ca ^ (4 * (p & 1))) * 16;
+#pragma unroll
+  for (int p = 0; p < 2; ++p)
+    off[4 + p] = (uint32_t)min(16 * p + (lane >> 2), g.N - 1 - n0) * (uint32_t)g.ldb + cb * 16;
+  // Elements beyond K (a partial last step, steps beyond the last) are fetched from beyond the
+  // descriptor: zeros.
+  auto dma = [&](int kt, int stage) {
+    const int left = g.K - kt * BKE;
+    const uint32_t a0 = ca * 8 < left ? 0u : 0x80000000u, a1 = (ca ^ 4) * 8 < left ? 0u : 0x80000000u;
+    const uint32_t b0 = cb * 16 < left ? 0u : 0x80000000u;
+    __attribute__((address_space(3))) uint8_t* st =
+        (__attribute__((address_space(3))) uint8_t*)(smem) + stage;
+#pragma unroll
+    for (int p = 0; p < 4; ++p)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (__attribute__((address_space(3))) void*)(st + p * 1024), 16,
+                                               (int)(off[p] | (p & 1 ? a1 : a0)), kt * 2 * BKE, 0, 0);
+#pragma unroll
+    for (int p = 0; p < 2; ++p)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (__attribute__((address_space(3))) void*)(st + A_BYTES + p * 1024),
+                                               16, (int)(off[4 + p] | b0), kt * BKE, 0, 0);
+  };
+
+  // operand read maps, as in the wide kernel
+  const int wrow = 16 * ((r32 >> 2) & 1) + 4 * (r32 >> 3) + (r32 & 3);
+  uint32_t rd_a[4], rd_b[2];
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+      rd_a[2 * t + e] = r32 * (2 * BKE) + (((4 * t + 2 * h + e) ^ ((r32 >> 1) & 7)) << 4);
+    rd_b[t] = A_BYTES + wrow * BKE + (((2 * t + h) ^ ((wrow >> 2) & 3)) << 4);
+  }
+  struct Step {
+    v8bf a[4];
+    uint4 w[2];
+  };
+  // (__restrict__: see the wide kernel; without it every read would wait for the whole stream)
+  auto read = [&](const uint8_t* __restrict__ st) -> Step {
+    Step f;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) f.a[q] = *reinterpret_cast<const v8bf*>(st + rd_a[q]);
+#pragma unroll
+    for (int t = 0; t < 2; ++t) f.w[t] = *reinterpret_cast<const uint4*>(st + rd_b[t]);
+    return f;
+  };
+
+  v16f acc;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+#pragma unroll
+  for (int s = 0; s < D; ++s) dma(s, s * STAGE);
+  wait_vm<(D - 1) * NDMA>();
+  Step even = read(smem), odd;
+  wait_lgkm0();
+  dma(D, 0);
+  int stage = STAGE;  // of step kt + 1
+  // Step kt: its operands are in `f`; reads step kt + 1 into `nf` and sends for step kt + 1 + D.
+  auto step = [&](int kt, const Step& f, Step& nf) {
+    wait_vm<(D - 1) * NDMA>();  // steps up to kt + 1 have landed
+    nf = read(smem + stage);
+    __builtin_amdgcn_sched_barrier(0);
+    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(e4m3x8_to_bf16(f.w[0].x, f.w[0].y), f.a[0], acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(e4m3x8_to_bf16(f.w[0].z, f.w[0].w), f.a[1], acc, 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    wait_lgkm0();  // step kt + 1 is in registers: its stage can be filled again
+    dma(kt + 1 + D, stage);
+    __builtin_amdgcn_sched_barrier(0);
+    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(e4m3x8_to_bf16(f.w[1].x, f.w[1].y), f.a[2], acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(e4m3x8_to_bf16(f.w[1].z, f.w[1].w), f.a[3], acc, 0, 0, 0);
+    stage = stage + STAGE == D * STAGE ? 0 : stage + STAGE;
+  };
+  for (int kt = 0; kt < KT; kt += 2) {
+    step(kt, even, odd);
+    if (kt + 1 < KT) step(kt + 1, odd, even);
+  }
+  wait_vm<0>();  // no DMA outlives the workgroup
+
+  // acc[r] is out[m0 + r32][n0 + 16 h + r]
+  const int m = m0 + r32;
+  if (m >= g.M || !n_in) return;
+  const uint32_t bw[8] = {bi[0].x, bi[0].y, bi[0].z, bi[0].w, bi[1].x, bi[1].y, bi[1].z, bi[1].w};
+  uint32_t pk[8];
+#pragma unroll
+  for (int r = 0; r < 16; r += 2) {
+    float v0 = __fmaf_rn(acc[r], bs[r >> 2][r & 3], __uint_as_float(bw[r >> 1] << 16));
+    float v1 = __fmaf_rn(acc[r + 1], bs[r >> 2][(r + 1) & 3], __uint_as_float(bw[r >> 1] & 0xffff0000u));
+    if constexpr (GELU) {
+      v0 = gelu_tanh(v0);
+      v1 = gelu_tanh(v1);
+    }
+    pk[r >> 1] = pack_bf16x2(v0, v1);
+  }
+  uint4* dst = reinterpret_cast<uint4*>(g.out + (int64_t)m * g.ldo + nw);
+  dst[0] = uint4{pk[0], pk[1], pk[2], pk[3]};
+  dst[1] = uint4{pk[4], pk[5], pk[6], pk[7]};
+}
+
+int launch_wavetile(const GemmArgs& g, hipStream_t stream) {
+  const int tiles_m = (g.M + 31) / 32, tiles_n = (g.N + 31) / 32;
+  const dim3 grid((tiles_n + 7) / 8 * 8 * tiles_m), block(64);
+  if (g.epilogue & CDIT_EPI_GELU_TANH)
+    hipLaunchKernelGGL(gemm_w8a16_wavetile<true>, grid, block, kTileLds, stream, g, tiles_m, tiles_n);
+  else
+    hipLaunchKernelGGL(gemm_w8a16_wavetile<false>, grid, block, kTileLds, stream, g, tiles_m, tiles_n);
+  return 0;
+}
+
+// ---------------------------------------------------------------------------
 // Skinny kernel for 4 < M <= 16, and for fewer rows at K > 4096: weight streaming. A
 // workgroup of 4 waves owns 16 output channels, each wave a quarter of K. Per
 // 128-element chunk a lane (weight row l&15, K group l>>4) loads 32 e4m3 bytes
@@ -1254,6 +1415,12 @@ int launch_gemm_w8a16(const GemmArgs& g, int variant, hipStream_t stream) {
   auto wide_ok = [&](int depth) {
     return (k_tail || g.K >= (depth > 3 ? depth : 3) * BKE) && g.N % 16 == 0;
   };
+  // Two 32 x 32 tiles per CU and less: the wavefront-per-tile kernel (figures at the kernel; at
+  // three per CU it wins or loses with the shape, beyond that the CUs take a second round of it).
+  if (g.N % 16 == 0 &&
+      (variant == 13 || (variant < 0 && (int64_t)((g.M + 31) / 32) * ((g.N + 31) / 32) <=
+                                            2 * (int64_t)(cu_count() > 0 ? cu_count() : 256))))
+    return launch_wavetile(g, stream);
   if (variant < 0 || (k_tail && (variant < 7 || variant > 12))) {
     variant = choose_variant(
         [&](int bm, int bn) { return (int64_t)((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn); },

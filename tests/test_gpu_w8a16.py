@@ -145,6 +145,31 @@ def test_few_rows_kernel(M, N, K):
   _assert_close(_run(x, wq, ws * 8, b, epilogue=1), ref)
 
 
+@pytest.mark.parametrize("M,N,K", [(17, 16, 16), (32, 32, 64), (33, 48, 128), (77, 3072, 4096), (64, 272, 448),
+                                   (65, 1040, 512), (96, 528, 576), (100, 4096, 1088), (1, 264 + 8, 2224), (128, 16, 4464)])
+@pytest.mark.parametrize("gelu", [0, 1])
+def test_wavefront_tiles(M, N, K, gelu):
+  """The kernel with a wavefront per 32 x 32 tile: rows and columns that leave partial tiles, K
+  shorter than its ring of eight stages, an odd and an even number of steps, a partial last one.
+  Bit-equal to the wide kernel on random operands, to the oracle on integers; nothing is written
+  outside the output."""
+  from cache_dit_amd import _native, ops
+  x, wq, ws, b = _problem(M, N, K, seed=M + N + K)
+  _native.set_gemm_variant(13)
+  out = _run(x, wq, ws * 8, b, epilogue=gelu)
+  _native.set_gemm_variant(12)
+  assert torch.equal(out, _run(x, wq, ws * 8, b, epilogue=gelu))
+  g = torch.Generator().manual_seed(M * N + K)
+  x = torch.randint(-4, 5, (M, K), generator=g).to(torch.bfloat16)
+  w = torch.randint(-4, 5, (N, K), generator=g).float().to(FP8)
+  ws = torch.full((N, 1), 0.25)
+  buf = torch.full((M + 1, N + 8), 7.0, dtype=torch.bfloat16, device="cuda")
+  _native.set_gemm_variant(13)
+  ops.w8a16_into(x.cuda(), w.cuda(), ws.cuda().reshape(-1), None, buf[:M, :N], 0)
+  assert torch.equal(buf[:M, :N].cpu(), to.w8a16_linear(x, w, ws, fused=True))
+  assert (buf[M] == 7.0).all() and (buf[:, N:] == 7.0).all()
+
+
 def test_one_row_kernel_writes_only_its_row():
   from cache_dit_amd import _native
   N, K = 1040, 3072
