@@ -164,6 +164,13 @@ inline int cu_count() {
   return n;
 }
 
+// Modelled time of `tiles` tiles, one persistent workgroup per CU, for a tile whose full round
+// takes `round`: a last, partial round of r tiles counts 0.7 + 0.3 r/cus (small problems).
+inline int64_t rounds_time(int64_t tiles, int64_t cus, int round) {
+  const int64_t full = tiles / cus, rem = tiles % cus;
+  return (full * 10 * cus + (rem ? 7 * cus + 3 * rem : 0)) * round;
+}
+
 // Workgroup id -> output tile. Workgroups are handed to the 8 XCDs round-robin
 // and each XCD has its own L2, so ids that land on one XCD are first made
 // consecutive, then walked in column-major order inside groups of GROUP_M tile

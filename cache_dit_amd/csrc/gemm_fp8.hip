@@ -1587,10 +1587,9 @@ int launch_gemm_fp8_stamps(const GemmArgs& g, unsigned long long* stamps, int* w
 }
 
 // The tile for fp16 and fp32 outputs: one large, one middle and one small tile are built for
-// them, with the cost model of the small bf16-output problems (choose_bf16_variant: whole
-// rounds over the CUs times tile area, the small tile penalised by its lower MFMA rate; ties go
-// to the larger tile). The middle one is for a few hundred to a thousand rows, where the large
-// tile leaves CUs idle and the small one needs a second round.
+// them, chosen as the small bf16-output problems are (choose_bf16_variant). The middle one is
+// for a few hundred to a thousand rows, where the large tile leaves CUs idle and the small one
+// needs a second round.
 // fp16 at 1021 x 3072 x 3072: 25.1 us (64 x 128) -> 17.8 (128 x 128), 28.2 with 256 x 192;
 // 700 x 4096 x 3072 26.0 -> 17.2; fp32 at 256 x 12288 x 3072 31.0 -> 21.9; 4608 x 3072 x 3072,
 // fp16, 60.7 -> 51.0.
@@ -1598,16 +1597,16 @@ int launch_gemm_fp8_stamps(const GemmArgs& g, unsigned long long* stamps, int* w
 template <class WideOk>
 int choose_other_out_variant(const GemmArgs& g, int variant, WideOk wide_ok) {
   const int64_t cus = cu_count() > 0 ? cu_count() : 256;
-  const struct { int v, bm, bn, pen, depth; } cand[] = {
-      {15, 256, 192, 1000, V15::DEPTH}, {18, 128, 128, 1000, V18::DEPTH}, {17, 64, 128, 1493, V17::DEPTH}};
+  const struct { int v, bm, bn, us10, depth; } cand[] = {
+      {15, 256, 192, 245, V15::DEPTH}, {18, 128, 128, 145, V18::DEPTH}, {17, 64, 128, 110, V17::DEPTH}};
   int best = -1;
-  int64_t cost = INT64_MAX;
+  int64_t time = INT64_MAX;
   for (const auto& c : cand) {
     if (!wide_ok(c.depth)) continue;
     if (variant == c.v) return variant;
     const int64_t tiles = (int64_t)((g.M + c.bm - 1) / c.bm) * ((g.N + c.bn - 1) / c.bn);
-    const int64_t t = (tiles + cus - 1) / cus * c.bm * c.bn * c.pen;
-    if (t < cost) best = c.v, cost = t;
+    const int64_t t = rounds_time(tiles, cus, c.us10);
+    if (t < time) best = c.v, time = t;
   }
   return best;
 }
@@ -1709,19 +1708,29 @@ TileChoice choose_bf16_variant(Tiles tiles, WideOk wide_ok) {
       if (t < best.cost) best = {c.v, t};
     }
   } else {
-    // Smaller problems (the text-stream Linears, M of a few hundred to a few
-    // thousand): whole rounds over the CUs times tile area, the small tiles
-    // penalised by their measured lower MFMA rate (per mille); ties go to the
-    // larger tile. Tiles whose prefetch depth K cannot feed are left out.
-    const struct { int v, bm, bn, pen, depth; } cand[] = {
-        {12, 256, 256, 1000, 2}, {14, 288, 192, 1000, 2}, {15, 256, 192, 1000, 2},
-        {16, 128, 192, 1124, 3}, {18, 128, 128, 1000, 4}, {17, 64, 128, 1493, 5}};
+    // Smaller problems (the text-stream Linears, M of a few hundred to a few thousand): the
+    // time of a round of each tile, as measured (`us10`: tenths of a us at K of about 2200; only
+    // the ratios count), times the rounds over the CUs, a last round of r tiles counting
+    // 0.7 + 0.3 r/CUs. A large tile costs far less per element than its area says -- its round is
+    // bound by the same LDS-DMA latency and start-up --, so two or three rounds of a small tile
+    // lose to one of a large one: 1357 x 2224 x 4464 32.8 us (128 x 128, two rounds) against
+    // 27.8 (256 x 192), 1800 x 3056 x 4400 67.4 (64 x 128, four) against 34.4 (256 x 192). One
+    // round of the small tiles is still the best where it is enough: 512 x 2224 x 4464 19.3
+    // (128 x 128) against 24.2 and 27.9, 1000 x 2992 x 2000 18.7 (64 x 128) against 21.5 and 35.0.
+    // Tiles whose prefetch depth K cannot feed are left out; ties go to the larger tile.
+    const struct { int v, bm, bn, us10, depth; } cand[] = {
+        {12, 256, 256, 310, 2}, {14, 288, 192, 270, 2}, {15, 256, 192, 245, 2},
+        {16, 128, 192, 180, 3}, {18, 128, 128, 145, 4}, {17, 64, 128, 110, 5}};
     // K < 256: the kernels without a K stream across tiles (cost not modelled)
     best = {tiles(128, 128) >= cus ? 6 : 21, INT64_MAX / 8};
+    int64_t time = INT64_MAX;
     for (const auto& c : cand) {
       if (!wide_ok(c.depth)) continue;
-      const int64_t t = (tiles(c.bm, c.bn) + cus - 1) / cus * cus * c.bm * c.bn * c.pen;
-      if (t < best.cost) best = {c.v, t};
+      const int64_t t = rounds_time(tiles(c.bm, c.bn), cus, c.us10);
+      if (t >= time) continue;
+      time = t;
+      // in the unit of the large tiles (batches of activations of both kinds are compared)
+      best = {c.v, (tiles(c.bm, c.bn) + cus - 1) / cus * cus * c.bm * c.bn * 1000};
     }
   }
   return best;

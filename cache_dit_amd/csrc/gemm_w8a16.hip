@@ -1366,18 +1366,25 @@ TileChoice choose_variant(Tiles tiles, WideOk wide_ok) {
     const int64_t c8 = cost(256, 192, 102), c7 = cost(256, 256, 100);
     return c8 < c7 ? TileChoice{8, c8} : TileChoice{7, c7};
   }
-  // Smaller problems: whole rounds over the CUs times tile area, the small tiles
-  // penalised by their measured lower MFMA rate (per mille); ties go to the larger
-  // tile. Tiles whose prefetch depth K cannot feed are left out; without any wide
-  // tile (N not a multiple of 16, very short K) the 128x128 kernel runs.
-  const struct { int v, bm, bn, pen, depth; } cand[] = {
-      {7, 256, 256, 1000, 2}, {8, 256, 192, 1000, 2}, {10, 128, 192, 1300, 4},
-      {11, 128, 128, 1400, 5}, {12, 128, 64, 1700, 6}};
+  // Smaller problems: the time of a round of each tile, as measured (`us10`: tenths of a us at
+  // K of about 2200; only the ratios count), times the rounds over the CUs, as in the
+  // w8a8 entry point: 1357 x 2224 x 4464 47.6 us (128 x 128, two rounds) against 40.7
+  // (256 x 192); 512 x 2224 x 4464 27.1 (128 x 128) against 32.6, 34.7 and 40.4; 1000 x 2992 x
+  // 2000 27.6 (128 x 64) against 32.7. Ties go to the larger tile. Tiles whose prefetch depth K
+  // cannot feed are left out; without any wide tile (N not a multiple of 16, very short K) the
+  // 128x128 kernel runs.
+  const struct { int v, bm, bn, us10, depth; } cand[] = {
+      {7, 256, 256, 540, 2}, {8, 256, 192, 430, 2}, {10, 128, 192, 320, 4},
+      {11, 128, 128, 250, 5}, {12, 128, 64, 175, 6}};
   TileChoice best = {3, INT64_MAX / 8};  // the 128x128 kernel takes what no wide tile can
+  int64_t time = INT64_MAX;
   for (const auto& c : cand) {
     if (!wide_ok(c.depth)) continue;
-    const int64_t t = (tiles(c.bm, c.bn) + cus - 1) / cus * cus * c.bm * c.bn * c.pen;
-    if (t < best.cost) best = {c.v, t};
+    const int64_t t = rounds_time(tiles(c.bm, c.bn), cus, c.us10);
+    if (t >= time) continue;
+    time = t;
+    // in the unit of the large tiles (batches of activations of both kinds are compared)
+    best = {c.v, (tiles(c.bm, c.bn) + cus - 1) / cus * cus * c.bm * c.bn * 1000};
   }
   return best;
 }
