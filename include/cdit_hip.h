@@ -189,7 +189,7 @@ int cdit_fp8_ln_modulate_quant(const void* x_bf16, int64_t M, int64_t K, int64_t
  * adds it after the matmul in that case (_scaled_mm.py:71-81) and so must the
  * caller. Accumulation is fp32. Requires K % 16 == 0 (as the reference's FP8
  * matmul does) and 16-byte aligned a_q/b_q rows. bf16 is the tuned path; the
- * other two dtypes have two tile shapes of the same kernel and a generic
+ * other two dtypes have three tile shapes of the same kernel and a generic
  * fallback.
  */
 int cdit_fp8_gemm_rowwise(const void* a_q, const float* a_scale,
