@@ -660,8 +660,8 @@ def headline_kernels(device):
     del wb
   except Exception as e:
     res["w8a16_note"] = str(e)[:120]
-  # the per-tensor quantizer (float8_per_tensor and the policy's fallback pass): three launches
-  # (zero the amax word, amax over the tensor, cast), the tensor read twice: 5MK + 4M bytes
+  # the per-tensor quantizer (float8_per_tensor and the policy's fallback pass): two launches
+  # (amax over the tensor, cast), the tensor read twice: 5MK + 4M bytes
   try:
     amax_ws = torch.zeros(1, dtype=torch.int32, device=device)
 

@@ -302,7 +302,8 @@ __global__ __launch_bounds__(64) void quant_rowwise_generic(
 }
 
 // ---------------------------------------------------------------------------
-// Per-tensor variant (one scale for the whole [M,K] tensor): three launches.
+// Per-tensor variant (one scale for the whole [M,K] tensor): three launches for any shape and
+// alignment, two (further below) where the vector loads fit.
 //   zero_amax:           *amax_ws = 0 (a kernel, not a memset, so that the sequence
 //                        can be recorded into a hipGraph)
 //   tensor_amax:         amax over all elements, one wavefront per row at a time,
@@ -385,18 +386,23 @@ __global__ __launch_bounds__(64) void quant_tensorwise_cast(
 
 // The same two kernels for 16-byte aligned rows of up to 512 CH elements: all loads of a row
 // in flight at once (the row loop above issues them one by one), buffer accesses whose
-// descriptor drops what lies beyond the row, non-temporal stores of the codes. Atomics on one
-// address are served one after the other (measured: 15 ns each, 69 us for one per row of a
-// 4608-row activation), so the amax kernel runs on at most one workgroup of eight wavefronts
-// per CU, each wavefront with several rows, the eight maxima meet in LDS, and the workgroup
-// skips its atomic where the word already holds at least its maximum (a relaxed read at
-// device scope suffices: the word only grows).
+// descriptor drops what lies beyond the row, non-temporal stores of the codes. The amax kernel
+// runs on at most one workgroup of eight wavefronts per CU, each wavefront with several rows;
+// the eight maxima meet in LDS.
+// There is no word to clear and no atomic on one (they are served one after the other, 15 ns
+// each): workgroup i of the P <= M ones leaves its maximum in scale[i], tagged as a negative NaN
+// that no scale is, and every wavefront of the cast takes the maximum of the P words. Workgroup 0
+// of the cast alone replaces them by the scale; a wavefront that comes later finds a word
+// without the tag, which then is the scale itself. Against a launch that clears the word and an
+// atomic per workgroup, graph replays: 17 x 1024 7.3 -> 6.0 us, 512 x 3072 8.5 -> 6.4, 4608 x 3072
+// 17.8 -> 15.7 (4.5 TB/s over two reads and a write), 6889 x 12288 112.3 -> 113.3 (within noise).
 constexpr int kAmaxWaves = 8;  // wavefronts per workgroup of tensor_amax_rows
+constexpr uint32_t kPartTag = 0xffff0000u;
 
 template <int CH>
 __global__ __launch_bounds__(64 * kAmaxWaves) void tensor_amax_rows(const uint16_t* __restrict__ x,
                                                                      int64_t ld_x, int M, int K,
-                                                                     uint32_t* __restrict__ amax_ws) {
+                                                                     float* __restrict__ scale) {
   typedef unsigned int u4v __attribute__((ext_vector_type(4)));
   __shared__ uint32_t part[kAmaxWaves];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -421,24 +427,38 @@ __global__ __launch_bounds__(64 * kAmaxWaves) void tensor_amax_rows(const uint16
   if (threadIdx.x == 0) {
 #pragma unroll
     for (int w = 1; w < kAmaxWaves; ++w) m = m > part[w] ? m : part[w];
-    // (read at device scope: a plain load may be served by this CU's own cache with the value
-    // an earlier workgroup saw)
-    if (m > __hip_atomic_load(amax_ws, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(amax_ws, m);
+    scale[blockIdx.x] = __uint_as_float(kPartTag | m);
   }
 }
 
 template <int CH>
 __global__ __launch_bounds__(64) void quant_tensorwise_cast_rows(
     const uint16_t* __restrict__ x, int64_t ld_x, uint8_t* __restrict__ q, int64_t ld_q,
-    float* __restrict__ scale, int M, int K, int scale_mode, const uint32_t* __restrict__ amax_ws) {
+    float* scale, int parts, int M, int K, int scale_mode, uint32_t* __restrict__ amax_ws) {
   typedef unsigned int u4v __attribute__((ext_vector_type(4)));
   typedef unsigned int u2v __attribute__((ext_vector_type(2)));
   const int lane = threadIdx.x & 63;
-  const float s = row_scale(*amax_ws, scale_mode);
+  uint32_t* words = reinterpret_cast<uint32_t*>(scale);
+  uint32_t m = 0, done = 0;  // done: the bits of the scale (never 0), if a word holds it already
+  for (int i = lane; i < parts; i += 64) {
+    const uint32_t v = __hip_atomic_load(words + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (v >= kPartTag)
+      m = max(m, v & 0xffffu);
+    else
+      done = v;
+  }
+  m = wave_max_u32(m);
+  done = wave_max_u32(done);
+  const float s = done ? __uint_as_float(done) : row_scale(m, scale_mode);
+  if (blockIdx.x == 0) {
+    for (int i = lane; i < parts; i += 64)
+      __hip_atomic_store(words + i, __float_as_uint(s), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (lane == 0) *amax_ws = m;
+  }
   const bool fast = scale_in_fast_window(s);
   const Recip r = make_recip(s);
   for (int64_t row = blockIdx.x; row < M; row += gridDim.x) {
-    if (lane == 0) scale[row] = s;
+    if (lane == 0 && row >= parts) scale[row] = s;
     const __amdgpu_buffer_rsrc_t xb = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<uint16_t*>(x + row * ld_x), 0, K * 2, 0x00020000);
     const __amdgpu_buffer_rsrc_t qb = __builtin_amdgcn_make_buffer_rsrc(q + row * ld_q, 0, K, 0x00020000);
@@ -1116,22 +1136,22 @@ int launch_quant_tensorwise(const void* x, int64_t M, int64_t K, int64_t ld_x, v
   int64_t blocks = M;
   const int64_t kMaxBlocks = 256 * 64;  // the rest is picked up by the grid-stride loops
   if (blocks > kMaxBlocks) blocks = kMaxBlocks;
-  hipLaunchKernelGGL(zero_amax, dim3(1), dim3(1), 0, stream, amax_ws);
   if (vec && K <= 32 * 512) {
     const int need = (int)((K + 511) / 512);
+    const int parts = (int)std::min<int64_t>((M + kAmaxWaves - 1) / kAmaxWaves, cu_count_or(256));
 #define CDIT_PT_CASE(CH)                                                                           \
   if (need <= CH) {                                                                                \
-    hipLaunchKernelGGL(tensor_amax_rows<CH>,                                                       \
-                       dim3((unsigned)std::min<int64_t>((M + kAmaxWaves - 1) / kAmaxWaves, cu_count_or(256))), \
-                       dim3(64 * kAmaxWaves), 0, stream, xp, ld_x, (int)M, (int)K, amax_ws);        \
+    hipLaunchKernelGGL(tensor_amax_rows<CH>, dim3((unsigned)parts), dim3(64 * kAmaxWaves), 0, stream, \
+                       xp, ld_x, (int)M, (int)K, scale);                                           \
     hipLaunchKernelGGL(quant_tensorwise_cast_rows<CH>, dim3((unsigned)blocks), dim3(64), 0, stream,  \
-                       xp, ld_x, qp, ld_q, scale, (int)M, (int)K, scale_mode, amax_ws);            \
+                       xp, ld_x, qp, ld_q, scale, parts, (int)M, (int)K, scale_mode, amax_ws);     \
     return 0;                                                                                      \
   }
     CDIT_PT_CASE(1) CDIT_PT_CASE(2) CDIT_PT_CASE(3) CDIT_PT_CASE(4) CDIT_PT_CASE(6) CDIT_PT_CASE(8)
     CDIT_PT_CASE(12) CDIT_PT_CASE(16) CDIT_PT_CASE(24) CDIT_PT_CASE(32)
 #undef CDIT_PT_CASE
   }
+  hipLaunchKernelGGL(zero_amax, dim3(1), dim3(1), 0, stream, amax_ws);
   hipLaunchKernelGGL(tensor_amax, dim3((unsigned)blocks), dim3(64), 0, stream, xp, ld_x, (int)M,
                      (int)K, vec, amax_ws);
   hipLaunchKernelGGL(quant_tensorwise_cast, dim3((unsigned)blocks), dim3(64), 0, stream, xp, ld_x,

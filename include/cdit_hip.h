@@ -140,8 +140,8 @@ int cdit_fp8_quant_rowwise_cat2(const void* x1_bf16, int64_t K1, int64_t ld_x1,
  *   scale[m] = s for every m (the GEMM entry point takes per-row scales)
  *
  * amax_ws: 4 bytes of device memory owned by the caller, used as scratch (the
- * bf16 bit pattern of amax is left in it). Three kernels are enqueued; nothing is
- * allocated or synchronised.
+ * bf16 bit pattern of amax is left in it); scale carries partial maxima between the
+ * kernels. Two or three kernels are enqueued; nothing is allocated or synchronised.
  */
 int cdit_fp8_quant_tensorwise(const void* x_bf16, int64_t M, int64_t K, int64_t ld_x,
                               void* q_e4m3, int64_t ld_q, float* scale, void* amax_ws,

@@ -108,3 +108,30 @@ def test_forward_under_hip_graph_capture():
     torch.cuda.synchronize()
     assert torch.equal(y, expect)
   assert eager.shape == y.shape
+
+
+@pytest.mark.parametrize("M", [1, 7, 8, 9, 64, 65, 513, 2047, 2048, 2049, 4608, 16400])
+@pytest.mark.parametrize("K", [8, 520])
+def test_partial_maxima_by_row_count(M, K):
+  """The two-kernel form leaves a partial maximum per eight rows (at most one per CU) in the scale
+  vector: row counts around those limits, the tensor's maximum in the first, a middle and the last
+  row, the same buffers again each time (they hold the previous scale), a NaN and an infinity."""
+  from cache_dit_amd import ops
+  g = torch.Generator().manual_seed(M + K)
+  base = torch.randn(M, K, generator=g).clamp_(-3, 3).to(torch.bfloat16)
+  q = torch.empty((M, K), dtype=torch.float8_e4m3fn, device=_dev())
+  s = torch.empty((M + 4, ), dtype=torch.float32, device=_dev()).fill_(7.0)
+  ws = torch.empty((1, ), dtype=torch.int32, device=_dev())
+  for row, peak in ((0, 1000.0), (M // 2, -37.0), (M - 1, 5.0), (M - 1, float("inf")), (0, float("nan")), (M // 2, 4.0)):
+    x = base.clone()
+    x[row, K - 1] = peak
+    ops.quant_tensorwise_into(x.to(_dev()), q, s[:M], ws, 0)
+    torch.cuda.synchronize()
+    amax = x.abs().amax()
+    assert int(ws) == int(amax.view(torch.int16)) & 0x7fff
+    if not torch.isfinite(amax):
+      assert torch.isnan(s[:M]).all() if torch.isnan(amax) else torch.isinf(s[:M]).all()
+      continue
+    q_ref, s_ref = to.quantize_tensorwise(x, "bf16div")
+    assert torch.equal(s[:M].cpu(), s_ref.reshape(-1).expand(M)) and (s[M:] == 7.0).all()
+    assert torch.equal(q.cpu().view(torch.uint8), q_ref.view(torch.uint8))
