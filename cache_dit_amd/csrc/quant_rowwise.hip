@@ -395,7 +395,7 @@ __global__ __launch_bounds__(64) void quant_tensorwise_cast(
 // of the cast alone replaces them by the scale; a wavefront that comes later finds a word
 // without the tag, which then is the scale itself. Against a launch that clears the word and an
 // atomic per workgroup, graph replays: 17 x 1024 7.3 -> 6.0 us, 512 x 3072 8.5 -> 6.4, 4608 x 3072
-// 17.8 -> 15.7 (4.5 TB/s over two reads and a write), 6889 x 12288 112.3 -> 113.3 (within noise).
+// 17.8 -> 15.7 (4.5 TB/s over two reads and a write).
 constexpr int kAmaxWaves = 8;  // wavefronts per workgroup of tensor_amax_rows
 constexpr uint32_t kPartTag = 0xffff0000u;
 
@@ -431,6 +431,7 @@ __global__ __launch_bounds__(64 * kAmaxWaves) void tensor_amax_rows(const uint16
   }
 }
 
+// Workgroup (p, r): the 512 CH elements from p of rows r, r + gridDim.y, ...
 template <int CH>
 __global__ __launch_bounds__(64) void quant_tensorwise_cast_rows(
     const uint16_t* __restrict__ x, int64_t ld_x, uint8_t* __restrict__ q, int64_t ld_q,
@@ -450,33 +451,34 @@ __global__ __launch_bounds__(64) void quant_tensorwise_cast_rows(
   m = wave_max_u32(m);
   done = wave_max_u32(done);
   const float s = done ? __uint_as_float(done) : row_scale(m, scale_mode);
-  if (blockIdx.x == 0) {
+  if (blockIdx.x == 0 && blockIdx.y == 0) {
     for (int i = lane; i < parts; i += 64)
       __hip_atomic_store(words + i, __float_as_uint(s), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (lane == 0) *amax_ws = m;
   }
   const bool fast = scale_in_fast_window(s);
   const Recip r = make_recip(s);
-  for (int64_t row = blockIdx.x; row < M; row += gridDim.x) {
-    if (lane == 0 && row >= parts) scale[row] = s;
+  const int first = blockIdx.x * CH * 64 + lane;  // this lane's first group of eight elements
+  for (int64_t row = blockIdx.y; row < M; row += gridDim.y) {
+    if (lane == 0 && blockIdx.x == 0 && row >= parts) scale[row] = s;
     const __amdgpu_buffer_rsrc_t xb = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<uint16_t*>(x + row * ld_x), 0, K * 2, 0x00020000);
     const __amdgpu_buffer_rsrc_t qb = __builtin_amdgcn_make_buffer_rsrc(q + row * ld_q, 0, K, 0x00020000);
     u4v w[CH];
 #pragma unroll
-    for (int c = 0; c < CH; ++c) w[c] = __builtin_amdgcn_raw_buffer_load_b128(xb, 16 * (c * 64 + lane), 0, 0);
+    for (int c = 0; c < CH; ++c) w[c] = __builtin_amdgcn_raw_buffer_load_b128(xb, 16 * (c * 64 + first), 0, 0);
     if (fast) {
 #pragma unroll
       for (int c = 0; c < CH; ++c)
         __builtin_amdgcn_raw_buffer_store_b64(
             u2v{quant4<true>(w[c][0], w[c][1], s, r), quant4<true>(w[c][2], w[c][3], s, r)}, qb,
-            8 * (c * 64 + lane), 0, 2);
+            8 * (c * 64 + first), 0, 2);
     } else {
 #pragma unroll 1
       for (int c = 0; c < CH; ++c)
         __builtin_amdgcn_raw_buffer_store_b64(
             u2v{quant4<false>(w[c][0], w[c][1], s, Recip{}), quant4<false>(w[c][2], w[c][3], s, Recip{})}, qb,
-            8 * (c * 64 + lane), 0, 2);
+            8 * (c * 64 + first), 0, 2);
     }
   }
 }
@@ -1139,12 +1141,18 @@ int launch_quant_tensorwise(const void* x, int64_t M, int64_t K, int64_t ld_x, v
   if (vec && K <= 32 * 512) {
     const int need = (int)((K + 511) / 512);
     const int parts = (int)std::min<int64_t>((M + kAmaxWaves - 1) / kAmaxWaves, cu_count_or(256));
+    // The cast of rows beyond 4096 elements: a wavefront per 3072 of them. A whole row in one
+    // wavefront's registers leaves few wavefronts per SIMD and a last round of them that is nearly
+    // empty. Both passes, graph replays: 6889 x 12288 113.3 -> 71.4 us (5.9 TB/s), 4608 x 15360
+    // 91.0 -> 62.0; against three launches 4608 x 4112 38.1 -> 29.2, 300 x 15360 16.1 -> 10.1.
 #define CDIT_PT_CASE(CH)                                                                           \
   if (need <= CH) {                                                                                \
     hipLaunchKernelGGL(tensor_amax_rows<CH>, dim3((unsigned)parts), dim3(64 * kAmaxWaves), 0, stream, \
                        xp, ld_x, (int)M, (int)K, scale);                                           \
-    hipLaunchKernelGGL(quant_tensorwise_cast_rows<CH>, dim3((unsigned)blocks), dim3(64), 0, stream,  \
-                       xp, ld_x, qp, ld_q, scale, parts, (int)M, (int)K, scale_mode, amax_ws);     \
+    constexpr int CAST = CH <= 8 ? CH : 6;                                                         \
+    hipLaunchKernelGGL(quant_tensorwise_cast_rows<CAST>,                                           \
+                       dim3((unsigned)std::max(1, (need + CAST - 1) / CAST), (unsigned)blocks), dim3(64), 0, \
+                       stream, xp, ld_x, qp, ld_q, scale, parts, (int)M, (int)K, scale_mode, amax_ws); \
     return 0;                                                                                      \
   }
     CDIT_PT_CASE(1) CDIT_PT_CASE(2) CDIT_PT_CASE(3) CDIT_PT_CASE(4) CDIT_PT_CASE(6) CDIT_PT_CASE(8)
