@@ -1141,9 +1141,10 @@ int launch_quant_tensorwise(const void* x, int64_t M, int64_t K, int64_t ld_x, v
   if (vec && K <= 32 * 512) {
     const int need = (int)((K + 511) / 512);
     const int parts = (int)std::min<int64_t>((M + kAmaxWaves - 1) / kAmaxWaves, cu_count_or(256));
-    // The cast of rows beyond 4096 elements: a wavefront per 3072 of them. A whole row in one
-    // wavefront's registers leaves few wavefronts per SIMD and a last round of them that is nearly
-    // empty. Both passes, graph replays: 6889 x 12288 113.3 -> 71.4 us (5.9 TB/s), 4608 x 15360
+    // The cast of rows beyond 4096 elements: a wavefront per 3072 of them. With 12 and more vectors
+    // of a row per lane the compiler kept them in scratch memory too (for the indexed loop of
+    // the exact division: 400 bytes per lane at 24), and 2 to 6 wavefronts fitted a SIMD instead
+    // of 8. Both passes, graph replays: 6889 x 12288 113.3 -> 71.4 us (5.9 TB/s), 4608 x 15360
     // 91.0 -> 62.0; against three launches 4608 x 4112 38.1 -> 29.2, 300 x 15360 16.1 -> 10.1.
 #define CDIT_PT_CASE(CH)                                                                           \
   if (need <= CH) {                                                                                \

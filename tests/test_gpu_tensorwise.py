@@ -111,12 +111,14 @@ def test_forward_under_hip_graph_capture():
 
 
 @pytest.mark.parametrize("M", [1, 7, 8, 9, 64, 65, 513, 2047, 2048, 2049, 4608, 16400])
-@pytest.mark.parametrize("K", [8, 520])
+@pytest.mark.parametrize("K", [8, 520, 4104, 6152])
 def test_partial_maxima_by_row_count(M, K):
   """The two-kernel form leaves a partial maximum per eight rows (at most one per CU) in the scale
-  vector: row counts around those limits, the tensor's maximum in the first, a middle and the last
+  vector: row counts around those limits, rows that one or several wavefronts cast, the tensor's maximum in the first, a middle and the last
   row, the same buffers again each time (they hold the previous scale), a NaN and an infinity."""
   from cache_dit_amd import ops
+  if M * K > 1 << 24:
+    pytest.skip("the row counts are covered by the short rows")
   g = torch.Generator().manual_seed(M + K)
   base = torch.randn(M, K, generator=g).clamp_(-3, 3).to(torch.bfloat16)
   q = torch.empty((M, K), dtype=torch.float8_e4m3fn, device=_dev())
