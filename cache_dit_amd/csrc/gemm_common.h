@@ -80,6 +80,15 @@ __device__ __forceinline__ float gelu_tanh(float v) {
   return v * __builtin_amdgcn_rcpf(1.0f + e);
 }
 
+// Eight e4m3 values (two words) as bf16, exact. Not for operands of inline-assembly MFMAs.
+__device__ __forceinline__ v8bf e4m3x8_to_bf16(uint32_t lo, uint32_t hi) {
+  const v2bf c0 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 1.0f, false);
+  const v2bf c1 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 1.0f, true);
+  const v2bf c2 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 1.0f, false);
+  const v2bf c3 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 1.0f, true);
+  return v8bf{c0[0], c0[1], c1[0], c1[1], c2[0], c2[1], c3[0], c3[1]};
+}
+
 // s_waitcnt vmcnt(N) lgkmcnt(0) followed by a bare workgroup barrier. The memory
 // clobber keeps the compiler from moving LDS accesses across it.
 // The s_waitcnt is emitted through the builtin so that the compiler's own wait

@@ -409,6 +409,31 @@ __device__ __forceinline__ void mfma_16x16x128_fp8(v4f& acc, const v8i& b, const
   }
 }
 
+// The operands of K that is not a whole number of steps: the 32 e4m3 codes a lane holds of a
+// 128-byte step, converted to bf16 (exact), as four operands of v_mfma_f32_16x16x32_bf16. Which
+// of the 128 k a lane's byte is does not matter to a dot product, as long as it is the same in
+// both operands. The FP8 instructions (f8f6f4 and the unscaled ones alike) cut the bits of a sum
+// that lie some 13 places below its largest product: 200704 + 1 + 3 gives 200707, and a sum of
+// 2304 random products is 1.7e-5 off its 64-bit value (relative 2-norm), 5e-5 with rows of
+// mixed magnitudes. The bf16 instruction on the converted codes is 6.2e-8 and 1.5e-7 off, an
+// fp32 FMA per product (gemm_fp8_generic, the only other kernel that takes such a K) 6.4e-8 and
+// 1.6e-7; the same order from K = 128 to 15360.
+struct CodesBf16 {
+  v8bf k[4];
+};
+__device__ __forceinline__ CodesBf16 codes_to_bf16(const v8i& c) {
+  CodesBf16 f;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) f.k[q] = e4m3x8_to_bf16((uint32_t)c[2 * q], (uint32_t)c[2 * q + 1]);
+  return f;
+}
+__device__ __forceinline__ v4f mfma_codes_as_bf16(const v8i& b, const v8i& a, v4f acc) {
+  const CodesBf16 bb = codes_to_bf16(b), aa = codes_to_bf16(a);
+#pragma unroll
+  for (int q = 0; q < 4; ++q) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bb.k[q], aa.k[q], acc, 0, 0, 0);
+  return acc;
+}
+
 // A batch of GEMMs as one launch (GemmGroup, declared with the launchers): sibling Linears
 // that read one activation -- to_q / to_k / to_v, and proj_mlp next to them in FLUX single
 // blocks (reference dataflow: src/cache_dit/caching/patch_functors/functor_flux.py:60-67) --
@@ -434,8 +459,8 @@ struct NoGroup {};
 // which the last ones are all zeros. The chunk a lane fetches is the same for every DMA
 // instruction of a panel (swz_a / swz_b take the row bits that the lane and the parity of the
 // wave give), so a step costs one comparison per panel and one OR per DMA instruction.
-// Without it such a K ran one scalar FMA per element: 1357 x 2224 x 4464 16.8 ms (1.6
-// TFLOP/s); with it 25 us.
+// These instances multiply on the bf16 matrix instruction (mfma_codes_as_bf16): such a K has
+// its sums in full fp32, which the FP8 instruction's are not.
 struct StampArgs {
   unsigned long long* stamps;
 };
@@ -647,6 +672,7 @@ gemm_fp8_wide(GemmArgs g, int tiles_m, int tiles_n,
 
   v4f acc[TM][TN];
   v8i af[TM], bf[TN];
+  CodesBf16 bw[KTAIL ? TN : 1];  // KTAIL: this step's B operands as bf16
 
   // LDS offsets of the stages of steps kt-1 / kt / kt+1 (A) and kt / kt+1 (B);
   // step s lives in A stage s mod (D+1) and B stage s mod D
@@ -680,6 +706,27 @@ gemm_fp8_wide(GemmArgs g, int tiles_m, int tiles_n,
     v4f bs[TN];
     uint2 bi[TN];  // bias stays packed (bf16 pairs) until used: registers are scarce
     float as[TM];
+
+    // KTAIL: row i of blocks on the bf16 instruction, four MFMAs per block, a k group of all its
+    // blocks before the next (consecutive MFMAs are independent); items(b) is what the schedule
+    // puts in front of block b of the row. Row 0 converts the step's B operands on the way, so
+    // that every raw B fragment is free in the second half. Builtins: the compiler places the
+    // conversions and knows the wait states between them and the MFMAs.
+    auto row_as_bf16 = [&](int i, auto first_tag, auto items) {
+      constexpr bool FIRST = decltype(first_tag)::value;
+      const CodesBf16 a = codes_to_bf16(af[i]);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          if ((q * TN + j) % 4 == 0) items((q * TN + j) / 4);
+          if (i == 0) bw[j].k[q] = e4m3x8_to_bf16((uint32_t)bf[j][2 * q], (uint32_t)bf[j][2 * q + 1]);
+          v4f c = acc[i][j];
+          if (FIRST && q == 0) c = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bw[j].k[q], a.k[q], c, 0, 0, 0);
+        }
+      }
+    };
 
     // One K step; FIRST: step 0 of the tile (the accumulators start from zero).
     // EVENTS: the step may be one of the last max(D, 2) of the tile, where the DMA stream
@@ -749,19 +796,36 @@ gemm_fp8_wide(GemmArgs g, int tiles_m, int tiles_n,
       // first half: rows 0..H-1, row-major; meanwhile the other A fragments of this
       // step are read and the A panel D steps ahead goes into the stage that step
       // kt-1 read (schedule: CfgWide::slot1)
+      if constexpr (KTAIL) {
 #pragma unroll
-      for (int sl = 0; sl < C::S1; ++sl) {
+        for (int i = 0; i < H; ++i)
+          row_as_bf16(i, first_tag, [&](int b) {
 #pragma unroll
-        for (int t = 0; t < C::T1; ++t) {
-          if (C::slot1(t) != sl) continue;
-          if (C::is_read1(t)) {
-            af[C::read1_index(t) + 1] = read_a(st, C::read1_index(t) + 1);
-          } else {
-            dma_a(kd, a_prev, C::dma1_index(t));
-          }
-        }
-        mfma_16x16x128_fp8<FIRST>(acc[sl / TN][sl % TN], bf[sl % TN], af[sl / TN]);
+            for (int t = 0; t < C::T1; ++t) {
+              if (C::slot1(t) != i * TN + b) continue;
+              if (C::is_read1(t)) {
+                af[C::read1_index(t) + 1] = read_a(st, C::read1_index(t) + 1);
+              } else {
+                dma_a(kd, a_prev, C::dma1_index(t));
+              }
+            }
+          });
         __builtin_amdgcn_sched_barrier(0);
+      } else {
+#pragma unroll
+        for (int sl = 0; sl < C::S1; ++sl) {
+#pragma unroll
+          for (int t = 0; t < C::T1; ++t) {
+            if (C::slot1(t) != sl) continue;
+            if (C::is_read1(t)) {
+              af[C::read1_index(t) + 1] = read_a(st, C::read1_index(t) + 1);
+            } else {
+              dma_a(kd, a_prev, C::dma1_index(t));
+            }
+          }
+          mfma_16x16x128_fp8<FIRST>(acc[sl / TN][sl % TN], bf[sl % TN], af[sl / TN]);
+          __builtin_amdgcn_sched_barrier(0);
+        }
       }
       // own LDS reads of this step done, own DMA of the next step landed (the
       // steps after it and the A panel issued above may still fly); then
@@ -786,9 +850,14 @@ gemm_fp8_wide(GemmArgs g, int tiles_m, int tiles_n,
           if (C::slot_dma2(p) == sl) dma_b(kd, b_cur, p);
       };
       int a_after = 0, b_after = 0;  // stages of the step after the next
+      if constexpr (KTAIL) {
+#pragma unroll
+        for (int i = H; i < TM; ++i)
+          row_as_bf16(i, first_tag, [&](int b) { second_half_items((i - H) * TN + b); });
+      }
 #pragma unroll
       for (int sl = 0; sl < C::S2; ++sl) {
-        second_half_items(sl);
+        if constexpr (!KTAIL) second_half_items(sl);
         if (sl == C::S2 - 1) {
           // worked out in front of the last MFMA, not behind it
           a_after = a_next + C::A_BYTES == C::A_STAGES * C::A_BYTES ? 0 : a_next + C::A_BYTES;
@@ -796,8 +865,10 @@ gemm_fp8_wide(GemmArgs g, int tiles_m, int tiles_n,
                         ? C::B_BASE
                         : b_next + C::B_BYTES;
         }
-        mfma_16x16x128_fp8<FIRST>(acc[H + sl % C::R][sl / C::R], bf[sl / C::R], af[H + sl % C::R]);
-        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (!KTAIL) {
+          mfma_16x16x128_fp8<FIRST>(acc[H + sl % C::R][sl / C::R], bf[sl / C::R], af[H + sl % C::R]);
+          __builtin_amdgcn_sched_barrier(0);
+        }
       }
       second_half_items(C::S2);
       __builtin_amdgcn_sched_barrier(0);
@@ -1123,6 +1194,9 @@ int launch_wide_grouped(const GemmArgs& g, GemmGroup grp, hipStream_t stream) {
 // weights: every weight byte is used exactly once. The weight loads carry no
 // non-temporal hint: with this access pattern (16 rows x 64 bytes per instruction)
 // the hinted loads measured 17 % slower in a read-only loop and 10 % in the kernel.
+// KTAIL: K is not a multiple of 128; the products go through the bf16 instruction, as in the
+// wide kernel's instances.
+template <bool KTAIL>
 __global__ __launch_bounds__(256) void gemm_fp8_skinny(GemmArgs g) {
   __shared__ float part[4][16][17];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -1157,7 +1231,11 @@ __global__ __launch_bounds__(256) void gemm_fp8_skinny(GemmArgs g) {
         v8i wf = __builtin_shufflevector(w[u][0], w[u][1], 0, 1, 2, 3, 4, 5, 6, 7);
         v8i af = __builtin_shufflevector(a[u][0], a[u][1], 0, 1, 2, 3, 4, 5, 6, 7);
         if (!a_valid) af = v8i{0, 0, 0, 0, 0, 0, 0, 0};
-        acc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf, af, acc, 0, 0, 0, 0, 0, 0);
+        if constexpr (KTAIL) {
+          acc = mfma_codes_as_bf16(wf, af, acc);
+        } else {
+          acc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf, af, acc, 0, 0, 0, 0, 0, 0);
+        }
       }
     }
   }
@@ -1202,6 +1280,7 @@ __global__ __launch_bounds__(256) void gemm_fp8_skinny(GemmArgs g) {
 // workspaces. The first batch of weight loads is issued before that, so the HBM latency
 // of the weights covers it. g.a is the bf16 activation here, g.lda its leading dimension.
 constexpr int kFusedPad = 16;  // LDS row pitch K + 16 bytes: rows start 4 banks apart
+template <bool KTAIL>
 __global__ __launch_bounds__(256) void linear_fp8_skinny_fused(GemmArgs g, uint8_t* q_ws,
                                                                float* scale_ws, int scale_mode) {
   extern __shared__ __attribute__((aligned(16))) uint8_t codes[];  // [M][K + kFusedPad]
@@ -1290,7 +1369,11 @@ __global__ __launch_bounds__(256) void linear_fp8_skinny_fused(GemmArgs g, uint8
         v8i af = __builtin_shufflevector(a[0], a[1], 0, 1, 2, 3, 4, 5, 6, 7);
         if (!a_valid) af = v8i{0, 0, 0, 0, 0, 0, 0, 0};
         const v8i wf = __builtin_shufflevector(w[u][0], w[u][1], 0, 1, 2, 3, 4, 5, 6, 7);
-        acc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf, af, acc, 0, 0, 0, 0, 0, 0);
+        if constexpr (KTAIL) {
+          acc = mfma_codes_as_bf16(wf, af, acc);
+        } else {
+          acc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf, af, acc, 0, 0, 0, 0, 0, 0);
+        }
       }
     }
   }
@@ -1344,8 +1427,9 @@ __global__ __launch_bounds__(256) void linear_fp8_skinny_fused(GemmArgs g, uint8
 // FUSED: the row is quantized by every workgroup itself, as in linear_fp8_skinny_fused
 // (same codes, same scale, workgroup 0 writes them to the caller's workspaces); else
 // g.a holds the codes and g.a_scale the scale.
+// KTAIL: as in the 16-row kernels.
 constexpr int kRow1Rows = 3, kRow1Waves = 4;
-template <int CHK, bool FUSED>
+template <int CHK, bool FUSED, bool KTAIL>
 __global__ __launch_bounds__(64 * kRow1Waves) void linear_fp8_row1(GemmArgs g, uint8_t* q_ws,
                                                                    float* scale_ws, int scale_mode) {
   constexpr int R = kRow1Rows, WAVES = kRow1Waves, THREADS = 64 * WAVES;
@@ -1428,7 +1512,11 @@ __global__ __launch_bounds__(64 * kRow1Waves) void linear_fp8_row1(GemmArgs g, u
       const v4i w1 = c + 1 < CHK ? w[q][c + 1] : zero4, x1 = c + 1 < CHK ? xa[c + 1] : zero4;
       const v8i wf = __builtin_shufflevector(w[q][c], w1, 0, 1, 2, 3, 4, 5, 6, 7);
       const v8i af = __builtin_shufflevector(xa[c], x1, 0, 1, 2, 3, 4, 5, 6, 7);
-      acc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf, af, acc, 0, 0, 0, 0, 0, 0);
+      if constexpr (KTAIL) {
+        acc = mfma_codes_as_bf16(wf, af, acc);
+      } else {
+        acc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf, af, acc, 0, 0, 0, 0, 0, 0);
+      }
     }
     float d = 0.0f;
 #pragma unroll
@@ -1528,9 +1616,15 @@ int launch_row1(const GemmArgs& g, uint8_t* q_ws, float* scale_ws, int scale_mod
   if (!ok) return 1;
   constexpr int rows_wg = kRow1Rows * kRow1Waves;
   auto go = [&](auto chk_tag) {
-    hipLaunchKernelGGL((linear_fp8_row1<decltype(chk_tag)::value, FUSED>),
-                       dim3((g.N + rows_wg - 1) / rows_wg), dim3(64 * kRow1Waves), 0, stream, g, q_ws,
-                       scale_ws, scale_mode);
+    constexpr int CHK = decltype(chk_tag)::value;
+    const dim3 grid((g.N + rows_wg - 1) / rows_wg), block(64 * kRow1Waves);
+    if (g.K % BK) {
+      hipLaunchKernelGGL((linear_fp8_row1<CHK, FUSED, true>), grid, block, 0, stream, g, q_ws, scale_ws,
+                         scale_mode);
+    } else {
+      hipLaunchKernelGGL((linear_fp8_row1<CHK, FUSED, false>), grid, block, 0, stream, g, q_ws, scale_ws,
+                         scale_mode);
+    }
   };
   switch ((g.K + 1023) / 1024) {
     case 1: go(std::integral_constant<int, 1>{}); break;
@@ -1561,8 +1655,13 @@ int launch_linear_fp8_skinny_fused(const GemmArgs& g, void* q_ws, float* scale_w
                   reinterpret_cast<uintptr_t>(g.out) % 16 == 0 &&
                   reinterpret_cast<uintptr_t>(q_ws) % 8 == 0;
   if (!ok) return 1;
-  hipLaunchKernelGGL(linear_fp8_skinny_fused, dim3((g.N + 15) / 16), dim3(256), (size_t)lds, stream,
-                     g, static_cast<uint8_t*>(q_ws), scale_ws, scale_mode);
+  if (g.K % BK) {
+    hipLaunchKernelGGL(linear_fp8_skinny_fused<true>, dim3((g.N + 15) / 16), dim3(256), (size_t)lds, stream,
+                       g, static_cast<uint8_t*>(q_ws), scale_ws, scale_mode);
+  } else {
+    hipLaunchKernelGGL(linear_fp8_skinny_fused<false>, dim3((g.N + 15) / 16), dim3(256), (size_t)lds, stream,
+                       g, static_cast<uint8_t*>(q_ws), scale_ws, scale_mode);
+  }
   return 0;
 }
 
@@ -1633,7 +1732,11 @@ int launch_gemm_fp8(const GemmArgs& g, int variant, hipStream_t stream) {
       set_error("cdit_fp8_gemm_rowwise: the skinny kernel takes M <= 16, got %d", g.M);
       return CDIT_EINVAL;
     }
-    hipLaunchKernelGGL(gemm_fp8_skinny, dim3((g.N + 15) / 16), dim3(256), 0, stream, g);
+    if (g.K % BK) {
+      hipLaunchKernelGGL(gemm_fp8_skinny<true>, dim3((g.N + 15) / 16), dim3(256), 0, stream, g);
+    } else {
+      hipLaunchKernelGGL(gemm_fp8_skinny<false>, dim3((g.N + 15) / 16), dim3(256), 0, stream, g);
+    }
     return 0;
   }
   if (!tiled_ok(g)) return launch_gemm_fp8_ktail(g, variant, stream);
@@ -1662,19 +1765,33 @@ int launch_gemm_fp8(const GemmArgs& g, int variant, hipStream_t stream) {
 }
 
 // K a multiple of 16 but not of 128, or shorter than a step: the KTAIL instances of the wide
-// kernel (they take any K, so the choice of the tile is the one for a long K; fp16 and fp32
-// outputs have three tiles, as above).
+// kernel, which take any K. They run at the rate of the bf16 instruction and convert the codes,
+// so a round of a tile takes longer than that of the FP8 instances and grows more with its area;
+// the tile is chosen by their own round times (tenths of a us at K of about 2200; only the ratios
+// count). Within 0.1 % of the best tile over 90 shapes of M 17 to 6889, K 272 to 12288, N 272 to
+// 4592 (geometric mean; the worst 9 % off). 1357 x 4464 x 2224 (M x N x K): 38.9 us with 128 x 128
+// against 42.0 (256 x 192) and 50.4 (128 x 192); 256 x 3072 x 2992: 19.8 with 64 x 128 against
+// 24.8 (128 x 128); 4608 x 3072 x 3056: 68.5 with 288 x 192 against 87.6 (128 x 128) and 100.4
+// (256 x 192). The scalar FMA kernel took 16.8 ms for the first. There is no 256 x 256 instance:
+// its converted operands do not fit the registers. fp16 and fp32 outputs have three tiles.
 int launch_gemm_fp8_ktail(const GemmArgs& g, int variant, hipStream_t stream) {
-  auto tiles = [&](int bm, int bn) { return (int64_t)((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn); };
-  if (g.out_dtype != CDIT_DT_BF16) {
-    const int v = choose_other_out_variant(g, variant, [](int) { return true; });
-    return g.out_dtype == CDIT_DT_F16 ? launch_other_out<CDIT_DT_F16, true>(g, v, stream)
-                                      : launch_other_out<CDIT_DT_F32, true>(g, v, stream);
+  const int64_t cus = cu_count() > 0 ? cu_count() : 256;
+  const struct { int v, bm, bn, us10; bool other_out; } cand[] = {
+      {14, 288, 192, 530, false}, {15, 256, 192, 470, true}, {16, 128, 192, 290, false},
+      {18, 128, 128, 205, true}, {17, 64, 128, 150, true}};
+  const bool bf16 = g.out_dtype == CDIT_DT_BF16;
+  int best = 18;
+  int64_t time = INT64_MAX;
+  for (const auto& c : cand) {
+    if (!bf16 && !c.other_out) continue;
+    const int64_t tiles = (int64_t)((g.M + c.bm - 1) / c.bm) * ((g.N + c.bn - 1) / c.bn);
+    const int64_t t = variant == c.v ? -1 : rounds_time(tiles, cus, c.us10);
+    if (t < time) best = c.v, time = t;
   }
-  const bool forced = variant == 12 || (variant >= 14 && variant <= 18);
-  if (!forced) variant = choose_bf16_variant(tiles, [](int) { return true; }).variant;
-  switch (variant) {
-    case 12: return launch_wide<V12, CDIT_DT_BF16, true>(g, stream);
+  if (!bf16)
+    return g.out_dtype == CDIT_DT_F16 ? launch_other_out<CDIT_DT_F16, true>(g, best, stream)
+                                      : launch_other_out<CDIT_DT_F32, true>(g, best, stream);
+  switch (best) {
     case 14: return launch_wide<V14, CDIT_DT_BF16, true>(g, stream);
     case 15: return launch_wide<V15, CDIT_DT_BF16, true>(g, stream);
     case 16: return launch_wide<V16, CDIT_DT_BF16, true>(g, stream);

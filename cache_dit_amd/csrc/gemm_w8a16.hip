@@ -936,15 +936,6 @@ int launch_wide_grouped(const GemmArgs& g, GemmGroup grp, hipStream_t stream) {
   return 0;
 }
 
-// Eight e4m3 values (two words) as bf16, exact. Not for operands of inline-assembly MFMAs.
-__device__ __forceinline__ v8bf e4m3x8_to_bf16(uint32_t lo, uint32_t hi) {
-  const v2bf c0 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 1.0f, false);
-  const v2bf c1 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 1.0f, true);
-  const v2bf c2 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 1.0f, false);
-  const v2bf c3 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 1.0f, true);
-  return v8bf{c0[0], c0[1], c1[0], c1[1], c2[0], c2[1], c3[0], c3[1]};
-}
-
 // ---------------------------------------------------------------------------
 // A few dozen rows (the prompt's projections: M = 17 to 128 or so): one wavefront, alone in
 // its workgroup, per 32 x 32 tile. A 128 x 64 tile of the wide kernel gives such a problem to a

@@ -110,3 +110,54 @@ def test_other_output_types(out_dtype, variant):
     ops.gemm_rowwise_into(a, sa, w, sw, None, out, 0)
     torch.cuda.synchronize()
     assert torch.equal(out, (exact * sa.double()[:, None]).float().to(out_dtype)), (out_dtype, variant, K)
+
+
+def _wide_range_problem(M, N, K, seed, act_dtype):
+  """Products of 448 x 448 = 200704 next to products of a few units, all integers: in each run of
+  128 k, two k where every activation is 448 and the weights are +448 and -448, so the large
+  products cancel and the result is the sum of the small ones. At most K / 64 = 64 large products
+  of 200704 and 9 K small units: every partial sum in any order is an integer below 2^24, exact in
+  fp32. A unit that cuts low bits of a sum next to a large product is off by units."""
+  g = torch.Generator(device=DEV).manual_seed(seed)
+  a, w = _ints(-3, 4, (M, K), g), _ints(-3, 4, (N, K), g)
+  for k in range(0, K - 15, 128):
+    first = k + int(torch.randint(0, 8, (1, ), generator=g, device=DEV))
+    second = first + 8
+    a[:, first] = a[:, second] = 448.0
+    w[:, first], w[:, second] = 448.0, -448.0
+  assert (2 * ((K + 127) // 128)) * 448**2 + 9 * K < 2**24
+  exact = a.double() @ w.double().t()
+  return _framed(a, 32, act_dtype), _framed(w, 48, FP8), exact
+
+
+def _expect(run, exact, dtype, what):
+  out = torch.empty(exact.shape, dtype=dtype, device=DEV)
+  run(out)
+  torch.cuda.synchronize()
+  assert torch.equal(out, exact.float().to(dtype)), what
+
+
+@pytest.mark.parametrize("K", [144, 336, 1040, 2224, 4080])
+def test_sums_keep_fp32(K):
+  """Every kernel that takes such a K sums in full fp32, as the kernels for any shape do."""
+  from cache_dit_amd import _native, ops
+  for M in (1, 2, 16, 17, 300):
+    N = 264
+    a, w, exact = _wide_range_problem(M, N, K, K + M, FP8)
+    x = _framed(a.float(), 32, torch.bfloat16)
+    one, ones = torch.ones(M, device=DEV), torch.ones(N, device=DEV)
+    for dtype, variants in ((torch.bfloat16, (-1, 100, 12, 14, 15, 16, 17, 18)), (torch.float16, (-1, 15, 17, 18)),
+                            (torch.float32, (-1, 15, 17, 18))):
+      for variant in variants if M > 16 else (-1, 50):
+        _native.set_gemm_variant(variant)
+        _expect(lambda out: ops.gemm_rowwise_into(a, one, w, ones, None, out, 0), exact, dtype,
+                (M, K, dtype, variant))
+    for variant in (-1, 100, 7, 8, 9, 10, 11, 12) if M > 16 else (-1, 50):
+      _native.set_gemm_variant(variant)
+      _expect(lambda out: ops.w8a16_into(x, w, ones, None, out, 0), exact, torch.bfloat16, ("w8a16", M, K, variant))
+    _native.set_gemm_variant(-1)
+    q = torch.empty((M, K), dtype=FP8, device=DEV)
+    s = torch.empty((M, ), dtype=torch.float32, device=DEV)
+    _expect(lambda out: ops.linear_w8a8_into(x, w, ones, None, out, q, s, 0, 0), exact, torch.bfloat16,
+            ("linear", M, K))
+    assert torch.equal(q.float(), x.float()) and bool((s == 1.0).all())
