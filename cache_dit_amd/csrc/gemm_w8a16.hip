@@ -1104,6 +1104,11 @@ int launch_wavetile(const GemmArgs& g, hipStream_t stream) {
 // straight from HBM and the matching 32 bf16 activations (zero for rows >= M),
 // converts the weights to bf16 and issues four v_mfma_f32_16x16x32_bf16; the four
 // partial tiles are summed through LDS.
+// KTAIL: K is not a multiple of 128; what lies beyond it is masked. The masks are kept out of the
+// instance for whole chunks: each made the load a branch of its own, and the registers of the
+// masked loads cost two of seven wavefronts per SIMD (16 rows, N = 18432, K = 3072: 26.5 us
+// without, 32.4 with masks; K = 5120: 47.4 and 60.9).
+template <bool KTAIL>
 __global__ __launch_bounds__(256) void gemm_w8a16_skinny(GemmArgs g) {
   __shared__ float part[4][16][17];
   typedef float v4f_ __attribute__((ext_vector_type(4)));
@@ -1111,7 +1116,7 @@ __global__ __launch_bounds__(256) void gemm_w8a16_skinny(GemmArgs g) {
   const int r = lane & 15, kg = lane >> 4;
   const int n0 = blockIdx.x * 16;
   const int nrow = min(n0 + r, g.N - 1);
-  const int KT = (g.K + 127) / 128;  // the last 128-element chunk may be partial
+  const int KT = KTAIL ? (g.K + 127) / 128 : g.K / 128;
   const int per = (KT + 3) / 4;
   const int k_begin = wave * per, k_end = min(KT, k_begin + per);
   const uint8_t* __restrict__ wp = g.b + (int64_t)nrow * g.ldb + kg * 32;
@@ -1127,12 +1132,20 @@ __global__ __launch_bounds__(256) void gemm_w8a16_skinny(GemmArgs g) {
     for (int u = 0; u < U; ++u) {
       const int kt = min(k0 + u, k_end - 1);
       const v8bf* aq = reinterpret_cast<const v8bf*>(ap + (int64_t)kt * 128);
+      if constexpr (KTAIL) {
 #pragma unroll
-      for (int e = 0; e < 2; ++e) {  // (16 elements beyond K are zeros on both sides)
-        const bool in = kt * 128 + kg * 32 + e * 16 < g.K;
-        w[u][e] = in ? *reinterpret_cast<const uint4*>(wp + kt * 128 + e * 16) : uint4{0u, 0u, 0u, 0u};
+        for (int e = 0; e < 2; ++e) {  // (16 elements beyond K are zeros on both sides)
+          const bool in = kt * 128 + kg * 32 + e * 16 < g.K;
+          w[u][e] = in ? *reinterpret_cast<const uint4*>(wp + kt * 128 + e * 16) : uint4{0u, 0u, 0u, 0u};
 #pragma unroll
-        for (int t = 2 * e; t < 2 * e + 2; ++t) a[u][t] = in ? aq[t] : v8bf{0, 0, 0, 0, 0, 0, 0, 0};
+          for (int t = 2 * e; t < 2 * e + 2; ++t) a[u][t] = in ? aq[t] : v8bf{0, 0, 0, 0, 0, 0, 0, 0};
+        }
+      } else {
+        const uint4* wq = reinterpret_cast<const uint4*>(wp + (int64_t)kt * 128);
+        w[u][0] = wq[0];
+        w[u][1] = wq[1];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) a[u][t] = aq[t];
       }
     }
 #pragma unroll
@@ -1403,7 +1416,11 @@ int launch_gemm_w8a16(const GemmArgs& g, int variant, hipStream_t stream) {
       set_error("cdit_w8a16_gemm: the skinny kernel takes M <= 16");
       return CDIT_EINVAL;
     }
-    hipLaunchKernelGGL(gemm_w8a16_skinny, dim3((g.N + 15) / 16), dim3(256), 0, stream, g);
+    if (g.K % 128) {
+      hipLaunchKernelGGL(gemm_w8a16_skinny<true>, dim3((g.N + 15) / 16), dim3(256), 0, stream, g);
+    } else {
+      hipLaunchKernelGGL(gemm_w8a16_skinny<false>, dim3((g.N + 15) / 16), dim3(256), 0, stream, g);
+    }
     return 0;
   }
   // the wide kernels stream K two or more steps ahead and store 16 columns per lane
