@@ -173,11 +173,26 @@ inline int cu_count() {
   return n;
 }
 
-// Modelled time of `tiles` tiles, one persistent workgroup per CU, for a tile whose full round
-// takes `round`: a last, partial round of r tiles counts 0.7 + 0.3 r/cus (small problems).
-inline int64_t rounds_time(int64_t tiles, int64_t cus, int round) {
+// Rounds that `tiles` tiles take over the CUs, one persistent workgroup each, in thousandths. A
+// round of r tiles takes less than a full one (fewer CUs share the power and the memory): it
+// counts p + (1 - p) r/CUs with p = `lone` (in thousandths) if it is the only one, else `last`.
+inline int64_t rounds_permille(int64_t tiles, int64_t cus, int lone, int last) {
   const int64_t full = tiles / cus, rem = tiles % cus;
-  return (full * 10 * cus + (rem ? 7 * cus + 3 * rem : 0)) * round;
+  const int p = full ? last : lone;
+  return full * 1000 + (rem ? p + (1000 - p) * rem / cus : 0);
+}
+
+// A tile of a wide kernel and the measured time of a full round of it: start-up and epilogue,
+// and each K step (ns). Both the choice of a tile and the choice between one launch for a batch
+// and one per activation are made by launch_ns().
+struct TileTime {
+  int variant, bm, bn, depth, round_ns, step_ns;
+};
+struct LaunchModel {
+  int start_ns, lone, last;  // of a launch; see rounds_permille()
+};
+inline int64_t launch_ns(const LaunchModel& m, const TileTime& t, int64_t tiles, int64_t cus, int64_t steps) {
+  return m.start_ns + rounds_permille(tiles, cus, m.lone, m.last) * (t.round_ns + t.step_ns * steps) / 1000;
 }
 
 // Workgroup id -> output tile. Workgroups are handed to the 8 XCDs round-robin

@@ -1690,10 +1690,16 @@ int launch_linear_fp8_skinny_fused(const GemmArgs& g, void* q_ws, float* scale_w
 
 struct TileChoice {
   int variant;
-  int64_t cost;  // 1000 x CUs x tile area per full round over the CUs (K left out)
+  int64_t ns;  // modelled time of the launch
 };
 template <class Tiles, class WideOk>
-TileChoice choose_bf16_variant(Tiles tiles, WideOk wide_ok);
+TileChoice choose_bf16_variant(Tiles tiles, WideOk wide_ok, int K);
+// The wide kernel's tiles, larger ones first, fitted to 2060 times of single GEMMs and of batches
+// with every tile (M 17 to 7000, K 640 to 15360, N 1024 to 12288; 11 % rms).
+constexpr LaunchModel kLaunch = {4600, 700, 760};
+constexpr TileTime kTiles[] = {{12, 256, 256, V12::DEPTH, 6400, 1227}, {14, 288, 192, V14::DEPTH, 4600, 1029},
+                               {15, 256, 192, V15::DEPTH, 4400, 946},  {16, 128, 192, V16::DEPTH, 3500, 552},
+                               {18, 128, 128, V18::DEPTH, 2100, 445},  {17, 64, 128, V17::DEPTH, 1300, 332}};
 int launch_gemm_fp8_ktail(const GemmArgs& g, int variant, hipStream_t stream);
 template <class WideOk>
 int launch_bf16_variant(const GemmArgs& g, int variant, WideOk wide_ok, hipStream_t stream);
@@ -1719,16 +1725,14 @@ int launch_gemm_fp8_stamps(const GemmArgs& g, unsigned long long* stamps, int* w
 template <class WideOk>
 int choose_other_out_variant(const GemmArgs& g, int variant, WideOk wide_ok) {
   const int64_t cus = cu_count() > 0 ? cu_count() : 256;
-  const struct { int v, bm, bn, us10, depth; } cand[] = {
-      {15, 256, 192, 245, V15::DEPTH}, {18, 128, 128, 145, V18::DEPTH}, {17, 64, 128, 110, V17::DEPTH}};
   int best = -1;
   int64_t time = INT64_MAX;
-  for (const auto& c : cand) {
-    if (!wide_ok(c.depth)) continue;
-    if (variant == c.v) return variant;
+  for (const auto& c : kTiles) {
+    if ((c.variant != 15 && c.variant != 18 && c.variant != 17) || !wide_ok(c.depth)) continue;
+    if (variant == c.variant) return variant;
     const int64_t tiles = (int64_t)((g.M + c.bm - 1) / c.bm) * ((g.N + c.bn - 1) / c.bn);
-    const int64_t t = rounds_time(tiles, cus, c.us10);
-    if (t < time) best = c.v, time = t;
+    const int64_t t = launch_ns(kLaunch, c, tiles, cus, g.K / BK);
+    if (t < time) best = c.variant, time = t;
   }
   return best;
 }
@@ -1782,7 +1786,7 @@ int launch_gemm_fp8(const GemmArgs& g, int variant, hipStream_t stream) {
   if (variant < 0) {
     variant = choose_bf16_variant(
         [&](int bm, int bn) { return (int64_t)((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn); },
-        wide_ok).variant;
+        wide_ok, g.K).variant;
   }
   return launch_bf16_variant(g, variant, wide_ok, stream);
 }
@@ -1808,7 +1812,7 @@ int launch_gemm_fp8_ktail(const GemmArgs& g, int variant, hipStream_t stream) {
   for (const auto& c : cand) {
     if (!bf16 && !c.other_out) continue;
     const int64_t tiles = (int64_t)((g.M + c.bm - 1) / c.bm) * ((g.N + c.bn - 1) / c.bn);
-    const int64_t t = variant == c.v ? -1 : rounds_time(tiles, cus, c.us10);
+    const int64_t t = variant == c.v ? -1 : rounds_permille(tiles, cus, 700, 700) * c.us10;
     if (t < time) best = c.v, time = t;
   }
   if (!bf16)
@@ -1824,54 +1828,46 @@ int launch_gemm_fp8_ktail(const GemmArgs& g, int variant, hipStream_t stream) {
 }
 
 // Tile choice for a bf16-output problem whose tile count for a bm x bn tile is tiles(bm, bn)
-// (a single GEMM, or a batch of GEMMs walked as one tile stream), with the modelled cost of
-// that choice; both branches count in the same unit.
+// (a single GEMM, or a batch of GEMMs walked as one tile stream), with the modelled time of
+// that choice.
 template <class Tiles, class WideOk>
-TileChoice choose_bf16_variant(Tiles tiles, WideOk wide_ok) {
+TileChoice choose_bf16_variant(Tiles tiles, WideOk wide_ok, int K) {
   // workgroups a round holds: one per CU (what launch_wide starts)
   const int64_t cus = cu_count() > 0 ? cu_count() : 256;
-  TileChoice best;
+  auto ns = [&](const TileTime& c) { return launch_ns(kLaunch, c, tiles(c.bm, c.bn), cus, K / BK); };
   if (tiles(256, 256) * 256 >= 160 * cus) {
     // Large problems take one of the large-tile wide kernels. Cost model, fitted to
     // measured times: tile area times the number of rounds over the CUs, where a
     // last, partial round of r tiles counts 0.4 + 0.6 r/CUs (the chip is power
     // limited: with fewer CUs busy the clocks rise); ties go to the larger tile.
-    auto cost = [&](int bm, int bn, int pen) {
-      const int64_t t = tiles(bm, bn), full = t / cus, rem = t % cus;
-      return (full * 10 * cus + (rem ? 4 * cus + 6 * rem : 0)) * bm * bn * pen;
+    auto cost = [&](const TileTime& c, int pen) {
+      const int64_t t = tiles(c.bm, c.bn), full = t / cus, rem = t % cus;
+      return (full * 10 * cus + (rem ? 4 * cus + 6 * rem : 0)) * c.bm * c.bn * pen;
     };
-    best = {12, cost(256, 256, 100)};
-    const struct { int v, bm, bn, pen; } cand[] = {
-        {14, 288, 192, 101}, {15, 256, 192, 102}};
-    for (const auto& c : cand) {
-      const int64_t t = cost(c.bm, c.bn, c.pen);
-      if (t < best.cost) best = {c.v, t};
+    int best = 0;
+    int64_t least = cost(kTiles[0], 100);
+    for (int i = 1; i <= 2; ++i) {
+      const int64_t t = cost(kTiles[i], 100 + i);
+      if (t < least) best = i, least = t;
     }
-  } else {
-    // Smaller problems (the text-stream Linears, M of a few hundred to a few thousand): the
-    // time of a round of each tile, as measured (`us10`: tenths of a us at K of about 2200; only
-    // the ratios count), times the rounds over the CUs, a last round of r tiles counting
-    // 0.7 + 0.3 r/CUs. A large tile costs far less per element than its area says -- its round is
-    // bound by the same LDS-DMA latency and start-up --, so two or three rounds of a small tile
-    // lose to one of a large one: 1357 x 2224 x 4464 32.8 us (128 x 128, two rounds) against
-    // 27.8 (256 x 192), 1800 x 3056 x 4400 67.4 (64 x 128, four) against 34.4 (256 x 192). One
-    // round of the small tiles is still the best where it is enough: 512 x 2224 x 4464 19.3
-    // (128 x 128) against 24.2 and 27.9, 1000 x 2992 x 2000 18.7 (64 x 128) against 21.5 and 35.0.
-    // Tiles whose prefetch depth K cannot feed are left out; ties go to the larger tile.
-    const struct { int v, bm, bn, us10, depth; } cand[] = {
-        {12, 256, 256, 310, 2}, {14, 288, 192, 270, 2}, {15, 256, 192, 245, 2},
-        {16, 128, 192, 180, 3}, {18, 128, 128, 145, 4}, {17, 64, 128, 110, 5}};
-    // K < 256: the kernels without a K stream across tiles (cost not modelled)
-    best = {tiles(128, 128) >= cus ? 6 : 21, INT64_MAX / 8};
-    int64_t time = INT64_MAX;
-    for (const auto& c : cand) {
-      if (!wide_ok(c.depth)) continue;
-      const int64_t t = rounds_time(tiles(c.bm, c.bn), cus, c.us10);
-      if (t >= time) continue;
-      time = t;
-      // in the unit of the large tiles (batches of activations of both kinds are compared)
-      best = {c.v, (tiles(c.bm, c.bn) + cus - 1) / cus * cus * c.bm * c.bn * 1000};
-    }
+    return {kTiles[best].variant, ns(kTiles[best])};
+  }
+  // Smaller problems (the text-stream Linears, M of a few hundred to a few thousand): the tile
+  // with the least modelled time; ties go to the larger tile. A large tile costs far less per
+  // element than its area says -- its round is bound by the same LDS-DMA latency and start-up --,
+  // so two or three rounds of a small tile lose to one of a large one: 1800 x 4416 x 3072
+  // (M x N x K) 32 us with 256 x 192 against 64 with 64 x 128 (four rounds), 666 x 11328 x 8192 71
+  // against 144, 604 x 9920 x 15360 123 against 142 with 128 x 128. One round of the small tiles
+  // is still the best where it is enough: 512 x 4480 x 2176 17 us with 128 x 128 against 22 with
+  // 256 x 192. Within 0.6 % of the best tile over 360 problems with K from 640 to 15360 (geometric
+  // mean; tile area times rounds, with a penalty per tile, was 6.4 % off). Tiles whose prefetch
+  // depth K cannot feed are left out.
+  // K < 384: the kernels without a K stream across tiles (time not modelled)
+  TileChoice best = {tiles(128, 128) >= cus ? 6 : 21, INT64_MAX / 1024};
+  for (const auto& c : kTiles) {
+    if (!wide_ok(c.depth)) continue;
+    const int64_t t = ns(c);
+    if (t < best.ns) best = {c.variant, t};
   }
   return best;
 }
@@ -1933,7 +1929,7 @@ int launch_gemm_fp8_grouped(const GemmArgs& common, const GemmGroup& grp, int va
     return t;
   };
   if (variant < 0) {
-    const TileChoice whole = choose_bf16_variant(tiles, wide_ok);
+    const TileChoice whole = choose_bf16_variant(tiles, wide_ok, common.K);
     variant = whole.variant;
     if (grp.acts > 1) {
       // One tile stream is not always the cheaper form: the tiles of a small activation
@@ -1941,22 +1937,21 @@ int launch_gemm_fp8_grouped(const GemmArgs& common, const GemmGroup& grp, int va
       // (FLUX ff.net.0.proj: 4096 rows fill three rounds of 256 x 256 tiles exactly, the
       // 512 text rows add a fourth, nearly empty one; on its own the text GEMM is one round
       // of small tiles: measured 148 us as two launches, 173 as one). Compare with one
-      // launch per activation, each with the tile it would choose, plus what a further
-      // launch costs (about 3 us, in the unit of the model: a CU does about 4900 K-steps of
-      // one output element per us).
-      const int64_t cus = cu_count() > 0 ? cu_count() : 256;
-      int64_t apart = (grp.acts - 1) * (3 * 1000 * cus * 4900 / (common.K > 0 ? common.K : 1));
+      // launch per activation, each with the tile it would choose; the time of each launch
+      // counts its start. Over 70 joint-block stages (image 1024 to 6889, text 33 to 512
+      // rows, widths 1536 to 3072) the form chosen is 0.4 % slower than the better one
+      // (geometric mean): 1184 + 59 rows, three members, K 2816: 36 us as one launch, 42 as two.
+      int64_t apart = 0;
       for (int s = 0; s < grp.acts; ++s) {
         auto tiles_s = [&](int bm, int bn) {
           int64_t cols = 0;
           for (int p = grp.first_member[s]; p < grp.first_member[s + 1]; ++p) cols += (grp.N[p] + bn - 1) / bn;
           return (int64_t)((grp.M[s] + bm - 1) / bm) * cols;
         };
-        apart += choose_bf16_variant(tiles_s, wide_ok).cost;
+        apart += choose_bf16_variant(tiles_s, wide_ok, common.K).ns;
       }
-      // (the model is good to a few per cent: within 3 % the single stream is kept, which
-      // measured faster in every such case)
-      if (apart * 100 < whole.cost * 97) {
+      // (within 2 % the single stream is kept)
+      if (apart * 100 < whole.ns * 98) {
         for (int s = 0; s < grp.acts; ++s) {
           GemmGroup one = {};
           one.acts = 1;

@@ -1350,45 +1350,46 @@ typedef CfgWW<128, 64, 4, 6> W12;           // wide: 64x32 wave tiles, DMA 6 ste
 namespace {
 struct TileChoice {
   int variant;
-  int64_t cost;  // 1000 x CUs x tile area per full round over the CUs (K left out)
+  int64_t ns;  // modelled time of the launch
 };
+// The wide kernel's tiles, larger ones first, fitted to 1190 times of single GEMMs and of batches
+// (M 17 to 7000, K 640 to 15360, N 1024 to 12288; 6 % rms).
+constexpr LaunchModel kLaunch = {5700, 600, 690};
+constexpr TileTime kTiles[] = {{7, 256, 256, W7::DEPTH, 4400, 1271}, {8, 256, 192, W8::DEPTH, 2400, 1007},
+                               {10, 128, 192, W10::DEPTH, 3000, 583}, {11, 128, 128, W11::DEPTH, 2000, 444},
+                               {12, 128, 64, W12::DEPTH, 1100, 297}};
 
 // Tile choice for a problem whose tile count for a bm x bn tile is tiles(bm, bn) (one GEMM,
-// or a batch walked as one tile stream). Same cost model as the w8a8 entry point: tile area
-// times rounds over the CUs (one persistent workgroup each), a last partial round of r tiles
-// counting 0.4 + 0.6 r/CUs; both branches count in the same unit.
+// or a batch walked as one tile stream), with the modelled time of that choice.
 template <class Tiles, class WideOk>
-TileChoice choose_variant(Tiles tiles, WideOk wide_ok) {
+TileChoice choose_variant(Tiles tiles, WideOk wide_ok, int K) {
   const int64_t cus = cu_count() > 0 ? cu_count() : 256;
+  auto ns = [&](const TileTime& c) {
+    return launch_ns(kLaunch, c, tiles(c.bm, c.bn), cus, (K + BKE - 1) / BKE);
+  };
   if (tiles(256, 256) * 256 >= 160 * cus && wide_ok(2)) {
+    // Large problems: tile area times rounds over the CUs (one persistent workgroup each), a
+    // last partial round of r tiles counting 0.4 + 0.6 r/CUs, as in the w8a8 entry point.
     auto cost = [&](int bm, int bn, int pen) {
       const int64_t t = tiles(bm, bn), full = t / cus, rem = t % cus;
       return (full * 10 * cus + (rem ? 4 * cus + 6 * rem : 0)) * bm * bn * pen;
     };
     // (256 x 192 against 256 x 256, measured: 0.98 at 4608 x 3072 x 12288, 0.955 at N = 15360,
     // 1.03 at 4096 x 3072 x 12288, 1.05 at N = 9216; a penalty of 2 % puts all four on the right side)
-    const int64_t c8 = cost(256, 192, 102), c7 = cost(256, 256, 100);
-    return c8 < c7 ? TileChoice{8, c8} : TileChoice{7, c7};
+    const TileTime& c = cost(256, 192, 102) < cost(256, 256, 100) ? kTiles[1] : kTiles[0];
+    return {c.variant, ns(c)};
   }
-  // Smaller problems: the time of a round of each tile, as measured (`us10`: tenths of a us at
-  // K of about 2200; only the ratios count), times the rounds over the CUs, as in the
-  // w8a8 entry point: 1357 x 2224 x 4464 47.6 us (128 x 128, two rounds) against 40.7
-  // (256 x 192); 512 x 2224 x 4464 27.1 (128 x 128) against 32.6, 34.7 and 40.4; 1000 x 2992 x
-  // 2000 27.6 (128 x 64) against 32.7. Ties go to the larger tile. Tiles whose prefetch depth K
-  // cannot feed are left out; without any wide tile (N not a multiple of 16, very short K) the
-  // 128x128 kernel runs.
-  const struct { int v, bm, bn, us10, depth; } cand[] = {
-      {7, 256, 256, 540, 2}, {8, 256, 192, 430, 2}, {10, 128, 192, 320, 4},
-      {11, 128, 128, 250, 5}, {12, 128, 64, 175, 6}};
-  TileChoice best = {3, INT64_MAX / 8};  // the 128x128 kernel takes what no wide tile can
-  int64_t time = INT64_MAX;
-  for (const auto& c : cand) {
+  // Smaller problems: the tile with the least modelled time, ties to the larger one, as in the
+  // w8a8 entry point: within 0.2 % of the best tile over 360 problems with K from 640 to 15360
+  // (geometric mean). 2084 x 3200 x 1024 (M x N x K): 18.8 us with 256 x 192, 24.1 with 128 x 128;
+  // 634 x 10176 x 8192 the other way round, 115 with 128 x 128 and 120; 512 x 4480 x 2176 27.1
+  // with 128 x 128 against 33 to 40. Tiles whose prefetch depth K cannot feed are left out; without any
+  // wide tile (N not a multiple of 16, very short K) the 128x128 kernel runs.
+  TileChoice best = {3, INT64_MAX / 1024};  // the 128x128 kernel takes what no wide tile can
+  for (const auto& c : kTiles) {
     if (!wide_ok(c.depth)) continue;
-    const int64_t t = rounds_time(tiles(c.bm, c.bn), cus, c.us10);
-    if (t >= time) continue;
-    time = t;
-    // in the unit of the large tiles (batches of activations of both kinds are compared)
-    best = {c.v, (tiles(c.bm, c.bn) + cus - 1) / cus * cus * c.bm * c.bn * 1000};
+    const int64_t t = ns(c);
+    if (t < best.ns) best = {c.variant, t};
   }
   return best;
 }
@@ -1439,7 +1440,7 @@ int launch_gemm_w8a16(const GemmArgs& g, int variant, hipStream_t stream) {
   if (variant < 0 || (k_tail && (variant < 7 || variant > 12))) {
     variant = choose_variant(
         [&](int bm, int bn) { return (int64_t)((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn); },
-        wide_ok).variant;
+        wide_ok, g.K).variant;
   }
   if (k_tail) {  // the KTAIL instances of the wide kernel take any K
     switch (variant) {
@@ -1502,24 +1503,23 @@ int launch_gemm_w8a16_grouped(const GemmArgs& common, const GemmGroup& grp, int 
     return t;
   };
   if (variant < 0) {
-    const TileChoice whole = choose_variant(tiles, wide_ok);
+    const TileChoice whole = choose_variant(tiles, wide_ok, common.K);
     variant = whole.variant;
     if (grp.acts > 1) {
       // one tile stream against one launch per activation, as in the w8a8 launcher: a small
       // activation can push a batch that filled whole rounds into one more, nearly empty one
-      // (a further launch costs about 3 us; a CU does about 2450 K elements of one output
-      // element per us at the bf16 rate)
-      const int64_t cus = cu_count() > 0 ? cu_count() : 256;
-      int64_t apart = (grp.acts - 1) * (3 * 1000 * cus * 2450 / (common.K > 0 ? common.K : 1));
+      // (over 70 joint-block stages 0.9 % slower than the better form; 1104 + 100 rows, three
+      // members, K 2816: 63 us as one launch, 71 as two)
+      int64_t apart = 0;
       for (int s = 0; s < grp.acts; ++s) {
         auto tiles_s = [&](int bm, int bn) {
           int64_t cols = 0;
           for (int p = grp.first_member[s]; p < grp.first_member[s + 1]; ++p) cols += (grp.N[p] + bn - 1) / bn;
           return (int64_t)((grp.M[s] + bm - 1) / bm) * cols;
         };
-        apart += choose_variant(tiles_s, wide_ok).cost;
+        apart += choose_variant(tiles_s, wide_ok, common.K).ns;
       }
-      if (apart * 100 < whole.cost * 97) {
+      if (apart * 100 < whole.ns * 98) {
         for (int s = 0; s < grp.acts; ++s) {
           GemmGroup one = {};
           one.acts = 1;
