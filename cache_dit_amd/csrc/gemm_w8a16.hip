@@ -1397,11 +1397,12 @@ TileChoice choose_variant(Tiles tiles, WideOk wide_ok, int K) {
 
 int launch_gemm_w8a16(const GemmArgs& g, int variant, hipStream_t stream) {
   const bool k_tail = !tiled_ok(g);  // K not a whole number of steps
-  if (!aligned_ok(g) || (k_tail && g.M > 16 && g.N % 16 != 0) || variant == 100) {
+  auto launch_generic = [&]() {
     dim3 grid((g.N + 15) / 16, (g.M + 15) / 16);
     hipLaunchKernelGGL(gemm_w8a16_generic, grid, dim3(256), 0, stream, g);
     return 0;
-  }
+  };
+  if (!aligned_ok(g) || variant == 100) return launch_generic();
   if ((variant < 0 || variant == 51) && g.M <= 4 && g.K <= 4096) {
     // (aligned_ok has checked the alignment of the operands and of lda and ldb)
     switch ((g.K + 1023) / 1024) {
@@ -1424,6 +1425,8 @@ int launch_gemm_w8a16(const GemmArgs& g, int variant, hipStream_t stream) {
     }
     return 0;
   }
+  // what is left of K remainders is for the wide kernel, which stores 16 columns per lane
+  if (k_tail && g.N % 16 != 0) return launch_generic();
   // the wide kernels stream K two or more steps ahead and store 16 columns per lane
   // at least `depth` K steps to prefetch, and at least 3: the epilogue operands of a tile are
   // staged in LDS two steps before its end, which must be behind the first barrier of the

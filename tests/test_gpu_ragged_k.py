@@ -161,3 +161,15 @@ def test_sums_keep_fp32(K):
     _expect(lambda out: ops.linear_w8a8_into(x, w, ones, None, out, q, s, 0, 0), exact, torch.bfloat16,
             ("linear", M, K))
     assert torch.equal(q.float(), x.float()) and bool((s == 1.0).all())
+
+
+@pytest.mark.parametrize("variant", [0, 3, 7, 8, 9, 10, 11, 12])
+@pytest.mark.parametrize("M", [2, 16, 17])
+def test_w8a16_tiles_need_whole_columns(variant, M):
+  """N a multiple of 8 and not of 16: no tile of the wide kernel may be taken, whatever M is and
+  whichever is asked for (a lane of it owns 16 columns)."""
+  from cache_dit_amd import _native, ops
+  _native.set_gemm_variant(variant)
+  for N, K in ((264, 112), (8, 48), (1288, 656)):
+    a, w, _, sw, b, exact = _problem(M, N, K, N + K + M, torch.bfloat16)
+    _check(lambda out: ops.w8a16_into(a, w, sw, b, out, 0), exact + b.double()[None, :], M, N, (variant, M, N, K))
