@@ -1098,7 +1098,7 @@ int launch_wavetile(const GemmArgs& g, hipStream_t stream) {
 }
 
 // ---------------------------------------------------------------------------
-// Skinny kernel for 4 < M <= 16, and for fewer rows at K > 4096: weight streaming. A
+// Skinny kernel for M <= 16 where the whole-row kernel below is not taken: weight streaming. A
 // workgroup of 4 waves owns 16 output channels, each wave a quarter of K. Per
 // 128-element chunk a lane (weight row l&15, K group l>>4) loads 32 e4m3 bytes
 // straight from HBM and the matching 32 bf16 activations (zero for rows >= M),
@@ -1190,7 +1190,7 @@ __global__ __launch_bounds__(256) void gemm_w8a16_skinny(GemmArgs g) {
 }
 
 // One to four activation rows (the modulation Linears: one embedding per image, with guidance
-// and a batch a few), K <= 4096, with the access pattern of the w8a8 path's linear_fp8_row1: a
+// and a batch a few), K <= 4096 (whole_rows_better() below), with the access pattern of the w8a8 path's linear_fp8_row1: a
 // load instruction of the wavefront reads 1 KiB of one weight row (lane l bytes 16 l ..
 // 16 l + 15) where the 16-row arrangement above makes every lane a memory request of its own;
 // the MFMA's 16 "rows" are 16 interleaved K subsets of that row, the activation is fetched at
@@ -1395,6 +1395,23 @@ TileChoice choose_variant(Tiles tiles, WideOk wide_ok, int K) {
 }
 }  // namespace
 
+namespace {
+// Whether the whole-row kernel is the better one for up to four activation rows (K <= 4096). It
+// works in pieces of 1 KiB of a weight row, and each activation row costs its share of a piece
+// whether the piece is full or not: with a single piece that is mostly empty, or a second one
+// that is, it loses to the 16-row kernel. Measured with a different weight matrix per launch (640
+// MB of them) over K 256 to 4096, N 768 to 18432, time against the 16-row kernel for M = 2 / 3 / 4:
+// K 3072, N 9216 0.75 / 0.80 / 0.85; K 1792, N 768 0.78 / 0.83 / 0.87; K 1024, N 4608 0.74 / 0.80 /
+// 0.83; K 768, N 2304 0.88 / 0.92 / 0.94; K 512, N 1536 1.09 / 1.15 / 1.16; K 1152, N 18432 1.01 /
+// 1.21 / 1.40, N 4608 0.92 / 1.00 / 1.03; K 1280, N 4608 0.85 / 0.92 / 0.97, N 768 1.01 / 1.08 / 1.12.
+bool whole_rows_better(const GemmArgs& g) {
+  // (the 16-row kernel masks its loads where K is not a multiple of 128)
+  if (g.M == 1 || g.K >= 1600 || (g.K >= (g.K % 128 ? 640 : 768) && g.K <= 1024)) return true;
+  if (g.K > 1024) return g.N >= 1536 && g.N <= 16384 && (g.M == 2 || (g.M == 3 && g.K >= 1280));
+  return g.M == 2 && g.N >= 4608 && g.K >= 320;
+}
+}  // namespace
+
 int launch_gemm_w8a16(const GemmArgs& g, int variant, hipStream_t stream) {
   const bool k_tail = !tiled_ok(g);  // K not a whole number of steps
   auto launch_generic = [&]() {
@@ -1403,7 +1420,7 @@ int launch_gemm_w8a16(const GemmArgs& g, int variant, hipStream_t stream) {
     return 0;
   };
   if (!aligned_ok(g) || variant == 100) return launch_generic();
-  if ((variant < 0 || variant == 51) && g.M <= 4 && g.K <= 4096) {
+  if (g.M <= 4 && g.K <= 4096 && (variant == 51 || (variant < 0 && whole_rows_better(g)))) {
     // (aligned_ok has checked the alignment of the operands and of lda and ldb)
     switch ((g.K + 1023) / 1024) {
       case 1: launch_rows_chk<1>(g, stream); break;

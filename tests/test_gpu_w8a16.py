@@ -524,3 +524,22 @@ def test_weight_only_sibling_groups_and_stream_batches_in_a_model():
     assert cache_dit.group_sibling_linears_(wan, lambda: wan(**winp)) == 2 * 2
     assert wan.blocks[0].attn1.to_q.sibling_group.weight_only
     assert torch.equal(wan(**winp), w0)
+
+
+@pytest.mark.parametrize("M", [1, 2, 3, 4])
+@pytest.mark.parametrize("N,K", [(24, 624), (24, 640), (24, 656), (24, 768), (24, 1024), (1528, 1040), (1536, 1040), (1536, 1264), (1536, 1280),
+                                 (16384, 1280), (16392, 1280), (24, 1584), (24, 1600), (4600, 320), (4608, 304),
+                                 (4608, 320)])
+def test_few_rows_kernels_at_the_edges_of_their_rule(M, N, K):
+  """On both sides of each limit between the whole-row kernel and the 16-row one: integer operands
+  through the one that is chosen and through either, bit-equal to the oracle."""
+  from cache_dit_amd import _native
+  g = torch.Generator().manual_seed(M + N + K)
+  x = torch.randint(-4, 5, (M, K), generator=g).to(torch.bfloat16)
+  w = torch.randint(-4, 5, (N, K), generator=g).float().to(FP8)
+  ws = torch.full((N, 1), 0.25)
+  ref = to.w8a16_linear(x, w, ws, fused=True)
+  for variant in (-1, 50, 51):
+    _native.set_gemm_variant(variant)
+    assert torch.equal(_run(x, w, ws, None).cpu(), ref), variant
+  _native.set_gemm_variant(-1)
