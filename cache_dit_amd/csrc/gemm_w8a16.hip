@@ -1430,7 +1430,13 @@ int launch_gemm_w8a16(const GemmArgs& g, int variant, hipStream_t stream) {
     }
     return 0;
   }
-  if ((variant < 0 && g.M <= 16) || variant == 50) {
+  // K remainders: the 16-row kernel masks its loads, and its time grows with the rows and the
+  // columns; from some 41,000 outputs on the wavefront-per-tile kernel below is the faster one.
+  // Another weight matrix per launch, us (16-row / wavefront tiles / 128 x 64 tiles of the wide
+  // kernel), M x N x K: 16 x 18432 x 3136 40.6 / 18.1 / 31.2, 8 x 9216 x 5056 25.8 / 19.0 / 23.6,
+  // 12 x 4608 x 1600 9.7 / 7.9 / 10.2, 4 x 9216 x 1360 7.8 / 7.9, 16 x 2304 x 3136 10.6 / 12.2 / 15.4.
+  const bool few_on_tiles = g.K % 128 != 0 && g.N % 16 == 0 && g.M <= 16 && (int64_t)g.M * g.N > 40960;
+  if ((variant < 0 && g.M <= 16 && !few_on_tiles) || variant == 50) {
     if (g.M > 16) {
       set_error("cdit_w8a16_gemm: the skinny kernel takes M <= 16");
       return CDIT_EINVAL;
@@ -1454,8 +1460,8 @@ int launch_gemm_w8a16(const GemmArgs& g, int variant, hipStream_t stream) {
   // Two 32 x 32 tiles per CU and less: the wavefront-per-tile kernel (figures at the kernel; at
   // three per CU it wins or loses with the shape, beyond that the CUs take a second round of it).
   if (g.N % 16 == 0 &&
-      (variant == 13 || (variant < 0 && (int64_t)((g.M + 31) / 32) * ((g.N + 31) / 32) <=
-                                            2 * (int64_t)(cu_count() > 0 ? cu_count() : 256))))
+      (variant == 13 || (variant < 0 && (few_on_tiles || (int64_t)((g.M + 31) / 32) * ((g.N + 31) / 32) <=
+                                                             2 * (int64_t)(cu_count() > 0 ? cu_count() : 256)))))
     return launch_wavetile(g, stream);
   if (variant < 0 || (k_tail && (variant < 7 || variant > 12))) {
     variant = choose_variant(

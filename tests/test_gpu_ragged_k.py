@@ -173,3 +173,15 @@ def test_w8a16_tiles_need_whole_columns(variant, M):
   for N, K in ((264, 112), (8, 48), (1288, 656)):
     a, w, _, sw, b, exact = _problem(M, N, K, N + K + M, torch.bfloat16)
     _check(lambda out: ops.w8a16_into(a, w, sw, b, out, 0), exact + b.double()[None, :], M, N, (variant, M, N, K))
+
+
+@pytest.mark.parametrize("M,N,K", [(16, 2560, 320), (16, 2576, 320), (16, 18432, 832), (5, 8192, 1600), (5, 8208, 1600),
+                                   (3, 13648, 1360), (3, 13664, 1360), (9, 4552, 112), (9, 4568, 112), (9, 4560, 112)])
+def test_w8a16_few_rows_on_both_sides_of_the_tile_rule(M, N, K):
+  """Up to 16 rows with a K remainder: the 16-row kernel up to 40960 outputs and where N is not a
+  multiple of 16, a wavefront per 32 x 32 tile beyond."""
+  from cache_dit_amd import _native, ops
+  a, w, _, sw, b, exact = _problem(M, N, K, N + K + M, torch.bfloat16)
+  for variant in (-1, 50, 13) if N % 16 == 0 else (-1, 50):
+    _native.set_gemm_variant(variant)
+    _check(lambda out: ops.w8a16_into(a, w, sw, b, out, 0), exact + b.double()[None, :], M, N, (variant, M, N, K))
