@@ -1200,9 +1200,8 @@ __global__ __launch_bounds__(256) void gemm_w8a16_skinny(GemmArgs g) {
 // MFMAs and a diagonal sum per weight row and no memory traffic to speak of.
 // With a different weight matrix per launch, against the 16-row kernel below 5 rows: 2 rows
 // 16.4 -> 14.2 us at N = 18432, K = 3072 (4.0 TB/s of weights), 8.2 -> 4.4 at 4096 x 1088;
-// 4 rows 18.3 -> 17.6 and, at N = 9216, 12.3 -> 9.9; one row is as before (12.0 and 7.5).
-// The activations are fetched inside the K loop: held across it they took the registers of
-// the wavefronts that keep the weight loads in flight.
+// 4 rows 18.3 -> 17.6 and, at N = 9216, 12.3 -> 9.9. One row has a body of its own: through the
+// one for several it took 1 to 4 % longer (4.39 -> 4.55 us at N = 960, K = 4096).
 constexpr int kRow1Rows = 3, kRow1Waves = 4;
 template <int CHK, int MA>
 __global__ __launch_bounds__(64 * kRow1Waves, MA == 1 ? 1 : (MA == 2 ? 6 : 4) - (CHK == 4 ? MA / 2 : 0)) void
@@ -1227,46 +1226,71 @@ gemm_w8a16_rows(GemmArgs g) {
     }
   }
   const v8bf zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
-  v4f_ acc[R][MA];
-#pragma unroll
-  for (int q = 0; q < R; ++q) {
-#pragma unroll
-    for (int m = 0; m < MA; ++m) acc[q][m] = v4f_{0.0f, 0.0f, 0.0f, 0.0f};
-  }
-#pragma unroll
-  for (int c = 0; c < CHK; ++c) {
-    v8bf xa[MA][2];
+  // 1 KiB piece c of activation row m
+  auto load_x = [&](v8bf (&x)[2], int m, int c) {
     const bool in = c * 1024 + lane * 16 < g.K;
+    const v8bf* src = reinterpret_cast<const v8bf*>(static_cast<const uint16_t*>(g.a) + m * g.lda +
+                                                    c * 1024 + lane * 16);
+    x[0] = in ? src[0] : zero8;
+    x[1] = in ? src[1] : zero8;
+  };
+  // lane l holds D[4 (l >> 4) + e][l & 15]: the diagonal entry of lanes 0-3, 20-23, 40-43, 60-63
+  const int diag = (lane & 15) - 4 * (lane >> 4);
+  float mine = 0.0f;  // lane q * MA + m keeps the dot product of weight row row0 + q, row m
+  auto keep_diagonal = [&](const v4f_& acc, int q, int m) {
+    float d = 0.0f;
 #pragma unroll
-    for (int m = 0; m < MA; ++m) {
-      const v8bf* src = reinterpret_cast<const v8bf*>(static_cast<const uint16_t*>(g.a) + m * g.lda +
-                                                      c * 1024 + lane * 16);
-      xa[m][0] = in ? src[0] : zero8;
-      xa[m][1] = in ? src[1] : zero8;
+    for (int e = 0; e < 4; ++e) d = diag == e ? acc[e] : d;
+    const float sum = wave_sum_f32(d);
+    mine = lane == q * MA + m ? sum : mine;
+  };
+  if constexpr (MA == 1) {
+    // one row: all of it is fetched right behind the weights, and a weight row's sum is under way
+    // while the next one's MFMAs run
+    v8bf xa[CHK][2];
+#pragma unroll
+    for (int c = 0; c < CHK; ++c) load_x(xa[c], 0, c);
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      v4f_ acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int c = 0; c < CHK; ++c) {
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+          acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(e4m3x8_to_bf16(w[q][c][2 * t], w[q][c][2 * t + 1]),
+                                                        xa[c][t], acc, 0, 0, 0);
+      }
+      keep_diagonal(acc, q, 0);
+    }
+  } else {
+    // (more rows: fetched inside the K loop; held across it they took the registers of the
+    // wavefronts that keep the weight loads in flight)
+    v4f_ acc[R][MA];
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+#pragma unroll
+      for (int m = 0; m < MA; ++m) acc[q][m] = v4f_{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+#pragma unroll
+    for (int c = 0; c < CHK; ++c) {
+      v8bf xa[MA][2];
+#pragma unroll
+      for (int m = 0; m < MA; ++m) load_x(xa[m], m, c);
+#pragma unroll
+      for (int q = 0; q < R; ++q) {
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          const v8bf wf = e4m3x8_to_bf16(w[q][c][2 * t], w[q][c][2 * t + 1]);
+#pragma unroll
+          for (int m = 0; m < MA; ++m)
+            acc[q][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf, xa[m][t], acc[q][m], 0, 0, 0);
+        }
+      }
     }
 #pragma unroll
     for (int q = 0; q < R; ++q) {
 #pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        const v8bf wf = e4m3x8_to_bf16(w[q][c][2 * t], w[q][c][2 * t + 1]);
-#pragma unroll
-        for (int m = 0; m < MA; ++m)
-          acc[q][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf, xa[m][t], acc[q][m], 0, 0, 0);
-      }
-    }
-  }
-  // lane l holds D[4 (l >> 4) + e][l & 15]: the diagonal entry of lanes 0-3, 20-23, 40-43, 60-63
-  const int diag = (lane & 15) - 4 * (lane >> 4);
-  float mine = 0.0f;  // lane q * MA + m keeps the dot product of weight row row0 + q, row m
-#pragma unroll
-  for (int q = 0; q < R; ++q) {
-#pragma unroll
-    for (int m = 0; m < MA; ++m) {
-      float d = 0.0f;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) d = diag == e ? acc[q][m][e] : d;
-      const float sum = wave_sum_f32(d);
-      mine = lane == q * MA + m ? sum : mine;
+      for (int m = 0; m < MA; ++m) keep_diagonal(acc[q][m], q, m);
     }
   }
   const int n = row0 + lane / MA, m = lane % MA;
