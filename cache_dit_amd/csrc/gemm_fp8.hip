@@ -1715,23 +1715,32 @@ int launch_gemm_fp8_stamps(const GemmArgs& g, unsigned long long* stamps, int* w
 }
 
 // The tile for fp16 and fp32 outputs: one large, one middle and one small tile are built for
-// them, chosen as the small bf16-output problems are (choose_bf16_variant). The middle one is
-// for a few hundred to a thousand rows, where the large tile leaves CUs idle and the small one
-// needs a second round.
-// fp16 at 1021 x 3072 x 3072: 25.1 us (64 x 128) -> 17.8 (128 x 128), 28.2 with 256 x 192;
-// 700 x 4096 x 3072 26.0 -> 17.2; fp32 at 256 x 12288 x 3072 31.0 -> 21.9; 4608 x 3072 x 3072,
-// fp16, 60.7 -> 51.0.
+// them, chosen by modelled time as the small bf16-output problems are (choose_bf16_variant). The
+// middle one is for a few hundred to a thousand rows, where the large tile leaves CUs idle and the
+// small one needs a second round.
+// fp16, M x N x K: 1021 x 3072 x 3072 25.1 us (64 x 128) -> 17.8 (128 x 128), 28.2 with 256 x 192;
+// 700 x 3072 x 4096 26.0 -> 17.2; 4608 x 3072 x 3072 60.7 -> 51.0.
+// fp32 outputs of short K are bound by their stores, which a large tile issues all at once behind
+// its last MFMA, the longer the less its rows are whole 64-byte pieces: up to K = 1024 that time
+// is added, per round's share of tiles. Within 0.6 % of the best tile over 590 problems of K 384 to
+// 12288 (0.9 % where N is not a multiple of 16; without the addition 1.6 and 4.1 %). M x N x K: 4751 x
+// 3576 x 768 36.2 us with 64 x 128 against 63.4 (256 x 192), 2848 x 8072 x 640 57.3 against 84.2,
+// 2970 x 2560 x 640 14.6 with 128 x 128 against 17.6; but 1180 x 3696 x 2176 22.1 with 256 x 192
+// against 24.9 and 30.3.
 // -1: K is too short for any of them.
 template <class WideOk>
 int choose_other_out_variant(const GemmArgs& g, int variant, WideOk wide_ok) {
   const int64_t cus = cu_count() > 0 ? cu_count() : 256;
   int best = -1;
   int64_t time = INT64_MAX;
+  const bool stores = g.out_dtype == CDIT_DT_F32 && g.K <= 1024, pieces = g.N % 16 == 0;
   for (const auto& c : kTiles) {
     if ((c.variant != 15 && c.variant != 18 && c.variant != 17) || !wide_ok(c.depth)) continue;
     if (variant == c.variant) return variant;
     const int64_t tiles = (int64_t)((g.M + c.bm - 1) / c.bm) * ((g.N + c.bn - 1) / c.bn);
-    const int64_t t = launch_ns(kLaunch, c, tiles, cus, g.K / BK);
+    int64_t t = launch_ns(kLaunch, c, tiles, cus, g.K / BK);
+    if (stores && c.variant == 15) t += tiles * (pieces ? 6000 : 12000) / cus;
+    if (stores && c.variant == 18 && !pieces) t += tiles * 2000 / cus;
     if (t < time) best = c.variant, time = t;
   }
   return best;
