@@ -185,3 +185,41 @@ def test_w8a16_few_rows_on_both_sides_of_the_tile_rule(M, N, K):
   for variant in (-1, 50, 13) if N % 16 == 0 else (-1, 50):
     _native.set_gemm_variant(variant)
     _check(lambda out: ops.w8a16_into(a, w, sw, b, out, 0), exact + b.double()[None, :], M, N, (variant, M, N, K))
+
+
+def _second_tiles(variant, tiles, M, N):
+  bm, bn = tiles[variant]
+  return -(-M // bm) * -(-N // bn) > torch.cuda.get_device_properties(0).multi_processor_count
+
+
+@pytest.mark.parametrize("variant,M,N", [(14, 4700, 4112), (15, 4700, 4112), (16, 2500, 2680), (18, 2100, 2096),
+                                         (17, 2100, 1808)])
+@pytest.mark.parametrize("K", [48, 240, 656])
+def test_w8a8_workgroups_take_a_second_tile(variant, M, N, K):
+  """More tiles than CUs: the persistent workgroup goes on to another tile, with K below and above
+  the prefetch depth (the next tile's first steps are fetched during this one's last, padded
+  ones)."""
+  from cache_dit_amd import _native, ops
+  assert _second_tiles(variant, {14: (288, 192), 15: (256, 192), 16: (128, 192), 18: (128, 128), 17: (64, 128)}, M, N)
+  _native.set_gemm_variant(variant)
+  a, w, sa, sw, b, exact = _problem(M, N, K, K + variant, FP8)
+  exact *= sa.double()[:, None]
+  _check(lambda out: ops.gemm_rowwise_into(a, sa, w, sw, b, out, 0), exact + b.double()[None, :], M, N, (variant, K))
+  if variant in (15, 17, 18):
+    for dtype in (torch.float16, torch.float32):
+      out = torch.empty((M, N), dtype=dtype, device=DEV)
+      ops.gemm_rowwise_into(a, sa, w, sw, None, out, 0)
+      torch.cuda.synchronize()
+      assert torch.equal(out, exact.float().to(dtype)), (dtype, variant, K)
+
+
+@pytest.mark.parametrize("variant,M,N", [(7, 4700, 4112), (8, 4700, 4112), (9, 4700, 4112), (10, 2500, 2688),
+                                         (11, 2100, 2112), (12, 2100, 1808)])
+@pytest.mark.parametrize("K", [48, 240, 656])
+def test_w8a16_workgroups_take_a_second_tile(variant, M, N, K):
+  from cache_dit_amd import _native, ops
+  tiles = {7: (256, 256), 8: (256, 192), 9: (192, 256), 10: (128, 192), 11: (128, 128), 12: (128, 64)}
+  assert _second_tiles(variant, tiles, M, N)
+  _native.set_gemm_variant(variant)
+  a, w, _, sw, b, exact = _problem(M, N, K, K + variant, torch.bfloat16)
+  _check(lambda out: ops.w8a16_into(a, w, sw, b, out, 0), exact + b.double()[None, :], M, N, (variant, K))
