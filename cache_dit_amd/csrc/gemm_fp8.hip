@@ -6,7 +6,8 @@
 // Both operands are K-contiguous ("NT" GEMM), which is what the MFMA operand
 // registers want: per lane, 32 consecutive K bytes of one row. The production kernel
 // (gemm_fp8_wide) issues v_mfma_f32_16x16x128_f8f6f4: row lane&15, 32-byte K group
-// lane>>4 of a 128-byte K step; the older tiled kernel v_mfma_f32_32x32x64_f8f6f4: row
+// lane>>4 of a 128-byte K step (K remainders four v_mfma_f32_16x16x32_bf16 on the converted
+// bytes, see mfma_codes_as_bf16); the older tiled kernel v_mfma_f32_32x32x64_f8f6f4: row
 // lane&31, K half lane>>5 of a 64-byte step.
 //
 // Kernels in this file: gemm_fp8_wide (persistent, one wave per SIMD, the one every
@@ -386,6 +387,16 @@ struct CfgWide {
   static constexpr int slot_b(int j) { return (j + 1) * R + 1 < S2 ? (j + 1) * R + 1 : S2; }
   static constexpr int slot_a0 = S2 > 1 ? 1 : 0;
   static constexpr int slot_dma2(int p) { return (2 * p + 1) * S2 / (2 * NDB); }
+  // The instances for K remainders (row-major in the second half too, where every raw B fragment is
+  // free from the start) read B_j of the next step in front of the last row, which converts them.
+  static constexpr int slot_b_ktail(int j) { return j * (S2 - TN) / TN; }
+  // When half h of B operand k = q TN + j is converted: slots of the last row of a step (0 .. 4 TN - 1)
+  // and of the first row of the next (from 4 TN on, used at 4 TN + k). Not before its registers are
+  // free (slot k) and, with a second half of one row, the fragment has arrived; four MFMAs ahead.
+  static constexpr int ktail_b_time(int k, int h) {
+    const int t = 2 * k + h + (R > 1 ? 2 : 5), last = 4 * TN + k - 4;
+    return t < last ? t : last;
+  }
 };
 
 __device__ __forceinline__ int swz_a(int row) { return ((row >> 1) & 1) | (((row >> 3) & 1) * 6); }
@@ -427,11 +438,23 @@ __device__ __forceinline__ CodesBf16 codes_to_bf16(const v8i& c) {
   for (int q = 0; q < 4; ++q) f.k[q] = e4m3x8_to_bf16((uint32_t)c[2 * q], (uint32_t)c[2 * q + 1]);
   return f;
 }
+// (for the kernels whose MFMAs are builtins)
 __device__ __forceinline__ v4f mfma_codes_as_bf16(const v8i& b, const v8i& a, v4f acc) {
   const CodesBf16 bb = codes_to_bf16(b), aa = codes_to_bf16(a);
 #pragma unroll
   for (int q = 0; q < 4; ++q) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bb.k[q], aa.k[q], acc, 0, 0, 0);
   return acc;
+}
+
+// acc (+)= B-operand x A-operand, as mfma_16x16x128_fp8 and with the same obligations; neither
+// operand may have been written by one of the last four instructions.
+template <bool FIRST>
+__device__ __forceinline__ void mfma_16x16x32_bf16(v4f& acc, const v8bf& b, const v8bf& a) {
+  if constexpr (FIRST) {
+    asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=a"(acc) : "v"(b), "v"(a));
+  } else {
+    asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(b), "v"(a));
+  }
 }
 
 // A batch of GEMMs as one launch (GemmGroup, declared with the launchers): sibling Linears
@@ -672,7 +695,35 @@ gemm_fp8_wide(GemmArgs g, int tiles_m, int tiles_n,
 
   v4f acc[TM][TN];
   v8i af[TM], bf[TN];
-  CodesBf16 bw[KTAIL ? TN : 1];  // KTAIL: this step's B operands as bf16
+  // KTAIL: this step's B and this row's A operands as bf16; operand (j, q) is B fragment j, k group q
+  uint4 bw[KTAIL ? TN : 1][4], aw[4];
+  // Two e4m3 codes of a word. Inline assembly (volatile): as builtins, pure functions of loaded
+  // values, the compiler moved conversions across branches up to the MFMA that uses them.
+  auto cvt2 = [](int word, bool high) -> uint32_t {
+    uint32_t v;
+    if (high) {
+      asm volatile("v_cvt_scalef32_pk_bf16_fp8 %0, %1, 1.0 op_sel:[1,0,0]" : "=v"(v) : "v"(word));
+    } else {
+      asm volatile("v_cvt_scalef32_pk_bf16_fp8 %0, %1, 1.0" : "=v"(v) : "v"(word));
+    }
+    return v;
+  };
+  auto convert_a = [&](int i, int q, int c) {  // elements 2c and 2c + 1 of A operand q of row i
+    const uint32_t v = cvt2(af[i][2 * q + (c >> 1)], c & 1);
+    (c == 0 ? aw[q].x : c == 1 ? aw[q].y : c == 2 ? aw[q].z : aw[q].w) = v;
+  };
+  auto convert_b = [&](int j, int q, int h) {  // half h of operand (j, q)
+    const uint32_t lo = cvt2(bf[j][2 * q + h], false), hi = cvt2(bf[j][2 * q + h], true);
+    (h ? bw[j][q].z : bw[j][q].x) = lo;
+    (h ? bw[j][q].w : bw[j][q].y) = hi;
+  };
+  auto convert_b_at = [&](int t) {  // what the schedule puts at time t (CfgWide::ktail_b_time)
+#pragma unroll
+    for (int k = 0; k < 4 * TN; ++k)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        if (C::ktail_b_time(k, h) == t) convert_b(k % TN, k / TN, h);
+  };
 
   // LDS offsets of the stages of steps kt-1 / kt / kt+1 (A) and kt / kt+1 (B);
   // step s lives in A stage s mod (D+1) and B stage s mod D
@@ -698,6 +749,13 @@ gemm_fp8_wide(GemmArgs g, int tiles_m, int tiles_n,
 #pragma unroll
     for (int j = 0; j < TN; ++j) bf[j] = read_b(smem + b_cur, j);
     af[0] = read_a(smem + a_cur, 0);
+    if constexpr (KTAIL) {  // what the last row of the step before converts otherwise (row_as_bf16)
+#pragma unroll
+      for (int c = 0; c < 6; ++c) convert_a(0, c >> 2, c & 3);
+#pragma unroll
+      for (int t = 0; t < 4 * TN; ++t) convert_b_at(t);
+      __builtin_amdgcn_sched_barrier(0);
+    }
     // epilogue operands of this tile, fetched two steps before they are needed:
     // acc[i][4t+q][e] is out[m][n] with
     //   m = m0 + wm*WM + 16i + (lane&15),
@@ -708,22 +766,33 @@ gemm_fp8_wide(GemmArgs g, int tiles_m, int tiles_n,
     float as[TM];
 
     // KTAIL: row i of blocks on the bf16 instruction, four MFMAs per block, a k group of all its
-    // blocks before the next (consecutive MFMAs are independent); items(b) is what the schedule
-    // puts in front of block b of the row. Row 0 converts the step's B operands on the way, so
-    // that every raw B fragment is free in the second half. Builtins: the compiler places the
-    // conversions and knows the wait states between them and the MFMAs.
+    // blocks before the next: slot s = q TN + j; items(b) is what the schedule puts in front of block
+    // b of the row. Between two MFMAs (4 passes, 16 clocks) about one conversion (8 clocks) is free,
+    // so they are spread: A operand q + 1 of a row one conversion per slot from two slots before
+    // group q on (group 0 of the next row from group 3 of this), half a B operand of the next step
+    // per slot through the last row of this step and the first of the next. Every operand is
+    // complete four MFMAs before its use. In the last step of a tile what is converted for a next
+    // one is of no use; the next tile starts with its own.
     auto row_as_bf16 = [&](int i, auto first_tag, auto items) {
       constexpr bool FIRST = decltype(first_tag)::value;
-      const CodesBf16 a = codes_to_bf16(af[i]);
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
-          if ((q * TN + j) % 4 == 0) items((q * TN + j) / 4);
-          if (i == 0) bw[j].k[q] = e4m3x8_to_bf16((uint32_t)bf[j][2 * q], (uint32_t)bf[j][2 * q + 1]);
-          v4f c = acc[i][j];
-          if (FIRST && q == 0) c = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bw[j].k[q], a.k[q], c, 0, 0, 0);
+          const int s = q * TN + j;
+          if (s % 4 == 0) items(s / 4);
+          const int ahead = (s + 2) / TN + 1;  // k group of this row (4, 5: of the next one)
+          if ((s + 2) % TN < 4) convert_a(ahead < 4 ? i : (i + 1) % TM, ahead & 3, (s + 2) % TN);
+          if (i == TM - 1) convert_b_at(s);
+          if (i == 0) convert_b_at(4 * TN + s);
+          __builtin_amdgcn_sched_barrier(0);
+          const v8bf b = __builtin_bit_cast(v8bf, bw[j][q]), a = __builtin_bit_cast(v8bf, aw[q]);
+          if (FIRST && q == 0) {
+            mfma_16x16x32_bf16<true>(acc[i][j], b, a);
+          } else {
+            mfma_16x16x32_bf16<false>(acc[i][j], b, a);
+          }
+          __builtin_amdgcn_sched_barrier(0);
         }
       }
     };
@@ -844,7 +913,7 @@ gemm_fp8_wide(GemmArgs g, int tiles_m, int tiles_n,
         if (sl == C::slot_a0) af[0] = read_a(smem + a_next, 0);
 #pragma unroll
         for (int j = 0; j < TN; ++j)
-          if (C::slot_b(j) == sl) bf[j] = read_b(smem + b_next, j);
+          if ((KTAIL ? C::slot_b_ktail(j) : C::slot_b(j)) == sl) bf[j] = read_b(smem + b_next, j);
 #pragma unroll
         for (int p = 0; p < C::NDB; ++p)
           if (C::slot_dma2(p) == sl) dma_b(kd, b_cur, p);
@@ -1558,7 +1627,8 @@ __global__ __launch_bounds__(64 * kRow1Waves) void linear_fp8_row1(GemmArgs g, u
 
 // Any shape, any alignment: a 16x16 output tile per workgroup, one output
 // element per thread, scalar decode + FMA. Only for what the other kernels cannot take
-// (N not a multiple of 8, odd strides, misaligned operands).
+// (N not a multiple of 8, odd strides, misaligned operands; fp16 and fp32 outputs with K = 128
+// or 256 and M > 16).
 __global__ __launch_bounds__(256) void gemm_fp8_generic(GemmArgs g) {
   const int n = blockIdx.x * 16 + (threadIdx.x & 15);
   const int m = blockIdx.y * 16 + (threadIdx.x >> 4);
@@ -1804,10 +1874,10 @@ int launch_gemm_fp8(const GemmArgs& g, int variant, hipStream_t stream) {
 // kernel, which take any K. They run at the rate of the bf16 instruction and convert the codes,
 // so a round of a tile takes longer than that of the FP8 instances and grows more with its area;
 // the tile is chosen by their own round times (tenths of a us at K of about 2200; only the ratios
-// count). Within 0.1 % of the best tile over 90 shapes of M 17 to 6889, K 272 to 12288, N 272 to
-// 4592 (geometric mean; the worst 9 % off). 1357 x 4464 x 2224 (M x N x K): 38.9 us with 128 x 128
-// against 42.0 (256 x 192) and 50.4 (128 x 192); 256 x 3072 x 2992: 19.8 with 64 x 128 against
-// 24.8 (128 x 128); 4608 x 3072 x 3056: 68.5 with 288 x 192 against 87.6 (128 x 128) and 100.4
+// count). Within 0.2 % of the best tile over 90 shapes of M 17 to 6889, K 272 to 12288, N 272 to
+// 4592 (geometric mean; the worst 9 % off). 1357 x 4464 x 2224 (M x N x K): 40.6 us with 128 x 128
+// against 42.2 (256 x 192) and 50.4 (128 x 192); 256 x 3072 x 2992: 20.5 with 64 x 128 against
+// 26.2 (128 x 128); 4608 x 3072 x 3056: 69.8 with 288 x 192 against 92.9 (128 x 128) and 99.7
 // (256 x 192). The scalar FMA kernel took 16.8 ms for the first. There is no 256 x 256 instance:
 // its converted operands do not fit the registers. fp16 and fp32 outputs have three tiles.
 int launch_gemm_fp8_ktail(const GemmArgs& g, int variant, hipStream_t stream) {

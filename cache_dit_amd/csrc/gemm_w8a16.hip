@@ -948,7 +948,7 @@ int launch_wide_grouped(const GemmArgs& g, GemmGroup grp, hipStream_t stream) {
 // wide kernel, so the results are bit-identical to it (a member of a batch may run there).
 // What bounds it: a chain of four dependent MFMAs (128 clocks) and six DMA instructions per step.
 // One wavefront issues all of it in order: about 500 clocks per step.
-// Another weight matrix per launch, against 128 x 64 tiles: 77 x 4096 x 3072 22.1 -> 16.1 us,
+// Another weight matrix per launch (M x K x N), against 128 x 64 tiles: 77 x 4096 x 3072 22.1 -> 16.1 us,
 // 17 x 3072 x 3072 15.3 -> 12.1, 128 x 3072 x 3072 20.4 -> 13.2, 256 x 3072 x 1536 19.8 -> 12.9,
 // 512 x 4096 x 1024 20.4 -> 15.6, 32 x 3072 x 12288 18.3 -> 17.3; with 672 tiles
 // (200 x 4096 x 3072) 21.5 -> 22.2 and with 864 (77 x 3072 x 9216) 19.6 -> 29.9: not taken.
