@@ -429,25 +429,18 @@ __device__ __forceinline__ void mfma_16x16x128_fp8(v4f& acc, const v8i& b, const
 // mixed magnitudes. The bf16 instruction on the converted codes is 6.2e-8 and 1.5e-7 off, an
 // fp32 FMA per product (gemm_fp8_generic, the only other kernel that takes such a K) 6.4e-8 and
 // 1.6e-7; the same order from K = 128 to 15360.
-struct CodesBf16 {
-  v8bf k[4];
-};
-__device__ __forceinline__ CodesBf16 codes_to_bf16(const v8i& c) {
-  CodesBf16 f;
-#pragma unroll
-  for (int q = 0; q < 4; ++q) f.k[q] = e4m3x8_to_bf16((uint32_t)c[2 * q], (uint32_t)c[2 * q + 1]);
-  return f;
-}
-// (for the kernels whose MFMAs are builtins)
+// (This form is for the kernels whose MFMAs are builtins.)
 __device__ __forceinline__ v4f mfma_codes_as_bf16(const v8i& b, const v8i& a, v4f acc) {
-  const CodesBf16 bb = codes_to_bf16(b), aa = codes_to_bf16(a);
 #pragma unroll
-  for (int q = 0; q < 4; ++q) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bb.k[q], aa.k[q], acc, 0, 0, 0);
+  for (int q = 0; q < 4; ++q)
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(e4m3x8_to_bf16((uint32_t)b[2 * q], (uint32_t)b[2 * q + 1]),
+                                                  e4m3x8_to_bf16((uint32_t)a[2 * q], (uint32_t)a[2 * q + 1]),
+                                                  acc, 0, 0, 0);
   return acc;
 }
 
-// acc (+)= B-operand x A-operand, as mfma_16x16x128_fp8 and with the same obligations; neither
-// operand may have been written by one of the last four instructions.
+// The same for the wide kernel: acc (+)= B-operand x A-operand, as mfma_16x16x128_fp8 and with the
+// same obligations; neither operand may have been written by one of the last four instructions.
 template <bool FIRST>
 __device__ __forceinline__ void mfma_16x16x32_bf16(v4f& acc, const v8bf& b, const v8bf& a) {
   if constexpr (FIRST) {
@@ -482,8 +475,8 @@ struct NoGroup {};
 // which the last ones are all zeros. The chunk a lane fetches is the same for every DMA
 // instruction of a panel (swz_a / swz_b take the row bits that the lane and the parity of the
 // wave give), so a step costs one comparison per panel and one OR per DMA instruction.
-// These instances multiply on the bf16 matrix instruction (mfma_codes_as_bf16): such a K has
-// its sums in full fp32, which the FP8 instruction's are not.
+// These instances multiply on the bf16 matrix instruction (mfma_codes_as_bf16, row_as_bf16): such
+// a K has its sums in full fp32, which the FP8 instruction's are not.
 struct StampArgs {
   unsigned long long* stamps;
 };

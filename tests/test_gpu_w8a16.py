@@ -128,8 +128,9 @@ def test_one_row_kernel_exact_and_k_positions(N, K):
 @pytest.mark.parametrize("M", [2, 3, 4])
 @pytest.mark.parametrize("N,K", [(18432, 3072), (1008, 2048), (24, 16), (6160, 4096), (528, 1152), (272, 3968)])
 def test_few_rows_kernel(M, N, K):
-  """M = 2 to 4 with K <= 4096 runs the whole-row kernel too: integer operands bit-equal to the
-  oracle (every sum is exact in any order), random ones with GELU within the tolerance."""
+  """M = 2 to 4 with K <= 4096, through the kernel that is chosen, the 16-row and the whole-row one:
+  integer operands bit-equal to the oracle (every sum is exact in any order), random ones with
+  GELU within the tolerance."""
   from cache_dit_amd import _native
   g = torch.Generator().manual_seed(M + N + K)
   x = torch.randint(-4, 5, (M, K), generator=g).to(torch.bfloat16)
@@ -137,12 +138,14 @@ def test_few_rows_kernel(M, N, K):
   ws = torch.full((N, 1), 0.25)
   auto = _run(x, w, ws, None).cpu()
   assert torch.equal(auto, to.w8a16_linear(x, w, ws, fused=True))
-  _native.set_gemm_variant(50)
-  assert torch.equal(_run(x, w, ws, None).cpu(), auto)
-  _native.set_gemm_variant(-1)
+  for variant in (50, 51):
+    _native.set_gemm_variant(variant)
+    assert torch.equal(_run(x, w, ws, None).cpu(), auto)
   x, wq, ws, b = _problem(M, N, K, seed=M * 7 + N + K)
   ref = to.w8a16_linear(x, wq, ws * 8, b, gelu="fused", fused=True)
-  _assert_close(_run(x, wq, ws * 8, b, epilogue=1), ref)
+  for variant in (-1, 51):
+    _native.set_gemm_variant(variant)
+    _assert_close(_run(x, wq, ws * 8, b, epilogue=1), ref)
 
 
 @pytest.mark.parametrize("M,N,K", [(17, 16, 16), (32, 32, 64), (33, 48, 128), (77, 3072, 4096), (64, 272, 448),
