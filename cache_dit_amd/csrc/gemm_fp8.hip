@@ -1685,6 +1685,7 @@ typedef CfgWide<256, 192, 4> V15;                     // ... 128x96 wave tiles
 typedef CfgWide<128, 192, 4, 3> V16;                  // ... 64x96 wave tiles, DMA 3 steps ahead
 typedef CfgWide<64, 128, 8, 5> V17;                   // ... 32x64 wave tiles, DMA 5 steps ahead
 typedef CfgWide<128, 128, 4, 4> V18;                  // ... 64x64 wave tiles, DMA 4 steps ahead
+typedef CfgWide<256, 128, 4> V19;                     // ... 128x64 wave tiles, for K remainders only
 // the two large tiles with contiguous wave columns and half-line output stores (16 rows x 64
 // bytes per store instruction), kept to measure the whole-line stores against: variants 112, 114
 typedef CfgWide<256, 256, 4, 2, false> V12H;
@@ -1867,17 +1868,22 @@ int launch_gemm_fp8(const GemmArgs& g, int variant, hipStream_t stream) {
 // kernel, which take any K. They run at the rate of the bf16 instruction and convert the codes,
 // so a round of a tile takes longer than that of the FP8 instances and grows more with its area;
 // the tile is chosen by their own round times (tenths of a us at K of about 2200; only the ratios
-// count). Within 0.2 % of the best tile over 90 shapes of M 17 to 6889, K 272 to 12288, N 272 to
-// 4592 (geometric mean; the worst 9 % off). 1357 x 4464 x 2224 (M x N x K): 40.6 us with 128 x 128
-// against 42.2 (256 x 192) and 50.4 (128 x 192); 256 x 3072 x 2992: 20.5 with 64 x 128 against
-// 26.2 (128 x 128); 4608 x 3072 x 3056: 69.8 with 288 x 192 against 92.9 (128 x 128) and 99.7
-// (256 x 192). The scalar FMA kernel took 16.8 ms for the first. There is no 256 x 256 instance:
-// its converted operands do not fit the registers. fp16 and fp32 outputs have three tiles.
+// count). Within 0.2 % of the best tile over 110 shapes of M 300 to 6889, K 272 to 3056, N 1024 to
+// 9000 (geometric mean; the worst 5 % off). A wavefront converts the operands of its own tile, so
+// a step of 256 x 128 (wave tile 128 x 64: 1.5 conversions of 8 clocks per MFMA of 16) takes 1.45
+// times one of 128 x 128 (2 per MFMA) and does twice the work: the tile for problems that are more
+// than one round of 128 x 128 and less than one of the larger tiles (without it the choice was
+// 1.2 % off the best, the worst 39 %). 1357 x 4464 x 2224 (M x N x K): 35.6 us with 256 x 128
+// against 43.1 (128 x 128, two rounds), 44.5 (256 x 192) and 52.1 (128 x 192); 256 x 3072 x 2992:
+// 20.7 with 64 x 128 against 27.5 (128 x 128); 4608 x 3072 x 3056: 64.4 with 288 x 192 against
+// 75.1 (256 x 128) and 93.8 (128 x 128). The scalar FMA kernel took 16.8 ms for the first. There is
+// no 256 x 256 instance: its converted operands do not fit the registers. fp16 and fp32 outputs
+// have three tiles.
 int launch_gemm_fp8_ktail(const GemmArgs& g, int variant, hipStream_t stream) {
   const int64_t cus = cu_count() > 0 ? cu_count() : 256;
   const struct { int v, bm, bn, us10; bool other_out; } cand[] = {
       {14, 288, 192, 530, false}, {15, 256, 192, 470, true}, {16, 128, 192, 290, false},
-      {18, 128, 128, 205, true}, {17, 64, 128, 150, true}};
+      {19, 256, 128, 310, false}, {18, 128, 128, 205, true}, {17, 64, 128, 150, true}};
   const bool bf16 = g.out_dtype == CDIT_DT_BF16;
   int best = 18;
   int64_t time = INT64_MAX;
@@ -1895,6 +1901,7 @@ int launch_gemm_fp8_ktail(const GemmArgs& g, int variant, hipStream_t stream) {
     case 15: return launch_wide<V15, CDIT_DT_BF16, true>(g, stream);
     case 16: return launch_wide<V16, CDIT_DT_BF16, true>(g, stream);
     case 17: return launch_wide<V17, CDIT_DT_BF16, true>(g, stream);
+    case 19: return launch_wide<V19, CDIT_DT_BF16, true>(g, stream);
     default: return launch_wide<V18, CDIT_DT_BF16, true>(g, stream);
   }
 }

@@ -223,3 +223,22 @@ def test_w8a16_workgroups_take_a_second_tile(variant, M, N, K):
   _native.set_gemm_variant(variant)
   a, w, _, sw, b, exact = _problem(M, N, K, K + variant, torch.bfloat16)
   _check(lambda out: ops.w8a16_into(a, w, sw, b, out, 0), exact + b.double()[None, :], M, N, (variant, K))
+
+
+@pytest.mark.parametrize("M,N", [(17, 72), (255, 128), (257, 136), (577, 400), (2100, 4112)])
+@pytest.mark.parametrize("K", [16, 112, 240, 272, 656, 2224])
+def test_w8a8_tile_of_256_by_128(M, N, K):
+  """Edges of the tile, one and two tiles per workgroup (2100 x 4112: 297), K below and above the
+  prefetch depth: the exact result, and the bits of the 128 x 128 tile with a GELU epilogue."""
+  from cache_dit_amd import _native, ops
+  a, w, sa, sw, b, exact = _problem(M, N, K, N + K + M, FP8)
+  _native.set_gemm_variant(19)
+  _check(lambda out: ops.gemm_rowwise_into(a, sa, w, sw, b, out, 0),
+         exact * sa.double()[:, None] + b.double()[None, :], M, N, (M, N, K))
+  outs = []
+  for variant in (19, 18):
+    _native.set_gemm_variant(variant)
+    outs.append(torch.empty((M, N), dtype=torch.bfloat16, device=DEV))
+    ops.gemm_rowwise_into(a, sa, w, sw, b, outs[-1], 1)
+  torch.cuda.synchronize()
+  assert torch.equal(outs[0], outs[1]), (M, N, K)
