@@ -1,4 +1,5 @@
-"""ctypes binding of libcdit_hip.so (C ABI declared in include/cdit_hip.h).
+"""ctypes binding of libcdit_hip.so (C ABI declared in include/cdit_hip.h), and the Python
+extension `_cdit_host.so` (csrc/host_ext.cpp) through which the operators call it.
 
 The library is loaded lazily, on the first call that needs it, and only after
 `torch` has been imported so that it binds to the HIP runtime PyTorch already
@@ -15,6 +16,7 @@ import torch  # noqa: F401  (must be imported before the library is loaded)
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "lib", "libcdit_hip.so")
+HOST_PATH = os.path.join(_HERE, "lib", "_cdit_host.so")
 ABI_VERSION = 1
 
 SCALE_MODE_IDS = {"bf16div": 0, "fp32div": 1}
@@ -55,6 +57,7 @@ EXPORTS = (
 )
 
 _lib = None
+_host = None
 _lock = threading.Lock()
 
 
@@ -150,8 +153,30 @@ def load(path: str | None = None) -> ctypes.CDLL:
   return _lib
 
 
+def host():
+  """The Python extension, loaded once and bound to the library that load() gives."""
+  global _host
+  if _host is None:
+    lib = load()
+    with _lock:
+      if _host is None:
+        if not os.path.exists(HOST_PATH):
+          raise CditNativeError(
+              f"{HOST_PATH} not found: build it with `python -m cache_dit_amd.csrc.build`. "
+              "There is no fallback path.")
+        import importlib.machinery
+        import importlib.util
+        loader = importlib.machinery.ExtensionFileLoader("_cdit_host", HOST_PATH)
+        spec = importlib.util.spec_from_file_location("_cdit_host", HOST_PATH, loader=loader)
+        module = importlib.util.module_from_spec(spec)
+        loader.exec_module(module)
+        module.bind(lib._name)
+        _host = module
+  return _host
+
+
 def is_built() -> bool:
-  return os.path.exists(os.environ.get("CDIT_HIP_LIB", LIB_PATH))
+  return os.path.exists(os.environ.get("CDIT_HIP_LIB", LIB_PATH)) and os.path.exists(HOST_PATH)
 
 
 def last_error() -> str:

@@ -22,6 +22,11 @@ torch.library.define("cdit::fp8_comm_qkv_permute_dequant", "(Tensor quant_x) -> 
 
 @torch.library.impl("cdit::fp8_comm_per_token_quant", "CUDA")
 def _per_token_quant(x: torch.Tensor) -> torch.Tensor:
+  plain = _native.host().comm_per_token_quant(x)
+  if plain is not None:
+    if plain[0]:
+      _native.check(plain[0])
+    return plain[1]
   assert x.dtype == torch.bfloat16, f"expected bfloat16 but got {x.dtype}"
   *shape, H = x.shape
   x2 = x.reshape(-1, H).contiguous()
@@ -42,6 +47,11 @@ def _fake_per_token_quant(x):
 
 @torch.library.impl("cdit::fp8_comm_per_token_dequant", "CUDA")
 def _per_token_dequant(x: torch.Tensor) -> torch.Tensor:
+  plain = _native.host().comm_per_token_dequant(x)
+  if plain is not None:
+    if plain[0]:
+      _native.check(plain[0])
+    return plain[1]
   assert x.dtype == FP8, f"expected float8_e4m3fn but got {x.dtype}"
   *shape, H2 = x.shape
   if H2 < 2:
@@ -64,6 +74,11 @@ def _fake_per_token_dequant(x):
 
 @torch.library.impl("cdit::fp8_comm_qkv_permute_quant", "CUDA")
 def _qkv_permute_quant(x: torch.Tensor) -> torch.Tensor:
+  plain = _native.host().comm_qkv_permute_quant(x)
+  if plain is not None:
+    if plain[0]:
+      _native.check(plain[0])
+    return plain[1]
   assert x.dtype == torch.bfloat16, f"expected bfloat16 but got {x.dtype}"
   B, S, P, N, D = x.shape
   if x.stride(4) != 1 or x.stride(3) != D:  # heads and channels contiguous, as the kernel reads
@@ -84,6 +99,11 @@ def _fake_qkv_permute_quant(x):
 
 @torch.library.impl("cdit::fp8_comm_qkv_permute_dequant", "CUDA")
 def _qkv_permute_dequant(quant_x: torch.Tensor) -> torch.Tensor:
+  plain = _native.host().comm_qkv_permute_dequant(quant_x)
+  if plain is not None:
+    if plain[0]:
+      _native.check(plain[0])
+    return plain[1]
   assert quant_x.dtype == FP8, f"expected float8_e4m3fn but got {quant_x.dtype}"
   S, B, N, D4 = quant_x.shape
   D = D4 - 4
@@ -103,26 +123,33 @@ def _fake_qkv_permute_dequant(quant_x):
   return quant_x.new_empty((B, S, N, D4 - 4), dtype=torch.bfloat16)
 
 
+# (looked up once: a call through the packet resolves the overload again each time)
+_per_token_quant_op = torch.ops.cdit.fp8_comm_per_token_quant.default
+_per_token_dequant_op = torch.ops.cdit.fp8_comm_per_token_dequant.default
+_qkv_permute_quant_op = torch.ops.cdit.fp8_comm_qkv_permute_quant.default
+_qkv_permute_dequant_op = torch.ops.cdit.fp8_comm_qkv_permute_dequant.default
+
+
 def fp8_comm_per_token_quant(x: torch.Tensor) -> torch.Tensor:
   """bf16 [..., H] -> float8_e4m3fn [..., H + 2] (codes, then the row's scale as bf16)."""
   _require_cuda("fp8_comm_per_token_quant", x)
-  return torch.ops.cdit.fp8_comm_per_token_quant(x)
+  return _per_token_quant_op(x)
 
 
 def fp8_comm_per_token_dequant(x: torch.Tensor) -> torch.Tensor:
   """float8_e4m3fn [..., H + 2] -> bf16 [..., H]."""
   _require_cuda("fp8_comm_per_token_dequant", x)
-  return torch.ops.cdit.fp8_comm_per_token_dequant(x)
+  return _per_token_dequant_op(x)
 
 
 def fp8_comm_qkv_permute_quant(x: torch.Tensor) -> torch.Tensor:
   """bf16 [B, S, P, N, D] -> float8_e4m3fn [P, S, B, N, D + 4] (codes, then the head row's
   fp32 scale)."""
   _require_cuda("fp8_comm_qkv_permute_quant", x)
-  return torch.ops.cdit.fp8_comm_qkv_permute_quant(x)
+  return _qkv_permute_quant_op(x)
 
 
 def fp8_comm_qkv_permute_dequant(quant_x: torch.Tensor) -> torch.Tensor:
   """float8_e4m3fn [S, B, N, D + 4] -> bf16 [B, S, N, D]."""
   _require_cuda("fp8_comm_qkv_permute_dequant", quant_x)
-  return torch.ops.cdit.fp8_comm_qkv_permute_dequant(quant_x)
+  return _qkv_permute_dequant_op(quant_x)

@@ -1,7 +1,8 @@
-"""Builds libcdit_hip.so (the HIP kernels + C ABI) for gfx950 with hipcc.
+"""Builds libcdit_hip.so (the HIP kernels + C ABI) for gfx950 with hipcc, and the Python
+extension _cdit_host.so (host code only) with g++.
 
 Usage: python -m cache_dit_amd.csrc.build   (or call build())
-The library is written to cache_dit_amd/lib/libcdit_hip.so, in-tree.
+Both are written to cache_dit_amd/lib/, in-tree.
 """
 from __future__ import annotations
 
@@ -15,6 +16,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(os.path.dirname(HERE))
 LIB_DIR = os.path.join(os.path.dirname(HERE), "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libcdit_hip.so")
+HOST_PATH = os.path.join(LIB_DIR, "_cdit_host.so")
 SOURCES = ["capi.hip", "quant_rowwise.hip", "comm_quant.hip", "gemm_fp8.hip", "gemm_w8a16.hip"]
 
 # -ffp-contract=off: the quantizer's arithmetic is specified operation by
@@ -51,8 +53,10 @@ def build(verbose: bool = False) -> str:
       raise RuntimeError(f"hipcc failed on {src}:\n{r.stdout}\n{r.stderr}")
     return obj
 
-  with ThreadPoolExecutor(max_workers=4) as ex:
+  with ThreadPoolExecutor(max_workers=5) as ex:
+    host = ex.submit(build_host, verbose)
     objs = list(ex.map(compile_one, SOURCES))
+    host.result()
   tmp = LIB_PATH + ".tmp"
   cmd = [hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", tmp, *objs]
   r = subprocess.run(cmd, capture_output=True, text=True)
@@ -60,6 +64,31 @@ def build(verbose: bool = False) -> str:
     raise RuntimeError(f"link failed:\n{r.stdout}\n{r.stderr}")
   os.replace(tmp, LIB_PATH)
   return LIB_PATH
+
+
+def build_host(verbose: bool = False) -> str:
+  """The Python extension (host_ext.cpp), against the installed torch's headers."""
+  import sysconfig
+
+  import torch
+  from torch.utils import cpp_extension
+
+  rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+  lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+  inc = [*cpp_extension.include_paths(), os.path.join(rocm, "include"), sysconfig.get_paths()["include"],
+         os.path.join(ROOT, "include")]
+  tmp = HOST_PATH + ".tmp"
+  cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-w", "-DUSE_ROCM",
+         f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}", *("-I" + i for i in inc),
+         os.path.join(HERE, "host_ext.cpp"), "-o", tmp, "-L" + lib, "-ltorch_python", "-ltorch",
+         "-ltorch_cpu", "-lc10", "-lc10_hip", "-ldl"]
+  if verbose:
+    print(" ".join(cmd), flush=True)
+  r = subprocess.run(cmd, capture_output=True, text=True)
+  if r.returncode != 0:
+    raise RuntimeError(f"{cmd[0]} failed on host_ext.cpp:\n{r.stdout}\n{r.stderr}")
+  os.replace(tmp, HOST_PATH)
+  return HOST_PATH
 
 
 if __name__ == "__main__":

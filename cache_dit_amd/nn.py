@@ -449,8 +449,8 @@ def linear_batch(pairs):
   for x, lins in pairs:
     x2 = ops._as_rows(x)
     M = x2.shape[0]
-    outs = [torch.empty((M, lin.out_features), dtype=torch.bfloat16, device=x2.device) for lin in lins]
-    result.append([o.view(*x.shape[:-1], lin.out_features) for o, lin in zip(outs, lins)])
+    outs = _native.host().outputs(x, [lin.out_features for lin in lins])
+    result.append(outs)
     if M == 0:
       continue
     rows.append(x2)
@@ -569,8 +569,8 @@ def linear_on_cat(linear: nn.Module, xs) -> torch.Tensor:
   xs = list(xs)
   if (type(linear) is Fp8DynamicLinear and len(xs) == 2 and linear.sibling_group is None
       and all(x.is_cuda and x.dtype == torch.bfloat16 for x in xs)):
-    return torch.ops.cdit.linear_w8a8_cat2(xs[0], xs[1], linear.weight, linear.weight_scale,
-                                           linear.bias, linear._scale_mode_id, linear.epilogue)
+    return ops.linear_w8a8_cat2_op(xs[0], xs[1], linear.weight, linear.weight_scale,
+                                   linear.bias, linear._scale_mode_id, linear.epilogue)
   return linear(torch.cat(xs, dim=-1))
 
 

@@ -90,7 +90,8 @@ def _require_cuda(name: str, *tensors: Optional[torch.Tensor]) -> None:
 
 
 # --------------------------------------------------------------------------- raw launchers
-# These take already-validated 2-D tensors and write into caller-provided outputs.
+# These take already-validated matrices (or contiguous tensors whose leading dimensions are the
+# rows) and write into caller-provided outputs, on the tensors' device and its current stream.
 
 
 #: Buffers whose bf16 values were never written: ln_modulate_quant(materialize=False) returns
@@ -138,12 +139,9 @@ def quant_tensorwise_into(x2: torch.Tensor, q: torch.Tensor, scale: torch.Tensor
   """Per-tensor quantizer: one scale for all of x2, written to every scale[m].
   amax_ws: 4 bytes of device scratch (an int32 tensor of one element)."""
   _reject_codes_only("quant_tensorwise_into", x2)
-  M, K = x2.shape
-  with _DeviceOf(x2):
-    _native.check(_native.load().cdit_fp8_quant_tensorwise(x2.data_ptr(), M, K, x2.stride(0),
-                                                           q.data_ptr(), q.stride(0),
-                                                           scale.data_ptr(), amax_ws.data_ptr(),
-                                                           scale_mode_id, _stream_ptr(x2)))
+  rc = _native.host().quant_tensorwise(x2, q, scale, amax_ws, scale_mode_id)
+  if rc:
+    _native.check(rc)
 
 
 def quant_rowwise_into(x2: torch.Tensor, q: torch.Tensor, scale: torch.Tensor,
@@ -152,13 +150,10 @@ def quant_rowwise_into(x2: torch.Tensor, q: torch.Tensor, scale: torch.Tensor,
   hint for the quantizer; the results are the same)."""
   if _codes_only:
     _reject_codes_only("quant_rowwise_into", x2)
-  M, K = x2.shape
   mode = scale_mode_id | (_native.QUANT_GEMM_FOLLOWS if gemm_follows else 0)
-  with _DeviceOf(x2):
-    _native.check(_native.load().cdit_fp8_quant_rowwise(x2.data_ptr(), M, K, x2.stride(0),
-                                                        q.data_ptr(), q.stride(0),
-                                                        scale.data_ptr(), mode,
-                                                        _stream_ptr(x2)))
+  rc = _native.host().quant_rowwise(x2, q, scale, mode)
+  if rc:
+    _native.check(rc)
 
 
 def quant_rowwise_batched_into(items, scale_mode_id: int) -> None:
@@ -167,19 +162,9 @@ def quant_rowwise_batched_into(items, scale_mode_id: int) -> None:
   one device; the codes are taken to be read by a GEMM launched next. Bit-identical to one
   quant_rowwise_into per item."""
   _reject_codes_only("quant_rowwise_batched_into", *[x for x, _, _ in items])
-  import ctypes
-  n = len(items)
-  x0 = items[0][0]
-  K = x0.shape[1]
-  if any(x.shape[1] != K or x.device != x0.device for x, _, _ in items):
-    raise ValueError("quant_rowwise_batched_into: the activations must share K and the device")
-  vp, i64 = ctypes.c_void_p, ctypes.c_int64
-  with _DeviceOf(x0):
-    _native.check(_native.load().cdit_fp8_quant_rowwise_batched(
-        n, (vp * n)(*[x.data_ptr() for x, _, _ in items]), (i64 * n)(*[x.shape[0] for x, _, _ in items]),
-        K, (i64 * n)(*[x.stride(0) for x, _, _ in items]), (vp * n)(*[q.data_ptr() for _, q, _ in items]),
-        (i64 * n)(*[q.stride(0) for _, q, _ in items]), (vp * n)(*[s.data_ptr() for _, _, s in items]),
-        scale_mode_id, _stream_ptr(x0)))
+  rc = _native.host().quant_rowwise_batched(items, scale_mode_id)
+  if rc:
+    _native.check(rc)
 
 
 def quant_rowwise_cat2_into(x1: torch.Tensor, x2: torch.Tensor, q: torch.Tensor, scale: torch.Tensor,
@@ -187,10 +172,9 @@ def quant_rowwise_cat2_into(x1: torch.Tensor, x2: torch.Tensor, q: torch.Tensor,
   """Quantizes the rows [x1 | x2] (bf16 [M,K1] and [M,K2]) into q [M,K1+K2] / scale [M] without
   the concatenated tensor; the results are those of quant_rowwise_into on torch.cat."""
   _reject_codes_only("quant_rowwise_cat2_into", x1, x2)
-  with _DeviceOf(x1):
-    _native.check(_native.load().cdit_fp8_quant_rowwise_cat2(
-        x1.data_ptr(), x1.shape[1], x1.stride(0), x2.data_ptr(), x2.shape[1], x2.stride(0),
-        x1.shape[0], q.data_ptr(), q.stride(0), scale.data_ptr(), scale_mode_id, _stream_ptr(x1)))
+  rc = _native.host().quant_rowwise_cat2(x1, x2, q, scale, scale_mode_id)
+  if rc:
+    _native.check(rc)
 
 
 def cat2_quant_ok(x1: torch.Tensor, x2: torch.Tensor) -> bool:
@@ -205,13 +189,10 @@ def gemm_rowwise_into(a: torch.Tensor, a_scale: torch.Tensor, w: torch.Tensor,
                       epilogue: int) -> None:
   """a [M,K] e4m3, w [N,K] e4m3 (row-major), scales fp32 contiguous, out [M,N] fp16,
   bf16 or fp32; bias in the output's dtype (none for an fp32 output)."""
-  M, K = a.shape
-  N = w.shape[0]
-  with _DeviceOf(a):
-    _native.check(_native.load().cdit_fp8_gemm_rowwise(
-        a.data_ptr(), a_scale.data_ptr(), w.data_ptr(), w_scale.data_ptr(),
-        bias.data_ptr() if bias is not None else None, out.data_ptr(), M, N, K, a.stride(0),
-        w.stride(0), out.stride(0), epilogue, encode_output_dtype(out.dtype), _stream_ptr(a)))
+  rc = _native.host().gemm_rowwise(a, a_scale, w, w_scale, bias, out, epilogue,
+                                   encode_output_dtype(out.dtype))
+  if rc:
+    _native.check(rc)
 
 
 def gemm_rowwise_grouped_into(a: torch.Tensor, a_scale: torch.Tensor, weights, w_scales, biases,
@@ -243,32 +224,9 @@ def gemm_rowwise_batched_into(acts) -> None:
   activation, its members listed as for gemm_rowwise_grouped_into; all activations and
   weights share K and their row strides. Bit-identical to one gemm_rowwise_into per
   member."""
-  import ctypes
-  vp, i64, ci = ctypes.c_void_p, ctypes.c_int64, ctypes.c_int
-  a0 = acts[0][0]
-  K, lda, ldb = a0.shape[1], a0.stride(0), acts[0][2][0].stride(0)
-  ws, wss, bs, outs, epis, per_act = [], [], [], [], [], []
-  for a, a_s, weights, w_scales, biases, o, e in acts:
-    if a.shape[1] != K or a.stride(0) != lda or a.device != a0.device:
-      raise ValueError("gemm_rowwise_batched_into: the activations must share K, the row stride "
-                       "and the device")
-    if any(w.stride(0) != ldb or w.shape[1] != K for w in weights):
-      raise ValueError("gemm_rowwise_batched_into: the weights must share K and the row stride")
-    ws += weights
-    wss += w_scales
-    bs += biases
-    outs += o
-    epis += e
-    per_act.append(len(weights))
-  n, na = len(ws), len(acts)
-  with _DeviceOf(a0):
-    _native.check(_native.load().cdit_fp8_gemm_rowwise_batched(
-        na, (vp * na)(*[t[0].data_ptr() for t in acts]), (vp * na)(*[t[1].data_ptr() for t in acts]),
-        (i64 * na)(*[t[0].shape[0] for t in acts]), K, lda, (ci * na)(*per_act),
-        (vp * n)(*[w.data_ptr() for w in ws]), (vp * n)(*[s.data_ptr() for s in wss]),
-        (vp * n)(*[b.data_ptr() if b is not None else None for b in bs]),
-        (vp * n)(*[o.data_ptr() for o in outs]), (i64 * n)(*[w.shape[0] for w in ws]), ldb,
-        (i64 * n)(*[o.stride(0) for o in outs]), (ci * n)(*[int(e) for e in epis]), _stream_ptr(a0)))
+  rc = _native.host().gemm_batched(acts, False)
+  if rc:
+    _native.check(rc)
 
 
 def w8a16_batched_into(acts) -> None:
@@ -278,48 +236,23 @@ def w8a16_batched_into(acts) -> None:
   bf16 outputs [M,N_p] and epilogue flags. Activations whose row strides differ are
   launched apart. Bit-identical to one w8a16_into per member."""
   _reject_codes_only("w8a16_batched_into", *[t[0] for t in acts])
-  import ctypes
-  vp, i64, ci = ctypes.c_void_p, ctypes.c_int64, ctypes.c_int
   x0 = acts[0][0]
   if any(t[0].stride(0) != x0.stride(0) for t in acts[1:]):
     for t in acts:
       w8a16_batched_into([t])
     return
-  K, lda, ldb = x0.shape[1], x0.stride(0), acts[0][1][0].stride(0)
-  ws, wss, bs, outs, epis, per_act = [], [], [], [], [], []
-  for x, weights, w_scales, biases, o, e in acts:
-    if x.shape[1] != K or x.device != x0.device or x.dtype != torch.bfloat16 or x.stride(1) != 1:
-      raise ValueError("w8a16_batched_into: the activations must be bf16 rows of one K on one device")
-    if any(w.stride(0) != ldb or w.shape[1] != K for w in weights):
-      raise ValueError("w8a16_batched_into: the weights must share K and the row stride")
-    ws += weights
-    wss += w_scales
-    bs += biases
-    outs += o
-    epis += e
-    per_act.append(len(weights))
-  n, na = len(ws), len(acts)
-  with _DeviceOf(x0):
-    _native.check(_native.load().cdit_w8a16_gemm_batched(
-        na, (vp * na)(*[t[0].data_ptr() for t in acts]), (i64 * na)(*[t[0].shape[0] for t in acts]),
-        K, lda, (ci * na)(*per_act), (vp * n)(*[w.data_ptr() for w in ws]),
-        (vp * n)(*[s.data_ptr() for s in wss]),
-        (vp * n)(*[b.data_ptr() if b is not None else None for b in bs]),
-        (vp * n)(*[o.data_ptr() for o in outs]), (i64 * n)(*[w.shape[0] for w in ws]), ldb,
-        (i64 * n)(*[o.stride(0) for o in outs]), (ci * n)(*[int(e) for e in epis]), _stream_ptr(x0)))
+  rc = _native.host().gemm_batched([(t[0], None, *t[1:]) for t in acts], True)
+  if rc:
+    _native.check(rc)
 
 
 def w8a16_into(x2: torch.Tensor, w: torch.Tensor, w_scale: torch.Tensor,
                bias: Optional[torch.Tensor], out: torch.Tensor, epilogue: int) -> None:
   if _codes_only:
     _reject_codes_only("w8a16_into", x2)
-  M, K = x2.shape
-  N = w.shape[0]
-  with _DeviceOf(x2):
-    _native.check(_native.load().cdit_w8a16_gemm(
-        x2.data_ptr(), w.data_ptr(), w_scale.data_ptr(),
-        bias.data_ptr() if bias is not None else None, out.data_ptr(), M, N, K, x2.stride(0),
-        w.stride(0), out.stride(0), epilogue, _native.DT_BF16, _stream_ptr(x2)))
+  rc = _native.host().w8a16(x2, w, w_scale, bias, out, epilogue)
+  if rc:
+    _native.check(rc)
 
 
 class _SharedQuant:
@@ -390,8 +323,7 @@ def shared_activation_quant(x2: torch.Tensor, scale_mode_id: int):
   for e in entries:
     if e.matches(x2, scale_mode_id):
       return e.q, e.s
-  q = torch.empty((M, K), dtype=FP8, device=dev)
-  s = torch.empty((M, ), dtype=torch.float32, device=dev)
+  q, s = _native.host().workspace(x2)
   quant_rowwise_into(x2, q, s, scale_mode_id, gemm_follows=True)
   quant_launches += 1
   _remember_quant(entries, capture_id, x2, scale_mode_id, q, s)
@@ -423,10 +355,7 @@ def shared_activation_quant_many(x2s, scale_mode_id: int):
   elif missing:
     items = []
     for i in missing:
-      x = x2s[i]
-      q = torch.empty(x.shape, dtype=FP8, device=x.device)
-      s = torch.empty((x.shape[0], ), dtype=torch.float32, device=x.device)
-      items.append((x, q, s))
+      items.append((x2s[i], *_native.host().workspace(x2s[i])))
     quant_rowwise_batched_into(items, scale_mode_id)
     quant_launches += 1
     for i, (x, q, s) in zip(missing, items):
@@ -448,14 +377,7 @@ def linear_w8a8_into(x2: torch.Tensor, w: torch.Tensor, w_scale: torch.Tensor,
   """Quantizer + GEMM of one Linear forward in a single library call."""
   if _codes_only:
     _reject_codes_only("linear_w8a8_into", x2)
-  M, K = x2.shape
-  N = w.shape[0]
-  with _DeviceOf(x2):
-    rc = _native.load().cdit_fp8_linear_w8a8(
-        x2.data_ptr(), w.data_ptr(), w_scale.data_ptr(),
-        bias.data_ptr() if bias is not None else None, out.data_ptr(), q_ws.data_ptr(),
-        s_ws.data_ptr(), M, N, K, x2.stride(0), w.stride(0), out.stride(0), scale_mode_id,
-        epilogue, _native.DT_BF16, _stream_ptr(x2))
+  rc = _native.host().linear_w8a8(x2, w, w_scale, bias, out, q_ws, s_ws, scale_mode_id, epilogue)
   if rc:
     _native.check(rc)
 
@@ -526,6 +448,10 @@ def _fp8_rowwise_quant(x: torch.Tensor, scale_mode: int = 0) -> Tuple[torch.Tens
     raise ValueError("cdit::fp8_rowwise_quant: x must have at least one dimension")
   if scale_mode not in (0, 1):
     raise ValueError(f"cdit::fp8_rowwise_quant: scale_mode must be 0 or 1, got {scale_mode}")
+  plain = _native.host().quant_plain(x)
+  if plain is not None:
+    quant_rowwise_into(x, plain[0], plain[1], scale_mode)
+    return plain
   x2 = _as_rows(x)
   q = torch.empty(x2.shape, dtype=FP8, device=x.device)
   scale = torch.empty((x2.shape[0], ), dtype=torch.float32, device=x.device)
@@ -569,6 +495,11 @@ def _float8_inference_scaled_mm(a_data, a_scale, b_data, b_scale, bias, out_dtyp
   del use_fast_accum  # a cuBLASLt hint; fp32 accumulation is the only mode here
   name = "cdit::float8_inference_scaled_mm"
   out_dtype = decode_output_dtype(out_dtype_id)
+  plain = _native.host().scaled_mm_plain(a_data, a_scale, b_data, b_scale, bias, out_dtype_id)
+  if plain is not None:
+    out, w = plain
+    gemm_rowwise_into(a_data, a_scale, w, b_scale, bias, out, epilogue)
+    return out
   if a_data.dtype != FP8 or b_data.dtype != FP8:
     raise ValueError(f"{name}: a_data/b_data must be float8_e4m3fn, got {a_data.dtype}/"
                      f"{b_data.dtype}")
@@ -624,6 +555,11 @@ def _ln_modulate_quant(x, shift, scale, eps=1e-6, scale_mode=0, write_y=True):
   leading index of x (AdaLN: [B, 1, K] for x [B, S, K]). Returns (y bf16 like x -- left
   unwritten when write_y is False --, codes e4m3 like x, scales fp32 [..., 1])."""
   name = "cdit::ln_modulate_quant"
+  plain = _native.host().ln_modulate_quant(x, shift, scale, eps, scale_mode, write_y)
+  if plain is not None:
+    if plain[0]:
+      _native.check(plain[0])
+    return plain[1:]
   if x.dtype != torch.bfloat16 or shift.dtype != torch.bfloat16 or scale.dtype != torch.bfloat16:
     raise ValueError(f"{name}: x, shift and scale must be bfloat16, got {x.dtype}, {shift.dtype}, "
                      f"{scale.dtype}")
@@ -678,7 +614,7 @@ def ln_modulate_quant(x: torch.Tensor, shift: torch.Tensor, scale: torch.Tensor,
   no_handover = (x.is_inference() or torch.is_inference_mode_enabled()
                  or torch.compiler.is_compiling())
   write_y = bool(materialize or no_handover)
-  y, q, s = torch.ops.cdit.ln_modulate_quant(x, shift, scale, float(eps), mode_id, write_y)
+  y, q, s = _ln_modulate_quant_op(x, shift, scale, float(eps), mode_id, write_y)
   if not no_handover and y.numel() > 0:
     y2 = y.view(-1, y.shape[-1])
     entries, capture_id = _shared_entries(y2)
@@ -702,6 +638,17 @@ def _linear_w8a8(x, weight, weight_scale, bias, scale_mode=0, epilogue=0, granul
   activation scales, 1: one scale for the whole activation. Workspaces are taken inside
   the op, so a traced graph only sees tensors in and a tensor out."""
   name = "cdit::linear_w8a8"
+  if not share_input_quant and scale_mode in (0, 1) and granularity in (0, 1):
+    per_tensor = granularity == GRANULARITY_PER_TENSOR
+    plain = _native.host().linear_plain(x, weight, weight_scale, bias, per_tensor)
+    if plain is not None:
+      out, q, s = plain[:3]
+      if per_tensor:
+        quant_tensorwise_into(x, q, s, plain[3], scale_mode)
+        gemm_rowwise_into(q, s, weight, weight_scale, bias, out, epilogue)
+      else:
+        linear_w8a8_into(x, weight, weight_scale, bias, out, q, s, scale_mode, epilogue)
+      return out
   if x.dtype != torch.bfloat16:
     raise ValueError(f"{name}: x must be bfloat16, got {x.dtype}")
   if weight.dtype != FP8 or weight.dim() != 2:
@@ -745,6 +692,12 @@ def _linear_w8a8_cat2(x1, x2, weight, weight_scale, bias, scale_mode=0, epilogue
   src/cache_dit/caching/patch_functors/functor_flux.py:68-80). Bit-identical to the op on the
   concatenation; sources the kernel does not take are concatenated."""
   name = "cdit::linear_w8a8_cat2"
+  plain = _native.host().cat2_plain(x1, x2, weight, weight_scale, bias) if scale_mode in (0, 1) else None
+  if plain is not None:
+    out, q, s = plain
+    quant_rowwise_cat2_into(x1, x2, q, s, scale_mode)
+    gemm_rowwise_into(q, s, weight, weight_scale, bias, out, epilogue)
+    return out
   if x1.dtype != torch.bfloat16 or x2.dtype != torch.bfloat16:
     raise ValueError(f"{name}: x1 and x2 must be bfloat16, got {x1.dtype} and {x2.dtype}")
   if x1.shape[:-1] != x2.shape[:-1]:
@@ -895,6 +848,12 @@ def _fake_linear_w8a8(x, weight, weight_scale, bias, scale_mode=0, epilogue=0, g
 def _w8a16_mm(x, b_data, b_scale, bias, out_dtype_id, epilogue=0):
   name = "cdit::w8a16_mm"
   out_dtype = decode_output_dtype(out_dtype_id)
+  plain = (_native.host().w8a16_plain(x, b_data, b_scale, bias)
+           if out_dtype == torch.bfloat16 else None)
+  if plain is not None:
+    out, w = plain
+    w8a16_into(x, w, b_scale, bias, out, epilogue)
+    return out
   if out_dtype != torch.bfloat16 or x.dtype != torch.bfloat16:
     raise ValueError(f"{name}: only bfloat16 activations and output are built, got {x.dtype} -> "
                      f"{out_dtype}")
@@ -926,6 +885,8 @@ linear_w8a8_op = torch.ops.cdit.linear_w8a8.default
 w8a16_mm_op = torch.ops.cdit.w8a16_mm.default
 _fp8_rowwise_quant_op = torch.ops.cdit.fp8_rowwise_quant.default
 _scaled_mm_op = torch.ops.cdit.float8_inference_scaled_mm.default
+_ln_modulate_quant_op = torch.ops.cdit.ln_modulate_quant.default
+linear_w8a8_cat2_op = torch.ops.cdit.linear_w8a8_cat2.default
 
 # --------------------------------------------------------------------------- python-level API
 
