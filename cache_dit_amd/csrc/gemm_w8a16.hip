@@ -937,35 +937,87 @@ int launch_wide_grouped(const GemmArgs& g, GemmGroup grp, hipStream_t stream) {
 }
 
 // ---------------------------------------------------------------------------
-// A few dozen rows (the prompt's projections: M = 17 to 128 or so): one wavefront, alone in
-// its workgroup, per 32 x 32 tile. A 128 x 64 tile of the wide kernel gives such a problem to a
-// few dozen CUs, whose prefetch cannot keep the weight stream in flight; 32 x 32 tiles put it on
-// all of them. The wavefront has a ring of D stages (A 32 rows x 128 B, B 32 rows x 64 B, the
-// swizzles of the wide kernel) that LDS-DMA fills D steps ahead; nobody else touches them, so
-// there are no barriers, only waits on its own loads and LDS reads. Operands are read one step
-// ahead of their MFMAs, and a stage is refilled as soon as they are in registers, between the
-// second and the third MFMA of the step. MFMA, K order and epilogue arithmetic are those of the
-// wide kernel, so the results are bit-identical to it (a member of a batch may run there).
-// What bounds it: a chain of four dependent MFMAs (128 clocks) and six DMA instructions per step.
-// One wavefront issues all of it in order: about 500 clocks per step.
-// Another weight matrix per launch (M x K x N), against 128 x 64 tiles: 77 x 4096 x 3072 22.1 -> 16.1 us,
-// 17 x 3072 x 3072 15.3 -> 12.1, 128 x 3072 x 3072 20.4 -> 13.2, 256 x 3072 x 1536 19.8 -> 12.9,
-// 512 x 4096 x 1024 20.4 -> 15.6, 32 x 3072 x 12288 18.3 -> 17.3; with 672 tiles
-// (200 x 4096 x 3072) 21.5 -> 22.2 and with 864 (77 x 3072 x 9216) 19.6 -> 29.9: not taken.
-constexpr int kTileDepth = 8, kTileLds = kTileDepth * 32 * 3 * BKE;
+// A few dozen rows (the prompt's projections: M = 17 to 128 or so) and few rows on many columns: a
+// workgroup of two wavefronts per 32 x 32 tile. A 128 x 64 tile of the wide kernel gives such a
+// problem to a few dozen CUs, whose prefetch cannot keep the weight stream in flight (one CU has
+// some 60 GB/s from HBM); 32 x 32 tiles put it on all of them. A ring of D stages (A 32 rows x
+// 128 B, B 32 rows x 64 B, the swizzles of the wide kernel) is filled D steps ahead by LDS-DMA of
+// the one wavefront; the other reads the operands of a step one step ahead of their MFMAs. One
+// barrier per step: in front of it step kt + 1 has landed, behind it the operands of step kt are in
+// registers and its stage is free. MFMA, K order and epilogue arithmetic are those of the wide
+// kernel, so the results are bit-identical to it (a member of a batch may run there).
+// What bounds it: a chain of four dependent MFMAs (128 clocks) next to 16 conversions, and six DMA
+// instructions per step, each on a wavefront of its own: about 250 clocks per step (500 with one
+// wavefront issuing both in order). Two feeding wavefronts: 3 to 8 % faster with one tile per CU,
+// 4 to 8 % slower with two. Conversions a step ahead of their MFMAs: the same or slower. D = 6: four
+// workgroups fit a CU; 8 is 1 to 5 % slower up to two per CU (but up to 6 % faster where 40 MB of weights
+// come from HBM) and three per CU already take a second round; 4 is up to 27 % slower on such weights.
+// Another weight matrix per launch (M x K x N), us, one wavefront before -> now: 77 x 4096 x 3072
+// 15.9 -> 11.2, 17 x 3072 x 3072 12.3 -> 8.5, 128 x 3072 x 3072 13.2 -> 9.5, 256 x 15360 x 1024 47.4
+// -> 31, 100 x 1024 x 2048 6.3 -> 4.9; 128 x 64 tiles of the wide kernel -> now: 245 x 1664 x 2560 11.4 ->
+// 8.1, 299 x 3328 x 2368 (740 tiles) 18.1 -> 15.1, 103 x 2816 x 6016 (752) 15.6 -> 10.9, but
+// 158 x 6784 x 4352 (680) 30.0 -> 34.2, and beyond 768 tiles either way: 154 x 2560 x 5056 (790) 15.8 -> 13.7,
+// 592 x 1664 x 1600 (950) 11.9 -> 14.9.
+constexpr int kTileDepth = 6, kTileLds = kTileDepth * 32 * 3 * BKE;
 template <bool GELU>
-__global__ __launch_bounds__(64) void gemm_w8a16_wavetile(GemmArgs g, int tiles_m, int tiles_n) {
+__global__ __launch_bounds__(128) void gemm_w8a16_wavetile(GemmArgs g, int tiles_m, int tiles_n) {
   constexpr int D = kTileDepth, A_BYTES = 32 * 2 * BKE, STAGE = kTileLds / D, NDMA = 6;
-  static_assert((D - 1) * NDMA < 63 && D * STAGE <= 64 * 1024, "vmcnt has 6 bits; LDS without opt-in");
+  static_assert(D >= 3 && (D - 1) * NDMA < 63 && D * STAGE <= 64 * 1024, "vmcnt has 6 bits; LDS without opt-in");
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
   // the row tiles of one column tile on one XCD (workgroups go to the 8 XCDs in turn): its
   // weights come from HBM once
   const int id = blockIdx.x;
   const int tn = id / 8 / tiles_m * 8 + id % 8, tm = id / 8 % tiles_m;
   if (tn >= tiles_n) return;
-  const int lane = threadIdx.x, m0 = tm * 32, n0 = tn * 32;
+  const int lane = threadIdx.x & 63, m0 = tm * 32, n0 = tn * 32;
   const int h = lane >> 5, r32 = lane & 31;
   const int KT = (g.K + BKE - 1) / BKE;
+  if (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) == 1) {
+    // the feeding wavefront
+    // DMA maps: an instruction fills 8 A rows (chunk (lane & 7) ^ swizzle, which differs between
+    // even and odd instructions by 4) or 16 B rows
+    const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint8_t*>(static_cast<const uint8_t*>(g.a)) + (int64_t)m0 * g.lda * 2, 0, 0x7fffffff, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint8_t*>(g.b) + (int64_t)n0 * g.ldb, 0, 0x7fffffff, 0x00020000);
+    const int ca = (lane & 7) ^ (lane >> 4), cb = (lane & 3) ^ ((lane >> 4) & 3);
+    uint32_t off[NDMA];
+  #pragma unroll
+    for (int p = 0; p < 4; ++p)
+      off[p] = (uint32_t)min(8 * p + (lane >> 3), g.M - 1 - m0) * (uint32_t)(g.lda * 2) + (ca ^ (4 * (p & 1))) * 16;
+  #pragma unroll
+    for (int p = 0; p < 2; ++p)
+      off[4 + p] = (uint32_t)min(16 * p + (lane >> 2), g.N - 1 - n0) * (uint32_t)g.ldb + cb * 16;
+    // Elements beyond K (a partial last step, steps beyond the last) are fetched from beyond the
+    // descriptor: zeros.
+    auto dma = [&](int kt, int stage) {
+      const int left = g.K - kt * BKE;
+      const uint32_t a0 = ca * 8 < left ? 0u : 0x80000000u, a1 = (ca ^ 4) * 8 < left ? 0u : 0x80000000u;
+      const uint32_t b0 = cb * 16 < left ? 0u : 0x80000000u;
+      __attribute__((address_space(3))) uint8_t* st =
+          (__attribute__((address_space(3))) uint8_t*)(smem) + stage;
+  #pragma unroll
+      for (int p = 0; p < 4; ++p)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (__attribute__((address_space(3))) void*)(st + p * 1024), 16,
+                                                 (int)(off[p] | (p & 1 ? a1 : a0)), kt * 2 * BKE, 0, 0);
+  #pragma unroll
+      for (int p = 0; p < 2; ++p)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (__attribute__((address_space(3))) void*)(st + A_BYTES + p * 1024),
+                                                 16, (int)(off[4 + p] | b0), kt * BKE, 0, 0);
+    };
+#pragma unroll
+    for (int s = 0; s < D; ++s) dma(s, s * STAGE);
+    wait_and_barrier<(D - 1) * NDMA>();  // step 0 has landed
+    int stage = 0;                       // of step kt
+    for (int kt = 0; kt < KT; ++kt) {
+      // step kt + 1 has landed; behind the barrier the operands of step kt are in registers
+      wait_and_barrier<(D - 2) * NDMA>();
+      dma(kt + D, stage);
+      stage = stage + STAGE == D * STAGE ? 0 : stage + STAGE;
+    }
+    wait_vm<0>();  // no DMA outlives the workgroup
+    return;
+  }
 
   // scale and bias of the lane's 16 columns n0 + 16 h .. (N % 16 == 0: all in or all out)
   const int nw = n0 + 16 * h;
@@ -979,38 +1031,6 @@ __global__ __launch_bounds__(64) void gemm_w8a16_wavetile(GemmArgs g, int tiles_
     bi[0] = reinterpret_cast<const uint4*>(g.bias + nw)[0];
     bi[1] = reinterpret_cast<const uint4*>(g.bias + nw)[1];
   }
-
-  // DMA maps: an instruction fills 8 A rows (chunk (lane & 7) ^ swizzle, which differs between
-  // even and odd instructions by 4) or 16 B rows
-  const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<uint8_t*>(static_cast<const uint8_t*>(g.a)) + (int64_t)m0 * g.lda * 2, 0, 0x7fffffff, 0x00020000);
-  const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<uint8_t*>(g.b) + (int64_t)n0 * g.ldb, 0, 0x7fffffff, 0x00020000);
-  const int ca = (lane & 7) ^ (lane >> 4), cb = (lane & 3) ^ ((lane >> 4) & 3);
-  uint32_t off[NDMA];
-#pragma unroll
-  for (int p = 0; p < 4; ++p)
-    off[p] = (uint32_t)min(8 * p + (lane >> 3), g.M - 1 - m0) * (uint32_t)(g.lda * 2) + (ca ^ (4 * (p & 1))) * 16;
-#pragma unroll
-  for (int p = 0; p < 2; ++p)
-    off[4 + p] = (uint32_t)min(16 * p + (lane >> 2), g.N - 1 - n0) * (uint32_t)g.ldb + cb * 16;
-  // Elements beyond K (a partial last step, steps beyond the last) are fetched from beyond the
-  // descriptor: zeros.
-  auto dma = [&](int kt, int stage) {
-    const int left = g.K - kt * BKE;
-    const uint32_t a0 = ca * 8 < left ? 0u : 0x80000000u, a1 = (ca ^ 4) * 8 < left ? 0u : 0x80000000u;
-    const uint32_t b0 = cb * 16 < left ? 0u : 0x80000000u;
-    __attribute__((address_space(3))) uint8_t* st =
-        (__attribute__((address_space(3))) uint8_t*)(smem) + stage;
-#pragma unroll
-    for (int p = 0; p < 4; ++p)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (__attribute__((address_space(3))) void*)(st + p * 1024), 16,
-                                               (int)(off[p] | (p & 1 ? a1 : a0)), kt * 2 * BKE, 0, 0);
-#pragma unroll
-    for (int p = 0; p < 2; ++p)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (__attribute__((address_space(3))) void*)(st + A_BYTES + p * 1024),
-                                               16, (int)(off[4 + p] | b0), kt * BKE, 0, 0);
-  };
 
   // operand read maps, as in the wide kernel
   const int wrow = 16 * ((r32 >> 2) & 1) + 4 * (r32 >> 3) + (r32 & 3);
@@ -1039,33 +1059,24 @@ __global__ __launch_bounds__(64) void gemm_w8a16_wavetile(GemmArgs g, int tiles_
   v16f acc;
 #pragma unroll
   for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
-#pragma unroll
-  for (int s = 0; s < D; ++s) dma(s, s * STAGE);
-  wait_vm<(D - 1) * NDMA>();
+  wait_and_barrier<63>();
   Step even = read(smem), odd;
-  wait_lgkm0();
-  dma(D, 0);
   int stage = STAGE;  // of step kt + 1
-  // Step kt: its operands are in `f`; reads step kt + 1 into `nf` and sends for step kt + 1 + D.
-  auto step = [&](int kt, const Step& f, Step& nf) {
-    wait_vm<(D - 1) * NDMA>();  // steps up to kt + 1 have landed
+  // Step kt: its operands are in `f`; reads step kt + 1 into `nf`.
+  auto step = [&](const Step& f, Step& nf) {
+    wait_and_barrier<63>();
     nf = read(smem + stage);
     __builtin_amdgcn_sched_barrier(0);
     acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(e4m3x8_to_bf16(f.w[0].x, f.w[0].y), f.a[0], acc, 0, 0, 0);
     acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(e4m3x8_to_bf16(f.w[0].z, f.w[0].w), f.a[1], acc, 0, 0, 0);
-    __builtin_amdgcn_sched_barrier(0);
-    wait_lgkm0();  // step kt + 1 is in registers: its stage can be filled again
-    dma(kt + 1 + D, stage);
-    __builtin_amdgcn_sched_barrier(0);
     acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(e4m3x8_to_bf16(f.w[1].x, f.w[1].y), f.a[2], acc, 0, 0, 0);
     acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(e4m3x8_to_bf16(f.w[1].z, f.w[1].w), f.a[3], acc, 0, 0, 0);
     stage = stage + STAGE == D * STAGE ? 0 : stage + STAGE;
   };
   for (int kt = 0; kt < KT; kt += 2) {
-    step(kt, even, odd);
-    if (kt + 1 < KT) step(kt + 1, odd, even);
+    step(even, odd);
+    if (kt + 1 < KT) step(odd, even);
   }
-  wait_vm<0>();  // no DMA outlives the workgroup
 
   // acc[r] is out[m0 + r32][n0 + 16 h + r]
   const int m = m0 + r32;
@@ -1089,7 +1100,7 @@ __global__ __launch_bounds__(64) void gemm_w8a16_wavetile(GemmArgs g, int tiles_
 
 int launch_wavetile(const GemmArgs& g, hipStream_t stream) {
   const int tiles_m = (g.M + 31) / 32, tiles_n = (g.N + 31) / 32;
-  const dim3 grid((tiles_n + 7) / 8 * 8 * tiles_m), block(64);
+  const dim3 grid((tiles_n + 7) / 8 * 8 * tiles_m), block(128);
   if (g.epilogue & CDIT_EPI_GELU_TANH)
     hipLaunchKernelGGL(gemm_w8a16_wavetile<true>, grid, block, kTileLds, stream, g, tiles_m, tiles_n);
   else
@@ -1434,6 +1445,24 @@ bool whole_rows_better(const GemmArgs& g) {
   if (g.K > 1024) return g.N >= 1536 && g.N <= 16384 && (g.M == 2 || (g.M == 3 && g.K >= 1280));
   return g.M == 2 && g.N >= 4608 && g.K >= 320;
 }
+
+// Whether 2 to 16 rows go to the kernel with a workgroup per 32 x 32 tile instead of the 16-row
+// (or whole-row) kernel. The latter's time grows with the rows and the columns, the former's with
+// neither until the tiles are more than the CUs: few columns stay where they are, many do not. us,
+// another weight matrix per launch, 16-row / tiles: 16 x 18432 x 5120 (M x N x K) 48.4 / 30.6, 16 x 9216 x
+// 1024 8.9 / 5.0, 8 x 18432 x 3072 19.5 / 16.4, 8 x 5120 x 4608 12.6 / 12.2, 5 x 9216 x 3072 11.8 / 10.7;
+// 16 x 3072 x 3072 6.9 / 8.2, 8 x 4096 x 4608 8.6 / 12.3; whole-row / tiles: 4 x 18432 x 3072 17.6 /
+// 15.9, 3 x 9216 x 3072 9.1 / 10.7, 2 x 18432 x 3072 14.0 / 16.5. Over 610 shapes (K 1024 to 5120,
+// N 2048 to 18432) 0.8 % off the best of the three in the geometric mean (11 % without the tiles).
+// K remainders, where the 16-row kernel masks its loads: from some 41,000 outputs on. 16-row / tiles,
+// M x N x K: 16 x 18432 x 3136 40.6 / 17.0, 8 x 9216 x 5056 25.8 / 14.6, 4 x 9216 x 1360 7.8 / 7.9.
+bool tiles_better_for_few(const GemmArgs& g) {
+  if (g.K % 128) return (int64_t)g.M * g.N > 40960;
+  if (g.M >= 7) return g.N > 4500;
+  if (g.M >= 5) return g.N > 7000;
+  if (g.M >= 3) return g.N > (g.M == 4 ? 8000 : 10000);
+  return g.M == 2 && g.K > 4096 && g.N > 8000;
+}
 }  // namespace
 
 int launch_gemm_w8a16(const GemmArgs& g, int variant, hipStream_t stream) {
@@ -1444,7 +1473,8 @@ int launch_gemm_w8a16(const GemmArgs& g, int variant, hipStream_t stream) {
     return 0;
   };
   if (!aligned_ok(g) || variant == 100) return launch_generic();
-  if (g.M <= 4 && g.K <= 4096 && (variant == 51 || (variant < 0 && whole_rows_better(g)))) {
+  const bool few_on_tiles = g.M <= 16 && g.N % 16 == 0 && tiles_better_for_few(g);
+  if (g.M <= 4 && g.K <= 4096 && (variant == 51 || (variant < 0 && whole_rows_better(g) && (g.K % 128 || !few_on_tiles)))) {
     // (aligned_ok has checked the alignment of the operands and of lda and ldb)
     switch ((g.K + 1023) / 1024) {
       case 1: launch_rows_chk<1>(g, stream); break;
@@ -1454,12 +1484,6 @@ int launch_gemm_w8a16(const GemmArgs& g, int variant, hipStream_t stream) {
     }
     return 0;
   }
-  // K remainders: the 16-row kernel masks its loads, and its time grows with the rows and the
-  // columns; from some 41,000 outputs on the wavefront-per-tile kernel below is the faster one.
-  // Another weight matrix per launch, us (16-row / wavefront tiles / 128 x 64 tiles of the wide
-  // kernel), M x N x K: 16 x 18432 x 3136 40.6 / 18.1 / 31.2, 8 x 9216 x 5056 25.8 / 19.0 / 23.6,
-  // 12 x 4608 x 1600 9.7 / 7.9 / 10.2, 4 x 9216 x 1360 7.8 / 7.9, 16 x 2304 x 3136 10.6 / 12.2 / 15.4.
-  const bool few_on_tiles = g.K % 128 != 0 && g.N % 16 == 0 && g.M <= 16 && (int64_t)g.M * g.N > 40960;
   if ((variant < 0 && g.M <= 16 && !few_on_tiles) || variant == 50) {
     if (g.M > 16) {
       set_error("cdit_w8a16_gemm: the skinny kernel takes M <= 16");
@@ -1481,11 +1505,11 @@ int launch_gemm_w8a16(const GemmArgs& g, int variant, hipStream_t stream) {
   auto wide_ok = [&](int depth) {
     return (k_tail || g.K >= (depth > 3 ? depth : 3) * BKE) && g.N % 16 == 0;
   };
-  // Two 32 x 32 tiles per CU and less: the wavefront-per-tile kernel (figures at the kernel; at
-  // three per CU it wins or loses with the shape, beyond that the CUs take a second round of it).
+  // Three 32 x 32 tiles per CU and less: the workgroup-per-tile kernel (figures at the kernel; at
+  // four per CU it wins or loses with the shape, beyond that the CUs take a second round of it).
   if (g.N % 16 == 0 &&
       (variant == 13 || (variant < 0 && (few_on_tiles || (int64_t)((g.M + 31) / 32) * ((g.N + 31) / 32) <=
-                                                             2 * (int64_t)(cu_count() > 0 ? cu_count() : 256)))))
+                                                             3 * (int64_t)(cu_count() > 0 ? cu_count() : 256)))))
     return launch_wavetile(g, stream);
   if (variant < 0 || (k_tail && (variant < 7 || variant > 12))) {
     variant = choose_variant(

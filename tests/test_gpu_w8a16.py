@@ -546,3 +546,30 @@ def test_few_rows_kernels_at_the_edges_of_their_rule(M, N, K):
     _native.set_gemm_variant(variant)
     assert torch.equal(_run(x, w, ws, None).cpu(), ref), variant
   _native.set_gemm_variant(-1)
+
+
+@pytest.mark.parametrize("M,N", [(2, 8000), (2, 8016), (3, 10000), (3, 10016), (4, 8000), (4, 8016), (5, 7008), (6, 7024),
+                                 (7, 4496), (7, 4512), (16, 4496), (16, 4512), (16, 4520), (16, 24592)])
+@pytest.mark.parametrize("K", [128, 1152, 4224])
+def test_few_rows_on_both_sides_of_the_tile_rule(M, N, K):
+  """Whole K steps: the 16-row or whole-row kernel up to a number of columns, a workgroup per 32 x 32
+  tile beyond. Integers whose sums are exact in fp32 in any order (below 9 K < 2^24): bit for bit,
+  whichever kernel runs; K below and above the depth of its ring, one round of workgroups and
+  more (24592 columns: 769 tiles)."""
+  from cache_dit_amd import _native, ops
+  g = torch.Generator(device="cuda").manual_seed(M + N + K)
+  x = torch.randint(-3, 4, (M, K), generator=g, device="cuda").to(torch.bfloat16)
+  w = torch.randint(-3, 4, (N, K), generator=g, device="cuda").float().to(torch.float8_e4m3fn)
+  s = torch.pow(2.0, torch.randint(-3, 3, (N, ), generator=g, device="cuda").float())
+  want = ((x.double() @ w.double().t()) * s.double()).float().to(torch.bfloat16)
+  try:
+    for variant in (-1, 50, 13) if N % 16 == 0 else (-1, 50):
+      _native.set_gemm_variant(variant)
+      full = torch.full((M + 2, N + 8), 777.0, dtype=torch.bfloat16, device="cuda")
+      ops.w8a16_into(x, w, s, None, full[1:M + 1, :N], 0)
+      torch.cuda.synchronize()
+      assert torch.equal(full[1:M + 1, :N], want), variant
+      full[1:M + 1, :N] = 777.0
+      assert bool((full == 777.0).all()), variant
+  finally:
+    _native.set_gemm_variant(-1)
