@@ -1352,14 +1352,19 @@ __global__ __launch_bounds__(256) void gemm_fp8_skinny(GemmArgs g) {
 // cdit_fp8_quant_rowwise bit for bit; workgroup 0 also writes them to the caller's
 // workspaces. The first batch of weight loads is issued before that, so the HBM latency
 // of the weights covers it. g.a is the bf16 activation here, g.lda its leading dimension.
+// From three rows on each wavefront quantizes every fourth row on its own: with all four on one row, two barriers
+// and a chain of loads per row, a row cost 1 us (K = 3072), now four rows do: 8 x 1024 x 3072
+// (M x N x K) 12.8 -> 8.4 us, 8 x 9216 x 3072 17.4 -> 15.5, 16 x 3072 x 1024 15.9 -> 8.8. Where it
+// is taken instead of the two kernels: skinny_fused_better().
 constexpr int kFusedPad = 16;  // LDS row pitch K + 16 bytes: rows start 4 banks apart
-template <bool KTAIL>
+// ROW_PER_WAVE: from three rows on (its registers cost the instance for fewer 4 to 7 %).
+template <bool KTAIL, bool ROW_PER_WAVE>
 __global__ __launch_bounds__(256) void linear_fp8_skinny_fused(GemmArgs g, uint8_t* q_ws,
                                                                float* scale_ws, int scale_mode) {
   extern __shared__ __attribute__((aligned(16))) uint8_t codes[];  // [M][K + kFusedPad]
   __shared__ float part[4][16][17];
-  __shared__ uint32_t wave_amax[4];
   __shared__ float row_s[16];
+  __shared__ uint32_t wave_amax[4];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int r = lane & 15, kg = lane >> 4;
   const int n0 = blockIdx.x * 16;
@@ -1393,33 +1398,60 @@ __global__ __launch_bounds__(256) void linear_fp8_skinny_fused(GemmArgs g, uint8
   // ---- quantize the activation rows into LDS
   const uint16_t* x = static_cast<const uint16_t*>(g.a);
   const int nchunks = g.K >> 3;  // 16-byte chunks of 8 bf16
-  for (int m = 0; m < g.M; ++m) {
-    const uint4* xr = reinterpret_cast<const uint4*>(x + (int64_t)m * g.lda);
-    uint32_t am = 0;
-    for (int c = threadIdx.x; c < nchunks; c += 256) {
-      const uint4 v = xr[c];
-      am = absmax2(absmax2(absmax2(absmax2(am, v.x), v.y), v.z), v.w);
+  auto codes_of = [](uint4 v, float s, Recip rcp, bool fast) {
+    return fast ? uint2{quant4<true>(v.x, v.y, s, rcp), quant4<true>(v.z, v.w, s, rcp)}
+                : uint2{quant4<false>(v.x, v.y, s, Recip{}), quant4<false>(v.z, v.w, s, Recip{})};
+  };
+  if constexpr (!ROW_PER_WAVE) {  // the four wavefronts share each row
+    for (int m = 0; m < g.M; ++m) {
+      const uint4* xr = reinterpret_cast<const uint4*>(x + (int64_t)m * g.lda);
+      uint32_t am = 0;
+      for (int c = threadIdx.x; c < nchunks; c += 256) {
+        const uint4 v = xr[c];
+        am = absmax2(absmax2(absmax2(absmax2(am, v.x), v.y), v.z), v.w);
+      }
+      am = wave_max_u32(fold2(am));
+      if (lane == 0) wave_amax[wave] = am;
+      __syncthreads();
+      const uint32_t a01 = max(wave_amax[0], wave_amax[1]), a23 = max(wave_amax[2], wave_amax[3]);
+      const float s = row_scale(max(a01, a23), scale_mode);
+      if (threadIdx.x == 0) row_s[m] = s;
+      uint2* dst = reinterpret_cast<uint2*>(codes + m * pitch);
+      if (scale_in_fast_window(s)) {  // uniform
+        const Recip rcp = make_recip(s);
+        for (int c = threadIdx.x; c < nchunks; c += 256) dst[c] = codes_of(xr[c], s, rcp, true);
+      } else {
+        for (int c = threadIdx.x; c < nchunks; c += 256) dst[c] = codes_of(xr[c], s, Recip{}, false);
+      }
+      __syncthreads();  // codes of row m complete; wave_amax free for the next row
     }
-    am = wave_max_u32(fold2(am));
-    if (lane == 0) wave_amax[wave] = am;
-    __syncthreads();
-    const uint32_t a01 = max(wave_amax[0], wave_amax[1]), a23 = max(wave_amax[2], wave_amax[3]);
-    const float s = row_scale(max(a01, a23), scale_mode);
-    if (threadIdx.x == 0) row_s[m] = s;
-    uint2* dst = reinterpret_cast<uint2*>(codes + m * pitch);
-    if (scale_in_fast_window(s)) {  // uniform
+  } else {
+    constexpr int P = 4;  // chunks of a lane whose loads are in flight together
+    for (int m = wave; m < g.M; m += 4) {
+      const uint4* xr = reinterpret_cast<const uint4*>(x + (int64_t)m * g.lda);
+      uint32_t am = 0;
+      for (int c0 = lane; c0 < nchunks; c0 += 64 * P) {
+        uint4 v[P];
+#pragma unroll
+        for (int p = 0; p < P; ++p) v[p] = xr[min(c0 + 64 * p, nchunks - 1)];
+#pragma unroll
+        for (int p = 0; p < P; ++p) am = absmax2(absmax2(absmax2(absmax2(am, v[p].x), v[p].y), v[p].z), v[p].w);
+      }
+      const float s = row_scale(wave_max_u32(fold2(am)), scale_mode);
+      if (lane == 0) row_s[m] = s;
+      uint2* dst = reinterpret_cast<uint2*>(codes + m * pitch);
+      const bool fast = scale_in_fast_window(s);  // uniform
       const Recip rcp = make_recip(s);
-      for (int c = threadIdx.x; c < nchunks; c += 256) {
-        const uint4 v = xr[c];
-        dst[c] = uint2{quant4<true>(v.x, v.y, s, rcp), quant4<true>(v.z, v.w, s, rcp)};
-      }
-    } else {
-      for (int c = threadIdx.x; c < nchunks; c += 256) {
-        const uint4 v = xr[c];
-        dst[c] = uint2{quant4<false>(v.x, v.y, s, Recip{}), quant4<false>(v.z, v.w, s, Recip{})};
+      for (int c0 = lane; c0 < nchunks; c0 += 64 * P) {
+        uint4 v[P];
+#pragma unroll
+        for (int p = 0; p < P; ++p) v[p] = xr[min(c0 + 64 * p, nchunks - 1)];
+#pragma unroll
+        for (int p = 0; p < P; ++p)
+          if (c0 + 64 * p < nchunks) dst[c0 + 64 * p] = codes_of(v[p], s, rcp, fast);
       }
     }
-    __syncthreads();  // codes of row m complete; wave_amax free for the next row
+    __syncthreads();
   }
   if (blockIdx.x == 0) {  // the caller's workspaces get what cdit_fp8_quant_rowwise would write
     for (int m = 0; m < g.M; ++m) {
@@ -1722,6 +1754,19 @@ int launch_row1(const GemmArgs& g, uint8_t* q_ws, float* scale_ws, int scale_mod
   return 0;
 }
 
+// Whether quantizing the rows in every workgroup costs less than a launch of the quantizer in front:
+// it grows with the rows per wavefront, their length and the workgroups per CU, the launch does not
+// (2.2 to 3 us). us, one kernel / two, another weight matrix per launch, M x N x K: 4 x 9216 x 3072 12.6 / 12.6,
+// 4 x 1024 x 3072 6.4 / 7.5; 8 x 9216 x 2048 11.8 / 12.8, 8 x 6144 x 3072 11.9 / 10.7, 8 x 18432 x 3072 23.7 / 18.6;
+// 12 x 6144 x 2048 10.6 / 10.9, 12 x 3072 x 3072 10.7 / 8.2, 16 x 3072 x 2048 9.1 / 8.3, 16 x 9216 x 3072
+// 24.8 / 15.0. (Some 10 % are left to the single launch where both take about 10 us: a call of two launches takes
+// the host 2.7 us longer.)
+bool skinny_fused_better(const GemmArgs& g) {
+  if (g.M <= 4) return true;
+  if (g.M <= 8) return g.K <= 2048 || g.N <= 6144;
+  return g.K <= 2048 && g.N <= 9216;
+}
+
 int launch_linear_fp8_skinny_fused(const GemmArgs& g, void* q_ws, float* scale_ws, int scale_mode,
                                    int variant, hipStream_t stream) {
   // Bit-identical to the quantizer followed by cdit_fp8_gemm_rowwise only where that call
@@ -1734,20 +1779,22 @@ int launch_linear_fp8_skinny_fused(const GemmArgs& g, void* q_ws, float* scale_w
   if (!aligned_ok(two_step)) return 1;
   if (launch_row1<true>(g, static_cast<uint8_t*>(q_ws), scale_ws, scale_mode, variant, stream) == 0) return 0;
   const int64_t lds = (int64_t)g.M * (g.K + kFusedPad);
-  const bool ok = g.M >= 1 && g.M <= 16 && (variant < 0 || variant == 50) && g.K >= 16 &&
-                  g.K % 16 == 0 && g.N % 8 == 0 && lds <= 48 * 1024 && g.lda % 8 == 0 &&
+  const bool ok = g.M >= 1 && g.M <= 16 && (variant == 50 || (variant < 0 && skinny_fused_better(g))) && g.K >= 16 &&
+                  g.K % 16 == 0 && g.N % 8 == 0 && lds <= 56 * 1024 && g.lda % 8 == 0 &&
                   g.ldb % 16 == 0 && g.ldo % 8 == 0 &&
                   reinterpret_cast<uintptr_t>(g.a) % 16 == 0 &&
                   reinterpret_cast<uintptr_t>(g.b) % 16 == 0 &&
                   reinterpret_cast<uintptr_t>(g.out) % 16 == 0 &&
                   reinterpret_cast<uintptr_t>(q_ws) % 8 == 0;
   if (!ok) return 1;
-  if (g.K % BK) {
-    hipLaunchKernelGGL(linear_fp8_skinny_fused<true>, dim3((g.N + 15) / 16), dim3(256), (size_t)lds, stream,
-                       g, static_cast<uint8_t*>(q_ws), scale_ws, scale_mode);
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((g.N + 15) / 16), dim3(256), (size_t)lds, stream, g,
+                       static_cast<uint8_t*>(q_ws), scale_ws, scale_mode);
+  };
+  if (g.M > 2) {
+    g.K % BK ? go(&linear_fp8_skinny_fused<true, true>) : go(&linear_fp8_skinny_fused<false, true>);
   } else {
-    hipLaunchKernelGGL(linear_fp8_skinny_fused<false>, dim3((g.N + 15) / 16), dim3(256), (size_t)lds, stream,
-                       g, static_cast<uint8_t*>(q_ws), scale_ws, scale_mode);
+    g.K % BK ? go(&linear_fp8_skinny_fused<true, false>) : go(&linear_fp8_skinny_fused<false, false>);
   }
   return 0;
 }

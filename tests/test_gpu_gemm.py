@@ -729,3 +729,33 @@ def test_measurement_instance_with_time_stamps_gives_the_same_bits(M, N, K):
                                 b.data_ptr(), out.data_ptr(), 16, N, K, K, K, N,
                                 stamps.data_ptr(), ctypes.byref(n_wg), None)
   assert rc != 0 and b"288 x 192" in L.cdit_last_error()
+
+
+@pytest.mark.parametrize("scale_mode", [0, 1])
+@pytest.mark.parametrize("M", [2, 4, 5, 8, 9, 13, 16])
+@pytest.mark.parametrize("N,K", [(264, 16), (40, 528), (520, 2048), (9232, 2064), (6152, 3072)])
+def test_rows_quantized_one_per_wavefront(M, N, K, scale_mode):
+  """The Linear for few rows in one kernel (50), a row per wavefront, one to four rows each, K with
+  partial pieces of 64 chunks; and whichever of one and two kernels is chosen (-1): codes, scales and
+  outputs of the quantizer and the GEMM called one after the other, rows of zeros, of NaN and beyond
+  the fast division's window among them."""
+  from cache_dit_amd import _native, ops
+  g = torch.Generator(device="cuda").manual_seed(M * 7 + N + K + scale_mode)
+  x = (torch.randn(M, K, generator=g, device="cuda") * 2).to(torch.bfloat16)
+  x[0] = 0
+  x[1] *= 1e32
+  x[-1, K - 1] = float("nan")
+  wq, w_s = ops.fp8_rowwise_quant((torch.randn(N, K, generator=g, device="cuda") * 0.05).to(torch.bfloat16))
+  q2, s2 = torch.empty(M, K, dtype=FP8, device="cuda"), torch.empty(M, dtype=torch.float32, device="cuda")
+  out2 = torch.empty(M, N, dtype=torch.bfloat16, device="cuda")
+  ops.quant_rowwise_into(x, q2, s2, scale_mode)
+  ops.gemm_rowwise_into(q2, s2, wq, w_s, None, out2, 1)
+  for variant in (-1, 50):
+    _native.set_gemm_variant(variant)
+    q = torch.full((M, K), 0x55, dtype=torch.uint8, device="cuda").view(FP8)
+    s, out = torch.full_like(s2, -1.0), torch.zeros_like(out2)
+    ops.linear_w8a8_into(x, wq, w_s, None, out, q, s, scale_mode, 1)
+    torch.cuda.synchronize()
+    assert torch.equal(q.view(torch.uint8), q2.view(torch.uint8)), variant
+    assert torch.equal(s.view(torch.int32), s2.view(torch.int32)), variant
+    assert torch.equal(out.view(torch.int16), out2.view(torch.int16)), variant
