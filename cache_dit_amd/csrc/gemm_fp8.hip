@@ -1246,6 +1246,168 @@ int launch_wide_grouped(const GemmArgs& g, GemmGroup grp, hipStream_t stream) {
 }
 
 // ---------------------------------------------------------------------------
+// Small problems (a prompt's projections, few rows of long K, a few hundred rows of a narrow
+// Linear): a workgroup per 32 x 32 tile, four wavefronts with a 16 x 16 block each and two that
+// only feed them. The tiles of the wide kernel give such a problem to a few dozen CUs, and a step
+// of theirs waits for what one CU gets from beyond its L2 (60 GB/s from HBM, 130 from the
+// last-level cache) or, with K remainders, for the conversions of one wavefront (96 of 8 clocks
+// in the 64 x 128 tile; 32 here). A ring of D stages (A and B, 32 rows x 128 B each) is filled D
+// steps ahead; one barrier per step: in front of it step kt + 1 has landed, behind it the
+// operands of step kt are in registers and its stage is free. MFMA, K order and epilogue
+// arithmetic are those of the wide kernel and its instances for K remainders, so the results are
+// bit-identical to them (a member of a batch may run there).
+// What bounds it: the feeding wavefronts' DMA instructions (4 a step and wavefront) and the
+// barrier, about 250 clocks a step; K remainders the conversions as well. Four feeding wavefronts:
+// no faster. D = 5 against 4: up to 8 % faster where K is long (52 x 15104 x 2304, M x K x N: 17.9 us against
+// 19.2), up to 4 % slower on 600 tiles and more; against 6: 1 to 4 % faster there, the same elsewhere.
+// us, best tile of the wide kernel -> this one, M x K x N: 77 x 4096 x 3072 11.8 -> 8.7, 23 x 7168 x 3328
+// 16.4 -> 10.3, 303 x 4736 x 640 13.9 -> 8.1, 35 x 4864 x 8064 13.9 -> 10.6, 203 x 4992 x 3392 (742
+// tiles) 16.1 -> 15.3; K remainders 158 x 2656 x 304 17.2 -> 6.6, 22 x 2832 x 3984 18.9 -> 7.5, 300 x
+// 2224 x 3072 (960 tiles) 16.6 -> 14.3.
+constexpr int kTile32Depth = 5;
+template <int OUT, bool KTAIL, bool GELU>
+__global__ __launch_bounds__(384) void gemm_fp8_tile32(GemmArgs g, int tiles_m, int tiles_n) {
+  constexpr int D = kTile32Depth, BKW = 128, PANEL = 32 * BKW, STAGE = 2 * PANEL, NDMA = 4;
+  static_assert(D >= 3 && (D - 1) * NDMA <= 63 && D * STAGE <= 64 * 1024, "vmcnt has 6 bits; LDS without opt-in");
+  extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+  // the row tiles of one column tile on one XCD (workgroups go to the 8 XCDs in turn): its
+  // weights come from HBM once
+  const int id = blockIdx.x;
+  const int tn = id / 8 / tiles_m * 8 + id % 8, tm = id / 8 % tiles_m;
+  if (tn >= tiles_n) return;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int m0 = tm * 32, n0 = tn * 32;
+  const int KT = (g.K + BKW - 1) / BKW;
+
+  if (wave >= 4) {
+    // Feeding wavefronts: 4 the A panel, 5 the B panel. An instruction fills 8 panel rows; lane l lands
+    // on row l / 8, position l % 8 and fetches the chunk that the swizzle stores there (swz_a: the
+    // parity of the instruction gives row bit 3). What lies beyond K comes from beyond the descriptor:
+    // zeros.
+    const bool is_a = wave == 4;
+    const int64_t ld = is_a ? g.lda : g.ldb;
+    const int rows = is_a ? g.M - m0 : g.N - n0;
+    const uint8_t* base = is_a ? static_cast<const uint8_t*>(g.a) + (int64_t)m0 * g.lda : g.b + (int64_t)n0 * g.ldb;
+    const __amdgpu_buffer_rsrc_t src = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(base), 0, 0x7fffffff,
+                                                                         0x00020000);
+    const int even = (lane & 7) ^ swz_a(lane >> 3), odd = (lane & 7) ^ swz_a(8 + (lane >> 3));
+    uint32_t off[NDMA];
+#pragma unroll
+    for (int p = 0; p < NDMA; ++p)
+      off[p] = (uint32_t)min(8 * p + (lane >> 3), rows - 1) * (uint32_t)ld + (p & 1 ? odd : even) * 16;
+    auto dma = [&](int kt, int stage) {
+      const int left = g.K - kt * BKW;
+      const uint32_t none_even = even * 16 < left ? 0u : 0x80000000u, none_odd = odd * 16 < left ? 0u : 0x80000000u;
+      uint8_t* st = smem + stage + (is_a ? 0 : PANEL);
+#pragma unroll
+      for (int p = 0; p < NDMA; ++p)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(src, (__attribute__((address_space(3))) void*)(st + p * 1024), 16,
+                                                 (int)(off[p] | (p & 1 ? none_odd : none_even)), kt * BKW, 0, 0);
+    };
+#pragma unroll
+    for (int s = 0; s < D; ++s) dma(s, s * STAGE);
+    wait_and_barrier<(D - 1) * NDMA>();  // step 0 has landed
+    int stage = 0;                       // of step kt
+    for (int kt = 0; kt < KT; ++kt) {
+      // step kt + 1 has landed; behind the barrier the operands of step kt are in registers
+      wait_and_barrier<(D - 2) * NDMA>();
+      dma(kt + D, stage);
+      stage = stage + STAGE == D * STAGE ? 0 : stage + STAGE;
+    }
+    wait_vm<0>();  // no DMA outlives the workgroup
+    return;
+  }
+
+  const int wm = wave >> 1, wn = wave & 1, r16 = lane & 15, kg = lane >> 4;
+  // scale and bias of the lane's 4 columns (N % 8 == 0: all in or all out)
+  const int n = n0 + 16 * wn + 4 * kg, m = m0 + 16 * wm + r16;
+  const bool n_in = n < g.N;
+  v4f bs = {0.0f, 0.0f, 0.0f, 0.0f};
+  uint2 bi = {0u, 0u};
+  if (n_in) bs = *reinterpret_cast<const v4f*>(g.b_scale + n);
+  if (n_in && g.bias) bi = *reinterpret_cast<const uint2*>(g.bias + n);
+  const float as = g.a_scale[min(m, g.M - 1)];
+
+  uint32_t rd_a[2], rd_b[2];
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {
+    rd_a[e] = (16 * wm + r16) * BKW + (((2 * kg + e) ^ swz_a(16 * wm + r16)) << 4);
+    rd_b[e] = PANEL + (16 * wn + r16) * BKW + (((2 * kg + e) ^ swz_a(16 * wn + r16)) << 4);
+  }
+  struct Step {
+    v8i a, b;
+  };
+  // (__restrict__: see the wide kernel; without it every read would wait for the whole stream)
+  auto read = [&](const uint8_t* __restrict__ st) -> Step {
+    auto two = [&](const uint32_t (&rd)[2]) {
+      const v4i lo = *reinterpret_cast<const v4i*>(st + rd[0]), hi = *reinterpret_cast<const v4i*>(st + rd[1]);
+      return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+    };
+    return {two(rd_a), two(rd_b)};
+  };
+  v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
+  wait_and_barrier<63>();
+  Step even = read(smem), odd;
+  int stage = STAGE;  // of step kt + 1
+  auto step = [&](const Step& f, Step& nf) {
+    wait_and_barrier<63>();
+    nf = read(smem + stage);
+    __builtin_amdgcn_sched_barrier(0);
+    // operands swapped: result rows follow B (n), result columns follow A (m)
+    if constexpr (KTAIL) {
+      acc = mfma_codes_as_bf16(f.b, f.a, acc);
+    } else {
+      acc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(f.b, f.a, acc, 0, 0, 0, 0, 0, 0);
+    }
+    stage = stage + STAGE == D * STAGE ? 0 : stage + STAGE;
+  };
+  for (int kt = 0; kt < KT; kt += 2) {
+    step(even, odd);
+    if (kt + 1 < KT) step(odd, even);
+  }
+
+  // acc[e] is out[m][n + e]
+  if (m >= g.M || !n_in) return;
+  const float b4[4] = {bias_to_f32<OUT>(bi.x & 0xffffu), bias_to_f32<OUT>(bi.x >> 16), bias_to_f32<OUT>(bi.y & 0xffffu),
+                       bias_to_f32<OUT>(bi.y >> 16)};
+  float v[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    v[e] = __fmaf_rn(acc[e] * as, bs[e], b4[e]);
+    if constexpr (GELU) v[e] = gelu_tanh(v[e]);
+  }
+  const int64_t at = (int64_t)m * g.ldo + n;
+  if constexpr (OUT == CDIT_DT_F32) {
+    *reinterpret_cast<v4f*>(reinterpret_cast<float*>(g.out) + at) = v4f{v[0], v[1], v[2], v[3]};
+  } else if constexpr (OUT == CDIT_DT_F16) {
+    *reinterpret_cast<uint2*>(g.out + at) = uint2{pack_f16x2(v[0], v[1]), pack_f16x2(v[2], v[3])};
+  } else {
+    *reinterpret_cast<uint2*>(g.out + at) = uint2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+  }
+}
+
+template <int OUT, bool KTAIL>
+int launch_tile32(const GemmArgs& g, hipStream_t stream) {
+  const int tiles_m = (g.M + 31) / 32, tiles_n = (g.N + 31) / 32;
+  const dim3 grid((tiles_n + 7) / 8 * 8 * tiles_m), block(384);
+  constexpr int lds = kTile32Depth * 2 * 32 * 128;
+  if (g.epilogue & CDIT_EPI_GELU_TANH)
+    hipLaunchKernelGGL((gemm_fp8_tile32<OUT, KTAIL, true>), grid, block, lds, stream, g, tiles_m, tiles_n);
+  else
+    hipLaunchKernelGGL((gemm_fp8_tile32<OUT, KTAIL, false>), grid, block, lds, stream, g, tiles_m, tiles_n);
+  return 0;
+}
+
+template <bool KTAIL>
+int launch_tile32(const GemmArgs& g, hipStream_t stream) {
+  switch (g.out_dtype) {
+    case CDIT_DT_F16: return launch_tile32<CDIT_DT_F16, KTAIL>(g, stream);
+    case CDIT_DT_F32: return launch_tile32<CDIT_DT_F32, KTAIL>(g, stream);
+    default: return launch_tile32<CDIT_DT_BF16, KTAIL>(g, stream);
+  }
+}
+
+// ---------------------------------------------------------------------------
 // Skinny kernel for M <= 16 (the M = 1 modulation Linears `norm1.linear`,
 // `norm.linear` of every block): pure weight streaming. A workgroup of 4 waves
 // owns 16 output channels; each wave takes a quarter of K and reads its weight
@@ -1886,6 +2048,16 @@ int launch_gemm_fp8(const GemmArgs& g, int variant, hipStream_t stream) {
     }
     return 0;
   }
+  // Up to three 32 x 32 tiles per CU the workgroup-per-tile kernel (figures at the kernel; beyond, it
+  // wins with short K and loses with long: 864 tiles 7.1 us with the wide kernel, 6.4 with this one
+  // at K = 896, 816 tiles 30.1 and 32.9 at K = 10624), with K remainders up to five (1209 tiles 9.5 and
+  // 8.3, 1677 tiles 18.6 and 22.0). A K of one or two steps takes the instances for K remainders: fp16 and
+  // fp32 outputs of such a K have their sums in full fp32 (from the kernel for any shape), and the
+  // conversions of two steps cost nothing (36 x 3904 x 256, M x N x K: 7.4 us with the tiled kernel, 4.2).
+  const bool tail = g.K % BK != 0 || g.K < 3 * BK;
+  const int64_t tiles32 = (int64_t)((g.M + 31) / 32) * ((g.N + 31) / 32);
+  if (variant == 26 || (variant < 0 && tiles32 <= (tail ? 5 : 3) * (int64_t)(cu_count() > 0 ? cu_count() : 256)))
+    return tail ? launch_tile32<true>(g, stream) : launch_tile32<false>(g, stream);
   if (!tiled_ok(g)) return launch_gemm_fp8_ktail(g, variant, stream);
   // the wide kernels stream K two or more steps ahead: shorter K runs the 128x128 kernel
   // at least `depth` K steps to prefetch, and at least 3: the epilogue operands of a tile are
