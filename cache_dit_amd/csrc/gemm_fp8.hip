@@ -1517,7 +1517,7 @@ __global__ __launch_bounds__(256) void gemm_fp8_skinny(GemmArgs g) {
 // From three rows on each wavefront quantizes every fourth row on its own: with all four on one row, two barriers
 // and a chain of loads per row, a row cost 1 us (K = 3072), now four rows do: 8 x 1024 x 3072
 // (M x N x K) 12.8 -> 8.4 us, 8 x 9216 x 3072 17.4 -> 15.5, 16 x 3072 x 1024 15.9 -> 8.8. Where it
-// is taken instead of the two kernels: skinny_fused_better().
+// is taken instead of two kernels: few_on_tiles().
 constexpr int kFusedPad = 16;  // LDS row pitch K + 16 bytes: rows start 4 banks apart
 // ROW_PER_WAVE: from three rows on (its registers cost the instance for fewer 4 to 7 %).
 template <bool KTAIL, bool ROW_PER_WAVE>
@@ -1885,6 +1885,8 @@ typedef CfgWide<256, 128, 4> V19;                     // ... 128x64 wave tiles, 
 typedef CfgWide<256, 256, 4, 2, false> V12H;
 typedef CfgWide<288, 192, 4, 2, false> V14H;
 
+bool few_on_tiles(const GemmArgs& g);
+
 // The M = 1 kernel when the shape fits it (variant 51 forces it, 50 the 16-row kernel);
 // returns 1 when it is not taken.
 template <bool FUSED>
@@ -1916,17 +1918,24 @@ int launch_row1(const GemmArgs& g, uint8_t* q_ws, float* scale_ws, int scale_mod
   return 0;
 }
 
-// Whether quantizing the rows in every workgroup costs less than a launch of the quantizer in front:
-// it grows with the rows per wavefront, their length and the workgroups per CU, the launch does not
-// (2.2 to 3 us). us, one kernel / two, another weight matrix per launch, M x N x K: 4 x 9216 x 3072 12.6 / 12.6,
-// 4 x 1024 x 3072 6.4 / 7.5; 8 x 9216 x 2048 11.8 / 12.8, 8 x 6144 x 3072 11.9 / 10.7, 8 x 18432 x 3072 23.7 / 18.6;
-// 12 x 6144 x 2048 10.6 / 10.9, 12 x 3072 x 3072 10.7 / 8.2, 16 x 3072 x 2048 9.1 / 8.3, 16 x 9216 x 3072
-// 24.8 / 15.0. (Some 10 % are left to the single launch where both take about 10 us: a call of two launches takes
-// the host 2.7 us longer.)
-bool skinny_fused_better(const GemmArgs& g) {
-  if (g.M <= 4) return true;
-  if (g.M <= 8) return g.K <= 2048 || g.N <= 6144;
-  return g.K <= 2048 && g.N <= 9216;
+// Whether 2 to 16 rows go to the kernel with a workgroup per 32 x 32 tile, behind a launch of the
+// quantizer where they come as bf16, instead of the 16-row kernel, which quantizes them itself.
+// That grows with the rows per wavefront and their length in every workgroup, and its loads
+// take 64-byte pieces of 16 rows; the tiles cost a launch (2.2 to 3 us) and no more with 16 rows than with
+// 2. us, the whole Linear in one kernel / with tiles, another weight matrix per launch, M x N x K: 16 x 9216 x 3072
+// 24.8 / 12.7, 16 x 18432 x 5120 36.6 / 26.7, 12 x 3072 x 3072 10.7 / 8.3, 8 x 18432 x 3072 23.7 / 17.8, 8 x 6144 x
+// 5120 18.2 / 13.3, 4 x 9216 x 5120 20.3 / 16.9, 4 x 18432 x 2048 14.5 / 13.1, 2 x 9216 x 5120 18.6 / 16.9; 16 x 3072 x
+// 1024 8.8 / 6.5, 8 x 6144 x 3072 11.9 / 10.2, 4 x 9216 x 3072 12.6 / 11.9, 2 x 18432 x 3072 17.2 / 17.6. (What is near on
+// both sides and about 10 us is left to the single launch: a call of two takes the host 2.7 us longer.)
+// The distance from 64-bit sums is the same on both (1.5e-5 of normal rows, 2.5e-5 with outliers, K
+// 1024 to 5120). The rule looks at nothing that differs between the Linear and its GEMM alone, so
+// that both give the same bits.
+bool few_on_tiles(const GemmArgs& g) {
+  const int64_t weights = (int64_t)g.N * g.K;
+  if (g.M >= 9) return g.K > 2048 || g.N > 9216;
+  if (g.M >= 5) return weights > 20000000 || g.N > 12288;
+  if (g.M >= 3) return weights > 30000000;
+  return g.M == 2 && g.K > 4096 && weights > 40000000;
 }
 
 int launch_linear_fp8_skinny_fused(const GemmArgs& g, void* q_ws, float* scale_ws, int scale_mode,
@@ -1941,7 +1950,7 @@ int launch_linear_fp8_skinny_fused(const GemmArgs& g, void* q_ws, float* scale_w
   if (!aligned_ok(two_step)) return 1;
   if (launch_row1<true>(g, static_cast<uint8_t*>(q_ws), scale_ws, scale_mode, variant, stream) == 0) return 0;
   const int64_t lds = (int64_t)g.M * (g.K + kFusedPad);
-  const bool ok = g.M >= 1 && g.M <= 16 && (variant == 50 || (variant < 0 && skinny_fused_better(g))) && g.K >= 16 &&
+  const bool ok = g.M >= 1 && g.M <= 16 && (variant == 50 || (variant < 0 && !few_on_tiles(g))) && g.K >= 16 &&
                   g.K % 16 == 0 && g.N % 8 == 0 && lds <= 56 * 1024 && g.lda % 8 == 0 &&
                   g.ldb % 16 == 0 && g.ldo % 8 == 0 &&
                   reinterpret_cast<uintptr_t>(g.a) % 16 == 0 &&
@@ -2036,7 +2045,7 @@ int launch_gemm_fp8(const GemmArgs& g, int variant, hipStream_t stream) {
   if ((variant < 0 || variant == 51) &&
       launch_row1<false>(g, nullptr, nullptr, 0, variant, stream) == 0)
     return 0;
-  if ((variant < 0 && g.M <= 16) || variant == 50) {
+  if ((variant < 0 && g.M <= 16 && !few_on_tiles(g)) || variant == 50) {
     if (g.M > 16) {
       set_error("cdit_fp8_gemm_rowwise: the skinny kernel takes M <= 16, got %d", g.M);
       return CDIT_EINVAL;
@@ -2048,7 +2057,7 @@ int launch_gemm_fp8(const GemmArgs& g, int variant, hipStream_t stream) {
     }
     return 0;
   }
-  // Up to three 32 x 32 tiles per CU the workgroup-per-tile kernel (figures at the kernel; beyond, it
+  // Few rows (few_on_tiles) and up to three 32 x 32 tiles per CU: the workgroup-per-tile kernel (figures at the kernel; beyond, it
   // wins with short K and loses with long: 864 tiles 7.1 us with the wide kernel, 6.4 with this one
   // at K = 896, 816 tiles 30.1 and 32.9 at K = 10624), with K remainders up to five (1209 tiles 9.5 and
   // 8.3, 1677 tiles 18.6 and 22.0). A K of one or two steps takes the instances for K remainders: fp16 and
@@ -2056,7 +2065,7 @@ int launch_gemm_fp8(const GemmArgs& g, int variant, hipStream_t stream) {
   // conversions of two steps cost nothing (36 x 3904 x 256, M x N x K: 7.4 us with the tiled kernel, 4.2).
   const bool tail = g.K % BK != 0 || g.K < 3 * BK;
   const int64_t tiles32 = (int64_t)((g.M + 31) / 32) * ((g.N + 31) / 32);
-  if (variant == 26 || (variant < 0 && tiles32 <= (tail ? 5 : 3) * (int64_t)(cu_count() > 0 ? cu_count() : 256)))
+  if (variant == 26 || (variant < 0 && (g.M <= 16 || tiles32 <= (tail ? 5 : 3) * (int64_t)(cu_count() > 0 ? cu_count() : 256))))
     return tail ? launch_tile32<true>(g, stream) : launch_tile32<false>(g, stream);
   if (!tiled_ok(g)) return launch_gemm_fp8_ktail(g, variant, stream);
   // the wide kernels stream K two or more steps ahead: shorter K runs the 128x128 kernel

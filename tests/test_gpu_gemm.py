@@ -749,9 +749,9 @@ def test_rows_quantized_one_per_wavefront(M, N, K, scale_mode):
   q2, s2 = torch.empty(M, K, dtype=FP8, device="cuda"), torch.empty(M, dtype=torch.float32, device="cuda")
   out2 = torch.empty(M, N, dtype=torch.bfloat16, device="cuda")
   ops.quant_rowwise_into(x, q2, s2, scale_mode)
-  ops.gemm_rowwise_into(q2, s2, wq, w_s, None, out2, 1)
   for variant in (-1, 50):
     _native.set_gemm_variant(variant)
+    ops.gemm_rowwise_into(q2, s2, wq, w_s, None, out2, 1)
     q = torch.full((M, K), 0x55, dtype=torch.uint8, device="cuda").view(FP8)
     s, out = torch.full_like(s2, -1.0), torch.zeros_like(out2)
     ops.linear_w8a8_into(x, wq, w_s, None, out, q, s, scale_mode, 1)
