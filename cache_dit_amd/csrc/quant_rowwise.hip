@@ -395,31 +395,43 @@ __global__ __launch_bounds__(64) void quant_tensorwise_cast(
 // of the cast alone replaces them by the scale; a wavefront that comes later finds a word
 // without the tag, which then is the scale itself. Against a launch that clears the word and an
 // atomic per workgroup, graph replays: 17 x 1024 7.3 -> 6.0 us, 512 x 3072 8.5 -> 6.4, 4608 x 3072
-// 17.8 -> 15.7 (4.5 TB/s over two reads and a write).
+// 17.8 -> 15.7 (4.5 TB/s over two reads and a write). With several rows of a wavefront in flight in the
+// amax kernel, and the cast fetching its row ahead of the scale, on the XCD that read it before:
+// 1357 x 2224 7.1 -> 6.3, 4608 x 3072 15.3 -> 12.7 (5.6 TB/s), 32760 x 5120 156 -> 135.
 constexpr int kAmaxWaves = 8;  // wavefronts per workgroup of tensor_amax_rows
 constexpr uint32_t kPartTag = 0xffff0000u;
 
-template <int CH>
+// R rows of a wavefront are in flight together (as many as it has, up to four and 24 vectors: with
+// one after the other 4608 x 3072 was three latencies); a row beyond the last reads as zeros.
+constexpr int amax_rows_in_flight(int ch) { return ch <= 6 ? 4 : ch <= 12 ? 2 : 1; }
+template <int CH, int R>
 __global__ __launch_bounds__(64 * kAmaxWaves) void tensor_amax_rows(const uint16_t* __restrict__ x,
                                                                      int64_t ld_x, int M, int K,
                                                                      float* __restrict__ scale) {
   typedef unsigned int u4v __attribute__((ext_vector_type(4)));
   __shared__ uint32_t part[kAmaxWaves];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t stride = (int64_t)gridDim.x * kAmaxWaves;
   uint32_t m = 0;
-  for (int64_t row = (int64_t)blockIdx.x * kAmaxWaves + wave; row < M; row += (int64_t)gridDim.x * kAmaxWaves) {
-    const __amdgpu_buffer_rsrc_t xb = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint16_t*>(x + row * ld_x), 0, K * 2, 0x00020000);
-    u4v w[CH];
+  for (int64_t row0 = (int64_t)blockIdx.x * kAmaxWaves + wave; row0 < M; row0 += R * stride) {
+    u4v w[R][CH];
 #pragma unroll
-    for (int c = 0; c < CH; ++c) w[c] = __builtin_amdgcn_raw_buffer_load_b128(xb, 16 * (c * 64 + lane), 0, 0);
+    for (int i = 0; i < R; ++i) {
+      const int64_t row = row0 + i * stride;
+      const __amdgpu_buffer_rsrc_t xb = __builtin_amdgcn_make_buffer_rsrc(
+          const_cast<uint16_t*>(x + (row < M ? row : row0) * ld_x), 0, row < M ? K * 2 : 0, 0x00020000);
 #pragma unroll
-    for (int c = 0; c < CH; ++c) {
-      m = absmax2(m, w[c][0]);
-      m = absmax2(m, w[c][1]);
-      m = absmax2(m, w[c][2]);
-      m = absmax2(m, w[c][3]);
+      for (int c = 0; c < CH; ++c) w[i][c] = __builtin_amdgcn_raw_buffer_load_b128(xb, 16 * (c * 64 + lane), 0, 0);
     }
+#pragma unroll
+    for (int i = 0; i < R; ++i)
+#pragma unroll
+      for (int c = 0; c < CH; ++c) {
+        m = absmax2(m, w[i][c][0]);
+        m = absmax2(m, w[i][c][1]);
+        m = absmax2(m, w[i][c][2]);
+        m = absmax2(m, w[i][c][3]);
+      }
   }
   m = wave_max_u32(fold2(m));
   if (lane == 0) part[wave] = m;
@@ -439,6 +451,21 @@ __global__ __launch_bounds__(64) void quant_tensorwise_cast_rows(
   typedef unsigned int u4v __attribute__((ext_vector_type(4)));
   typedef unsigned int u2v __attribute__((ext_vector_type(2)));
   const int lane = threadIdx.x & 63;
+  const int first = blockIdx.x * CH * 64 + lane;  // this lane's first group of eight elements
+  // The first row is on its way while the scale is worked out. In whole groups of 64 rows a row is
+  // cast on the XCD that the amax kernel read it on (row / 8 there, this kernel's id here, modulo
+  // 8; one wavefront per row), whose L2 may still have it.
+  const int64_t row_first = gridDim.x == 1 && (int)gridDim.y == M && ((int)blockIdx.y | 63) < M
+                                ? (blockIdx.y & ~63u) | (blockIdx.y & 7u) << 3 | (blockIdx.y >> 3 & 7u)
+                                : blockIdx.y;
+  u4v w[CH];
+  auto load_row = [&](int64_t row) {
+    const __amdgpu_buffer_rsrc_t xb = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint16_t*>(x + row * ld_x), 0, K * 2, 0x00020000);
+#pragma unroll
+    for (int c = 0; c < CH; ++c) w[c] = __builtin_amdgcn_raw_buffer_load_b128(xb, 16 * (c * 64 + first), 0, 0);
+  };
+  load_row(row_first);
   uint32_t* words = reinterpret_cast<uint32_t*>(scale);
   uint32_t m = 0, done = 0;  // done: the bits of the scale (never 0), if a word holds it already
   for (int i = lane; i < parts; i += 64) {
@@ -458,15 +485,10 @@ __global__ __launch_bounds__(64) void quant_tensorwise_cast_rows(
   }
   const bool fast = scale_in_fast_window(s);
   const Recip r = make_recip(s);
-  const int first = blockIdx.x * CH * 64 + lane;  // this lane's first group of eight elements
-  for (int64_t row = blockIdx.y; row < M; row += gridDim.y) {
+  for (int64_t row = row_first; row < M; row += gridDim.y) {
+    if (row != row_first) load_row(row);
     if (lane == 0 && blockIdx.x == 0 && row >= parts) scale[row] = s;
-    const __amdgpu_buffer_rsrc_t xb = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint16_t*>(x + row * ld_x), 0, K * 2, 0x00020000);
     const __amdgpu_buffer_rsrc_t qb = __builtin_amdgcn_make_buffer_rsrc(q + row * ld_q, 0, K, 0x00020000);
-    u4v w[CH];
-#pragma unroll
-    for (int c = 0; c < CH; ++c) w[c] = __builtin_amdgcn_raw_buffer_load_b128(xb, 16 * (c * 64 + first), 0, 0);
     if (fast) {
 #pragma unroll
       for (int c = 0; c < CH; ++c)
@@ -1141,6 +1163,7 @@ int launch_quant_tensorwise(const void* x, int64_t M, int64_t K, int64_t ld_x, v
   if (vec && K <= 32 * 512) {
     const int need = (int)((K + 511) / 512);
     const int parts = (int)std::min<int64_t>((M + kAmaxWaves - 1) / kAmaxWaves, cu_count_or(256));
+    const int64_t per_wave = (M + (int64_t)parts * kAmaxWaves - 1) / ((int64_t)parts * kAmaxWaves);
     // The cast of rows beyond 4096 elements: a wavefront per 3072 of them. With 12 and more vectors
     // of a row per lane the compiler kept them in scratch memory too (for the indexed loop of
     // the exact division: 400 bytes per lane at 24), and 2 to 6 wavefronts fitted a SIMD instead
@@ -1148,8 +1171,11 @@ int launch_quant_tensorwise(const void* x, int64_t M, int64_t K, int64_t ld_x, v
     // 91.0 -> 62.0; against three launches 4608 x 4112 38.1 -> 29.2, 300 x 15360 16.1 -> 10.1.
 #define CDIT_PT_CASE(CH)                                                                           \
   if (need <= CH) {                                                                                \
-    hipLaunchKernelGGL(tensor_amax_rows<CH>, dim3((unsigned)parts), dim3(64 * kAmaxWaves), 0, stream, \
-                       xp, ld_x, (int)M, (int)K, scale);                                           \
+    constexpr int RMAX = amax_rows_in_flight(CH), R2 = RMAX < 2 ? RMAX : 2;                         \
+    auto* amax = per_wave <= 1 ? &tensor_amax_rows<CH, 1>                                          \
+                               : per_wave <= 2 ? &tensor_amax_rows<CH, R2> : &tensor_amax_rows<CH, RMAX>; \
+    hipLaunchKernelGGL(amax, dim3((unsigned)parts), dim3(64 * kAmaxWaves), 0, stream, xp, ld_x, (int)M, \
+                       (int)K, scale);                                                             \
     constexpr int CAST = CH <= 8 ? CH : 6;                                                         \
     hipLaunchKernelGGL(quant_tensorwise_cast_rows<CAST>,                                           \
                        dim3((unsigned)std::max(1, (need + CAST - 1) / CAST), (unsigned)blocks), dim3(64), 0, \

@@ -137,3 +137,21 @@ def test_partial_maxima_by_row_count(M, K):
     q_ref, s_ref = to.quantize_tensorwise(x, "bf16div")
     assert torch.equal(s[:M].cpu(), s_ref.reshape(-1).expand(M)) and (s[M:] == 7.0).all()
     assert torch.equal(q.cpu().view(torch.uint8), q_ref.view(torch.uint8))
+
+
+@pytest.mark.parametrize("M,K", [(63, 64), (64, 64), (65, 64), (130, 1024), (2048, 72), (2049, 512), (4097, 1024),
+                                 (8193, 200), (4100, 3080), (2050, 4104), (2100, 6152), (2100, 8200)])
+def test_rows_in_flight_together(M, K):
+  """Whole and partial groups of 64 rows, one to four rows and more per wavefront of the amax kernel
+  (2048 wavefronts), rows of one and several wavefronts of the cast: the outlier that sets the scale
+  is in turn in the first, the last and a middle row, in its first and its last element."""
+  from cache_dit_amd import ops
+  x = torch.randn(M, K, generator=torch.Generator().manual_seed(M + K)).to(torch.bfloat16)
+  for row, col in ((0, 0), (M - 1, K - 1), (M // 2 + 1, K - 1), (min(2047, M - 1), 0)):
+    y = x.clone()
+    y[row, col] = -57.0
+    q_ref, s_ref = to.quantize_tensorwise(y, "bf16div")
+    q, s = ops.fp8_tensorwise_quant(y.to(_dev()), "bf16div")
+    torch.cuda.synchronize()
+    assert torch.equal(s.cpu(), s_ref), (row, col)
+    assert torch.equal(q.cpu().view(torch.uint8), q_ref.view(torch.uint8)), (row, col)
