@@ -118,17 +118,18 @@ PyObject* wrap(std::initializer_list<at::Tensor> ts) {
   return t;
 }
 
-// Calls a library entry point with `t`'s device current, on its current stream, without the GIL
-// (a full launch queue blocks); gives the status.
-template <class F>
-PyObject* launch(const at::Tensor& t, F call) {
-  TORCH_CHECK(lib.linear_w8a8, "libcdit_hip.so is not bound");
+// Calls a library entry point with `t`'s device current, on its current stream (every entry point's
+// last argument), without the GIL (a full launch queue blocks); gives the status. The arguments are
+// values: tensors are read while the GIL is held.
+template <class F, class... A>
+PyObject* launch(const at::Tensor& t, F f, A... a) {
+  TORCH_CHECK(f, "libcdit_hip.so is not bound");
   TORCH_CHECK_VALUE(t.is_cuda(), "expected tensors on the GPU, got a ", t.device(), " tensor");
   const c10::DeviceGuard guard(t.device());
   void* stream = c10::hip::getCurrentHIPStream(t.device().index()).stream();
   int rc;
   Py_BEGIN_ALLOW_THREADS;
-  rc = call(stream);
+  rc = f(a..., stream);
   Py_END_ALLOW_THREADS;
   return PyLong_FromLong(rc);
 }
@@ -274,11 +275,9 @@ PyObject* linear_w8a8(PyObject*, PyObject* const* a, Py_ssize_t n) {
   void* bias = bias_ptr(a[3]);
   const Rows r = rows(x);
   const int mode = (int)integer(a[7]), epi = (int)integer(a[8]);
-  return launch(x, [&](void* stream) {
-    return lib.linear_w8a8(x.data_ptr(), w.data_ptr(), (const float*)ws.data_ptr(), bias, out.data_ptr(),
-                           q.data_ptr(), (float*)s.data_ptr(), r.M, w.size(0), r.K, r.ld, w.stride(0), out_ld(out),
-                           mode, epi, CDIT_DT_BF16, stream);
-  });
+  return launch(x, lib.linear_w8a8, x.data_ptr(), w.data_ptr(), (const float*)ws.data_ptr(), bias, out.data_ptr(),
+                q.data_ptr(), (float*)s.data_ptr(), r.M, w.size(0), r.K, r.ld, w.stride(0), out_ld(out), mode, epi,
+                CDIT_DT_BF16);
   END_HANDLE_TH_ERRORS
 }
 
@@ -290,10 +289,9 @@ PyObject* gemm_rowwise(PyObject*, PyObject* const* a, Py_ssize_t n) {
   void* bias = bias_ptr(a[4]);
   const Rows r = rows(x);
   const int epi = (int)integer(a[6]), id = (int)integer(a[7]);
-  return launch(x, [&](void* stream) {
-    return lib.gemm_rowwise(x.data_ptr(), (const float*)xs.data_ptr(), w.data_ptr(), (const float*)ws.data_ptr(), bias,
-                            out.data_ptr(), r.M, w.size(0), r.K, r.ld, w.stride(0), out_ld(out), epi, id, stream);
-  });
+  return launch(x, lib.gemm_rowwise, x.data_ptr(), (const float*)xs.data_ptr(), w.data_ptr(),
+                (const float*)ws.data_ptr(), bias, out.data_ptr(), r.M, w.size(0), r.K, r.ld, w.stride(0),
+                out_ld(out), epi, id);
   END_HANDLE_TH_ERRORS
 }
 
@@ -305,10 +303,8 @@ PyObject* w8a16(PyObject*, PyObject* const* a, Py_ssize_t n) {
   void* bias = bias_ptr(a[3]);
   const Rows r = rows(x);
   const int epi = (int)integer(a[5]);
-  return launch(x, [&](void* stream) {
-    return lib.w8a16_gemm(x.data_ptr(), w.data_ptr(), (const float*)ws.data_ptr(), bias, out.data_ptr(), r.M,
-                          w.size(0), r.K, r.ld, w.stride(0), out_ld(out), epi, CDIT_DT_BF16, stream);
-  });
+  return launch(x, lib.w8a16_gemm, x.data_ptr(), w.data_ptr(), (const float*)ws.data_ptr(), bias, out.data_ptr(), r.M,
+                w.size(0), r.K, r.ld, w.stride(0), out_ld(out), epi, CDIT_DT_BF16);
   END_HANDLE_TH_ERRORS
 }
 
@@ -320,9 +316,7 @@ PyObject* quant_rowwise(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const Rows r = rows(x);
   const int64_t ldq = rows(q).ld;
   const int mode = (int)integer(a[3]);
-  return launch(x, [&](void* stream) {
-    return lib.quant_rowwise(x.data_ptr(), r.M, r.K, r.ld, q.data_ptr(), ldq, (float*)s.data_ptr(), mode, stream);
-  });
+  return launch(x, lib.quant_rowwise, x.data_ptr(), r.M, r.K, r.ld, q.data_ptr(), ldq, (float*)s.data_ptr(), mode);
   END_HANDLE_TH_ERRORS
 }
 
@@ -334,10 +328,8 @@ PyObject* quant_tensorwise(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const Rows r = rows(x);
   const int64_t ldq = rows(q).ld;
   const int mode = (int)integer(a[4]);
-  return launch(x, [&](void* stream) {
-    return lib.quant_tensorwise(x.data_ptr(), r.M, r.K, r.ld, q.data_ptr(), ldq, (float*)s.data_ptr(),
-                                amax.data_ptr(), mode, stream);
-  });
+  return launch(x, lib.quant_tensorwise, x.data_ptr(), r.M, r.K, r.ld, q.data_ptr(), ldq, (float*)s.data_ptr(),
+                amax.data_ptr(), mode);
   END_HANDLE_TH_ERRORS
 }
 
@@ -349,10 +341,8 @@ PyObject* quant_rowwise_cat2(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const Rows r1 = rows(x1), r2 = rows(x2);
   const int64_t ldq = rows(q).ld;
   const int mode = (int)integer(a[4]);
-  return launch(x1, [&](void* stream) {
-    return lib.quant_rowwise_cat2(x1.data_ptr(), r1.K, r1.ld, x2.data_ptr(), r2.K, r2.ld, r1.M, q.data_ptr(), ldq,
-                                  (float*)s.data_ptr(), mode, stream);
-  });
+  return launch(x1, lib.quant_rowwise_cat2, x1.data_ptr(), r1.K, r1.ld, x2.data_ptr(), r2.K, r2.ld, r1.M,
+                q.data_ptr(), ldq, (float*)s.data_ptr(), mode);
   END_HANDLE_TH_ERRORS
 }
 
@@ -396,9 +386,7 @@ PyObject* quant_rowwise_batched(PyObject*, PyObject* const* a, Py_ssize_t n) {
     ldx[i] = r.ld;
     ldq[i] = rows(qi).ld;
   }
-  return launch(x0, [&](void* stream) {
-    return lib.quant_rowwise_batched((int)items.size(), x, m, K, ldx, q, ldq, s, mode, stream);
-  });
+  return launch(x0, lib.quant_rowwise_batched, (int)items.size(), x, m, K, ldx, q, ldq, s, mode);
   END_HANDLE_TH_ERRORS
 }
 
@@ -457,12 +445,10 @@ PyObject* gemm_batched(PyObject*, PyObject* const* args, Py_ssize_t n) {
       epi[p] = (int)integer(e[j]);
     }
   }
-  return launch(a0, [&](void* stream) {
-    const int na = (int)acts.size();
-    return weight_only ? lib.w8a16_gemm_batched(na, a, M, K, lda, members, b, bs, bias, out, N, ldb, ldo, epi, stream)
-                       : lib.gemm_rowwise_batched(na, a, as, M, K, lda, members, b, bs, bias, out, N, ldb, ldo, epi,
-                                                  stream);
-  });
+  const int na = (int)acts.size();
+  return weight_only ? launch(a0, lib.w8a16_gemm_batched, na, a, M, K, lda, members, b, bs, bias, out, N, ldb, ldo, epi)
+                     : launch(a0, lib.gemm_rowwise_batched, na, a, as, M, K, lda, members, b, bs, bias, out, N, ldb,
+                              ldo, epi);
   END_HANDLE_TH_ERRORS
 }
 
@@ -506,11 +492,9 @@ PyObject* ln_modulate_quant(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const int64_t nb = sh.numel() / r.K;
   if (nb != 1 && !(nb > 0 && x.dim() >= 2 && nb == x.size(0) && r.M % nb == 0)) Py_RETURN_NONE;
   at::Tensor y = empty(x.sizes(), kBf16, x), q = empty(x.sizes(), kFp8, x), s = empty_like_rows(x, 1, kF32);
-  return with_status(launch(x, [&](void* stream) {
-    return lib.ln_modulate_quant(x.data_ptr(), r.M, r.K, r.ld, sh.data_ptr(), sc.data_ptr(), r.K,
-                                 nb == 1 ? r.M : r.M / nb, (float)eps, write_y ? y.data_ptr() : nullptr, r.K,
-                                 q.data_ptr(), r.K, (float*)s.data_ptr(), mode, stream);
-  }), {y, q, s});
+  return with_status(launch(x, lib.ln_modulate_quant, x.data_ptr(), r.M, r.K, r.ld, sh.data_ptr(), sc.data_ptr(), r.K,
+                            nb == 1 ? r.M : r.M / nb, (float)eps, write_y ? y.data_ptr() : nullptr, r.K, q.data_ptr(),
+                            r.K, (float*)s.data_ptr(), mode), {y, q, s});
   END_HANDLE_TH_ERRORS
 }
 
@@ -522,9 +506,7 @@ PyObject* comm_per_token_quant(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (x.scalar_type() != kBf16 || x.dim() < 1 || x.numel() == 0 || !x.is_contiguous()) Py_RETURN_NONE;
   const int64_t H = x.size(-1), M = x.numel() / H;
   at::Tensor y = empty_like_rows(x, H + 2, kFp8);
-  return with_status(launch(x, [&](void* stream) {
-    return lib.comm_per_token_quant(x.data_ptr(), M, H, y.data_ptr(), stream);
-  }), {y});
+  return with_status(launch(x, lib.comm_per_token_quant, x.data_ptr(), M, H, y.data_ptr()), {y});
   END_HANDLE_TH_ERRORS
 }
 PyObject* comm_per_token_dequant(PyObject*, PyObject* const* a, Py_ssize_t n) {
@@ -534,9 +516,7 @@ PyObject* comm_per_token_dequant(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (x.scalar_type() != kFp8 || x.dim() < 1 || x.numel() == 0 || !x.is_contiguous() || x.size(-1) < 3) Py_RETURN_NONE;
   const int64_t H = x.size(-1) - 2, M = x.numel() / (H + 2);
   at::Tensor y = empty_like_rows(x, H, kBf16);
-  return with_status(launch(x, [&](void* stream) {
-    return lib.comm_per_token_dequant(x.data_ptr(), M, H, y.data_ptr(), stream);
-  }), {y});
+  return with_status(launch(x, lib.comm_per_token_dequant, x.data_ptr(), M, H, y.data_ptr()), {y});
   END_HANDLE_TH_ERRORS
 }
 PyObject* comm_qkv_permute_quant(PyObject*, PyObject* const* a, Py_ssize_t n) {
@@ -546,10 +526,8 @@ PyObject* comm_qkv_permute_quant(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (x.scalar_type() != kBf16 || x.dim() != 5 || x.stride(4) != 1 || x.stride(3) != x.size(4)) Py_RETURN_NONE;
   const int64_t B = x.size(0), S = x.size(1), P = x.size(2), N = x.size(3), D = x.size(4);
   at::Tensor y = empty({P, S, B, N, D + 4}, kFp8, x);
-  return with_status(launch(x, [&](void* stream) {
-    return lib.comm_qkv_permute_quant(x.data_ptr(), B, S, P, N, D, x.stride(0), x.stride(1), x.stride(2), y.data_ptr(),
-                                      stream);
-  }), {y});
+  return with_status(launch(x, lib.comm_qkv_permute_quant, x.data_ptr(), B, S, P, N, D, x.stride(0), x.stride(1),
+                            x.stride(2), y.data_ptr()), {y});
   END_HANDLE_TH_ERRORS
 }
 PyObject* comm_qkv_permute_dequant(PyObject*, PyObject* const* a, Py_ssize_t n) {
@@ -559,10 +537,8 @@ PyObject* comm_qkv_permute_dequant(PyObject*, PyObject* const* a, Py_ssize_t n) 
   if (x.scalar_type() != kFp8 || x.dim() != 4 || x.stride(3) != 1 || x.size(3) < 4) Py_RETURN_NONE;
   const int64_t S = x.size(0), B = x.size(1), N = x.size(2), D = x.size(3) - 4;
   at::Tensor y = empty({B, S, N, D}, kBf16, x);
-  return with_status(launch(x, [&](void* stream) {
-    return lib.comm_qkv_permute_dequant(x.data_ptr(), S, B, N, D, x.stride(0), x.stride(1), x.stride(2), y.data_ptr(),
-                                        stream);
-  }), {y});
+  return with_status(launch(x, lib.comm_qkv_permute_dequant, x.data_ptr(), S, B, N, D, x.stride(0), x.stride(1),
+                            x.stride(2), y.data_ptr()), {y});
   END_HANDLE_TH_ERRORS
 }
 
