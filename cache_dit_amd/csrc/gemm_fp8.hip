@@ -1255,7 +1255,12 @@ int launch_wide_grouped(const GemmArgs& g, GemmGroup grp, hipStream_t stream) {
 // steps ahead; one barrier per step: in front of it step kt + 1 has landed, behind it the
 // operands of step kt are in registers and its stage is free. MFMA, K order and epilogue
 // arithmetic are those of the wide kernel and its instances for K remainders, so the results are
-// bit-identical to them (a member of a batch may run there).
+// bit-identical to them (a member of a batch may run there). Up to 16 rows they are those of the
+// 16-row kernel instead, bit for bit: four sums over a quarter of the steps each, added at the end
+// (one chain over all of K is further from the 64-bit sum, with K remainders, whose sums are in
+// full fp32, by more the longer it is: 16 x 512 x 15376, M x N x K, 1.9e-7 against 9.6e-8 of normal
+// values, 5.1e-7 against 9.8e-8 of positive ones). That costs 0.1 us, with K remainders 0.4: 16 x 3072 x
+3072 5.7 -> 5.8, 16 x 3072 x 2992 6.7 -> 7.2.
 // What bounds it: the feeding wavefronts' DMA instructions (4 a step and wavefront) and the
 // barrier, about 250 clocks a step; K remainders the conversions as well. Four feeding wavefronts:
 // no faster. D = 5 against 4: up to 8 % faster where K is long (52 x 15104 x 2304, M x K x N: 17.9 us against
@@ -1265,7 +1270,7 @@ int launch_wide_grouped(const GemmArgs& g, GemmGroup grp, hipStream_t stream) {
 // tiles) 16.1 -> 15.3; K remainders 158 x 2656 x 304 17.2 -> 6.6, 22 x 2832 x 3984 18.9 -> 7.5, 300 x
 // 2224 x 3072 (960 tiles) 16.6 -> 14.3.
 constexpr int kTile32Depth = 5;
-template <int OUT, bool KTAIL, bool GELU>
+template <int OUT, bool KTAIL, bool GELU, bool FEW>
 __global__ __launch_bounds__(384) void gemm_fp8_tile32(GemmArgs g, int tiles_m, int tiles_n) {
   constexpr int D = kTile32Depth, BKW = 128, PANEL = 32 * BKW, STAGE = 2 * PANEL, NDMA = 4;
   static_assert(D >= 3 && (D - 1) * NDMA <= 63 && D * STAGE <= 64 * 1024, "vmcnt has 6 bits; LDS without opt-in");
@@ -1361,9 +1366,31 @@ __global__ __launch_bounds__(384) void gemm_fp8_tile32(GemmArgs g, int tiles_m, 
     }
     stage = stage + STAGE == D * STAGE ? 0 : stage + STAGE;
   };
-  for (int kt = 0; kt < KT; kt += 2) {
-    step(even, odd);
-    if (kt + 1 < KT) step(odd, even);
+  if constexpr (!FEW) {
+    for (int kt = 0; kt < KT; kt += 2) {
+      step(even, odd);
+      if (kt + 1 < KT) step(odd, even);
+    }
+  } else {
+    const int per = (KT + 3) / 4;
+    v4f part[4];
+    int kt = 0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int end = min(KT, (q + 1) * per);
+      for (; kt + 1 < end; kt += 2) {
+        step(even, odd);
+        step(odd, even);
+      }
+      if (kt < end) {
+        step(even, odd);
+        even = odd;
+        ++kt;
+      }
+      part[q] = acc;
+      acc = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+    acc = (part[0] + part[1]) + (part[2] + part[3]);
   }
 
   // acc[e] is out[m][n + e]
@@ -1373,7 +1400,12 @@ __global__ __launch_bounds__(384) void gemm_fp8_tile32(GemmArgs g, int tiles_m, 
   float v[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
-    v[e] = __fmaf_rn(acc[e] * as, bs[e], b4[e]);
+    if constexpr (!FEW) {
+      v[e] = __fmaf_rn(acc[e] * as, bs[e], b4[e]);
+    } else {
+      v[e] = acc[e] * as * bs[e];
+      if (g.bias) v[e] += b4[e];
+    }
     if constexpr (GELU) v[e] = gelu_tanh(v[e]);
   }
   const int64_t at = (int64_t)m * g.ldo + n;
@@ -1391,10 +1423,13 @@ int launch_tile32(const GemmArgs& g, hipStream_t stream) {
   const int tiles_m = (g.M + 31) / 32, tiles_n = (g.N + 31) / 32;
   const dim3 grid((tiles_n + 7) / 8 * 8 * tiles_m), block(384);
   constexpr int lds = kTile32Depth * 2 * 32 * 128;
-  if (g.epilogue & CDIT_EPI_GELU_TANH)
-    hipLaunchKernelGGL((gemm_fp8_tile32<OUT, KTAIL, true>), grid, block, lds, stream, g, tiles_m, tiles_n);
-  else
-    hipLaunchKernelGGL((gemm_fp8_tile32<OUT, KTAIL, false>), grid, block, lds, stream, g, tiles_m, tiles_n);
+  auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, lds, stream, g, tiles_m, tiles_n); };
+  const bool gelu = g.epilogue & CDIT_EPI_GELU_TANH;
+  if (g.M <= 16) {
+    gelu ? go(&gemm_fp8_tile32<OUT, KTAIL, true, true>) : go(&gemm_fp8_tile32<OUT, KTAIL, false, true>);
+  } else {
+    gelu ? go(&gemm_fp8_tile32<OUT, KTAIL, true, false>) : go(&gemm_fp8_tile32<OUT, KTAIL, false, false>);
+  }
   return 0;
 }
 
@@ -1927,9 +1962,8 @@ int launch_row1(const GemmArgs& g, uint8_t* q_ws, float* scale_ws, int scale_mod
 // 5120 18.2 / 13.3, 4 x 9216 x 5120 20.3 / 16.9, 4 x 18432 x 2048 14.5 / 13.1, 2 x 9216 x 5120 18.6 / 16.9; 16 x 3072 x
 // 1024 8.8 / 6.5, 8 x 6144 x 3072 11.9 / 10.2, 4 x 9216 x 3072 12.6 / 11.9, 2 x 18432 x 3072 17.2 / 17.6. (What is near on
 // both sides and about 10 us is left to the single launch: a call of two takes the host 2.7 us longer.)
-// The distance from 64-bit sums is the same on both (1.5e-5 of normal rows, 2.5e-5 with outliers, K
-// 1024 to 5120). The rule looks at nothing that differs between the Linear and its GEMM alone, so
-// that both give the same bits.
+// Both give the same bits (for K of 128 and 256 the tiles' sums are the more exact ones), and the rule looks at
+// nothing that differs between the Linear and its GEMM alone.
 bool few_on_tiles(const GemmArgs& g) {
   const int64_t weights = (int64_t)g.N * g.K;
   if (g.M >= 9) return g.K > 2048 || g.N > 9216;

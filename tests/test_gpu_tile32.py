@@ -87,3 +87,40 @@ def test_on_both_sides_of_the_tile_rule(M, N, K):
     ops.gemm_rowwise_into(a, one_m, w, one_n, None, out, 0)
     torch.cuda.synchronize()
     assert torch.equal(out, want.to(dtype)), dtype
+
+
+@pytest.mark.parametrize("positive", [False, True])
+@pytest.mark.parametrize("M,N", [(2, 40), (9, 264), (16, 8)])
+def test_few_rows_have_the_16_row_kernels_bits(M, N, positive):
+  """Up to 16 rows either kernel may run, and a sum is in four parts on both: same bits for every type, bias and
+  epilogue, with no, one, two and three empty parts. fp32 outputs against 64-bit sums: with K remainders a part is a
+  chain of fp32 roundings, at most one per 8 products, each of 2^-24 of what is summed by then; for whole steps
+  the FP8 instruction drops what is some 13 places below its largest product, from each product at most 2^-13
+  of that, in either direction (as often up as down for normal values, all one way for positive ones)."""
+  from cache_dit_amd import _native, ops
+  for K in (16, 112, 128, 144, 256, 400, 640, 1152, 1296, 5120, 15360, 15376):
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    a, w = (torch.randn(n, K, generator=g, device=DEV) for n in (M, N))
+    a, w = ((t.abs() if positive else t).mul_(100.0).clamp_(-448, 448).to(FP8) for t in (a, w))
+    sa, sw = torch.rand(M, generator=g, device=DEV), torch.rand(N, generator=g, device=DEV)
+    for dtype in (torch.float32, torch.bfloat16, torch.float16):
+      b = None if dtype == torch.float32 else torch.randn(N, generator=g, device=DEV).to(dtype)
+      scale = sa * (1e-4 if dtype == torch.float16 else 1.0)  # (within fp16's range)
+      for bias in (None, b):
+        for epilogue in (0, 1):
+          outs = []
+          for variant in (50, 26):
+            _native.set_gemm_variant(variant)
+            outs.append(torch.empty(M, N, dtype=dtype, device=DEV))
+            ops.gemm_rowwise_into(a, scale, w, sw, bias, outs[-1], epilogue)
+          torch.cuda.synchronize()
+          if K % 128 or K >= 384:  # (whole steps shorter than that take the instance for remainders)
+            assert torch.equal(outs[0], outs[1]), (K, dtype, bias is None, epilogue)
+          if dtype == torch.float32 and epilogue == 0:
+            ad, wd = a.double() * sa.double()[:, None], w.double() * sw.double()[:, None]
+            err = (outs[1].double() - ad @ wd.t()).abs()
+            if K % 128 or K < 384:
+              bound = (K / 32 + 8) * 2.0**-24 * (ad.abs() @ wd.abs().t())
+            else:
+              bound = K * 2.0**-13 * ad.abs().amax(1)[:, None] * wd.abs().amax(1)
+            assert bool((err <= bound).all()), K
