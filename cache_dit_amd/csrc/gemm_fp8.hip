@@ -1260,7 +1260,7 @@ int launch_wide_grouped(const GemmArgs& g, GemmGroup grp, hipStream_t stream) {
 // (one chain over all of K is further from the 64-bit sum, with K remainders, whose sums are in
 // full fp32, by more the longer it is: 16 x 512 x 15376, M x N x K, 1.9e-7 against 9.6e-8 of normal
 // values, 5.1e-7 against 9.8e-8 of positive ones). That costs 0.1 us, with K remainders 0.4: 16 x 3072 x
-3072 5.7 -> 5.8, 16 x 3072 x 2992 6.7 -> 7.2.
+// 3072 5.7 -> 5.8, 16 x 3072 x 2992 6.7 -> 7.2.
 // What bounds it: the feeding wavefronts' DMA instructions (4 a step and wavefront) and the
 // barrier, about 250 clocks a step; K remainders the conversions as well. Four feeding wavefronts:
 // no faster. D = 5 against 4: up to 8 % faster where K is long (52 x 15104 x 2304, M x K x N: 17.9 us against
