@@ -51,6 +51,8 @@ EXPORTS = (
     "cdit_fp8_comm_qkv_permute_dequant",
     "cdit_debug_set_gemm_variant",
     "cdit_debug_set_quant_hints",
+    "cdit_debug_gemm_choice",
+    "cdit_debug_linear_launches",
     "cdit_debug_mfma_only",
     "cdit_debug_gemm_stamps",
     "cdit_stream_capture_id",
@@ -79,6 +81,10 @@ def _bind(L: ctypes.CDLL) -> None:
   L.cdit_debug_set_gemm_variant.argtypes = [ci]
   L.cdit_debug_set_quant_hints.restype = ci
   L.cdit_debug_set_quant_hints.argtypes = [ci]
+  L.cdit_debug_gemm_choice.restype = ci
+  L.cdit_debug_gemm_choice.argtypes = [ci, i64, i64, i64, ci]
+  L.cdit_debug_linear_launches.restype = ci
+  L.cdit_debug_linear_launches.argtypes = [i64, i64, i64]
   L.cdit_debug_mfma_only.restype = ci
   L.cdit_debug_mfma_only.argtypes = [vp, ci, ci, ci, ctypes.POINTER(ctypes.c_double), vp]
   L.cdit_debug_gemm_stamps.restype = ci

@@ -154,6 +154,32 @@ int cdit_debug_set_gemm_variant(int variant) {
   return prev;
 }
 
+// A problem with contiguous, aligned operands; false: not one that an entry point takes.
+static bool shape_only(GemmArgs* g, int64_t M, int64_t N, int64_t K, int out_dtype_id) {
+  if (M < 1 || N < 1 || K < 1 || M > INT32_MAX || N > INT32_MAX || K > INT32_MAX || out_dtype_id < CDIT_DT_F16 ||
+      out_dtype_id > CDIT_DT_F32)
+    return false;
+  *g = GemmArgs{};
+  g->M = (int)M;
+  g->N = (int)N;
+  g->K = (int)K;
+  g->lda = g->ldb = K;
+  g->ldo = N;
+  g->out_dtype = out_dtype_id;
+  return true;
+}
+
+int cdit_debug_gemm_choice(int weight_only, int64_t M, int64_t N, int64_t K, int out_dtype_id) {
+  GemmArgs g;
+  if (!shape_only(&g, M, N, K, out_dtype_id) || weight_only) return -1;
+  return choose_gemm_fp8(g);
+}
+
+int cdit_debug_linear_launches(int64_t M, int64_t N, int64_t K) {
+  GemmArgs g;
+  return shape_only(&g, M, N, K, CDIT_DT_BF16) ? linear_fp8_launches(g) : -1;
+}
+
 int cdit_debug_set_quant_hints(int hints) {
   int prev = cdit::g_quant_variant;
   cdit::g_quant_variant = hints >= 0 && hints <= 7 ? hints : -1;
@@ -574,8 +600,8 @@ int cdit_fp8_linear_w8a8(const void* x_bf16, const void* w_q, const float* w_sca
                          const void* bias, void* out, void* q_ws, float* scale_ws, int64_t M,
                          int64_t N, int64_t K, int64_t ld_x, int64_t ldw, int64_t ldo,
                          int scale_mode, int epilogue, int out_dtype_id, void* stream) {
-  // M <= 16 (the M = 1 modulation Linears): one kernel that quantizes the rows itself,
-  // when every argument passes the checks of the two entry points it stands for
+  // M <= 16 (the M = 1 modulation Linears): one kernel that quantizes the rows itself where
+  // that is faster than two (few_quantized_apart()), when every argument passes the checks of the two entry points it stands for
   if (M >= 1 && M <= 16 && N > 0 && K > 0 && K <= INT32_MAX && N <= INT32_MAX && x_bf16 && q_ws &&
       scale_ws && w_scale && ld_x >= K &&
       (scale_mode == CDIT_SCALE_BF16DIV || scale_mode == CDIT_SCALE_FP32DIV) &&

@@ -95,6 +95,10 @@ struct GemmGroup {
   int epilogue[kMaxGroup];
 };
 
+// The kernel variant for a problem, and the launches of a w8a8 Linear of a problem's shape (1: the GEMM's kernel
+// quantizes the rows itself).
+int choose_gemm_fp8(const GemmArgs& g);
+int linear_fp8_launches(const GemmArgs& g);
 // variant < 0: choose by shape.
 int launch_gemm_fp8(const GemmArgs& g, int variant, hipStream_t stream);
 // the 288 x 192 kernel with per-workgroup time stamps (measurement only; gemm_fp8.hip)
@@ -109,10 +113,10 @@ int launch_gemm_w8a16(const GemmArgs& g, int variant, hipStream_t stream);
 // The same for the weight-only GEMM (grp.a: bf16 activations; grp.a_scale unused).
 int launch_gemm_w8a16_grouped(const GemmArgs& common, const GemmGroup& grp, int variant,
                               hipStream_t stream);
-// One w8a8 Linear forward at M <= 16 in a single kernel (per-token quantizer + GEMM);
+// One w8a8 Linear forward of few rows in a single kernel (per-token quantizer + GEMM);
 // g.a is the bf16 activation, g.lda its leading dimension in elements. Returns 0 when
-// launched, 1 when the shape or alignment is not taken (the caller then runs the
-// quantizer and the GEMM one after the other).
+// launched, 1 when the shape or alignment is not taken or two launches are faster (the caller then
+// runs the quantizer and the GEMM one after the other).
 int launch_linear_fp8_skinny_fused(const GemmArgs& g, void* q_ws, float* scale_ws, int scale_mode,
                                    int variant, hipStream_t stream);
 

@@ -1920,18 +1920,17 @@ typedef CfgWide<256, 128, 4> V19;                     // ... 128x64 wave tiles, 
 typedef CfgWide<256, 256, 4, 2, false> V12H;
 typedef CfgWide<288, 192, 4, 2, false> V14H;
 
-bool few_on_tiles(const GemmArgs& g);
-
+// Whether the M = 1 kernel takes a shape whose operands are aligned as it asks.
+bool row1_ok(const GemmArgs& g) {
+  return g.M == 1 && g.K >= 16 && g.K % 16 == 0 && g.K <= 4096 && g.ldb % 16 == 0 &&
+         reinterpret_cast<uintptr_t>(g.a) % 16 == 0 && reinterpret_cast<uintptr_t>(g.b) % 16 == 0;
+}
 // The M = 1 kernel when the shape fits it (variant 51 forces it, 50 the 16-row kernel);
 // returns 1 when it is not taken.
 template <bool FUSED>
 int launch_row1(const GemmArgs& g, uint8_t* q_ws, float* scale_ws, int scale_mode, int variant,
                 hipStream_t stream) {
-  const bool ok = g.M == 1 && g.K >= 16 && g.K % 16 == 0 && g.K <= 4096 && g.ldb % 16 == 0 &&
-                  reinterpret_cast<uintptr_t>(g.a) % 16 == 0 && reinterpret_cast<uintptr_t>(g.b) % 16 == 0 &&
-                  (!FUSED || reinterpret_cast<uintptr_t>(q_ws) % 8 == 0) &&
-                  (variant < 0 || variant == 51);
-  if (!ok) return 1;
+  if (!row1_ok(g) || (FUSED && reinterpret_cast<uintptr_t>(q_ws) % 8 != 0) || (variant >= 0 && variant != 51)) return 1;
   constexpr int rows_wg = kRow1Rows * kRow1Waves;
   auto go = [&](auto chk_tag) {
     constexpr int CHK = decltype(chk_tag)::value;
@@ -1953,24 +1952,46 @@ int launch_row1(const GemmArgs& g, uint8_t* q_ws, float* scale_ws, int scale_mod
   return 0;
 }
 
-// Whether 2 to 16 rows go to the kernel with a workgroup per 32 x 32 tile, behind a launch of the
-// quantizer where they come as bf16, instead of the 16-row kernel, which quantizes them itself.
-// That grows with the rows per wavefront and their length in every workgroup, and its loads
-// take 64-byte pieces of 16 rows; the tiles cost a launch (2.2 to 3 us) and no more with 16 rows than with
-// 2. us, the whole Linear in one kernel / with tiles, another weight matrix per launch, M x N x K: 16 x 9216 x 3072
-// 24.8 / 12.7, 16 x 18432 x 5120 36.6 / 26.7, 12 x 3072 x 3072 10.7 / 8.3, 8 x 18432 x 3072 23.7 / 17.8, 8 x 6144 x
-// 5120 18.2 / 13.3, 4 x 9216 x 5120 20.3 / 16.9, 4 x 18432 x 2048 14.5 / 13.1, 2 x 9216 x 5120 18.6 / 16.9; 16 x 3072 x
-// 1024 8.8 / 6.5, 8 x 6144 x 3072 11.9 / 10.2, 4 x 9216 x 3072 12.6 / 11.9, 2 x 18432 x 3072 17.2 / 17.6. (What is near on
-// both sides and about 10 us is left to the single launch: a call of two takes the host 2.7 us longer.)
-// Both give the same bits (for K of 128 and 256 the tiles' sums are the more exact ones), and the rule looks at
-// nothing that differs between the Linear and its GEMM alone.
-bool few_on_tiles(const GemmArgs& g) {
+// 2 to 16 rows on many weights, where the kernel with a workgroup per 32 x 32 tile is faster than the 16-row
+// kernel. The latter's loads take 64-byte pieces of 16 rows, and with the quantizer inside it grows
+// with the rows per wavefront and their length in every workgroup.
+// us, the whole Linear in one kernel / with tiles, another weight matrix per launch, M x N x K: 16 x 9216 x 3072
+// 24.8 / 12.7, 16 x 18432 x 5120 36.6 / 26.7, 8 x 18432 x 3072 23.7 / 17.8, 8 x 6144 x 5120 18.2 / 13.3,
+// 4 x 9216 x 5120 20.3 / 16.9, 4 x 18432 x 2048 14.5 / 13.1, 2 x 9216 x 5120 18.6 / 16.9, 2 x 18432 x 3072 17.2 / 17.6.
+bool few_on_many(const GemmArgs& g) {
   const int64_t weights = (int64_t)g.N * g.K;
   if (g.M >= 9) return g.K > 2048 || g.N > 9216;
   if (g.M >= 5) return weights > 20000000 || g.N > 12288;
   if (g.M >= 3) return weights > 30000000;
   return g.M == 2 && g.K > 4096 && weights > 40000000;
 }
+// The GEMM of 2 to 16 rows on tiles. Up to 4096 columns either kernel is one round of the CUs, and the time that
+// of one workgroup: a tile takes its steps of 128 elements one after the other, 130 to 170 ns each as the weights come from
+// the last-level cache or from HBM (with K remainders 175 to 200), the 16-row kernel splits K over four wavefronts
+// with six steps of each in flight, 2.3 to 3 us (2.7 to 4.5) for 24 steps. So the tiles are faster only
+// where the last batch of 24 is nearly empty. us, 16-row / tiles, M x N x K: 9 x 576 x 14608 15.7 / 22.3, 8 x 2048 x
+// 12288 14.4 / 19.0, 4 x 2048 x 15360 16.3 / 22.7, 2 x 4096 x 15360 17.3 / 24.1, 9 x 1024 x 3072 5.3 / 5.6;
+// 9 x 256 x 3200 7.0 / 6.1, 16 x 384 x 8736 17.2 / 15.2. Over 600 shapes of up to 4500 columns it is 1 % off the
+// better one.
+// Both kernels give the same bits (for K of 128 and 256 the tiles' sums are the more exact ones).
+bool few_on_tiles(const GemmArgs& g) {
+  if (!few_on_many(g)) return false;
+  if (g.N > 4096) return true;
+  const bool tail = g.K % BK != 0;
+  const int64_t steps = (g.K + BK - 1) / BK, batches = (steps + 23) / 24;
+  return steps * (tail ? 190 : 158) < batches * (tail ? 2450 + 125 * g.M : 2250 + 45 * g.M);
+}
+// A Linear of 2 to 16 bf16 rows as the quantizer's launch (2.2 to 3 us) and the GEMM's, instead of the 16-row kernel that
+// quantizes them itself. What is near on both sides and about 10 us is left to the single launch: a
+// call of two takes the host 2.7 us longer. Rows beyond 16384 elements are long to quantize apart (140 us, where
+// the single kernel takes two of them: 2 x 16192 x 16512, M x N x K, 73 us in one kernel and 176 in two); on up to
+// 4096 columns the single kernel is the faster one below five rows (2 x 2816 x 15360 22.6 / 26.5).
+bool few_quantized_apart(const GemmArgs& g) {
+  return few_on_many(g) && g.K <= 16384 && (g.N > 4096 || g.M >= 5);
+}
+
+constexpr int kFusedLds = 56 * 1024;
+int64_t fused_lds(const GemmArgs& g) { return (int64_t)g.M * (g.K + kFusedPad); }
 
 int launch_linear_fp8_skinny_fused(const GemmArgs& g, void* q_ws, float* scale_ws, int scale_mode,
                                    int variant, hipStream_t stream) {
@@ -1983,9 +2004,9 @@ int launch_linear_fp8_skinny_fused(const GemmArgs& g, void* q_ws, float* scale_w
   two_step.lda = g.K;
   if (!aligned_ok(two_step)) return 1;
   if (launch_row1<true>(g, static_cast<uint8_t*>(q_ws), scale_ws, scale_mode, variant, stream) == 0) return 0;
-  const int64_t lds = (int64_t)g.M * (g.K + kFusedPad);
-  const bool ok = g.M >= 1 && g.M <= 16 && (variant == 50 || (variant < 0 && !few_on_tiles(g))) && g.K >= 16 &&
-                  g.K % 16 == 0 && g.N % 8 == 0 && lds <= 56 * 1024 && g.lda % 8 == 0 &&
+  const int64_t lds = fused_lds(g);
+  const bool ok = g.M >= 1 && g.M <= 16 && (variant == 50 || (variant < 0 && !few_quantized_apart(g))) && g.K >= 16 &&
+                  g.K % 16 == 0 && g.N % 8 == 0 && lds <= kFusedLds && g.lda % 8 == 0 &&
                   g.ldb % 16 == 0 && g.ldo % 8 == 0 &&
                   reinterpret_cast<uintptr_t>(g.a) % 16 == 0 &&
                   reinterpret_cast<uintptr_t>(g.b) % 16 == 0 &&
@@ -2016,6 +2037,7 @@ constexpr LaunchModel kLaunch = {4600, 700, 760};
 constexpr TileTime kTiles[] = {{12, 256, 256, V12::DEPTH, 6400, 1227}, {14, 288, 192, V14::DEPTH, 4600, 1029},
                                {15, 256, 192, V15::DEPTH, 4400, 946},  {16, 128, 192, V16::DEPTH, 3500, 552},
                                {18, 128, 128, V18::DEPTH, 2100, 445},  {17, 64, 128, V17::DEPTH, 1300, 332}};
+int choose_ktail_variant(const GemmArgs& g, int variant);
 int launch_gemm_fp8_ktail(const GemmArgs& g, int variant, hipStream_t stream);
 template <class WideOk>
 int launch_bf16_variant(const GemmArgs& g, int variant, WideOk wide_ok, hipStream_t stream);
@@ -2070,16 +2092,59 @@ int launch_other_out(const GemmArgs& g, int variant, hipStream_t stream) {
   }
 }
 
+// Whether K takes the tile kernel's instances for K remainders. A K of one or two steps does as well: fp16 and
+// fp32 outputs of such a K have their sums in full fp32 (from the kernel for any shape), and the
+// conversions of two steps cost nothing (36 x 3904 x 256, M x N x K: 7.4 us with the tiled kernel, 4.2).
+bool tile32_tail(const GemmArgs& g) { return g.K % BK != 0 || g.K < 3 * BK; }
+
+// at least `depth` K steps to prefetch, and at least 3: the epilogue operands of a tile are
+// staged in LDS two steps before its end, which must be behind the first barrier of the
+// tile (before it, slower waves may still be reading the previous tile's)
+struct WideOk {
+  int K;
+  bool operator()(int depth) const { return K >= 128 * (depth > 3 ? depth : 3); }
+};
+
+// The kernel for a problem: 100 for any shape and alignment, 51 one row, 50 up to 16 rows, 26 a workgroup per
+// 32 x 32 tile, else a tile of the wide kernel (K remainders: of its instances for them) or of the tiled one.
+int choose_gemm_fp8(const GemmArgs& g) {
+  if (!aligned_ok(g)) return 100;
+  if (row1_ok(g)) return 51;
+  if (g.M <= 16) return few_on_tiles(g) ? 26 : 50;
+  // Up to three 32 x 32 tiles per CU: the workgroup-per-tile kernel (figures at the kernel; beyond, it
+  // wins with short K and loses with long: 864 tiles 7.1 us with the wide kernel, 6.4 with this one
+  // at K = 896, 816 tiles 30.1 and 32.9 at K = 10624), with K remainders up to five (1209 tiles 9.5 and
+  // 8.3, 1677 tiles 18.6 and 22.0).
+  const int64_t tiles32 = (int64_t)((g.M + 31) / 32) * ((g.N + 31) / 32);
+  if (tiles32 <= (tile32_tail(g) ? 5 : 3) * (int64_t)(cu_count() > 0 ? cu_count() : 256)) return 26;
+  if (!tiled_ok(g)) return choose_ktail_variant(g, -1);
+  // the wide kernels stream K two or more steps ahead: shorter K runs the 128x128 kernel
+  const WideOk wide_ok{g.K};
+  if (g.out_dtype != CDIT_DT_BF16) {
+    // fp16 / fp32 outputs (the op's other two out_dtype ids); what no wide tile can take
+    // runs the generic kernel.
+    const int v = choose_other_out_variant(g, -1, wide_ok);
+    return v >= 0 ? v : 100;
+  }
+  return choose_bf16_variant(
+      [&](int bm, int bn) { return (int64_t)((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn); }, wide_ok, g.K).variant;
+}
+
+int linear_fp8_launches(const GemmArgs& g) {
+  if (!aligned_ok(g) || g.M > 16) return 2;
+  return row1_ok(g) || (!few_quantized_apart(g) && fused_lds(g) <= kFusedLds) ? 1 : 2;
+}
+
 int launch_gemm_fp8(const GemmArgs& g, int variant, hipStream_t stream) {
-  if (!aligned_ok(g) || variant == 100) {
+  if (!aligned_ok(g)) variant = 100;
+  if (variant < 0) variant = choose_gemm_fp8(g);
+  if (variant == 100) {
     dim3 grid((g.N + 15) / 16, (g.M + 15) / 16);
     hipLaunchKernelGGL(gemm_fp8_generic, grid, dim3(256), 0, stream, g);
     return 0;
   }
-  if ((variant < 0 || variant == 51) &&
-      launch_row1<false>(g, nullptr, nullptr, 0, variant, stream) == 0)
-    return 0;
-  if ((variant < 0 && g.M <= 16 && !few_on_tiles(g)) || variant == 50) {
+  if (variant == 51 && launch_row1<false>(g, nullptr, nullptr, 0, variant, stream) == 0) return 0;
+  if (variant == 50) {
     if (g.M > 16) {
       set_error("cdit_fp8_gemm_rowwise: the skinny kernel takes M <= 16, got %d", g.M);
       return CDIT_EINVAL;
@@ -2091,25 +2156,10 @@ int launch_gemm_fp8(const GemmArgs& g, int variant, hipStream_t stream) {
     }
     return 0;
   }
-  // Few rows (few_on_tiles) and up to three 32 x 32 tiles per CU: the workgroup-per-tile kernel (figures at the kernel; beyond, it
-  // wins with short K and loses with long: 864 tiles 7.1 us with the wide kernel, 6.4 with this one
-  // at K = 896, 816 tiles 30.1 and 32.9 at K = 10624), with K remainders up to five (1209 tiles 9.5 and
-  // 8.3, 1677 tiles 18.6 and 22.0). A K of one or two steps takes the instances for K remainders: fp16 and
-  // fp32 outputs of such a K have their sums in full fp32 (from the kernel for any shape), and the
-  // conversions of two steps cost nothing (36 x 3904 x 256, M x N x K: 7.4 us with the tiled kernel, 4.2).
-  const bool tail = g.K % BK != 0 || g.K < 3 * BK;
-  const int64_t tiles32 = (int64_t)((g.M + 31) / 32) * ((g.N + 31) / 32);
-  if (variant == 26 || (variant < 0 && (g.M <= 16 || tiles32 <= (tail ? 5 : 3) * (int64_t)(cu_count() > 0 ? cu_count() : 256))))
-    return tail ? launch_tile32<true>(g, stream) : launch_tile32<false>(g, stream);
+  if (variant == 26) return tile32_tail(g) ? launch_tile32<true>(g, stream) : launch_tile32<false>(g, stream);
   if (!tiled_ok(g)) return launch_gemm_fp8_ktail(g, variant, stream);
-  // the wide kernels stream K two or more steps ahead: shorter K runs the 128x128 kernel
-  // at least `depth` K steps to prefetch, and at least 3: the epilogue operands of a tile are
-  // staged in LDS two steps before its end, which must be behind the first barrier of the
-  // tile (before it, slower waves may still be reading the previous tile's)
-  auto wide_ok = [&](int depth) { return g.K >= 128 * (depth > 3 ? depth : 3); };
+  const WideOk wide_ok{g.K};
   if (g.out_dtype != CDIT_DT_BF16) {
-    // fp16 / fp32 outputs (the op's other two out_dtype ids); what no wide tile can take
-    // runs the generic kernel.
     const int v = choose_other_out_variant(g, variant, wide_ok);
     if (v >= 0)
       return g.out_dtype == CDIT_DT_F16 ? launch_other_out<CDIT_DT_F16, false>(g, v, stream)
@@ -2117,11 +2167,6 @@ int launch_gemm_fp8(const GemmArgs& g, int variant, hipStream_t stream) {
     dim3 grid((g.N + 15) / 16, (g.M + 15) / 16);
     hipLaunchKernelGGL(gemm_fp8_generic, grid, dim3(256), 0, stream, g);
     return 0;
-  }
-  if (variant < 0) {
-    variant = choose_bf16_variant(
-        [&](int bm, int bn) { return (int64_t)((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn); },
-        wide_ok, g.K).variant;
   }
   return launch_bf16_variant(g, variant, wide_ok, stream);
 }
@@ -2141,7 +2186,7 @@ int launch_gemm_fp8(const GemmArgs& g, int variant, hipStream_t stream) {
 // 75.1 (256 x 128) and 93.8 (128 x 128). The scalar FMA kernel took 16.8 ms for the first. There is
 // no 256 x 256 instance: its converted operands do not fit the registers. fp16 and fp32 outputs
 // have three tiles.
-int launch_gemm_fp8_ktail(const GemmArgs& g, int variant, hipStream_t stream) {
+int choose_ktail_variant(const GemmArgs& g, int variant) {
   const int64_t cus = cu_count() > 0 ? cu_count() : 256;
   const struct { int v, bm, bn, us10; bool other_out; } cand[] = {
       {14, 288, 192, 530, false}, {15, 256, 192, 470, true}, {16, 128, 192, 290, false},
@@ -2155,7 +2200,12 @@ int launch_gemm_fp8_ktail(const GemmArgs& g, int variant, hipStream_t stream) {
     const int64_t t = variant == c.v ? -1 : rounds_permille(tiles, cus, 700, 700) * c.us10;
     if (t < time) best = c.v, time = t;
   }
-  if (!bf16)
+  return best;
+}
+
+int launch_gemm_fp8_ktail(const GemmArgs& g, int variant, hipStream_t stream) {
+  const int best = choose_ktail_variant(g, variant);
+  if (g.out_dtype != CDIT_DT_BF16)
     return g.out_dtype == CDIT_DT_F16 ? launch_other_out<CDIT_DT_F16, true>(g, best, stream)
                                       : launch_other_out<CDIT_DT_F32, true>(g, best, stream);
   switch (best) {
@@ -2259,7 +2309,7 @@ int launch_gemm_fp8_grouped(const GemmArgs& common, const GemmGroup& grp, int va
       if (!tiled_ok(g) || g.N <= 0) return -1;
     }
   }
-  auto wide_ok = [&](int depth) { return common.K >= 128 * (depth > 3 ? depth : 3); };
+  const WideOk wide_ok{common.K};
   auto tiles = [&](int bm, int bn) {
     int64_t t = 0;
     for (int s = 0; s < grp.acts; ++s) {

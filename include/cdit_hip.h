@@ -282,8 +282,8 @@ int cdit_w8a16_gemm_batched(int n_act, const void* const* x_bf16, const int64_t*
  * One quantized nn.Linear forward in the w8a8 dynamic mode: the two calls above
  * back to back on `stream` (per-token quantization of x into the caller's
  * workspace, then the scaled GEMM), saving one trip through the caller's FFI;
- * at M <= 16 a single kernel that quantizes the rows itself, with the same
- * results and the same workspace contents.
+ * at M <= 16 and where that is faster (one row always) a single kernel that
+ * quantizes the rows itself, with the same results and workspace contents.
  * This is what torchao's Float8Tensor `aten.linear` override does for a Linear
  * that cache-dit converted with `quantize_(..., Float8DynamicActivation
  * Float8WeightConfig(granularity=(PerRow(), PerRow())))`
@@ -378,6 +378,15 @@ int cdit_stream_capture_id(void* stream, uint64_t* id);
  */
 int cdit_debug_set_gemm_variant(int variant);
 int cdit_debug_set_quant_hints(int hints);
+
+/*
+ * What the automatic choice is for a shape with contiguous, aligned operands, on the current
+ * device (without one: 256 compute units). Nothing is launched. -1: no such problem.
+ * cdit_debug_gemm_choice: the variant that cdit_fp8_gemm_rowwise runs.
+ * cdit_debug_linear_launches: kernels that cdit_fp8_linear_w8a8 launches, 1 or 2.
+ */
+int cdit_debug_gemm_choice(int weight_only, int64_t M, int64_t N, int64_t K, int out_dtype_id);
+int cdit_debug_linear_launches(int64_t M, int64_t N, int64_t K);
 
 /*
  * Measurement aid, not part of the operator interface (no counterpart in the reference):

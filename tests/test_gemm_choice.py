@@ -1,0 +1,38 @@
+"""The kernels that the GEMM entry points choose by shape, at shapes where the rule was measured on both
+sides (figures beside the rules in csrc/gemm_fp8.hip). No GPU: the choice of 256 compute
+units."""
+import pytest
+
+F16, BF16, F32 = 0, 1, 2
+ROWS16, TILE32, ROW1 = 50, 26, 51
+
+
+@pytest.fixture(scope="module")
+def lib():
+  from cache_dit_amd import _native
+  if not _native.is_built():
+    pytest.skip("libcdit_hip.so not built")
+  return _native.load()
+
+
+@pytest.mark.parametrize("M,N,K,want", [
+    # long K on few columns: the 16-row kernel splits K over four wavefronts
+    (9, 576, 14608, ROWS16), (8, 2048, 12288, ROWS16), (4, 2048, 15360, ROWS16), (2, 4096, 15360, ROWS16),
+    (9, 1024, 3072, ROWS16), (16, 1024, 12288, ROWS16),
+    # a last batch of its steps that is nearly empty
+    (9, 256, 3200, TILE32), (16, 384, 8736, TILE32),
+    # many columns
+    (16, 9216, 3072, TILE32), (16, 18432, 5120, TILE32), (8, 18432, 3072, TILE32), (4, 9216, 5120, TILE32),
+    (2, 18432, 3072, ROWS16), (2, 9216, 5120, TILE32), (1, 9216, 3072, ROW1), (1, 9216, 4112, ROWS16)])
+def test_few_rows(lib, M, N, K, want):
+  for dtype in (F16, BF16, F32):
+    assert lib.cdit_debug_gemm_choice(0, M, N, K, dtype) == want
+
+
+@pytest.mark.parametrize("M,N,K,want", [
+    # rows beyond 16384 elements are quantized in the GEMM's kernel where they fit its LDS
+    (2, 16192, 16512, 1), (2, 22592, 17472, 1), (3, 7936, 18688, 1), (2, 9216, 5120, 2),
+    (2, 2816, 15360, 1), (4, 3456, 14320, 1), (1, 9216, 3072, 1), (8, 3072, 3072, 1),
+    (16, 9216, 3072, 2), (16, 3072, 3072, 2), (8, 2048, 12288, 2), (17, 64, 64, 2)])
+def test_launches_of_few_rows(lib, M, N, K, want):
+  assert lib.cdit_debug_linear_launches(M, N, K) == want
