@@ -1990,8 +1990,12 @@ bool few_quantized_apart(const GemmArgs& g) {
   return few_on_many(g) && g.K <= 16384 && (g.N > 4096 || g.M >= 5);
 }
 
-constexpr int kFusedLds = 56 * 1024;
+// LDS of the codes, and how much of it the kernel may take. From 48 KiB on the rows are so long that quantizing them in
+// every workgroup takes longer than a launch for it: 8 x 192 x 6784 (M x N x K) 14.7 us in one kernel and
+// 11.7 in two, 6 x 256 x 8384 18.1 and 12.3, 4 x 2304 x 12480 24.2 and 20.4. Rows beyond 16384 elements, which are long to
+// quantize apart (few_quantized_apart()), may take 56.
 int64_t fused_lds(const GemmArgs& g) { return (int64_t)g.M * (g.K + kFusedPad); }
+bool fused_fits(const GemmArgs& g) { return fused_lds(g) <= (g.K > 16384 ? 56 : 48) * 1024; }
 
 int launch_linear_fp8_skinny_fused(const GemmArgs& g, void* q_ws, float* scale_ws, int scale_mode,
                                    int variant, hipStream_t stream) {
@@ -2006,7 +2010,7 @@ int launch_linear_fp8_skinny_fused(const GemmArgs& g, void* q_ws, float* scale_w
   if (launch_row1<true>(g, static_cast<uint8_t*>(q_ws), scale_ws, scale_mode, variant, stream) == 0) return 0;
   const int64_t lds = fused_lds(g);
   const bool ok = g.M >= 1 && g.M <= 16 && (variant == 50 || (variant < 0 && !few_quantized_apart(g))) && g.K >= 16 &&
-                  g.K % 16 == 0 && g.N % 8 == 0 && lds <= kFusedLds && g.lda % 8 == 0 &&
+                  g.K % 16 == 0 && g.N % 8 == 0 && fused_fits(g) && g.lda % 8 == 0 &&
                   g.ldb % 16 == 0 && g.ldo % 8 == 0 &&
                   reinterpret_cast<uintptr_t>(g.a) % 16 == 0 &&
                   reinterpret_cast<uintptr_t>(g.b) % 16 == 0 &&
@@ -2132,7 +2136,7 @@ int choose_gemm_fp8(const GemmArgs& g) {
 
 int linear_fp8_launches(const GemmArgs& g) {
   if (!aligned_ok(g) || g.M > 16) return 2;
-  return row1_ok(g) || (!few_quantized_apart(g) && fused_lds(g) <= kFusedLds) ? 1 : 2;
+  return row1_ok(g) || (!few_quantized_apart(g) && fused_fits(g)) ? 1 : 2;
 }
 
 int launch_gemm_fp8(const GemmArgs& g, int variant, hipStream_t stream) {

@@ -32,7 +32,9 @@ def test_few_rows(lib, M, N, K, want):
 @pytest.mark.parametrize("M,N,K,want", [
     # rows beyond 16384 elements are quantized in the GEMM's kernel where they fit its LDS
     (2, 16192, 16512, 1), (2, 22592, 17472, 1), (3, 7936, 18688, 1), (2, 9216, 5120, 2),
-    (2, 2816, 15360, 1), (4, 3456, 14320, 1), (1, 9216, 3072, 1), (8, 3072, 3072, 1),
+    # codes of more than 48 KiB in every workgroup's LDS
+    (8, 256, 6128, 1), (8, 256, 6144, 2), (8, 256, 6464, 2), (6, 256, 8384, 2), (4, 2304, 12480, 2),
+    (2, 2816, 15360, 1), (4, 2304, 12272, 1), (1, 9216, 3072, 1), (8, 3072, 3072, 1),
     (16, 9216, 3072, 2), (16, 3072, 3072, 2), (8, 2048, 12288, 2), (17, 64, 64, 2)])
 def test_launches_of_few_rows(lib, M, N, K, want):
   assert lib.cdit_debug_linear_launches(M, N, K) == want
