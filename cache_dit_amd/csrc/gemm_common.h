@@ -182,6 +182,16 @@ inline int64_t rounds_permille(int64_t tiles, int64_t cus, int lone, int last) {
   return full * 1000 + (rem ? p + (1000 - p) * rem / cus : 0);
 }
 
+// The kernels with a workgroup per 32 x 32 tile. The 8 XCDs take their column tiles in turn, all rows of a column on one
+// XCD, so what a CU gets follows from the columns rounded up to a multiple of 8: `padded`.
+struct Tiles32 {
+  int64_t tiles, padded;
+};
+inline Tiles32 tiles32(int M, int N) {
+  const int64_t rows = (M + 31) / 32, cols = (N + 31) / 32;
+  return {rows * cols, rows * ((cols + 7) / 8 * 8)};
+}
+
 // A tile of a wide kernel and the measured time of a full round of it: start-up and epilogue,
 // and each K step (ns). Both the choice of a tile and the choice between one launch for a batch
 // and one per activation are made by launch_ns().

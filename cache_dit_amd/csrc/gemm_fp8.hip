@@ -2101,6 +2101,22 @@ int launch_other_out(const GemmArgs& g, int variant, hipStream_t stream) {
 // conversions of two steps cost nothing (36 x 3904 x 256, M x N x K: 7.4 us with the tiled kernel, 4.2).
 bool tile32_tail(const GemmArgs& g) { return g.K % BK != 0 || g.K < 3 * BK; }
 
+// More than 16 rows on the workgroup-per-tile kernel: up to three tiles per CU (figures at the kernel; beyond, it wins with short
+// K and loses with long: 864 tiles 7.1 us with the wide kernel, 6.4 with this one at K = 896, 816 tiles 30.1
+// and 32.9 at K = 10624). With K remainders, where the wide kernel's wavefronts convert, up to five for short
+// K (1209 tiles 9.5 and 8.3), but 144 x 1680 x 8032 (1255 tiles) 15.4 and 17.3, 72 x 8992 x 11840 (1110) 52.9
+// and 65.4. From K = 2048 on it counts if some XCDs get so many more columns than others (Tiles32::padded) that
+// theirs are more than three per CU: 1579 x 12032 x 352 (550 tiles, 800 padded) 26.9 and 41.8, 1631 x 9600 x 480
+// (765 and 816) 30.4 and 37.2; but 203 x 4992 x 3392 (742 and 784) 16.1 and 15.3, 1107 x 384 x 592 7.1 and 4.5. (M x K x
+// N.) Over 500 shapes it is 0.2 % off the better one (geometric mean), the worst 12 %.
+bool tile32_better(const GemmArgs& g) {
+  const int64_t cus = cu_count() > 0 ? cu_count() : 256;
+  const Tiles32 t = tiles32(g.M, g.N);
+  if (g.K % BK != 0) return t.tiles <= (g.K > 4096 ? 3 : g.K > 1024 ? 4 : 5) * cus;
+  if (g.K < 3 * BK) return t.tiles <= 5 * cus;
+  return t.tiles <= 3 * cus && (g.K <= 2048 || t.padded <= 3 * cus || (g.K <= 6144 && t.padded * 10 <= t.tiles * 11));
+}
+
 // at least `depth` K steps to prefetch, and at least 3: the epilogue operands of a tile are
 // staged in LDS two steps before its end, which must be behind the first barrier of the
 // tile (before it, slower waves may still be reading the previous tile's)
@@ -2115,12 +2131,7 @@ int choose_gemm_fp8(const GemmArgs& g) {
   if (!aligned_ok(g)) return 100;
   if (row1_ok(g)) return 51;
   if (g.M <= 16) return few_on_tiles(g) ? 26 : 50;
-  // Up to three 32 x 32 tiles per CU: the workgroup-per-tile kernel (figures at the kernel; beyond, it
-  // wins with short K and loses with long: 864 tiles 7.1 us with the wide kernel, 6.4 with this one
-  // at K = 896, 816 tiles 30.1 and 32.9 at K = 10624), with K remainders up to five (1209 tiles 9.5 and
-  // 8.3, 1677 tiles 18.6 and 22.0).
-  const int64_t tiles32 = (int64_t)((g.M + 31) / 32) * ((g.N + 31) / 32);
-  if (tiles32 <= (tile32_tail(g) ? 5 : 3) * (int64_t)(cu_count() > 0 ? cu_count() : 256)) return 26;
+  if (tile32_better(g)) return 26;
   if (!tiled_ok(g)) return choose_ktail_variant(g, -1);
   // the wide kernels stream K two or more steps ahead: shorter K runs the 128x128 kernel
   const WideOk wide_ok{g.K};

@@ -38,3 +38,17 @@ def test_few_rows(lib, M, N, K, want):
     (16, 9216, 3072, 2), (16, 3072, 3072, 2), (8, 2048, 12288, 2), (17, 64, 64, 2)])
 def test_launches_of_few_rows(lib, M, N, K, want):
   assert lib.cdit_debug_linear_launches(M, N, K) == want
+
+
+@pytest.mark.parametrize("M,N,K,tiles", [
+    (77, 3072, 4096, True), (303, 640, 4736, True), (203, 3392, 4992, True), (300, 3072, 2224, True),
+    # three (K remainders: five and four) tiles per CU and beyond
+    (96, 8192, 3072, True), (97, 8192, 3072, False), (160, 8192, 400, True), (161, 8192, 400, False),
+    (144, 8032, 1680, False), (128, 8192, 1680, True), (72, 11840, 8992, False), (898, 1088, 11536, False),
+    (160, 8192, 256, True), (161, 8192, 256, False),
+    # few columns, of which some XCDs get twice as many as others
+    (1579, 352, 12032, False), (1631, 480, 9600, False), (1806, 304, 3840, False), (639, 1168, 3200, True),
+    (1848, 400, 1024, True), (1107, 592, 384, True)])
+def test_tiles_of_more_than_16_rows(lib, M, N, K, tiles):
+  for dtype in (F16, BF16, F32):
+    assert (lib.cdit_debug_gemm_choice(0, M, N, K, dtype) == TILE32) == tiles
