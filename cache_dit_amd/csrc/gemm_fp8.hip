@@ -2190,22 +2190,25 @@ int launch_gemm_fp8(const GemmArgs& g, int variant, hipStream_t stream) {
 // kernel, which take any K. They run at the rate of the bf16 instruction and convert the codes,
 // so a round of a tile takes longer than that of the FP8 instances and grows more with its area;
 // the tile is chosen by their own round times (tenths of a us at K of about 2200; only the ratios
-// count). Within 0.2 % of the best tile over 110 shapes of M 300 to 6889, K 272 to 3056, N 1024 to
-// 9000 (geometric mean; the worst 5 % off). A wavefront converts the operands of its own tile, so
+// count). Within 0.1 % of the best tile over 510 shapes of M 300 to 6889, K 272 to 15344, N 256 to
+// 12288 (geometric mean; the worst 10 % off). A wavefront converts the operands of its own tile, so
 // a step of 256 x 128 (wave tile 128 x 64: 1.5 conversions of 8 clocks per MFMA of 16) takes 1.45
 // times one of 128 x 128 (2 per MFMA) and does twice the work: the tile for problems that are more
 // than one round of 128 x 128 and less than one of the larger tiles (without it the choice was
-// 1.2 % off the best, the worst 39 %). 1357 x 4464 x 2224 (M x N x K): 35.6 us with 256 x 128
+// 2.7 % off the best, the worst 41 %). 1357 x 4464 x 2224 (M x N x K): 35.6 us with 256 x 128
 // against 43.1 (128 x 128, two rounds), 44.5 (256 x 192) and 52.1 (128 x 192); 256 x 3072 x 2992:
 // 20.7 with 64 x 128 against 27.5 (128 x 128); 4608 x 3072 x 3056: 64.4 with 288 x 192 against
-// 75.1 (256 x 128) and 93.8 (128 x 128). The scalar FMA kernel took 16.8 ms for the first. There is
+// 75.1 (256 x 128) and 93.8 (128 x 128). Two rounds of 256 x 192 take less than three of 256 x 128
+// and one of 128 x 192 less than one of it (3261 x 7280 x 1040 49.8 and 55.3, 947 x 5216 x 3728 41.3
+// and 44.4): a round counts 340; with the 310 that it had at first, 56 of the 510 shapes were 4 to 16 %
+// slower than without the tile, with 340 none (1.7 % the worst). The scalar FMA kernel took 16.8 ms for the first. There is
 // no 256 x 256 instance: its converted operands do not fit the registers. fp16 and fp32 outputs
 // have three tiles.
 int choose_ktail_variant(const GemmArgs& g, int variant) {
   const int64_t cus = cu_count() > 0 ? cu_count() : 256;
   const struct { int v, bm, bn, us10; bool other_out; } cand[] = {
       {14, 288, 192, 530, false}, {15, 256, 192, 470, true}, {16, 128, 192, 290, false},
-      {19, 256, 128, 310, false}, {18, 128, 128, 205, true}, {17, 64, 128, 150, true}};
+      {19, 256, 128, 340, false}, {18, 128, 128, 205, true}, {17, 64, 128, 150, true}};
   const bool bf16 = g.out_dtype == CDIT_DT_BF16;
   int best = 18;
   int64_t time = INT64_MAX;

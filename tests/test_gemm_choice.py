@@ -52,3 +52,11 @@ def test_launches_of_few_rows(lib, M, N, K, want):
 def test_tiles_of_more_than_16_rows(lib, M, N, K, tiles):
   for dtype in (F16, BF16, F32):
     assert (lib.cdit_debug_gemm_choice(0, M, N, K, dtype) == TILE32) == tiles
+
+
+@pytest.mark.parametrize("M,N,K,want", [
+    # 256 x 128 tiles between one round of 128 x 128 and two of 256 x 192, not in their place
+    (1357, 4464, 2224, 19), (3261, 7280, 1040, 15), (5499, 3440, 1296, 15), (1678, 12080, 4000, 15), (947, 5216, 3728, 16),
+    (2269, 7248, 1344, 16), (4608, 3072, 3056, 14), (256, 12288, 2992, 18)])
+def test_tiles_for_k_remainders(lib, M, N, K, want):
+  assert lib.cdit_debug_gemm_choice(0, M, N, K, BF16) == want
