@@ -1971,15 +1971,21 @@ bool few_on_many(const GemmArgs& g) {
 // with six steps of each in flight, 2.3 to 3 us (2.7 to 4.5) for 24 steps. So the tiles are faster only
 // where the last batch of 24 is nearly empty. us, 16-row / tiles, M x N x K: 9 x 576 x 14608 15.7 / 22.3, 8 x 2048 x
 // 12288 14.4 / 19.0, 4 x 2048 x 15360 16.3 / 22.7, 2 x 4096 x 15360 17.3 / 24.1, 9 x 1024 x 3072 5.3 / 5.6;
-// 9 x 256 x 3200 7.0 / 6.1, 16 x 384 x 8736 17.2 / 15.2. Over 600 shapes of up to 4500 columns it is 1 % off the
-// better one.
+// 10 x 608 x 3328 7.1 / 6.2, 16 x 2112 x 4096 8.9 / 7.2, 16 x 944 x 11024 22.1 / 18.6. Batches after the second take the
+// 16-row kernel less each (16 x 832 x 9600 13.2 / 15.0, 16 x 2304 x 9344 13.6 / 15.2). With K remainders its time
+// grows more with the rows, and less where rows start on 64-byte boundaries: 9 x 416 x 2224 4.5 / 5.5, 11 x 2016 x
+// 2448 6.3 / 6.6, 10 x 1120 x 7232 12.3 / 13.2, 14 x 1600 x 2752 6.7 / 6.9, but 15 x 528 x 4544 10.0 / 9.4; on some 20
+// workgroups and fewer it stays short (12 x 272 x 3616 6.7 / 7.4, 16 x 288 x 5280 8.5 / 9.6). Over 208 shapes of up to
+// 4096 columns, matrices from HBM, 0.8 % off the better one and nowhere more than 5 % slower than the 16-row kernel.
 // Both kernels give the same bits (for K of 128 and 256 the tiles' sums are the more exact ones).
 bool few_on_tiles(const GemmArgs& g) {
   if (!few_on_many(g)) return false;
   if (g.N > 4096) return true;
   const bool tail = g.K % BK != 0;
+  if (tail && (g.N <= 320 || g.M < (g.K % 64 ? 12 : 15))) return false;
   const int64_t steps = (g.K + BK - 1) / BK, batches = (steps + 23) / 24;
-  return steps * (tail ? 190 : 158) < batches * (tail ? 2450 + 125 * g.M : 2250 + 45 * g.M);
+  const int64_t batch = tail ? 2450 + 125 * g.M : (steps > 40 ? 1800 : 2250) + 45 * g.M;
+  return steps * (tail ? 190 : 158) < batches * batch;
 }
 // A Linear of 2 to 16 bf16 rows as the quantizer's launch (2.2 to 3 us) and the GEMM's, instead of the 16-row kernel that
 // quantizes them itself. What is near on both sides and about 10 us is left to the single launch: a

@@ -21,6 +21,11 @@ def lib():
     (9, 1024, 3072, ROWS16), (16, 1024, 12288, ROWS16),
     # a last batch of its steps that is nearly empty
     (9, 256, 3200, TILE32), (16, 384, 8736, TILE32),
+    # longer K: a later batch of the 16-row kernel costs less
+    (16, 832, 9600, ROWS16), (16, 2304, 9344, ROWS16), (13, 3184, 6272, ROWS16), (16, 2112, 4096, TILE32),
+    # K remainders: up to 11 rows, rows that start on 64-byte boundaries, some 20 workgroups and fewer
+    (9, 416, 2224, ROWS16), (11, 2016, 2448, ROWS16), (12, 320, 2144, ROWS16), (16, 288, 5280, ROWS16),
+    (10, 1120, 7232, ROWS16), (14, 1600, 2752, ROWS16), (15, 528, 4544, TILE32), (16, 944, 11024, TILE32),
     # many columns
     (16, 9216, 3072, TILE32), (16, 18432, 5120, TILE32), (8, 18432, 3072, TILE32), (4, 9216, 5120, TILE32),
     (2, 18432, 3072, ROWS16), (2, 9216, 5120, TILE32), (1, 9216, 3072, ROW1), (1, 9216, 4112, ROWS16)])
