@@ -2114,10 +2114,13 @@ bool tile32_tail(const GemmArgs& g) { return g.K % BK != 0 || g.K < 3 * BK; }
 // and 65.4. From K = 2048 on it counts if some XCDs get so many more columns than others (Tiles32::padded) that
 // theirs are more than three per CU: 1579 x 12032 x 352 (550 tiles, 800 padded) 26.9 and 41.8, 1631 x 9600 x 480
 // (765 and 816) 30.4 and 37.2; but 203 x 4992 x 3392 (742 and 784) 16.1 and 15.3, 1107 x 384 x 592 7.1 and 4.5. (M x K x
-// N.) Over 500 shapes it is 0.2 % off the better one (geometric mean), the worst 12 %.
+// N.) Four per CU of an XCD are the limit for shorter K too: 2280 x 1408 x 320 (720 and 1152) 7.3 and 9.0, 2416 x
+// 896 x 288 5.8 and 6.4; with K remainders six below K = 1024: 2240 x 15136 x 288 74 and 89, 1366 x 3920 x 576 23.5 and
+// 26.8. Over 1900 shapes it is 0.7 % off the better one (geometric mean), the worst 14 % (1398 x 11392 x 496).
 bool tile32_better(const GemmArgs& g) {
   const int64_t cus = cu_count() > 0 ? cu_count() : 256;
   const Tiles32 t = tiles32(g.M, g.N);
+  if (t.padded > (g.K % BK != 0 && g.K <= 1024 ? 6 : 4) * cus && g.K >= 3 * BK) return false;
   if (g.K % BK != 0) return t.tiles <= (g.K > 4096 ? 3 : g.K > 1024 ? 4 : 5) * cus;
   if (g.K < 3 * BK) return t.tiles <= 5 * cus;
   return t.tiles <= 3 * cus && (g.K <= 2048 || t.padded <= 3 * cus || (g.K <= 6144 && t.padded * 10 <= t.tiles * 11));
