@@ -171,8 +171,8 @@ static bool shape_only(GemmArgs* g, int64_t M, int64_t N, int64_t K, int out_dty
 
 int cdit_debug_gemm_choice(int weight_only, int64_t M, int64_t N, int64_t K, int out_dtype_id) {
   GemmArgs g;
-  if (!shape_only(&g, M, N, K, out_dtype_id) || weight_only) return -1;
-  return choose_gemm_fp8(g);
+  if (!shape_only(&g, M, N, K, out_dtype_id)) return -1;
+  return weight_only ? choose_gemm_w8a16(g) : choose_gemm_fp8(g);
 }
 
 int cdit_debug_linear_launches(int64_t M, int64_t N, int64_t K) {

@@ -950,14 +950,14 @@ int launch_wide_grouped(const GemmArgs& g, GemmGroup grp, hipStream_t stream) {
 // instructions per step, each on a wavefront of its own: about 250 clocks per step (500 with one
 // wavefront issuing both in order). Two feeding wavefronts: 3 to 8 % faster with one tile per CU,
 // 4 to 8 % slower with two. Conversions a step ahead of their MFMAs: the same or slower. D = 6: four
-// workgroups fit a CU; 8 is 1 to 5 % slower up to two per CU (but up to 6 % faster where 40 MB of weights
-// come from HBM) and three per CU already take a second round; 4 is up to 27 % slower on such weights.
+// workgroups fit the LDS of a CU (4 x 36 KiB), with 8 three, and a fourth is a second round; 8 is 1 to 5 %
+// slower up to two per CU (but up to 6 % faster where 40 MB of weights come from HBM), 4 up to 27 % on such weights.
 // Another weight matrix per launch (M x K x N), us, one wavefront before -> now: 77 x 4096 x 3072
 // 15.9 -> 11.2, 17 x 3072 x 3072 12.3 -> 8.5, 128 x 3072 x 3072 13.2 -> 9.5, 256 x 15360 x 1024 47.4
 // -> 31, 100 x 1024 x 2048 6.3 -> 4.9; 128 x 64 tiles of the wide kernel -> now: 245 x 1664 x 2560 11.4 ->
-// 8.1, 299 x 3328 x 2368 (740 tiles) 18.1 -> 15.1, 103 x 2816 x 6016 (752) 15.6 -> 10.9, but
-// 158 x 6784 x 4352 (680) 30.0 -> 34.2, and beyond 768 tiles either way: 154 x 2560 x 5056 (790) 15.8 -> 13.7,
-// 592 x 1664 x 1600 (950) 11.9 -> 14.9.
+// 8.1, 299 x 3328 x 2368 (740 tiles) 18.1 -> 15.1, 103 x 2816 x 6016 (752) 15.6 -> 10.9; beyond 768 tiles
+// either way: 154 x 2560 x 5056 (790) 15.8 -> 13.7, 592 x 1664 x 1600 (950) 11.9 -> 14.9. Where it is taken:
+// wavetile_better().
 constexpr int kTileDepth = 6, kTileLds = kTileDepth * 32 * 3 * BKE;
 template <bool GELU>
 __global__ __launch_bounds__(128) void gemm_w8a16_wavetile(GemmArgs g, int tiles_m, int tiles_n) {
@@ -1459,22 +1459,68 @@ bool whole_rows_better(const GemmArgs& g) {
 bool tiles_better_for_few(const GemmArgs& g) {
   if (g.K % 128) return (int64_t)g.M * g.N > 40960;
   if (g.M >= 7) return g.N > 4500;
-  if (g.M >= 5) return g.N > 7000;
-  if (g.M >= 3) return g.N > (g.M == 4 ? 8000 : 10000);
+  if (g.M == 6) return g.N > 7000;
+  if (g.M >= 4) return g.N > 8000;  // (5 x 7952 x 2944 9.1 / 9.7, 5 x 7120 x 14208 28.1 / 32.2)
+  if (g.M >= 3) return g.N > 10000;
   return g.M == 2 && g.K > 4096 && g.N > 8000;
+}
+
+// More than 16 rows on the workgroup-per-tile kernel; us, wide kernel / this one, M x N x K. Two tiles per CU and less: always,
+// unless some XCDs get so many more columns than others (Tiles32::padded) that theirs are more than three per CU, from K
+// = 1024 on (1738 x 272 x 2944, 476 tiles and 880 padded, 16.4 / 18.7; up to K = 4096 not for the last tenth, 299 x 2368 x 3328,
+// 740 and 800, 18.1 / 15.1); below, more than four (1524 x 288 x 256 7.1 / 4.0).
+// Beyond four the CUs take a second round: 2257 x 272 x 15680, 639 and 1136, 63 / 133. Up to three per CU on weights of up to
+// 20 MB (486 shapes: 0.73 of the time in the middle, 0.95 at the 95th percentile); on more where there are few of the wide
+// kernel's smallest tiles (254 x 2896 x 7744, 92 of 128 x 64, 43.5 / 32.1) or they are mostly empty (42 x 11008 x 9536 42.9 /
+// 37.4), else a round of those is the faster one: 158 x 4800 x 14400 59.2 / 72.1, 152 x 4768 x 6320 38.7 / 49.3, 146 x 3520 x
+// 11392 46.5 / 55.0. At four per CU it wins or loses with the shape. Over 720 shapes of two to three per CU 1 % off the better one
+// (geometric mean), 7 are more than 4 % slower than the wide kernel (17 % the worst, 1327 x 496 x 15424).
+bool wavetile_better(const GemmArgs& g) {
+  if (g.N % 16) return false;
+  const int64_t cus = cu_count() > 0 ? cu_count() : 256;
+  const Tiles32 t = tiles32(g.M, g.N);
+  if (t.tiles > 3 * cus || t.padded > 4 * cus) return false;
+  if (g.K > 1024 && t.padded > 3 * cus && (g.K > 4096 || t.padded * 10 > t.tiles * 11)) return false;
+  if (t.tiles <= 2 * cus || (int64_t)g.N * g.K <= 20000000 || g.M <= 48) return true;
+  return (int64_t)((g.M + 127) / 128) * ((g.N + 63) / 64) * 11 <= 4 * cus;
+}
+
+// at least `depth` K steps to prefetch, and at least 3: the epilogue operands of a tile are
+// staged in LDS two steps before its end, which must be behind the first barrier of the
+// tile (before it, slower waves may still be reading the previous tile's)
+struct WideOk {
+  bool any_k;  // the instances for K remainders
+  int K, N;
+  bool operator()(int depth) const { return (any_k || K >= (depth > 3 ? depth : 3) * BKE) && N % 16 == 0; }
+};
+int choose_tile(const GemmArgs& g) {
+  return choose_variant([&](int bm, int bn) { return (int64_t)((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn); },
+                        WideOk{!tiled_ok(g), g.K, g.N}, g.K).variant;
 }
 }  // namespace
 
+// The kernel for a problem: 100 for any shape and alignment, 51 whole rows (up to four), 50 up to 16 rows, 13 a workgroup
+// per 32 x 32 tile, else a tile of the wide kernel (K remainders: of its instances for them) or of the tiled one.
+int choose_gemm_w8a16(const GemmArgs& g) {
+  if (!aligned_ok(g)) return 100;
+  const bool few_on_tiles = g.M <= 16 && g.N % 16 == 0 && tiles_better_for_few(g);
+  if (g.M <= 4 && g.K <= 4096 && whole_rows_better(g) && (g.K % 128 || !few_on_tiles)) return 51;
+  if (g.M <= 16 && !few_on_tiles) return 50;
+  // what is left of K remainders is for the wide kernel, which stores 16 columns per lane
+  if (!tiled_ok(g) && g.N % 16 != 0) return 100;
+  return few_on_tiles || wavetile_better(g) ? 13 : choose_tile(g);
+}
+
 int launch_gemm_w8a16(const GemmArgs& g, int variant, hipStream_t stream) {
   const bool k_tail = !tiled_ok(g);  // K not a whole number of steps
+  if (variant < 0) variant = choose_gemm_w8a16(g);
   auto launch_generic = [&]() {
     dim3 grid((g.N + 15) / 16, (g.M + 15) / 16);
     hipLaunchKernelGGL(gemm_w8a16_generic, grid, dim3(256), 0, stream, g);
     return 0;
   };
   if (!aligned_ok(g) || variant == 100) return launch_generic();
-  const bool few_on_tiles = g.M <= 16 && g.N % 16 == 0 && tiles_better_for_few(g);
-  if (g.M <= 4 && g.K <= 4096 && (variant == 51 || (variant < 0 && whole_rows_better(g) && (g.K % 128 || !few_on_tiles)))) {
+  if (g.M <= 4 && g.K <= 4096 && variant == 51) {
     // (aligned_ok has checked the alignment of the operands and of lda and ldb)
     switch ((g.K + 1023) / 1024) {
       case 1: launch_rows_chk<1>(g, stream); break;
@@ -1484,7 +1530,7 @@ int launch_gemm_w8a16(const GemmArgs& g, int variant, hipStream_t stream) {
     }
     return 0;
   }
-  if ((variant < 0 && g.M <= 16 && !few_on_tiles) || variant == 50) {
+  if (variant == 50) {
     if (g.M > 16) {
       set_error("cdit_w8a16_gemm: the skinny kernel takes M <= 16");
       return CDIT_EINVAL;
@@ -1496,26 +1542,10 @@ int launch_gemm_w8a16(const GemmArgs& g, int variant, hipStream_t stream) {
     }
     return 0;
   }
-  // what is left of K remainders is for the wide kernel, which stores 16 columns per lane
   if (k_tail && g.N % 16 != 0) return launch_generic();
-  // the wide kernels stream K two or more steps ahead and store 16 columns per lane
-  // at least `depth` K steps to prefetch, and at least 3: the epilogue operands of a tile are
-  // staged in LDS two steps before its end, which must be behind the first barrier of the
-  // tile (before it, slower waves may still be reading the previous tile's)
-  auto wide_ok = [&](int depth) {
-    return (k_tail || g.K >= (depth > 3 ? depth : 3) * BKE) && g.N % 16 == 0;
-  };
-  // Three 32 x 32 tiles per CU and less: the workgroup-per-tile kernel (figures at the kernel; at
-  // four per CU it wins or loses with the shape, beyond that the CUs take a second round of it).
-  if (g.N % 16 == 0 &&
-      (variant == 13 || (variant < 0 && (few_on_tiles || (int64_t)((g.M + 31) / 32) * ((g.N + 31) / 32) <=
-                                                             3 * (int64_t)(cu_count() > 0 ? cu_count() : 256)))))
-    return launch_wavetile(g, stream);
-  if (variant < 0 || (k_tail && (variant < 7 || variant > 12))) {
-    variant = choose_variant(
-        [&](int bm, int bn) { return (int64_t)((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn); },
-        wide_ok, g.K).variant;
-  }
+  if (variant == 13 && g.N % 16 == 0) return launch_wavetile(g, stream);
+  const WideOk wide_ok{k_tail, g.K, g.N};
+  if (k_tail && (variant < 7 || variant > 12)) variant = choose_tile(g);
   if (k_tail) {  // the KTAIL instances of the wide kernel take any K
     switch (variant) {
       case 7: return launch_wide<W7, true>(g, stream);
@@ -1566,7 +1596,7 @@ int launch_gemm_w8a16_grouped(const GemmArgs& common, const GemmGroup& grp, int 
       n16 = n16 && g.N % 16 == 0;
     }
   }
-  auto wide_ok = [&](int depth) { return common.K >= (depth > 3 ? depth : 3) * BKE && n16; };
+  const WideOk wide_ok{false, common.K, n16 ? 16 : 1};
   auto tiles = [&](int bm, int bn) {
     int64_t t = 0;
     for (int s = 0; s < grp.acts; ++s) {

@@ -1,5 +1,5 @@
 """The kernels that the GEMM entry points choose by shape, at shapes where the rule was measured on both
-sides (figures beside the rules in csrc/gemm_fp8.hip). No GPU: the choice of 256 compute
+sides (figures beside the rules in csrc/gemm_fp8.hip and csrc/gemm_w8a16.hip). No GPU: the choice of 256 compute
 units."""
 import pytest
 
@@ -66,3 +66,16 @@ def test_tiles_of_more_than_16_rows(lib, M, N, K, tiles):
     (2269, 7248, 1344, 16), (4608, 3072, 3056, 14), (256, 12288, 2992, 18)])
 def test_tiles_for_k_remainders(lib, M, N, K, want):
   assert lib.cdit_debug_gemm_choice(0, M, N, K, BF16) == want
+
+
+@pytest.mark.parametrize("M,N,K,want", [
+    # few columns, of which some XCDs get twice as many as others
+    (2257, 272, 15680, 12), (2346, 288, 3392, 12), (2277, 272, 1408, 12), (1738, 272, 2944, 12), (1524, 288, 256, 13),
+    # two to three tiles per CU on many weights
+    (158, 4800, 14400, 12), (152, 4768, 6320, 12), (146, 3520, 11392, 12), (254, 2896, 7744, 13), (42, 11008, 9536, 13),
+    (245, 2560, 1664, 13), (299, 2368, 3328, 13), (77, 3072, 4096, 13), (154, 5056, 2560, 12),
+    # up to 16 rows
+    (5, 7952, 2944, 50), (5, 9216, 3072, 13), (6, 7952, 2944, 13), (16, 18432, 5120, 13), (16, 3072, 3072, 50),
+    (2, 18432, 3072, 51), (1, 9216, 3072, 51), (16, 18432, 3136, 13)])
+def test_weight_only(lib, M, N, K, want):
+  assert lib.cdit_debug_gemm_choice(1, M, N, K, BF16) == want
