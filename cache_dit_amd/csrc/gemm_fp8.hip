@@ -2111,7 +2111,7 @@ bool tile32_tail(const GemmArgs& g) { return g.K % BK != 0 || g.K < 3 * BK; }
 // K and loses with long: 864 tiles 7.1 us with the wide kernel, 6.4 with this one at K = 896, 816 tiles 30.1
 // and 32.9 at K = 10624). With K remainders, where the wide kernel's wavefronts convert, up to five for short
 // K (1209 tiles 9.5 and 8.3), but 144 x 1680 x 8032 (1255 tiles) 15.4 and 17.3, 72 x 8992 x 11840 (1110) 52.9
-// and 65.4. From K = 2048 on it counts if some XCDs get so many more columns than others (Tiles32::padded) that
+// and 65.4; four to K = 6144: 1199 x 4160 x 704 (836) 24.5 and 21.9, 75 x 4528 x 9088 (852) 28.9 and 30.5. From K = 2048 on it counts if some XCDs get so many more columns than others (Tiles32::padded) that
 // theirs are more than three per CU: 1579 x 12032 x 352 (550 tiles, 800 padded) 26.9 and 41.8, 1631 x 9600 x 480
 // (765 and 816) 30.4 and 37.2; but 203 x 4992 x 3392 (742 and 784) 16.1 and 15.3, 1107 x 384 x 592 7.1 and 4.5. (M x K x
 // N.) Four per CU of an XCD are the limit for shorter K too: 2280 x 1408 x 320 (720 and 1152) 7.3 and 9.0, 2416 x
@@ -2121,7 +2121,7 @@ bool tile32_better(const GemmArgs& g) {
   const int64_t cus = cu_count() > 0 ? cu_count() : 256;
   const Tiles32 t = tiles32(g.M, g.N);
   if (t.padded > (g.K % BK != 0 && g.K <= 1024 ? 6 : 4) * cus && g.K >= 3 * BK) return false;
-  if (g.K % BK != 0) return t.tiles <= (g.K > 4096 ? 3 : g.K > 1024 ? 4 : 5) * cus;
+  if (g.K % BK != 0) return t.tiles <= (g.K > 6144 ? 3 : g.K > 1024 ? 4 : 5) * cus;
   if (g.K < 3 * BK) return t.tiles <= 5 * cus;
   return t.tiles <= 3 * cus && (g.K <= 2048 || t.padded <= 3 * cus || (g.K <= 6144 && t.padded * 10 <= t.tiles * 11));
 }

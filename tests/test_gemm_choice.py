@@ -54,7 +54,8 @@ def test_launches_of_few_rows(lib, M, N, K, want):
     # few columns, of which some XCDs get twice as many as others
     (1579, 352, 12032, False), (1631, 480, 9600, False), (1806, 304, 3840, False), (639, 1168, 3200, True),
     (1848, 400, 1024, True), (1107, 592, 384, True), (2280, 320, 1408, False), (2416, 288, 896, False),
-    (2048, 320, 1408, True), (2240, 288, 15136, False), (1366, 576, 3920, False), (1366, 576, 784, True)])
+    (2048, 320, 1408, True), (2240, 288, 15136, False), (1366, 576, 3920, False), (1366, 576, 784, True), (1199, 704, 4160, True),
+    (1199, 704, 6160, False)])
 def test_tiles_of_more_than_16_rows(lib, M, N, K, tiles):
   for dtype in (F16, BF16, F32):
     assert (lib.cdit_debug_gemm_choice(0, M, N, K, dtype) == TILE32) == tiles
