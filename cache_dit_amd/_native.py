@@ -159,6 +159,20 @@ def load(path: str | None = None) -> ctypes.CDLL:
   return _lib
 
 
+def host_built_for() -> str:
+  """What the extension depends on beyond the library: it is compiled against torch's C++ classes and
+  CPython's, neither of which is stable from one version to the next."""
+  import sysconfig
+  return f"cdit_host for torch {torch.__version__}, {sysconfig.get_config_var('SOABI')}"
+
+
+def _host_is_current() -> bool:
+  """Whether the extension was built for this torch and Python. Looked for in the file: loading one
+  that was not fails with an unresolved symbol, or works until a class of another layout is used."""
+  with open(HOST_PATH, "rb") as f:
+    return host_built_for().encode() + b"\0" in f.read()
+
+
 def host():
   """The Python extension, loaded once and bound to the library that load() gives."""
   global _host
@@ -170,6 +184,9 @@ def host():
           raise CditNativeError(
               f"{HOST_PATH} not found: build it with `python -m cache_dit_amd.csrc.build`. "
               "There is no fallback path.")
+        if not _host_is_current():
+          raise CditNativeError(f"{HOST_PATH}: not built for this torch and Python ({host_built_for()}); rebuild "
+                                "with `python -m cache_dit_amd.csrc.build`")
         import importlib.machinery
         import importlib.util
         loader = importlib.machinery.ExtensionFileLoader("_cdit_host", HOST_PATH)
@@ -182,7 +199,8 @@ def host():
 
 
 def is_built() -> bool:
-  return os.path.exists(os.environ.get("CDIT_HIP_LIB", LIB_PATH)) and os.path.exists(HOST_PATH)
+  return (os.path.exists(os.environ.get("CDIT_HIP_LIB", LIB_PATH)) and os.path.exists(HOST_PATH)
+          and _host_is_current())
 
 
 def last_error() -> str:

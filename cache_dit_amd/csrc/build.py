@@ -73,13 +73,16 @@ def build_host(verbose: bool = False) -> str:
   import torch
   from torch.utils import cpp_extension
 
+  from cache_dit_amd import _native
+
   rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
   lib = os.path.join(os.path.dirname(torch.__file__), "lib")
   inc = [*cpp_extension.include_paths(), os.path.join(rocm, "include"), sysconfig.get_paths()["include"],
          os.path.join(ROOT, "include")]
   tmp = HOST_PATH + ".tmp"
   cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-w", "-DUSE_ROCM",
-         f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}", *("-I" + i for i in inc),
+         f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}",
+         f'-DCDIT_HOST_BUILT_FOR="{_native.host_built_for()}"', *("-I" + i for i in inc),
          os.path.join(HERE, "host_ext.cpp"), "-o", tmp, "-L" + lib, "-ltorch_python", "-ltorch",
          "-ltorch_cpu", "-lc10", "-lc10_hip", "-ldl"]
   if verbose:

@@ -23,6 +23,9 @@
 
 #include "cdit_hip.h"
 
+// The torch and Python this is compiled against (_native.host_built_for()); looked for in the file before it is loaded.
+extern "C" __attribute__((used, visibility("default"))) const char cdit_host_built_for[] = CDIT_HOST_BUILT_FOR;
+
 namespace {
 
 constexpr int kMaxActs = 4, kMaxGroup = 8;
