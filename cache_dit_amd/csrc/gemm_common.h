@@ -107,12 +107,6 @@ __device__ __forceinline__ void wait_vm() {
   __builtin_amdgcn_s_waitcnt((VM & 0xf) | (7 << 4) | (0xf << 8) | ((VM >> 4) << 14));
   asm volatile("" ::: "memory");
 }
-// The wave's LDS reads have arrived.
-__device__ __forceinline__ void wait_lgkm0() {
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_waitcnt(0xf | (7 << 4) | (0 << 8) | (3 << 14));
-  asm volatile("" ::: "memory");
-}
 // Waits until at most `later` steps (of D DMA instructions each) are in flight,
 // `later` in [0, MAXL]; the count has to be an immediate, hence the switch.
 template <int D, int MAXL, bool BARRIER>
