@@ -600,8 +600,8 @@ int cdit_fp8_linear_w8a8(const void* x_bf16, const void* w_q, const float* w_sca
                          const void* bias, void* out, void* q_ws, float* scale_ws, int64_t M,
                          int64_t N, int64_t K, int64_t ld_x, int64_t ldw, int64_t ldo,
                          int scale_mode, int epilogue, int out_dtype_id, void* stream) {
-  // M <= 16 (the M = 1 modulation Linears): one kernel that quantizes the rows itself where
-  // that is faster than two (few_quantized_apart()), when every argument passes the checks of the two entry points it stands for
+  // M <= 16 (the M = 1 modulation Linears): one kernel that quantizes the rows itself where that is faster
+  // than two (linear_fp8_launches()), when every argument passes the checks of the two entry points it stands for
   if (M >= 1 && M <= 16 && N > 0 && K > 0 && K <= INT32_MAX && N <= INT32_MAX && x_bf16 && q_ws &&
       scale_ws && w_scale && ld_x >= K &&
       (scale_mode == CDIT_SCALE_BF16DIV || scale_mode == CDIT_SCALE_FP32DIV) &&

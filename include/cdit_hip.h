@@ -282,8 +282,8 @@ int cdit_w8a16_gemm_batched(int n_act, const void* const* x_bf16, const int64_t*
  * One quantized nn.Linear forward in the w8a8 dynamic mode: the two calls above
  * back to back on `stream` (per-token quantization of x into the caller's
  * workspace, then the scaled GEMM), saving one trip through the caller's FFI;
- * at M <= 16 and where that is faster (one row always) a single kernel that
- * quantizes the rows itself, with the same results and workspace contents.
+ * at M <= 16, where that is faster (cdit_debug_linear_launches), a single kernel
+ * that quantizes the rows itself, with the same results and workspace contents.
  * This is what torchao's Float8Tensor `aten.linear` override does for a Linear
  * that cache-dit converted with `quantize_(..., Float8DynamicActivation
  * Float8WeightConfig(granularity=(PerRow(), PerRow())))`
