@@ -950,8 +950,9 @@ int launch_wide_grouped(const GemmArgs& g, GemmGroup grp, hipStream_t stream) {
 // instructions per step, each on a wavefront of its own: about 250 clocks per step (500 with one
 // wavefront issuing both in order). Two feeding wavefronts: 3 to 8 % faster with one tile per CU,
 // 4 to 8 % slower with two. Conversions a step ahead of their MFMAs: the same or slower. D = 6: four
-// workgroups fit the LDS of a CU (4 x 36 KiB), with 8 three, and a fourth is a second round; 8 is 1 to 5 %
-// slower up to two per CU (but up to 6 % faster where 40 MB of weights come from HBM), 4 up to 27 % on such weights.
+// workgroups fit the LDS of a CU (4 x 36 KiB), with 8 three, and a fourth is a second round. With up to two per CU 8
+// is 1 to 5 % slower on matrices in the last-level cache; from HBM the same up to K = 4096 and 4 % faster beyond (geometric
+// mean of 325 shapes); 4 is up to 27 % slower there.
 // Another weight matrix per launch (M x K x N), us, one wavefront before -> now: 77 x 4096 x 3072
 // 15.9 -> 11.2, 17 x 3072 x 3072 12.3 -> 8.5, 128 x 3072 x 3072 13.2 -> 9.5, 256 x 15360 x 1024 47.4
 // -> 31, 100 x 1024 x 2048 6.3 -> 4.9; 128 x 64 tiles of the wide kernel -> now: 245 x 1664 x 2560 11.4 ->
