@@ -246,13 +246,21 @@ def w8a16_batched_into(acts) -> None:
     _native.check(rc)
 
 
-def w8a16_into(x2: torch.Tensor, w: torch.Tensor, w_scale: torch.Tensor,
-               bias: Optional[torch.Tensor], out: torch.Tensor, epilogue: int) -> None:
+def w8a16_into(x2: torch.Tensor, w: torch.Tensor, w_scale: torch.Tensor, bias: Optional[torch.Tensor],
+               out: Optional[torch.Tensor], epilogue: int) -> Optional[torch.Tensor]:
+  """out None (w is then the operator's [K, N] view of the weight): as in linear_w8a8_into."""
   if _codes_only:
     _reject_codes_only("w8a16_into", x2)
-  rc = _native.host().w8a16(x2, w, w_scale, bias, out, epilogue)
+  if out is None:
+    plain = _native.host().w8a16_plain(x2, w, w_scale, bias, epilogue)
+    if plain is None:
+      return None
+    rc, out = plain
+  else:
+    rc = _native.host().w8a16(x2, w, w_scale, bias, out, epilogue)
   if rc:
     _native.check(rc)
+  return out
 
 
 class _SharedQuant:
@@ -372,14 +380,23 @@ def clear_shared_activation_quant() -> None:
 
 
 def linear_w8a8_into(x2: torch.Tensor, w: torch.Tensor, w_scale: torch.Tensor,
-                     bias: Optional[torch.Tensor], out: torch.Tensor, q_ws: torch.Tensor,
-                     s_ws: torch.Tensor, scale_mode_id: int, epilogue: int) -> None:
-  """Quantizer + GEMM of one Linear forward in a single library call."""
+                     bias: Optional[torch.Tensor], out: Optional[torch.Tensor], q_ws: Optional[torch.Tensor],
+                     s_ws: Optional[torch.Tensor], scale_mode_id: int, epilogue: int) -> Optional[torch.Tensor]:
+  """Quantizer + GEMM of one Linear forward in a single library call. out None: the result and the
+  workspaces are allocated with the launch, in one call of the extension, and the result is
+  returned; None, with nothing launched, where the arguments are not plain."""
   if _codes_only:
     _reject_codes_only("linear_w8a8_into", x2)
-  rc = _native.host().linear_w8a8(x2, w, w_scale, bias, out, q_ws, s_ws, scale_mode_id, epilogue)
+  if out is None:
+    plain = _native.host().linear_plain(x2, w, w_scale, bias, scale_mode_id, epilogue, False)
+    if plain is None:
+      return None
+    rc, out = plain
+  else:
+    rc = _native.host().linear_w8a8(x2, w, w_scale, bias, out, q_ws, s_ws, scale_mode_id, epilogue)
   if rc:
     _native.check(rc)
+  return out
 
 
 # --------------------------------------------------------------------------- op definitions
@@ -448,10 +465,14 @@ def _fp8_rowwise_quant(x: torch.Tensor, scale_mode: int = 0) -> Tuple[torch.Tens
     raise ValueError("cdit::fp8_rowwise_quant: x must have at least one dimension")
   if scale_mode not in (0, 1):
     raise ValueError(f"cdit::fp8_rowwise_quant: scale_mode must be 0 or 1, got {scale_mode}")
-  plain = _native.host().quant_plain(x)
+  if _codes_only:
+    _reject_codes_only("quant_rowwise_into", x)
+  plain = _native.host().quant_plain(x, scale_mode)
   if plain is not None:
-    quant_rowwise_into(x, plain[0], plain[1], scale_mode)
-    return plain
+    rc, q, scale = plain
+    if rc:
+      _native.check(rc)
+    return q, scale
   x2 = _as_rows(x)
   q = torch.empty(x2.shape, dtype=FP8, device=x.device)
   scale = torch.empty((x2.shape[0], ), dtype=torch.float32, device=x.device)
@@ -495,10 +516,11 @@ def _float8_inference_scaled_mm(a_data, a_scale, b_data, b_scale, bias, out_dtyp
   del use_fast_accum  # a cuBLASLt hint; fp32 accumulation is the only mode here
   name = "cdit::float8_inference_scaled_mm"
   out_dtype = decode_output_dtype(out_dtype_id)
-  plain = _native.host().scaled_mm_plain(a_data, a_scale, b_data, b_scale, bias, out_dtype_id)
+  plain = _native.host().scaled_mm_plain(a_data, a_scale, b_data, b_scale, bias, out_dtype_id, epilogue)
   if plain is not None:
-    out, w = plain
-    gemm_rowwise_into(a_data, a_scale, w, b_scale, bias, out, epilogue)
+    rc, out = plain
+    if rc:
+      _native.check(rc)
     return out
   if a_data.dtype != FP8 or b_data.dtype != FP8:
     raise ValueError(f"{name}: a_data/b_data must be float8_e4m3fn, got {a_data.dtype}/"
@@ -627,6 +649,19 @@ def ln_modulate_quant(x: torch.Tensor, shift: torch.Tensor, scale: torch.Tensor,
 GRANULARITY_PER_ROW, GRANULARITY_PER_TENSOR = 0, 1
 
 
+def _linear_per_tensor(x, weight, weight_scale, bias, scale_mode, epilogue):
+  """A Linear with one activation scale, on plain arguments (else None)."""
+  if _codes_only:
+    _reject_codes_only("quant_tensorwise_into", x)
+  plain = _native.host().linear_plain(x, weight, weight_scale, bias, scale_mode, epilogue, True)
+  if plain is None:
+    return None
+  rc, out = plain
+  if rc:
+    _native.check(rc)
+  return out
+
+
 @torch.library.impl("cdit::linear_w8a8", "CUDA")
 def _linear_w8a8(x, weight, weight_scale, bias, scale_mode=0, epilogue=0, granularity=0,
                  share_input_quant=False):
@@ -639,15 +674,11 @@ def _linear_w8a8(x, weight, weight_scale, bias, scale_mode=0, epilogue=0, granul
   the op, so a traced graph only sees tensors in and a tensor out."""
   name = "cdit::linear_w8a8"
   if not share_input_quant and scale_mode in (0, 1) and granularity in (0, 1):
-    per_tensor = granularity == GRANULARITY_PER_TENSOR
-    plain = _native.host().linear_plain(x, weight, weight_scale, bias, per_tensor)
-    if plain is not None:
-      out, q, s = plain[:3]
-      if per_tensor:
-        quant_tensorwise_into(x, q, s, plain[3], scale_mode)
-        gemm_rowwise_into(q, s, weight, weight_scale, bias, out, epilogue)
-      else:
-        linear_w8a8_into(x, weight, weight_scale, bias, out, q, s, scale_mode, epilogue)
+    if granularity == GRANULARITY_PER_ROW:
+      out = linear_w8a8_into(x, weight, weight_scale, bias, None, None, None, scale_mode, epilogue)
+    else:
+      out = _linear_per_tensor(x, weight, weight_scale, bias, scale_mode, epilogue)
+    if out is not None:
       return out
   if x.dtype != torch.bfloat16:
     raise ValueError(f"{name}: x must be bfloat16, got {x.dtype}")
@@ -848,12 +879,10 @@ def _fake_linear_w8a8(x, weight, weight_scale, bias, scale_mode=0, epilogue=0, g
 def _w8a16_mm(x, b_data, b_scale, bias, out_dtype_id, epilogue=0):
   name = "cdit::w8a16_mm"
   out_dtype = decode_output_dtype(out_dtype_id)
-  plain = (_native.host().w8a16_plain(x, b_data, b_scale, bias)
-           if out_dtype == torch.bfloat16 else None)
-  if plain is not None:
-    out, w = plain
-    w8a16_into(x, w, b_scale, bias, out, epilogue)
-    return out
+  if out_dtype == torch.bfloat16:
+    out = w8a16_into(x, b_data, b_scale, bias, None, epilogue)
+    if out is not None:
+      return out
   if out_dtype != torch.bfloat16 or x.dtype != torch.bfloat16:
     raise ValueError(f"{name}: only bfloat16 activations and output are built, got {x.dtype} -> "
                      f"{out_dtype}")
