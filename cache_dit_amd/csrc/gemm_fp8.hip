@@ -1443,6 +1443,263 @@ int launch_tile32(const GemmArgs& g, hipStream_t stream) {
 }
 
 // ---------------------------------------------------------------------------
+// Problems that one round of tiles covers (a prompt's or a few hundred tokens' projections, K a whole number of
+// steps): a workgroup per tile, four (three, five) wavefronts that multiply and two that only feed them.
+// What bounds such a problem is what one CU gets through its vector memory path: some 64 KB in flight, whatever
+// the instructions issued ahead and whatever their cache policy, i.e. 58 GB/s of panels that come from HBM, 85 to 100
+// from the last-level cache (loads alone, without the arithmetic, of 256 x 12288 x 3072, M x N x K, on 192 tiles of 128 x
+// 128: 18.4 us from HBM of the kernel's 20.4). Lines that the other workgroups of the XCD have in flight or in the L2 count
+// like the rest, and touching them ahead from another wavefront takes as much of the path as it saves. So the time of a round
+// is (BM + BN) K bytes of the fullest CU, and the tile to take is the one with the shortest sides of which every CU gets
+// at most one: 96 x 96, 48 x 48, 32 x 48, 80 x 48 ... next to the wide kernel's and the 32 x 32 one. us, another weight
+// matrix per launch, the best of those -> this kernel, M x N x K: 77 x 3072 x 4096 10.6 -> 8.0 (32 x 48; on 288 tiles of 32 x 32 some
+// CUs get two), 200 x 2560 x 8192 20.7 -> 15.3, 512 x 3072 x 3072 14.8 -> 12.7 (96 x 96, 192 tiles; 64 x 128 as many), 512 x 3072 x
+// 12288 47.0 -> 37.4, 263 x 1216 x 8832 18.8 -> 13.1. With a second round of tiles it loses to the wide kernel, whose
+// stream of panels runs on from one tile to the next: chosen only for one (choose_one_round()).
+// The ring, its barrier and the order of K are those of gemm_fp8_tile32, MFMA and epilogue arithmetic the wide kernel's:
+// the same bits. Stages: as many as keep 64 KB in flight; one more or less is within 2 % (32 x 48: 5 stages 4 % slower
+// than 6), and where two workgroups then fit a CU's LDS a partial second round costs less (64 x 64 with 5 stages in place
+// of 6, 96 x 64 with 4: 9 %). Feeding wavefronts: with the multiplying ones issuing the DMA themselves the same time where the
+// panels come from HBM, 22 % longer K steps where they are in the L2 (0.25 us against 0.32 with 128 x 128).
+template <int BM_, int BN_, int WGM_, int WGN_, int DEPTH_, int GROUP_M_>
+struct CfgFed {
+  static constexpr int BM = BM_, BN = BN_, WGM = WGM_, WGN = WGN_, DEPTH = DEPTH_, GROUP_M = GROUP_M_;
+  static constexpr int WAVES = WGM * WGN, FEEDERS = 2, THREADS = 64 * (WAVES + FEEDERS);
+  static constexpr int WM = BM / WGM, WN = BN / WGN, TM = WM / 16, TN = WN / 16;  // wave tile, in fragments of 16 rows
+  static constexpr int A_BYTES = BM * 128, STAGE = (BM + BN) * 128, LDS_BYTES = DEPTH * STAGE;
+  static constexpr int NDMA = (BM + BN) / 8 / FEEDERS;  // DMA instructions (8 panel rows) per feeding wavefront and step
+  // Columns of a wave tile: LP blocks of 64 and NH of 32 in pairs of fragments as in the wide kernel, with an odd TN
+  // one fragment of 16 in its natural order behind them.
+  static constexpr int LP = TN / 4, NH = TN % 4 / 2, ODD = TN % 2;
+  static_assert(BM % (16 * WGM) == 0 && BN % (16 * WGN) == 0 && (BM + BN) / 8 % FEEDERS == 0, "whole fragments, whole instructions");
+  static_assert(DEPTH >= 3 && (DEPTH - 1) * NDMA <= 63 && LDS_BYTES <= 160 * 1024, "vmcnt has 6 bits; LDS");
+  // first of the four columns (of the wave tile) that lane group q holds of fragment j
+  __device__ static constexpr int col(int j, int q) {
+    return ODD && j == TN - 1 ? 16 * j + 4 * q : 32 * (j >> 1) + 8 * q + 4 * (j & 1);
+  }
+  // chunk c of B panel row r is stored at c ^ swizzle (for the rows that a fragment reads: conflict free)
+  __device__ static int swz_b_row(int r) { return ODD && r % WN >= 16 * (TN - 1) ? swz_a(r) : swz_b(r); }
+};
+
+template <class C, int OUT>
+__global__ __launch_bounds__(C::THREADS) __attribute__((amdgpu_waves_per_eu(2))) void
+gemm_fp8_fed(GemmArgs g, int tiles_m, int tiles_n) {
+  extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+  constexpr int D = C::DEPTH, BKW = 128, TM = C::TM, TN = C::TN;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int KT = g.K / BKW;
+  // workgroups go to the 8 XCDs in turn; each XCD gets consecutive tiles (any number of them), which share panels
+  const int ntiles = tiles_m * tiles_n, xcd = blockIdx.x % 8;
+  int tm, tn;
+  tile_of_linear<C::GROUP_M>(xcd * (ntiles / 8) + min(xcd, ntiles % 8) + blockIdx.x / 8, tiles_m, tiles_n, &tm, &tn);
+  const int m0 = tm * C::BM, n0 = tn * C::BN;
+
+  if (wave >= C::WAVES) {
+    // Feeding wavefront f: its instruction p fills the 8 panel rows from 8 (f NDMA + p) on, A's rows before B's; lane l
+    // lands on row l / 8, position l % 8 and fetches the chunk that the swizzle stores there.
+    const int f = wave - C::WAVES;
+    const uint8_t* const a = static_cast<const uint8_t*>(g.a) + (int64_t)m0 * g.lda;
+    const uint8_t* const b = g.b + (int64_t)n0 * g.ldb;
+    uint32_t off[C::NDMA];
+#pragma unroll
+    for (int p = 0; p < C::NDMA; ++p) {
+      const int row = (f * C::NDMA + p) * 8 + (lane >> 3), brow = row - C::BM;
+      off[p] = row < C::BM
+                   ? (uint32_t)min(row, g.M - m0 - 1) * (uint32_t)g.lda + ((lane & 7) ^ swz_a(row)) * 16
+                   : (uint32_t)min(brow, g.N - n0 - 1) * (uint32_t)g.ldb + ((lane & 7) ^ C::swz_b_row(brow)) * 16;
+    }
+    auto dma = [&](int kt, int stage) {
+      const int nrec = kt < KT ? 0x7fffffff : 0;  // steps beyond the last fetch nothing
+#pragma unroll
+      for (int p = 0; p < C::NDMA; ++p) {
+        const int q = f * C::NDMA + p;
+        const __amdgpu_buffer_rsrc_t src = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<uint8_t*>(q < C::BM / 8 ? a : b), 0, nrec, 0x00020000);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(
+            src, (__attribute__((address_space(3))) void*)(smem + stage + q * 1024), 16, (int)off[p], kt * BKW, 0, 0);
+      }
+    };
+#pragma unroll
+    for (int s = 0; s < D; ++s) dma(s, s * C::STAGE);
+    wait_and_barrier<(D - 1) * C::NDMA>();  // step 0 has landed
+    int stage = 0;                          // of step kt
+    for (int kt = 0; kt < KT; ++kt) {
+      // step kt + 1 has landed; behind the barrier the operands of step kt are in registers
+      wait_and_barrier<(D - 2) * C::NDMA>();
+      dma(kt + D, stage);
+      stage = stage + C::STAGE == D * C::STAGE ? 0 : stage + C::STAGE;
+    }
+    wait_vm<0>();  // no DMA outlives the workgroup
+    return;
+  }
+
+  const int wm = wave / C::WGN, wn = wave % C::WGN, r16 = lane & 15, kg = lane >> 4;
+  const int mw = m0 + wm * C::WM, nw = n0 + wn * C::WN;
+  // scales and bias; what lies beyond N (M) reads as zero, a null bias is an empty buffer
+  auto vec = [](const void* p, int bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00020000);
+  };
+  const __amdgpu_buffer_rsrc_t bs_buf = vec(g.b_scale, g.N * 4), bi_buf = vec(g.bias, g.bias ? g.N * 2 : 0),
+                               as_buf = vec(g.a_scale, g.M * 4);
+  v4f bs[TN];
+  uint2 bi[TN];
+  float as[TM];
+#pragma unroll
+  for (int j = 0; j < TN; ++j) {
+    const int n = nw + C::col(j, kg);
+    bs[j] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(bs_buf, n * 4, 0, 0));
+    bi[j] = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(bi_buf, n * 2, 0, 0));
+  }
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+    as[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(as_buf, (mw + 16 * i + r16) * 4, 0, 0));
+
+  struct Step {
+    v8i a[TM], b[TN];
+  };
+  // (__restrict__: see the wide kernel; without it every read would wait for the whole stream)
+  auto fragment = [&](const uint8_t* __restrict__ st, int row, int swz) -> v8i {
+    const v4i lo = *reinterpret_cast<const v4i*>(st + row * BKW + (((2 * kg) ^ swz) << 4));
+    const v4i hi = *reinterpret_cast<const v4i*>(st + row * BKW + (((2 * kg + 1) ^ swz) << 4));
+    return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+  };
+  // fragment q of a step, in the order of their first use: A_0, B_0 .. B_{TN-1}, A_1 ..
+  const int arow = wm * C::WM + r16, brow = wn * C::WN + 8 * (r16 >> 2) + (r16 & 3);
+  auto read = [&](const uint8_t* st, Step& f, int q) {
+    if (q == 0 || q > TN) {
+      const int i = q ? q - TN : 0;
+      f.a[i] = fragment(st, arow + 16 * i, swz_a(arow));
+    } else {
+      const int j = q - 1, row = C::ODD && j == TN - 1 ? wn * C::WN + 16 * j + r16 : brow + 32 * (j >> 1) + 4 * (j & 1);
+      f.b[j] = fragment(st + C::A_BYTES, row, C::swz_b_row(row));
+    }
+  };
+  v4f acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) acc[i][j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+  wait_and_barrier<63>();
+  Step even, odd;
+#pragma unroll
+  for (int q = 0; q < TM + TN; ++q) read(smem, even, q);
+  int stage = C::STAGE;  // of step kt + 1
+  // Step kt: its operands are in `f`; reads step kt + 1 into `nf`, spread over the first three quarters of the MFMAs.
+  auto step = [&](const Step& f, Step& nf) {
+    wait_and_barrier<63>();
+    const uint8_t* st = smem + stage;
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int s = 0; s < TM * TN; ++s) {
+#pragma unroll
+      for (int q = 0; q < TM + TN; ++q)
+        if (q * TM * TN * 3 / 4 / (TM + TN) == s) read(st, nf, q);
+      // operands swapped: result rows follow B (n), result columns follow A (m)
+      acc[s / TN][s % TN] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(f.b[s % TN], f.a[s / TN], acc[s / TN][s % TN],
+                                                                             0, 0, 0, 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    stage = stage + C::STAGE == D * C::STAGE ? 0 : stage + C::STAGE;
+  };
+  for (int kt = 0; kt < KT; kt += 2) {
+    step(even, odd);
+    if (kt + 1 < KT) step(odd, even);
+  }
+
+  // acc[i][j][e] is out[mw + 16 i + r16][nw + col(j, kg) + e]. 16-bit outputs change lanes before they are stored, as in
+  // the wide kernel, so that adjacent lanes hold adjacent bytes. Rows beyond M are beyond the descriptor, columns beyond N
+  // get an offset that is (N % 8 == 0: the 4 or 8 columns of a lane are all in or all out).
+  constexpr int OB = OUT == CDIT_DT_F32 ? 4 : 2;
+  const uint32_t ldo = (uint32_t)g.ldo * OB;
+  uint8_t* const out_wave = reinterpret_cast<uint8_t*>(g.out) + ((int64_t)mw * g.ldo + nw) * OB;
+  const int rows_wave = g.M - mw, cols_wave = g.N - nw;
+  auto at = [&](int row, int c) { return (int)(c < cols_wave ? (uint32_t)row * ldo + (uint32_t)(c * OB) : 0x80000000u); };
+  const int bp_line = 4 * (16 * (lane & 3) + 8 * ((lane >> 2) & 1) + (lane >> 3));
+  const int bp_half = 4 * (16 * (lane & 3) + (lane >> 2));
+  auto epilogue = [&](auto gelu_tag) {
+    constexpr bool GELU = decltype(gelu_tag)::value;
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      const int rows = __builtin_amdgcn_readfirstlane(min(max(rows_wave - 16 * i, 0), 16));
+      const __amdgpu_buffer_rsrc_t out_row = __builtin_amdgcn_make_buffer_rsrc(
+          out_wave + (int64_t)(16 * i) * ldo, 0, rows * (int)ldo, 0x00020000);
+      uint32_t pk[TN][2];
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        const float b4[4] = {bias_to_f32<OUT>(bi[j].x & 0xffffu), bias_to_f32<OUT>(bi[j].x >> 16),
+                             bias_to_f32<OUT>(bi[j].y & 0xffffu), bias_to_f32<OUT>(bi[j].y >> 16)};
+        float v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          v[e] = __fmaf_rn(acc[i][j][e] * as[i], bs[j][e], b4[e]);
+          if constexpr (GELU) v[e] = gelu_tanh(v[e]);
+        }
+        if constexpr (OUT == CDIT_DT_F32) {
+          __builtin_amdgcn_raw_buffer_store_b128(
+              v4u{__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), __float_as_uint(v[3])}, out_row,
+              at(r16, C::col(j, kg)), 0, 0);
+        } else {
+#pragma unroll
+          for (int k = 0; k < 2; ++k)
+            pk[j][k] = OUT == CDIT_DT_F16 ? pack_f16x2(v[2 * k], v[2 * k + 1]) : pack_bf16x2(v[2 * k], v[2 * k + 1]);
+        }
+      }
+      if constexpr (OUT != CDIT_DT_F32) {
+#pragma unroll
+        for (int v = 0; v < C::LP; ++v) {
+          v4u x, y;
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            const int w0 = (int)pk[4 * v + (k >> 1)][k & 1], w1 = (int)pk[4 * v + 2 + (k >> 1)][k & 1];
+            const int p = __builtin_amdgcn_update_dpp(w0, w1, 0x128, 0xf, 0xc, false);
+            const int q = __builtin_amdgcn_update_dpp(w1, w0, 0x128, 0xf, 0x3, false);
+            x[k] = (uint32_t)__builtin_amdgcn_ds_bpermute(bp_line, p);
+            y[k] = (uint32_t)__builtin_amdgcn_ds_bpermute(bp_line, q);
+          }
+          const int c = 64 * v + 8 * (lane & 7);
+          __builtin_amdgcn_raw_buffer_store_b128(x, out_row, at(lane >> 3, c), 0, 2);
+          __builtin_amdgcn_raw_buffer_store_b128(y, out_row, at(8 + (lane >> 3), c), 0, 2);
+        }
+        if constexpr (C::NH) {
+          v4u x;
+#pragma unroll
+          for (int k = 0; k < 4; ++k)
+            x[k] = (uint32_t)__builtin_amdgcn_ds_bpermute(bp_half, (int)pk[4 * C::LP + (k >> 1)][k & 1]);
+          __builtin_amdgcn_raw_buffer_store_b128(x, out_row, at(lane >> 2, 64 * C::LP + 8 * (lane & 3)), 0, 0);
+        }
+        if constexpr (C::ODD)
+          __builtin_amdgcn_raw_buffer_store_b64(v2u{pk[TN - 1][0], pk[TN - 1][1]}, out_row, at(r16, C::col(TN - 1, kg)),
+                                                0, 0);
+      }
+    }
+  };
+  if (g.epilogue & CDIT_EPI_GELU_TANH) {
+    epilogue(std::true_type{});
+  } else {
+    epilogue(std::false_type{});
+  }
+}
+
+template <class C, int OUT>
+int launch_fed_out(const GemmArgs& g, hipStream_t stream) {
+  static bool lds_allowed[64];
+  if (int rc = allow_dynamic_lds(reinterpret_cast<const void*>(&gemm_fp8_fed<C, OUT>), C::LDS_BYTES, lds_allowed))
+    return rc;
+  const int tiles_m = (g.M + C::BM - 1) / C::BM, tiles_n = (g.N + C::BN - 1) / C::BN;
+  hipLaunchKernelGGL((gemm_fp8_fed<C, OUT>), dim3(tiles_m * tiles_n), dim3(C::THREADS), C::LDS_BYTES, stream, g, tiles_m,
+                     tiles_n);
+  return 0;
+}
+template <class C>
+int launch_fed(const GemmArgs& g, hipStream_t stream) {
+  switch (g.out_dtype) {
+    case CDIT_DT_F16: return launch_fed_out<C, CDIT_DT_F16>(g, stream);
+    case CDIT_DT_F32: return launch_fed_out<C, CDIT_DT_F32>(g, stream);
+    default: return launch_fed_out<C, CDIT_DT_BF16>(g, stream);
+  }
+}
+
+// ---------------------------------------------------------------------------
 // Skinny kernel for M <= 16 (the M = 1 modulation Linears `norm1.linear`,
 // `norm.linear` of every block): pure weight streaming. A workgroup of 4 waves
 // owns 16 output channels; each wave takes a quarter of K and reads its weight
@@ -1915,6 +2172,14 @@ typedef CfgWide<128, 192, 4, 3> V16;                  // ... 64x96 wave tiles, D
 typedef CfgWide<64, 128, 8, 5> V17;                   // ... 32x64 wave tiles, DMA 5 steps ahead
 typedef CfgWide<128, 128, 4, 4> V18;                  // ... 64x64 wave tiles, DMA 4 steps ahead
 typedef CfgWide<256, 128, 4> V19;                     // ... 128x64 wave tiles, for K remainders only
+//         BM   BN  waves depth groupM
+typedef CfgFed<32, 48, 1, 3, 6, 8> V31;
+typedef CfgFed<48, 48, 1, 3, 6, 8> V32;
+typedef CfgFed<80, 48, 5, 1, 5, 8> V33;
+typedef CfgFed<64, 64, 2, 2, 5, 8> V34;
+typedef CfgFed<96, 64, 2, 2, 4, 8> V35;
+typedef CfgFed<96, 96, 2, 2, 5, 4> V36;
+typedef CfgFed<128, 96, 2, 2, 5, 4> V37;
 // the two large tiles with contiguous wave columns and half-line output stores (16 rows x 64
 // bytes per store instruction), kept to measure the whole-line stores against: variants 112, 114
 typedef CfgWide<256, 256, 4, 2, false> V12H;
@@ -2134,8 +2399,52 @@ struct WideOk {
   bool operator()(int depth) const { return K >= 128 * (depth > 3 ? depth : 3); }
 };
 
-// The kernel for a problem: 100 for any shape and alignment, 51 one row, 50 up to 16 rows, 26 a workgroup per
-// 32 x 32 tile, else a tile of the wide kernel (K remainders: of its instances for them) or of the tiled one.
+// Tiles for problems that one round of them covers, with their measured round times: the kernel above (31 to 37), the
+// 32 x 32 one (26) and the wide kernel's. Fitted to the times of 400 problems with every tile (M 17 to 4000, K 1024 to 15360,
+// N 1024 to 12288, at most 160 tiles of 256 x 256, weights from HBM; 8.5 % rms): of those that one round covers it takes one
+// that is 1.1 % off the best (geometric mean), 0.89 of the time that the choice among the older tiles gives (0.94 over all
+// problems of M 17 to 6889, K 256 to 15360, N 256 to 12288, bf16 and fp32 outputs), with 4 of 220 more than 4 % slower (8 %
+// the worst, 28 x 7712 x 14976, M x N x K).
+constexpr LaunchModel kOneLaunch = {1425, 907, 907};
+constexpr TileTime kOneRound[] = {{15, 256, 192, V15::DEPTH, 5000, 987}, {16, 128, 192, V16::DEPTH, 3710, 676},
+                                  {18, 128, 128, V18::DEPTH, 3100, 517}, {17, 64, 128, V17::DEPTH, 2620, 434},
+                                  {37, 128, 96, 3, 3260, 428},           {36, 96, 96, 3, 2920, 389},
+                                  {35, 96, 64, 3, 2510, 305},            {34, 64, 64, 3, 2340, 263},
+                                  {33, 80, 48, 3, 2310, 244},            {32, 48, 48, 3, 1910, 198},
+                                  {31, 32, 48, 3, 1640, 183},            {26, 32, 32, 3, 1430, 184}};
+
+// The tile of a problem that one round covers, -1 if there is none. fp32 outputs of short K are bound by their stores: the
+// other rules know them (1116 x 6016 x 512, M x N x K: 13.7 us, 15.4 by this one).
+int choose_one_round(const GemmArgs& g) {
+  if (!tiled_ok(g) || g.M <= 16 || g.K < (g.out_dtype == CDIT_DT_F32 ? 9 : 3) * BK) return -1;
+  const int64_t cus = cu_count() > 0 ? cu_count() : 256;
+  int best = -1;
+  int64_t time = INT64_MAX;
+  for (const auto& c : kOneRound) {
+    if (g.K < c.depth * BK || (c.variant == 16 && g.out_dtype != CDIT_DT_BF16)) continue;
+    const int64_t tiles = c.variant == 26 ? tiles32(g.M, g.N).padded
+                                          : (int64_t)((g.M + c.bm - 1) / c.bm) * ((g.N + c.bn - 1) / c.bn);
+    if (tiles > cus) continue;
+    const int64_t t = launch_ns(kOneLaunch, c, tiles, cus, g.K / BK);
+    if (t < time) best = c.variant, time = t;
+  }
+  return best;
+}
+
+int launch_gemm_fp8_fed(const GemmArgs& g, int variant, hipStream_t stream) {
+  switch (variant) {
+    case 31: return launch_fed<V31>(g, stream);
+    case 32: return launch_fed<V32>(g, stream);
+    case 33: return launch_fed<V33>(g, stream);
+    case 34: return launch_fed<V34>(g, stream);
+    case 35: return launch_fed<V35>(g, stream);
+    case 36: return launch_fed<V36>(g, stream);
+    default: return launch_fed<V37>(g, stream);
+  }
+}
+
+// The kernel for a problem that one round does not cover (choose_one_round()): 100 for any shape and alignment, 51 one
+// row, 50 up to 16 rows, 26 a workgroup per 32 x 32 tile, else a tile of the wide kernel (K remainders: of its instances for them) or of the tiled one.
 int choose_gemm_fp8(const GemmArgs& g) {
   if (!aligned_ok(g)) return 100;
   if (row1_ok(g)) return 51;
@@ -2161,6 +2470,7 @@ int linear_fp8_launches(const GemmArgs& g) {
 
 int launch_gemm_fp8(const GemmArgs& g, int variant, hipStream_t stream) {
   if (!aligned_ok(g)) variant = 100;
+  if (variant < 0) variant = choose_one_round(g);
   if (variant < 0) variant = choose_gemm_fp8(g);
   if (variant == 100) {
     dim3 grid((g.N + 15) / 16, (g.M + 15) / 16);
@@ -2182,6 +2492,7 @@ int launch_gemm_fp8(const GemmArgs& g, int variant, hipStream_t stream) {
   }
   if (variant == 26) return tile32_tail(g) ? launch_tile32<true>(g, stream) : launch_tile32<false>(g, stream);
   if (!tiled_ok(g)) return launch_gemm_fp8_ktail(g, variant, stream);
+  if (variant >= 31 && variant <= 37) return launch_gemm_fp8_fed(g, variant, stream);
   const WideOk wide_ok{g.K};
   if (g.out_dtype != CDIT_DT_BF16) {
     const int v = choose_other_out_variant(g, variant, wide_ok);

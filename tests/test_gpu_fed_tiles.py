@@ -1,0 +1,83 @@
+"""The FP8 GEMM's tiles for problems that one round covers (a workgroup per tile, fed by wavefronts of its own):
+every tile at partial rows and columns, K shorter than its ring, odd and even numbers of steps, every output type,
+bit for bit against the wide kernel; and which problems take them."""
+import pytest
+import torch
+
+FP8 = torch.float8_e4m3fn
+DEV = "cuda"
+TILES = {31: (32, 48), 32: (48, 48), 33: (80, 48), 34: (64, 64), 35: (96, 64), 36: (96, 96), 37: (128, 96)}
+
+
+@pytest.fixture(autouse=True)
+def _auto_variant():
+  from cache_dit_amd import _native
+  if not _native.is_built():
+    pytest.skip("libcdit_hip.so not built")
+  _native.set_gemm_variant(-1)
+  yield
+  _native.set_gemm_variant(-1)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("variant", sorted(TILES))
+def test_bits_of_the_wide_kernel(variant, dtype):
+  """The output is a window of a buffer of sentinels; what lies beyond K in the operands' rows is NaN. 384 and 640: K of
+  which every tile of the wide kernel (3 to 5 steps ahead) takes one."""
+  from cache_dit_amd import _native, ops
+  bm, bn = TILES[variant]
+  for M, N, K in ((17, 8, 640), (bm, bn, 384), (bm + 1, bn + 8, 768), (3 * bm - 15, 9 * bn - 40, 640),
+                  (2 * bm + 16, 17 * bn + 16, 1152)):
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    a, w = torch.full((M, K + 16), float("nan"), device=DEV).to(FP8), torch.full((N, K + 32), float("nan"), device=DEV).to(FP8)
+    a[:, :K] = torch.randn(M, K, generator=g, device=DEV).to(FP8)
+    w[:, :K] = torch.randn(N, K, generator=g, device=DEV).to(FP8)
+    sa, sw = torch.rand(M, generator=g, device=DEV), torch.rand(N, generator=g, device=DEV)
+    for bias in ((False, ) if dtype == torch.float32 else (False, True)):
+      b = torch.randn(N, generator=g, device=DEV).to(dtype) if bias else None
+      for epilogue in (0, 1):
+        outs = []
+        for v in (variant, 17 if K >= 640 else 15):
+          _native.set_gemm_variant(v)
+          outs.append(torch.full((M + 2, N + 8), 777.0, dtype=dtype, device=DEV))
+          ops.gemm_rowwise_into(a[:, :K], sa, w[:, :K], sw, b, outs[-1][1:M + 1, :N], epilogue)
+        torch.cuda.synchronize()
+        assert torch.equal(outs[0], outs[1]), (M, N, K, bias, epilogue)
+        outs[0][1:M + 1, :N] = 777.0
+        assert bool((outs[0] == 777.0).all()), (M, N, K, bias, epilogue)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(77, 3072, 4096), (200, 2560, 8192), (512, 3072, 3072), (250, 12288, 1024)])
+def test_the_choice_and_its_neighbours(M, N, K):
+  """By shape, against the wide kernel, on both sides of a round: M rows and as many as need one more."""
+  from cache_dit_amd import _native, ops
+  tile = TILES[_native.load().cdit_debug_gemm_choice(2, M, N, K, 1)]
+  g = torch.Generator(device=DEV).manual_seed(M)
+  rows = -(-M // tile[0]) * tile[0] + 1
+  a = torch.randn(rows, K, generator=g, device=DEV).to(FP8)
+  w = torch.randn(N, K, generator=g, device=DEV).to(FP8)
+  sa, sw = torch.rand(rows, generator=g, device=DEV), torch.rand(N, generator=g, device=DEV)
+  for m in (M, rows - 1, rows):
+    outs = []
+    for v in (-1, 17):
+      _native.set_gemm_variant(v)
+      outs.append(torch.empty(m, N, dtype=torch.bfloat16, device=DEV))
+      ops.gemm_rowwise_into(a[:m], sa[:m].clone(), w, sw, None, outs[-1], 0)
+    torch.cuda.synchronize()
+    assert torch.equal(outs[0], outs[1]), m
+
+
+@pytest.mark.parametrize("M,N,K,want", [
+    (77, 3072, 4096, 31), (200, 2560, 8192, 33), (512, 3072, 3072, 36), (512, 3072, 12288, 36), (1021, 3072, 3072, 37),
+    (512, 12288, 3072, 16), (100, 1024, 3072, 26), (4608, 3072, 3072, 0), (2048, 12288, 3072, 0),
+    # up to 16 rows, K remainders and K of one or two steps have other rules
+    (16, 3072, 3072, 0), (77, 3072, 4112, 0), (77, 3072, 256, 0)])
+def test_tile_of_one_round(M, N, K, want):
+  from cache_dit_amd import _native
+  lib = _native.load()
+  assert lib.cdit_debug_gemm_choice(2, M, N, K, 1) == want
+  if want != 16:  # built for bf16 outputs only
+    assert lib.cdit_debug_gemm_choice(2, M, N, K, 0) == want
+  assert lib.cdit_debug_gemm_choice(2, M, N, 1024, 2) == 0  # short K, fp32 outputs: bound by the stores
