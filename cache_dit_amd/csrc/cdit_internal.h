@@ -99,6 +99,7 @@ struct GemmGroup {
 // quantizes the rows itself).
 int choose_one_round(const GemmArgs& g);
 int choose_gemm_fp8(const GemmArgs& g);
+int choose_one_round_w8a16(const GemmArgs& g);
 int choose_gemm_w8a16(const GemmArgs& g);
 int linear_fp8_launches(const GemmArgs& g);
 // variant < 0: choose by shape.

@@ -1461,15 +1461,16 @@ int launch_tile32(const GemmArgs& g, hipStream_t stream) {
 // than 6), and where two workgroups then fit a CU's LDS a partial second round costs less (64 x 64 with 5 stages in place
 // of 6, 96 x 64 with 4: 9 %). Feeding wavefronts: with the multiplying ones issuing the DMA themselves the same time where the
 // panels come from HBM, 22 % longer K steps where they are in the L2 (0.25 us against 0.32 with 128 x 128).
-template <int BM_, int BN_, int WGM_, int WGN_, int DEPTH_, int GROUP_M_>
+template <int BM_, int BN_, int WGM_, int WGN_, int DEPTH_>
 struct CfgFed {
-  static constexpr int BM = BM_, BN = BN_, WGM = WGM_, WGN = WGN_, DEPTH = DEPTH_, GROUP_M = GROUP_M_;
+  static constexpr int BM = BM_, BN = BN_, WGM = WGM_, WGN = WGN_, DEPTH = DEPTH_;
+  static constexpr int GROUP_M = 8;  // (4: the same time)
   static constexpr int WAVES = WGM * WGN, FEEDERS = 2, THREADS = 64 * (WAVES + FEEDERS);
   static constexpr int WM = BM / WGM, WN = BN / WGN, TM = WM / 16, TN = WN / 16;  // wave tile, in fragments of 16 rows
   static constexpr int A_BYTES = BM * 128, STAGE = (BM + BN) * 128, LDS_BYTES = DEPTH * STAGE;
   static constexpr int NDMA = (BM + BN) / 8 / FEEDERS;  // DMA instructions (8 panel rows) per feeding wavefront and step
   // Columns of a wave tile: LP blocks of 64 and NH of 32 in pairs of fragments as in the wide kernel, with an odd TN
-  // one fragment of 16 in its natural order behind them.
+  // one fragment of 16 in its natural order behind them (store_fed_tile).
   static constexpr int LP = TN / 4, NH = TN % 4 / 2, ODD = TN % 2;
   static_assert(BM % (16 * WGM) == 0 && BN % (16 * WGN) == 0 && (BM + BN) / 8 % FEEDERS == 0, "whole fragments, whole instructions");
   static_assert(DEPTH >= 3 && (DEPTH - 1) * NDMA <= 63 && LDS_BYTES <= 160 * 1024, "vmcnt has 6 bits; LDS");
@@ -1606,77 +1607,12 @@ gemm_fp8_fed(GemmArgs g, int tiles_m, int tiles_n) {
     if (kt + 1 < KT) step(odd, even);
   }
 
-  // acc[i][j][e] is out[mw + 16 i + r16][nw + col(j, kg) + e]. 16-bit outputs change lanes before they are stored, as in
-  // the wide kernel, so that adjacent lanes hold adjacent bytes. Rows beyond M are beyond the descriptor, columns beyond N
-  // get an offset that is (N % 8 == 0: the 4 or 8 columns of a lane are all in or all out).
-  constexpr int OB = OUT == CDIT_DT_F32 ? 4 : 2;
-  const uint32_t ldo = (uint32_t)g.ldo * OB;
-  uint8_t* const out_wave = reinterpret_cast<uint8_t*>(g.out) + ((int64_t)mw * g.ldo + nw) * OB;
-  const int rows_wave = g.M - mw, cols_wave = g.N - nw;
-  auto at = [&](int row, int c) { return (int)(c < cols_wave ? (uint32_t)row * ldo + (uint32_t)(c * OB) : 0x80000000u); };
-  const int bp_line = 4 * (16 * (lane & 3) + 8 * ((lane >> 2) & 1) + (lane >> 3));
-  const int bp_half = 4 * (16 * (lane & 3) + (lane >> 2));
-  auto epilogue = [&](auto gelu_tag) {
-    constexpr bool GELU = decltype(gelu_tag)::value;
-#pragma unroll
-    for (int i = 0; i < TM; ++i) {
-      const int rows = __builtin_amdgcn_readfirstlane(min(max(rows_wave - 16 * i, 0), 16));
-      const __amdgpu_buffer_rsrc_t out_row = __builtin_amdgcn_make_buffer_rsrc(
-          out_wave + (int64_t)(16 * i) * ldo, 0, rows * (int)ldo, 0x00020000);
-      uint32_t pk[TN][2];
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        const float b4[4] = {bias_to_f32<OUT>(bi[j].x & 0xffffu), bias_to_f32<OUT>(bi[j].x >> 16),
-                             bias_to_f32<OUT>(bi[j].y & 0xffffu), bias_to_f32<OUT>(bi[j].y >> 16)};
-        float v[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          v[e] = __fmaf_rn(acc[i][j][e] * as[i], bs[j][e], b4[e]);
-          if constexpr (GELU) v[e] = gelu_tanh(v[e]);
-        }
-        if constexpr (OUT == CDIT_DT_F32) {
-          __builtin_amdgcn_raw_buffer_store_b128(
-              v4u{__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), __float_as_uint(v[3])}, out_row,
-              at(r16, C::col(j, kg)), 0, 0);
-        } else {
-#pragma unroll
-          for (int k = 0; k < 2; ++k)
-            pk[j][k] = OUT == CDIT_DT_F16 ? pack_f16x2(v[2 * k], v[2 * k + 1]) : pack_bf16x2(v[2 * k], v[2 * k + 1]);
-        }
-      }
-      if constexpr (OUT != CDIT_DT_F32) {
-#pragma unroll
-        for (int v = 0; v < C::LP; ++v) {
-          v4u x, y;
-#pragma unroll
-          for (int k = 0; k < 4; ++k) {
-            const int w0 = (int)pk[4 * v + (k >> 1)][k & 1], w1 = (int)pk[4 * v + 2 + (k >> 1)][k & 1];
-            const int p = __builtin_amdgcn_update_dpp(w0, w1, 0x128, 0xf, 0xc, false);
-            const int q = __builtin_amdgcn_update_dpp(w1, w0, 0x128, 0xf, 0x3, false);
-            x[k] = (uint32_t)__builtin_amdgcn_ds_bpermute(bp_line, p);
-            y[k] = (uint32_t)__builtin_amdgcn_ds_bpermute(bp_line, q);
-          }
-          const int c = 64 * v + 8 * (lane & 7);
-          __builtin_amdgcn_raw_buffer_store_b128(x, out_row, at(lane >> 3, c), 0, 2);
-          __builtin_amdgcn_raw_buffer_store_b128(y, out_row, at(8 + (lane >> 3), c), 0, 2);
-        }
-        if constexpr (C::NH) {
-          v4u x;
-#pragma unroll
-          for (int k = 0; k < 4; ++k)
-            x[k] = (uint32_t)__builtin_amdgcn_ds_bpermute(bp_half, (int)pk[4 * C::LP + (k >> 1)][k & 1]);
-          __builtin_amdgcn_raw_buffer_store_b128(x, out_row, at(lane >> 2, 64 * C::LP + 8 * (lane & 3)), 0, 0);
-        }
-        if constexpr (C::ODD)
-          __builtin_amdgcn_raw_buffer_store_b64(v2u{pk[TN - 1][0], pk[TN - 1][1]}, out_row, at(r16, C::col(TN - 1, kg)),
-                                                0, 0);
-      }
-    }
-  };
+  uint8_t* const out_wave =
+      reinterpret_cast<uint8_t*>(g.out) + ((int64_t)mw * g.ldo + nw) * (OUT == CDIT_DT_F32 ? 4 : 2);
   if (g.epilogue & CDIT_EPI_GELU_TANH) {
-    epilogue(std::true_type{});
+    store_fed_tile<C, OUT, true>(acc, as, bs, bi, out_wave, g.ldo, g.M - mw, g.N - nw, lane);
   } else {
-    epilogue(std::false_type{});
+    store_fed_tile<C, OUT, false>(acc, as, bs, bi, out_wave, g.ldo, g.M - mw, g.N - nw, lane);
   }
 }
 
@@ -2172,14 +2108,14 @@ typedef CfgWide<128, 192, 4, 3> V16;                  // ... 64x96 wave tiles, D
 typedef CfgWide<64, 128, 8, 5> V17;                   // ... 32x64 wave tiles, DMA 5 steps ahead
 typedef CfgWide<128, 128, 4, 4> V18;                  // ... 64x64 wave tiles, DMA 4 steps ahead
 typedef CfgWide<256, 128, 4> V19;                     // ... 128x64 wave tiles, for K remainders only
-//         BM   BN  waves depth groupM
-typedef CfgFed<32, 48, 1, 3, 6, 8> V31;
-typedef CfgFed<48, 48, 1, 3, 6, 8> V32;
-typedef CfgFed<80, 48, 5, 1, 5, 8> V33;
-typedef CfgFed<64, 64, 2, 2, 5, 8> V34;
-typedef CfgFed<96, 64, 2, 2, 4, 8> V35;
-typedef CfgFed<96, 96, 2, 2, 5, 4> V36;
-typedef CfgFed<128, 96, 2, 2, 5, 4> V37;
+//             BM  BN  waves depth
+typedef CfgFed<32, 48, 1, 3, 6> V31;
+typedef CfgFed<48, 48, 1, 3, 6> V32;
+typedef CfgFed<80, 48, 5, 1, 5> V33;
+typedef CfgFed<64, 64, 2, 2, 5> V34;
+typedef CfgFed<96, 64, 2, 2, 4> V35;
+typedef CfgFed<96, 96, 2, 2, 5> V36;
+typedef CfgFed<128, 96, 2, 2, 5> V37;
 // the two large tiles with contiguous wave columns and half-line output stores (16 rows x 64
 // bytes per store instruction), kept to measure the whole-line stores against: variants 112, 114
 typedef CfgWide<256, 256, 4, 2, false> V12H;

@@ -1110,6 +1110,198 @@ int launch_wavetile(const GemmArgs& g, hipStream_t stream) {
 }
 
 // ---------------------------------------------------------------------------
+// Problems that one round of tiles covers, as gemm_fp8_fed: bound by what one CU gets through its vector memory path (64 KB
+// in flight: 58 GB/s from HBM, 85 to 100 from the last-level cache), here (2 BM + BN) K bytes of the fullest CU. So tiles that
+// are wider than they are high, and of as many shapes as it takes for every CU to get at most one. A wavefront multiplies all
+// rows of the tile with its share of the columns, whose weights are then converted once per workgroup (8 conversions per 16
+// columns and 64 elements next to 2 MFMAs per 16 x 16 block); one or two wavefronts only feed. A step is SUB times 64
+// elements between two barriers: with 128 the small tiles, whose steps are short, take 4 % (48 x 64) to 20 % (32 x 32) less;
+// the larger ones, with room for fewer stages then, 2 to 4 % more (64 x 96, 48 x 96).
+// v_mfma_f32_16x16x32_bf16 adds its 32 products in the order of the lane groups that hold them, eight at a time, after
+// the accumulator: a chain of them over the pieces in the order in which the wide kernel's 32x32x16 instructions take theirs
+// (in each 32 elements the first, third, second and fourth eight) gives the same bits, which is what the swap of the piece's
+// two low bits in the swizzle is for.
+// us, another weight matrix per launch, the best of the other kernels -> this one, M x N x K: 77 x 3072 x 4096 13.9 -> 10.9 (16 x
+// 64: 240 tiles; of the 288 of 32 x 32 some CUs get two), 200 x 2560 x 8192 31.5 -> 26.1 (48 x 64), 17 x 3072 x 3072 9.2 -> 8.7
+// (32 x 32), 342 x 2752 x 12352 61.1 -> 46.3 (80 x 64).
+template <int BM_, int BN_, int WAVES_, int SUB_, int DEPTH_>
+struct CfgFedW {
+  static constexpr int BM = BM_, BN = BN_, WAVES = WAVES_, SUB = SUB_, DEPTH = DEPTH_;
+  static constexpr int GROUP_M = 8;  // (4: the same time)
+  static constexpr int DMA_A = BM / 8, DMA_B = BN / 16;  // DMA instructions per 64 elements
+  static constexpr int FEEDERS = (DMA_A + DMA_B) % 2 ? 1 : 2, NDMA = (DMA_A + DMA_B) / FEEDERS, THREADS = 64 * (WAVES + FEEDERS);
+  static constexpr int WN = BN / WAVES, TM = BM / 16, TN = WN / 16;
+  static constexpr int A_BYTES = BM * 2 * BKE, PART = A_BYTES + BN * BKE, STAGE = SUB * PART, LDS_BYTES = DEPTH * STAGE;
+  static constexpr int LP = TN / 4, NH = TN % 4 / 2, ODD = TN % 2;  // as in store_fed_tile
+  static_assert(BM % 16 == 0 && BN % (16 * WAVES) == 0, "whole fragments");
+  static_assert(DEPTH >= 3 && (DEPTH - 1) * NDMA * SUB <= 63 && LDS_BYTES <= 160 * 1024, "vmcnt has 6 bits; LDS");
+  // first of the four columns (of the wavefront's) that lane group q holds of fragment j
+  __device__ static constexpr int col(int j, int q) {
+    return ODD && j == TN - 1 ? 16 * j + 4 * q : 32 * (j >> 1) + 8 * q + 4 * (j & 1);
+  }
+  // chunk c of B panel row r is stored at c ^ swizzle
+  __device__ static int swz_b(int r) { return ODD && r % WN >= 16 * (TN - 1) ? (r >> 2) & 3 : (r >> 3) & 3; }
+};
+
+template <class C>
+__global__ __launch_bounds__(C::THREADS) __attribute__((amdgpu_waves_per_eu(2))) void
+gemm_w8a16_fed(GemmArgs g, int tiles_m, int tiles_n) {
+  extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+  constexpr int D = C::DEPTH, TM = C::TM, TN = C::TN, SUB = C::SUB;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int KT = (g.K + SUB * BKE - 1) / (SUB * BKE);
+  // workgroups go to the 8 XCDs in turn; each XCD gets consecutive tiles (any number of them), which share panels
+  const int ntiles = tiles_m * tiles_n, xcd = blockIdx.x % 8;
+  int tm, tn;
+  tile_of_linear<C::GROUP_M>(xcd * (ntiles / 8) + min(xcd, ntiles % 8) + blockIdx.x / 8, tiles_m, tiles_n, &tm, &tn);
+  const int m0 = tm * C::BM, n0 = tn * C::BN;
+
+  if (wave >= C::WAVES) {
+    // Feeding wavefront f: its instruction p is number f NDMA + p of a part of 64 elements: 8 A rows (lane l lands on row
+    // l / 8, position l % 8) or, behind all of those, 16 B rows (row l / 4, position l % 4).
+    const int f = wave - C::WAVES;
+    const uint8_t* const a = static_cast<const uint8_t*>(g.a) + (int64_t)m0 * g.lda * 2;
+    const uint8_t* const b = g.b + (int64_t)n0 * g.ldb;
+    uint32_t off[C::NDMA];
+    int first[C::NDMA];  // first element of the lane's piece
+#pragma unroll
+    for (int p = 0; p < C::NDMA; ++p) {
+      const int q = f * C::NDMA + p;
+      if (q < C::DMA_A) {
+        const int row = 8 * q + (lane >> 3), c = (lane & 7) ^ ((row >> 1) & 7);
+        const int piece = (c & 4) | ((c & 1) << 1) | ((c >> 1) & 1);
+        off[p] = (uint32_t)min(row, g.M - 1 - m0) * (uint32_t)(g.lda * 2) + piece * 16;
+        first[p] = piece * 8;
+      } else {
+        const int row = 16 * (q - C::DMA_A) + (lane >> 2), c = (lane & 3) ^ C::swz_b(row);
+        off[p] = (uint32_t)min(row, g.N - 1 - n0) * (uint32_t)g.ldb + c * 16;
+        first[p] = c * 16;
+      }
+    }
+    // Elements beyond K (a partial last step, steps beyond the last) are fetched from beyond the descriptor: zeros.
+    auto dma = [&](int kt, int stage) {
+#pragma unroll
+      for (int u = 0; u < SUB; ++u) {
+        const int k = kt * SUB + u, left = g.K - k * BKE;
+#pragma unroll
+        for (int p = 0; p < C::NDMA; ++p) {
+          const int q = f * C::NDMA + p;
+          const bool is_a = q < C::DMA_A;
+          const __amdgpu_buffer_rsrc_t src =
+              __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(is_a ? a : b), 0, 0x7fffffff, 0x00020000);
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(
+              src, (__attribute__((address_space(3))) void*)(smem + stage + u * C::PART + q * 1024), 16,
+              (int)(off[p] | (first[p] < left ? 0u : 0x80000000u)), k * (is_a ? 2 * BKE : BKE), 0, 0);
+        }
+      }
+    };
+#pragma unroll
+    for (int s = 0; s < D; ++s) dma(s, s * C::STAGE);
+    wait_and_barrier<(D - 1) * C::NDMA * SUB>();  // step 0 has landed
+    int stage = 0;                                // of step kt
+    for (int kt = 0; kt < KT; ++kt) {
+      // step kt + 1 has landed; behind the barrier the operands of step kt are in registers
+      wait_and_barrier<(D - 2) * C::NDMA * SUB>();
+      dma(kt + D, stage);
+      stage = stage + C::STAGE == D * C::STAGE ? 0 : stage + C::STAGE;
+    }
+    wait_vm<0>();  // no DMA outlives the workgroup
+    return;
+  }
+
+  const int r16 = lane & 15, kg = lane >> 4, h = kg & 1, e = kg >> 1;
+  const int nw = n0 + wave * C::WN;
+  // scale and bias; what lies beyond N reads as zero, a null bias is an empty buffer
+  auto vec = [](const void* p, int bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00020000);
+  };
+  const __amdgpu_buffer_rsrc_t bs_buf = vec(g.b_scale, g.N * 4), bi_buf = vec(g.bias, g.bias ? g.N * 2 : 0);
+  v4f bs[TN];
+  uint2 bi[TN];
+  float as[TM];
+#pragma unroll
+  for (int j = 0; j < TN; ++j) {
+    const int n = nw + C::col(j, kg);
+    bs[j] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(bs_buf, n * 4, 0, 0));
+    bi[j] = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(bi_buf, n * 2, 0, 0));
+  }
+#pragma unroll
+  for (int i = 0; i < TM; ++i) as[i] = 1.0f;
+
+  struct Step {
+    v8bf a[2 * SUB][TM];
+    uint2 w[2 * SUB][TN];
+  };
+  const int a_swz = (r16 >> 1) & 7, brow = wave * C::WN + 8 * (r16 >> 2) + (r16 & 3);
+  // operands of the 32 elements x of a step (__restrict__: see the wide kernel)
+  auto read = [&](const uint8_t* __restrict__ stage_at, Step& f, int x) {
+    const uint8_t* st = stage_at + (x >> 1) * C::PART;
+    const int t = x & 1;
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      const int row = C::ODD && j == TN - 1 ? wave * C::WN + 16 * j + r16 : brow + 32 * (j >> 1) + 4 * (j & 1);
+      f.w[x][j] = *reinterpret_cast<const uint2*>(st + C::A_BYTES + row * BKE + (((2 * t + h) ^ C::swz_b(row)) << 4) + 8 * e);
+    }
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+      f.a[x][i] = *reinterpret_cast<const v8bf*>(st + (16 * i + r16) * (2 * BKE) + (((4 * t + kg) ^ a_swz) << 4));
+  };
+  v4f acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) acc[i][j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+  wait_and_barrier<63>();
+  Step even, odd;
+#pragma unroll
+  for (int x = 0; x < 2 * SUB; ++x) read(smem, even, x);
+  int stage = C::STAGE;  // of step kt + 1
+  // Step kt: its operands are in `f`; reads step kt + 1 into `nf`, 32 elements in front of each 32 of the MFMAs, or, where
+  // a step has few of those, all in front of the first.
+  constexpr bool kReadsFirst = SUB * TM * TN <= 4;
+  auto step = [&](const Step& f, Step& nf) {
+    wait_and_barrier<63>();
+#pragma unroll
+    for (int x = 0; x < 2 * SUB; ++x) {
+      if (x == 0 || !kReadsFirst) {
+#pragma unroll
+        for (int y = x; y < (kReadsFirst ? 2 * SUB : x + 1); ++y) read(smem + stage, nf, y);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        const v8bf b = e4m3x8_to_bf16(f.w[x][j].x, f.w[x][j].y);
+        // operands swapped: result rows follow B (n), result columns follow A (m)
+#pragma unroll
+        for (int i = 0; i < TM; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b, f.a[x][i], acc[i][j], 0, 0, 0);
+      }
+      if (!kReadsFirst) __builtin_amdgcn_sched_barrier(0);
+    }
+    stage = stage + C::STAGE == D * C::STAGE ? 0 : stage + C::STAGE;
+  };
+  for (int kt = 0; kt < KT; kt += 2) {
+    step(even, odd);
+    if (kt + 1 < KT) step(odd, even);
+  }
+
+  uint8_t* const out_wave = reinterpret_cast<uint8_t*>(g.out) + ((int64_t)m0 * g.ldo + nw) * 2;
+  if (g.epilogue & CDIT_EPI_GELU_TANH) {
+    store_fed_tile<C, CDIT_DT_BF16, true>(acc, as, bs, bi, out_wave, g.ldo, g.M - m0, g.N - nw, lane);
+  } else {
+    store_fed_tile<C, CDIT_DT_BF16, false>(acc, as, bs, bi, out_wave, g.ldo, g.M - m0, g.N - nw, lane);
+  }
+}
+
+template <class C>
+int launch_fed(const GemmArgs& g, hipStream_t stream) {
+  static bool lds_allowed[64];
+  if (int rc = allow_dynamic_lds(reinterpret_cast<const void*>(&gemm_w8a16_fed<C>), C::LDS_BYTES, lds_allowed)) return rc;
+  const int tiles_m = (g.M + C::BM - 1) / C::BM, tiles_n = (g.N + C::BN - 1) / C::BN;
+  hipLaunchKernelGGL(gemm_w8a16_fed<C>, dim3(tiles_m * tiles_n), dim3(C::THREADS), C::LDS_BYTES, stream, g, tiles_m, tiles_n);
+  return 0;
+}
+
+// ---------------------------------------------------------------------------
 // Skinny kernel for M <= 16 where the whole-row kernel below is not taken: weight streaming. A
 // workgroup of 4 waves owns 16 output channels, each wave a quarter of K. Per
 // 128-element chunk a lane (weight row l&15, K group l>>4) loads 32 e4m3 bytes
@@ -1382,6 +1574,16 @@ typedef CfgWW<192, 256, 4> W9;              // wide: 96x128 wave tiles
 typedef CfgWW<128, 192, 4, 4> W10;          // wide: 64x96 wave tiles, DMA 4 steps ahead
 typedef CfgWW<128, 128, 4, 5> W11;          // wide: 64x64 wave tiles, DMA 5 steps ahead
 typedef CfgWW<128, 64, 4, 6> W12;           // wide: 64x32 wave tiles, DMA 6 steps ahead
+//              BM  BN  waves sub depth
+typedef CfgFedW<16, 64, 4, 2, 5> W21;
+typedef CfgFedW<32, 32, 2, 2, 5> W22;
+typedef CfgFedW<48, 32, 2, 2, 4> W23;
+typedef CfgFedW<32, 64, 4, 2, 4> W24;
+typedef CfgFedW<48, 64, 4, 2, 4> W25;
+typedef CfgFedW<80, 64, 4, 1, 5> W26;
+typedef CfgFedW<64, 96, 6, 1, 5> W27;
+typedef CfgFedW<96, 96, 6, 1, 4> W28;
+typedef CfgFedW<96, 128, 8, 1, 4> W29;
 
 namespace {
 struct TileChoice {
@@ -1500,7 +1702,58 @@ int choose_tile(const GemmArgs& g) {
 }
 }  // namespace
 
-// The kernel for a problem: 100 for any shape and alignment, 51 whole rows (up to four), 50 up to 16 rows, 13 a workgroup
+// Tiles for problems that one round of them covers, with their measured round times: the kernel above (21 to 29) and the
+// wide kernel's. Fitted, with a start of 3 us, to the times of 300 problems with every tile (M 17 to 3000, K 1024 to 15360, N 1024
+// to 12288, at most 128 tiles of 256 x 256, weights from HBM; 7 % rms): of those that one round covers it takes one that is
+// 0.7 % off the best (geometric mean), 0.88 of the time that the choice among the older tiles gives, with 9 of 300 more than
+// 4 % slower (14 % the worst, 2004 x 1408 x 1088, M x N x K). With K remainders from K = 320 on 0.86 (113 problems).
+constexpr LaunchModel kOneLaunch = {2960, 852, 852};
+constexpr TileTime kOneRound[] = {{8, 256, 192, W8::DEPTH, 3218, 912}, {10, 128, 192, W10::DEPTH, 3134, 560}, {11, 128, 128, W11::DEPTH, 2395, 424},
+                                  {12, 128, 64, W12::DEPTH, 1467, 299},  {29, 96, 128, 0, 2087, 389},  {28, 96, 96, 0, 1366, 332},
+                                  {27, 64, 96, 0, 953, 287},    {26, 80, 64, 0, 686, 252},    {25, 48, 64, 0, 1025, 178},
+                                  {24, 32, 64, 0, 593, 163},    {23, 48, 32, 0, 362, 142},    {21, 16, 64, 0, 227, 125},
+                                  {22, 32, 32, 0, 0, 105}};
+
+// The tile of a problem that one round covers, -1 if there is none. Shorter K than 5 steps stays with the other rules (127 x
+// 5584 x 192, M x N x K, 3.8 us and 5.2 with this one), than 10 where those take two or three 32 x 32 tiles per CU (53 x 6016 x
+// 320 4.0 and 4.6; from there to K = 1024 0.96 of the time of those, from K = 1600 on 0.81). Up to 16 rows only in place of the 32 x 32 tiles, whose sums it
+// gives bit for bit (tiles_better_for_few): 0.82 of their time where 32 x 32 tiles are one round, 0.96 with 16 x 64 (122
+// problems, none slower; 16 x 96 and 16 x 128: 1.13 and 1.49).
+int choose_one_round_w8a16(const GemmArgs& g) {
+  if (!aligned_ok(g) || g.N % 16 || g.K < 5 * BKE) return -1;
+  const int64_t cus = cu_count() > 0 ? cu_count() : 256;
+  if (g.M <= 16) {
+    if (choose_gemm_w8a16(g) != 13) return -1;
+    return (g.N + 31) / 32 <= cus ? 22 : (g.N + 63) / 64 <= cus ? 21 : -1;
+  }
+  if (g.K < 10 * BKE && tiles32(g.M, g.N).tiles > cus && wavetile_better(g)) return -1;
+  int best = -1;
+  int64_t time = INT64_MAX;
+  for (const auto& c : kOneRound) {
+    const int64_t tiles = (int64_t)((g.M + c.bm - 1) / c.bm) * ((g.N + c.bn - 1) / c.bn);
+    if (tiles > cus || (c.variant < 21 && !WideOk{!tiled_ok(g), g.K, g.N}(c.depth))) continue;
+    const int64_t t = launch_ns(kOneLaunch, c, tiles, cus, g.K / BKE);
+    if (t < time) best = c.variant, time = t;
+  }
+  return best;
+}
+
+int launch_gemm_w8a16_fed(const GemmArgs& g, int variant, hipStream_t stream) {
+  switch (variant) {
+    case 21: return launch_fed<W21>(g, stream);
+    case 22: return launch_fed<W22>(g, stream);
+    case 23: return launch_fed<W23>(g, stream);
+    case 24: return launch_fed<W24>(g, stream);
+    case 25: return launch_fed<W25>(g, stream);
+    case 26: return launch_fed<W26>(g, stream);
+    case 27: return launch_fed<W27>(g, stream);
+    case 28: return launch_fed<W28>(g, stream);
+    default: return launch_fed<W29>(g, stream);
+  }
+}
+
+// The kernel for a problem that one round does not cover (choose_one_round_w8a16()): 100 for any shape and alignment, 51
+// whole rows (up to four), 50 up to 16 rows, 13 a workgroup
 // per 32 x 32 tile, else a tile of the wide kernel (K remainders: of its instances for them) or of the tiled one.
 int choose_gemm_w8a16(const GemmArgs& g) {
   if (!aligned_ok(g)) return 100;
@@ -1514,6 +1767,7 @@ int choose_gemm_w8a16(const GemmArgs& g) {
 
 int launch_gemm_w8a16(const GemmArgs& g, int variant, hipStream_t stream) {
   const bool k_tail = !tiled_ok(g);  // K not a whole number of steps
+  if (variant < 0) variant = choose_one_round_w8a16(g);
   if (variant < 0) variant = choose_gemm_w8a16(g);
   auto launch_generic = [&]() {
     dim3 grid((g.N + 15) / 16, (g.M + 15) / 16);
@@ -1544,6 +1798,7 @@ int launch_gemm_w8a16(const GemmArgs& g, int variant, hipStream_t stream) {
     return 0;
   }
   if (k_tail && g.N % 16 != 0) return launch_generic();
+  if (variant >= 21 && variant <= 29 && g.N % 16 == 0) return launch_gemm_w8a16_fed(g, variant, stream);
   if (variant == 13 && g.N % 16 == 0) return launch_wavetile(g, stream);
   const WideOk wide_ok{k_tail, g.K, g.N};
   if (k_tail && (variant < 7 || variant > 12)) variant = choose_tile(g);

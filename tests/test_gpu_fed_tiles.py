@@ -1,12 +1,14 @@
-"""The FP8 GEMM's tiles for problems that one round covers (a workgroup per tile, fed by wavefronts of its own):
-every tile at partial rows and columns, K shorter than its ring, odd and even numbers of steps, every output type,
-bit for bit against the wide kernel; and which problems take them."""
+"""The GEMMs' tiles for problems that one round covers (a workgroup per tile, fed by wavefronts of its own): every tile
+at partial rows and columns, K shorter than its ring, odd and even numbers of steps, every output type, bit for bit
+against the wide kernel; and which problems take them."""
 import pytest
 import torch
 
 FP8 = torch.float8_e4m3fn
 DEV = "cuda"
 TILES = {31: (32, 48), 32: (48, 48), 33: (80, 48), 34: (64, 64), 35: (96, 64), 36: (96, 96), 37: (128, 96)}
+WEIGHT_ONLY = {21: (16, 64), 22: (32, 32), 23: (48, 32), 24: (32, 64), 25: (48, 64), 26: (80, 64), 27: (64, 96), 28: (96, 96),
+               29: (96, 128)}
 
 
 @pytest.fixture(autouse=True)
@@ -81,3 +83,60 @@ def test_tile_of_one_round(M, N, K, want):
   if want != 16:  # built for bf16 outputs only
     assert lib.cdit_debug_gemm_choice(2, M, N, K, 0) == want
   assert lib.cdit_debug_gemm_choice(2, M, N, 1024, 2) == 0  # short K, fp32 outputs: bound by the stores
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("variant", sorted(WEIGHT_ONLY))
+def test_weight_only_bits_of_the_wide_kernel(variant):
+  """As above; K of whole steps of the ring (128 or 64 elements) and of half ones, with remainders, and shorter than a step. The
+  wide kernel takes a K remainder with its masked instances."""
+  from cache_dit_amd import _native, ops
+  bm, bn = WEIGHT_ONLY[variant]
+  for M, N, K in ((17, 16, 640), (bm, bn, 384), (bm + 1, bn + 16, 448), (3 * bm - 15, 9 * bn - 48, 656), (5, 2 * bn, 48),
+                  (2 * bm + 16, 17 * bn + 16, 1104)):
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    x = torch.full((M, K + 8), float("nan"), device=DEV, dtype=torch.bfloat16)
+    w = torch.full((N, K + 32), float("nan"), device=DEV).to(FP8)
+    x[:, :K] = torch.randn(M, K, generator=g, device=DEV).bfloat16()
+    w[:, :K] = torch.randn(N, K, generator=g, device=DEV).to(FP8)
+    sw = torch.rand(N, generator=g, device=DEV)
+    for b in (None, torch.randn(N, generator=g, device=DEV).bfloat16()):
+      for epilogue in (0, 1):
+        outs = []
+        for v in (variant, 11):
+          _native.set_gemm_variant(v)
+          outs.append(torch.full((M + 2, N + 8), 777.0, dtype=torch.bfloat16, device=DEV))
+          ops.w8a16_into(x[:, :K], w[:, :K], sw, b, outs[-1][1:M + 1, :N], epilogue)
+        torch.cuda.synchronize()
+        assert torch.equal(outs[0], outs[1]), (M, N, K, b is None, epilogue)
+        outs[0][1:M + 1, :N] = 777.0
+        assert bool((outs[0] == 777.0).all()), (M, N, K, b is None, epilogue)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(77, 3072, 4096), (200, 2560, 8192), (512, 3072, 3088), (16, 9216, 3072), (16, 6144, 1040)])
+def test_weight_only_choice(M, N, K):
+  """By shape, against the kernel that had such problems before: the same bits."""
+  from cache_dit_amd import _native, ops
+  lib = _native.load()
+  assert lib.cdit_debug_gemm_choice(3, M, N, K, 1) in WEIGHT_ONLY
+  g = torch.Generator(device=DEV).manual_seed(M)
+  x = torch.randn(M, K, generator=g, device=DEV).bfloat16()
+  w, sw = torch.randn(N, K, generator=g, device=DEV).to(FP8), torch.rand(N, generator=g, device=DEV)
+  outs = []
+  for v in (-1, lib.cdit_debug_gemm_choice(1, M, N, K, 1)):
+    _native.set_gemm_variant(v)
+    outs.append(torch.empty(M, N, dtype=torch.bfloat16, device=DEV))
+    ops.w8a16_into(x, w, sw, None, outs[-1], 0)
+  torch.cuda.synchronize()
+  assert torch.equal(outs[0], outs[1])
+
+
+@pytest.mark.parametrize("M,N,K,want", [
+    (77, 3072, 4096, 21), (200, 2560, 8192, 25), (17, 3072, 3072, 22), (342, 2752, 12352, 26), (6889, 3072, 12288, 0),
+    # up to 16 rows where they were on 32 x 32 tiles; K of fewer than five steps has other rules
+    (16, 8192, 3072, 22), (16, 9216, 3072, 21), (16, 18432, 5120, 0), (16, 3072, 3072, 0), (1, 9216, 3072, 0), (77, 3072, 256, 0),
+    (77, 3080, 4096, 0)])
+def test_weight_only_tile_of_one_round(M, N, K, want):
+  from cache_dit_amd import _native
+  assert _native.load().cdit_debug_gemm_choice(3, M, N, K, 1) == want
