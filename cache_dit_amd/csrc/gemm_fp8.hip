@@ -1452,28 +1452,30 @@ int launch_tile32(const GemmArgs& g, hipStream_t stream) {
 // like the rest, and touching them ahead from another wavefront takes as much of the path as it saves. So the time of a round
 // is (BM + BN) K bytes of the fullest CU, and the tile to take is the one with the shortest sides of which every CU gets
 // at most one: 96 x 96, 48 x 48, 32 x 48, 80 x 48 ... next to the wide kernel's and the 32 x 32 one. us, another weight
-// matrix per launch, the best of those -> this kernel, M x N x K: 77 x 3072 x 4096 10.6 -> 8.0 (32 x 48; on 288 tiles of 32 x 32 some
+// matrix per launch, the best of those -> this kernel, M x N x K: 77 x 3072 x 4096 10.6 -> 8.0 (48 x 32; on 288 tiles of 32 x 32 some
 // CUs get two), 200 x 2560 x 8192 20.7 -> 15.3, 512 x 3072 x 3072 14.8 -> 12.7 (96 x 96, 192 tiles; 64 x 128 as many), 512 x 3072 x
 // 12288 47.0 -> 37.4, 263 x 1216 x 8832 18.8 -> 13.1. With a second round of tiles it loses to the wide kernel, whose
 // stream of panels runs on from one tile to the next: chosen only for one (choose_one_round()).
 // The ring, its barrier and the order of K are those of gemm_fp8_tile32, MFMA and epilogue arithmetic the wide kernel's:
 // the same bits. Stages: as many as keep 64 KB in flight; one more or less is within 2 % (32 x 48: 5 stages 4 % slower
 // than 6), and where two workgroups then fit a CU's LDS a partial second round costs less (64 x 64 with 5 stages in place
-// of 6, 96 x 64 with 4: 9 %). Feeding wavefronts: with the multiplying ones issuing the DMA themselves the same time where the
+// of 6, 96 x 64 with 4: 9 %). A step is SUB times 128 bytes of K between two barriers: with 256 the shortest steps, those of
+// 32 x 32, take 10 % less (62 x 2560 x 4480, M x N x K: 8.9 us with gemm_fp8_tile32, 8.2), those of 32 x 48 and 48 x 48 1 to
+// 2 % more, of 80 x 48 and 64 x 64, with room for three stages then, 4 to 6 %. Feeding wavefronts: with the multiplying ones issuing the DMA themselves the same time where the
 // panels come from HBM, 22 % longer K steps where they are in the L2 (0.25 us against 0.32 with 128 x 128).
-template <int BM_, int BN_, int WGM_, int WGN_, int DEPTH_>
+template <int BM_, int BN_, int WGM_, int WGN_, int SUB_, int DEPTH_>
 struct CfgFed {
-  static constexpr int BM = BM_, BN = BN_, WGM = WGM_, WGN = WGN_, DEPTH = DEPTH_;
+  static constexpr int BM = BM_, BN = BN_, WGM = WGM_, WGN = WGN_, SUB = SUB_, DEPTH = DEPTH_;
   static constexpr int GROUP_M = 8;  // (4: the same time)
   static constexpr int WAVES = WGM * WGN, FEEDERS = 2, THREADS = 64 * (WAVES + FEEDERS);
   static constexpr int WM = BM / WGM, WN = BN / WGN, TM = WM / 16, TN = WN / 16;  // wave tile, in fragments of 16 rows
-  static constexpr int A_BYTES = BM * 128, STAGE = (BM + BN) * 128, LDS_BYTES = DEPTH * STAGE;
-  static constexpr int NDMA = (BM + BN) / 8 / FEEDERS;  // DMA instructions (8 panel rows) per feeding wavefront and step
+  static constexpr int A_BYTES = BM * 128, PART = (BM + BN) * 128, STAGE = SUB * PART, LDS_BYTES = DEPTH * STAGE;
+  static constexpr int NDMA = (BM + BN) / 8 / FEEDERS;  // DMA instructions (8 panel rows) per feeding wavefront and part
   // Columns of a wave tile: LP blocks of 64 and NH of 32 in pairs of fragments as in the wide kernel, with an odd TN
   // one fragment of 16 in its natural order behind them (store_fed_tile).
   static constexpr int LP = TN / 4, NH = TN % 4 / 2, ODD = TN % 2;
   static_assert(BM % (16 * WGM) == 0 && BN % (16 * WGN) == 0 && (BM + BN) / 8 % FEEDERS == 0, "whole fragments, whole instructions");
-  static_assert(DEPTH >= 3 && (DEPTH - 1) * NDMA <= 63 && LDS_BYTES <= 160 * 1024, "vmcnt has 6 bits; LDS");
+  static_assert(DEPTH >= 3 && (DEPTH - 1) * NDMA * SUB <= 63 && LDS_BYTES <= 160 * 1024, "vmcnt has 6 bits; LDS");
   // first of the four columns (of the wave tile) that lane group q holds of fragment j
   __device__ static constexpr int col(int j, int q) {
     return ODD && j == TN - 1 ? 16 * j + 4 * q : 32 * (j >> 1) + 8 * q + 4 * (j & 1);
@@ -1486,9 +1488,9 @@ template <class C, int OUT>
 __global__ __launch_bounds__(C::THREADS) __attribute__((amdgpu_waves_per_eu(2))) void
 gemm_fp8_fed(GemmArgs g, int tiles_m, int tiles_n) {
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
-  constexpr int D = C::DEPTH, BKW = 128, TM = C::TM, TN = C::TN;
+  constexpr int D = C::DEPTH, BKW = 128, TM = C::TM, TN = C::TN, SUB = C::SUB, ND = C::NDMA * SUB;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int KT = g.K / BKW;
+  const int parts = g.K / BKW, KT = (parts + SUB - 1) / SUB;
   // workgroups go to the 8 XCDs in turn; each XCD gets consecutive tiles (any number of them), which share panels
   const int ntiles = tiles_m * tiles_n, xcd = blockIdx.x % 8;
   int tm, tn;
@@ -1510,23 +1512,27 @@ gemm_fp8_fed(GemmArgs g, int tiles_m, int tiles_n) {
                    : (uint32_t)min(brow, g.N - n0 - 1) * (uint32_t)g.ldb + ((lane & 7) ^ C::swz_b_row(brow)) * 16;
     }
     auto dma = [&](int kt, int stage) {
-      const int nrec = kt < KT ? 0x7fffffff : 0;  // steps beyond the last fetch nothing
 #pragma unroll
-      for (int p = 0; p < C::NDMA; ++p) {
-        const int q = f * C::NDMA + p;
-        const __amdgpu_buffer_rsrc_t src = __builtin_amdgcn_make_buffer_rsrc(
-            const_cast<uint8_t*>(q < C::BM / 8 ? a : b), 0, nrec, 0x00020000);
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(
-            src, (__attribute__((address_space(3))) void*)(smem + stage + q * 1024), 16, (int)off[p], kt * BKW, 0, 0);
+      for (int u = 0; u < SUB; ++u) {
+        const int x = kt * SUB + u, nrec = x < parts ? 0x7fffffff : 0;  // parts beyond the last: zeros, nothing fetched
+#pragma unroll
+        for (int p = 0; p < C::NDMA; ++p) {
+          const int q = f * C::NDMA + p;
+          const __amdgpu_buffer_rsrc_t src = __builtin_amdgcn_make_buffer_rsrc(
+              const_cast<uint8_t*>(q < C::BM / 8 ? a : b), 0, nrec, 0x00020000);
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(
+              src, (__attribute__((address_space(3))) void*)(smem + stage + u * C::PART + q * 1024), 16, (int)off[p],
+              x * BKW, 0, 0);
+        }
       }
     };
 #pragma unroll
     for (int s = 0; s < D; ++s) dma(s, s * C::STAGE);
-    wait_and_barrier<(D - 1) * C::NDMA>();  // step 0 has landed
+    wait_and_barrier<(D - 1) * ND>();  // step 0 has landed
     int stage = 0;                          // of step kt
     for (int kt = 0; kt < KT; ++kt) {
       // step kt + 1 has landed; behind the barrier the operands of step kt are in registers
-      wait_and_barrier<(D - 2) * C::NDMA>();
+      wait_and_barrier<(D - 2) * ND>();
       dma(kt + D, stage);
       stage = stage + C::STAGE == D * C::STAGE ? 0 : stage + C::STAGE;
     }
@@ -1556,7 +1562,7 @@ gemm_fp8_fed(GemmArgs g, int tiles_m, int tiles_n) {
     as[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(as_buf, (mw + 16 * i + r16) * 4, 0, 0));
 
   struct Step {
-    v8i a[TM], b[TN];
+    v8i a[SUB][TM], b[SUB][TN];
   };
   // (__restrict__: see the wide kernel; without it every read would wait for the whole stream)
   auto fragment = [&](const uint8_t* __restrict__ st, int row, int swz) -> v8i {
@@ -1564,15 +1570,16 @@ gemm_fp8_fed(GemmArgs g, int tiles_m, int tiles_n) {
     const v4i hi = *reinterpret_cast<const v4i*>(st + row * BKW + (((2 * kg + 1) ^ swz) << 4));
     return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
   };
-  // fragment q of a step, in the order of their first use: A_0, B_0 .. B_{TN-1}, A_1 ..
+  // fragment q of part u of a step, in the order of their first use: A_0, B_0 .. B_{TN-1}, A_1 ..
   const int arow = wm * C::WM + r16, brow = wn * C::WN + 8 * (r16 >> 2) + (r16 & 3);
-  auto read = [&](const uint8_t* st, Step& f, int q) {
+  auto read = [&](const uint8_t* stage_at, Step& f, int u, int q) {
+    const uint8_t* st = stage_at + u * C::PART;
     if (q == 0 || q > TN) {
       const int i = q ? q - TN : 0;
-      f.a[i] = fragment(st, arow + 16 * i, swz_a(arow));
+      f.a[u][i] = fragment(st, arow + 16 * i, swz_a(arow));
     } else {
       const int j = q - 1, row = C::ODD && j == TN - 1 ? wn * C::WN + 16 * j + r16 : brow + 32 * (j >> 1) + 4 * (j & 1);
-      f.b[j] = fragment(st + C::A_BYTES, row, C::swz_b_row(row));
+      f.b[u][j] = fragment(st + C::A_BYTES, row, C::swz_b_row(row));
     }
   };
   v4f acc[TM][TN];
@@ -1583,21 +1590,22 @@ gemm_fp8_fed(GemmArgs g, int tiles_m, int tiles_n) {
   wait_and_barrier<63>();
   Step even, odd;
 #pragma unroll
-  for (int q = 0; q < TM + TN; ++q) read(smem, even, q);
+  for (int q = 0; q < SUB * (TM + TN); ++q) read(smem, even, q / (TM + TN), q % (TM + TN));
   int stage = C::STAGE;  // of step kt + 1
   // Step kt: its operands are in `f`; reads step kt + 1 into `nf`, spread over the first three quarters of the MFMAs.
   auto step = [&](const Step& f, Step& nf) {
     wait_and_barrier<63>();
     const uint8_t* st = smem + stage;
     __builtin_amdgcn_sched_barrier(0);
+    constexpr int kFragments = SUB * (TM + TN), kMfmas = SUB * TM * TN;
 #pragma unroll
-    for (int s = 0; s < TM * TN; ++s) {
+    for (int s = 0; s < kMfmas; ++s) {
 #pragma unroll
-      for (int q = 0; q < TM + TN; ++q)
-        if (q * TM * TN * 3 / 4 / (TM + TN) == s) read(st, nf, q);
+      for (int q = 0; q < kFragments; ++q)
+        if (q * kMfmas * 3 / 4 / kFragments == s) read(st, nf, q / (TM + TN), q % (TM + TN));
       // operands swapped: result rows follow B (n), result columns follow A (m)
-      acc[s / TN][s % TN] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(f.b[s % TN], f.a[s / TN], acc[s / TN][s % TN],
-                                                                             0, 0, 0, 0, 0, 0);
+      const int u = s / (TM * TN), i = s / TN % TM, j = s % TN;
+      acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(f.b[u][j], f.a[u][i], acc[i][j], 0, 0, 0, 0, 0, 0);
       __builtin_amdgcn_sched_barrier(0);
     }
     stage = stage + C::STAGE == D * C::STAGE ? 0 : stage + C::STAGE;
@@ -2108,14 +2116,16 @@ typedef CfgWide<128, 192, 4, 3> V16;                  // ... 64x96 wave tiles, D
 typedef CfgWide<64, 128, 8, 5> V17;                   // ... 32x64 wave tiles, DMA 5 steps ahead
 typedef CfgWide<128, 128, 4, 4> V18;                  // ... 64x64 wave tiles, DMA 4 steps ahead
 typedef CfgWide<256, 128, 4> V19;                     // ... 128x64 wave tiles, for K remainders only
-//             BM  BN  waves depth
-typedef CfgFed<32, 48, 1, 3, 6> V31;
-typedef CfgFed<48, 48, 1, 3, 6> V32;
-typedef CfgFed<80, 48, 5, 1, 5> V33;
-typedef CfgFed<64, 64, 2, 2, 5> V34;
-typedef CfgFed<96, 64, 2, 2, 4> V35;
-typedef CfgFed<96, 96, 2, 2, 5> V36;
-typedef CfgFed<128, 96, 2, 2, 5> V37;
+//             BM  BN  waves sub depth
+typedef CfgFed<32, 48, 1, 3, 1, 6> V31;
+typedef CfgFed<48, 48, 1, 3, 1, 6> V32;
+typedef CfgFed<80, 48, 5, 1, 1, 5> V33;
+typedef CfgFed<64, 64, 2, 2, 1, 5> V34;
+typedef CfgFed<96, 64, 2, 2, 1, 4> V35;
+typedef CfgFed<96, 96, 2, 2, 1, 5> V36;
+typedef CfgFed<128, 96, 2, 2, 1, 5> V37;
+typedef CfgFed<32, 32, 1, 2, 2, 4> V38;
+typedef CfgFed<48, 32, 3, 1, 2, 4> V39;
 // the two large tiles with contiguous wave columns and half-line output stores (16 rows x 64
 // bytes per store instruction), kept to measure the whole-line stores against: variants 112, 114
 typedef CfgWide<256, 256, 4, 2, false> V12H;
@@ -2335,19 +2345,20 @@ struct WideOk {
   bool operator()(int depth) const { return K >= 128 * (depth > 3 ? depth : 3); }
 };
 
-// Tiles for problems that one round of them covers, with their measured round times: the kernel above (31 to 37), the
-// 32 x 32 one (26) and the wide kernel's. Fitted to the times of 400 problems with every tile (M 17 to 4000, K 1024 to 15360,
+// Tiles for problems that one round of them covers, with their measured round times: the kernel above (31 to 39)
+// and the wide kernel's. Fitted to the times of 250 to 400 problems with every tile (M 17 to 4000, K 1024 to 15360,
 // N 1024 to 12288, at most 160 tiles of 256 x 256, weights from HBM; 8.5 % rms): of those that one round covers it takes one
-// that is 1.1 % off the best (geometric mean), 0.89 of the time that the choice among the older tiles gives (0.94 over all
-// problems of M 17 to 6889, K 256 to 15360, N 256 to 12288, bf16 and fp32 outputs), with 4 of 220 more than 4 % slower (8 %
-// the worst, 28 x 7712 x 14976, M x N x K).
+// that is 1.1 % off the best (geometric mean), 0.87 of the time that the choice among the older tiles gives (0.94 over all
+// problems of M 17 to 6889, K 256 to 15360, N 256 to 12288, bf16 and fp32 outputs), with 6 of 500 more than 4 % slower (11 %
+// the worst, 1028 x 1792 x 6272, M x N x K: 96 x 96 tiles against 128 x 128).
 constexpr LaunchModel kOneLaunch = {1425, 907, 907};
 constexpr TileTime kOneRound[] = {{15, 256, 192, V15::DEPTH, 5000, 987}, {16, 128, 192, V16::DEPTH, 3710, 676},
                                   {18, 128, 128, V18::DEPTH, 3100, 517}, {17, 64, 128, V17::DEPTH, 2620, 434},
                                   {37, 128, 96, 3, 3260, 428},           {36, 96, 96, 3, 2920, 389},
                                   {35, 96, 64, 3, 2510, 305},            {34, 64, 64, 3, 2340, 263},
                                   {33, 80, 48, 3, 2310, 244},            {32, 48, 48, 3, 1910, 198},
-                                  {31, 32, 48, 3, 1640, 183},            {26, 32, 32, 3, 1430, 184}};
+                                  {31, 32, 48, 3, 1640, 183},            {39, 48, 32, 3, 1992, 153},
+                                  {38, 32, 32, 3, 1509, 147}};
 
 // The tile of a problem that one round covers, -1 if there is none. fp32 outputs of short K are bound by their stores: the
 // other rules know them (1116 x 6016 x 512, M x N x K: 13.7 us, 15.4 by this one).
@@ -2358,8 +2369,7 @@ int choose_one_round(const GemmArgs& g) {
   int64_t time = INT64_MAX;
   for (const auto& c : kOneRound) {
     if (g.K < c.depth * BK || (c.variant == 16 && g.out_dtype != CDIT_DT_BF16)) continue;
-    const int64_t tiles = c.variant == 26 ? tiles32(g.M, g.N).padded
-                                          : (int64_t)((g.M + c.bm - 1) / c.bm) * ((g.N + c.bn - 1) / c.bn);
+    const int64_t tiles = (int64_t)((g.M + c.bm - 1) / c.bm) * ((g.N + c.bn - 1) / c.bn);
     if (tiles > cus) continue;
     const int64_t t = launch_ns(kOneLaunch, c, tiles, cus, g.K / BK);
     if (t < time) best = c.variant, time = t;
@@ -2375,6 +2385,8 @@ int launch_gemm_fp8_fed(const GemmArgs& g, int variant, hipStream_t stream) {
     case 34: return launch_fed<V34>(g, stream);
     case 35: return launch_fed<V35>(g, stream);
     case 36: return launch_fed<V36>(g, stream);
+    case 38: return launch_fed<V38>(g, stream);
+    case 39: return launch_fed<V39>(g, stream);
     default: return launch_fed<V37>(g, stream);
   }
 }
@@ -2428,7 +2440,7 @@ int launch_gemm_fp8(const GemmArgs& g, int variant, hipStream_t stream) {
   }
   if (variant == 26) return tile32_tail(g) ? launch_tile32<true>(g, stream) : launch_tile32<false>(g, stream);
   if (!tiled_ok(g)) return launch_gemm_fp8_ktail(g, variant, stream);
-  if (variant >= 31 && variant <= 37) return launch_gemm_fp8_fed(g, variant, stream);
+  if (variant >= 31 && variant <= 39) return launch_gemm_fp8_fed(g, variant, stream);
   const WideOk wide_ok{g.K};
   if (g.out_dtype != CDIT_DT_BF16) {
     const int v = choose_other_out_variant(g, variant, wide_ok);

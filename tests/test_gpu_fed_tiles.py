@@ -6,7 +6,8 @@ import torch
 
 FP8 = torch.float8_e4m3fn
 DEV = "cuda"
-TILES = {31: (32, 48), 32: (48, 48), 33: (80, 48), 34: (64, 64), 35: (96, 64), 36: (96, 96), 37: (128, 96)}
+TILES = {31: (32, 48), 32: (48, 48), 33: (80, 48), 34: (64, 64), 35: (96, 64), 36: (96, 96), 37: (128, 96),
+         38: (32, 32), 39: (48, 32)}
 WEIGHT_ONLY = {21: (16, 64), 22: (32, 32), 23: (48, 32), 24: (32, 64), 25: (48, 64), 26: (80, 64), 27: (64, 96), 28: (96, 96),
                29: (96, 128)}
 
@@ -72,8 +73,8 @@ def test_the_choice_and_its_neighbours(M, N, K):
 
 
 @pytest.mark.parametrize("M,N,K,want", [
-    (77, 3072, 4096, 31), (200, 2560, 8192, 33), (512, 3072, 3072, 36), (512, 3072, 12288, 36), (1021, 3072, 3072, 37),
-    (512, 12288, 3072, 16), (100, 1024, 3072, 26), (4608, 3072, 3072, 0), (2048, 12288, 3072, 0),
+    (77, 3072, 4096, 39), (200, 2560, 8192, 33), (512, 3072, 3072, 36), (512, 3072, 12288, 36), (1021, 3072, 3072, 37),
+    (512, 12288, 3072, 16), (100, 1024, 3072, 38), (4608, 3072, 3072, 0), (2048, 12288, 3072, 0),
     # up to 16 rows, K remainders and K of one or two steps have other rules
     (16, 3072, 3072, 0), (77, 3072, 4112, 0), (77, 3072, 256, 0)])
 def test_tile_of_one_round(M, N, K, want):
