@@ -8,8 +8,6 @@
 
 #include <mutex>
 
-#include <algorithm>
-
 #include "cdit_internal.h"
 
 namespace cdit {
@@ -174,8 +172,6 @@ static bool shape_only(GemmArgs* g, int64_t M, int64_t N, int64_t K, int out_dty
 int cdit_debug_gemm_choice(int weight_only, int64_t M, int64_t N, int64_t K, int out_dtype_id) {
   GemmArgs g;
   if (!shape_only(&g, M, N, K, out_dtype_id)) return -1;
-  if (weight_only == 2) return std::max(choose_one_round(g), 0);
-  if (weight_only == 3) return std::max(choose_one_round_w8a16(g), 0);
   return weight_only ? choose_gemm_w8a16(g) : choose_gemm_fp8(g);
 }
 

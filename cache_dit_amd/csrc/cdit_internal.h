@@ -97,9 +97,7 @@ struct GemmGroup {
 
 // The kernel variant for a problem, and the launches of a w8a8 Linear of a problem's shape (1: the GEMM's kernel
 // quantizes the rows itself).
-int choose_one_round(const GemmArgs& g);
 int choose_gemm_fp8(const GemmArgs& g);
-int choose_one_round_w8a16(const GemmArgs& g);
 int choose_gemm_w8a16(const GemmArgs& g);
 int linear_fp8_launches(const GemmArgs& g);
 // variant < 0: choose by shape.

@@ -2362,8 +2362,8 @@ constexpr TileTime kOneRound[] = {{15, 256, 192, V15::DEPTH, 5000, 987}, {16, 12
 
 // The tile of a problem that one round covers, -1 if there is none. fp32 outputs of short K are bound by their stores: the
 // other rules know them (1116 x 6016 x 512, M x N x K: 13.7 us, 15.4 by this one).
-int choose_one_round(const GemmArgs& g) {
-  if (!tiled_ok(g) || g.M <= 16 || g.K < (g.out_dtype == CDIT_DT_F32 ? 9 : 3) * BK) return -1;
+static int choose_one_round(const GemmArgs& g) {
+  if (!tiled_ok(g) || g.K < (g.out_dtype == CDIT_DT_F32 ? 9 : 3) * BK) return -1;
   const int64_t cus = cu_count() > 0 ? cu_count() : 256;
   int best = -1;
   int64_t time = INT64_MAX;
@@ -2391,12 +2391,14 @@ int launch_gemm_fp8_fed(const GemmArgs& g, int variant, hipStream_t stream) {
   }
 }
 
-// The kernel for a problem that one round does not cover (choose_one_round()): 100 for any shape and alignment, 51 one
-// row, 50 up to 16 rows, 26 a workgroup per 32 x 32 tile, else a tile of the wide kernel (K remainders: of its instances for them) or of the tiled one.
+// The kernel for a problem: 100 for any shape and alignment, 51 one row, 50 up to 16 rows, 31 to 39 a tile of which one round
+// covers it, 26 a workgroup per 32 x 32 tile, else a tile of the wide kernel (K remainders: of its instances for them) or
+// of the tiled one.
 int choose_gemm_fp8(const GemmArgs& g) {
   if (!aligned_ok(g)) return 100;
   if (row1_ok(g)) return 51;
   if (g.M <= 16) return few_on_tiles(g) ? 26 : 50;
+  if (const int one = choose_one_round(g); one >= 0) return one;
   if (tile32_better(g)) return 26;
   if (!tiled_ok(g)) return choose_ktail_variant(g, -1);
   // the wide kernels stream K two or more steps ahead: shorter K runs the 128x128 kernel
@@ -2418,7 +2420,6 @@ int linear_fp8_launches(const GemmArgs& g) {
 
 int launch_gemm_fp8(const GemmArgs& g, int variant, hipStream_t stream) {
   if (!aligned_ok(g)) variant = 100;
-  if (variant < 0) variant = choose_one_round(g);
   if (variant < 0) variant = choose_gemm_fp8(g);
   if (variant == 100) {
     dim3 grid((g.N + 15) / 16, (g.M + 15) / 16);

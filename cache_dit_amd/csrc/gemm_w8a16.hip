@@ -1716,16 +1716,10 @@ constexpr TileTime kOneRound[] = {{8, 256, 192, W8::DEPTH, 3218, 912}, {10, 128,
 
 // The tile of a problem that one round covers, -1 if there is none. Shorter K than 5 steps stays with the other rules (127 x
 // 5584 x 192, M x N x K, 3.8 us and 5.2 with this one), than 10 where those take two or three 32 x 32 tiles per CU (53 x 6016 x
-// 320 4.0 and 4.6; from there to K = 1024 0.96 of the time of those, from K = 1600 on 0.81). Up to 16 rows only in place of the 32 x 32 tiles, whose sums it
-// gives bit for bit (tiles_better_for_few): 0.82 of their time where 32 x 32 tiles are one round, 0.96 with 16 x 64 (122
-// problems, none slower; 16 x 96 and 16 x 128: 1.13 and 1.49).
-int choose_one_round_w8a16(const GemmArgs& g) {
-  if (!aligned_ok(g) || g.N % 16 || g.K < 5 * BKE) return -1;
+// 320 4.0 and 4.6; from there to K = 1024 0.96 of the time of those, from K = 1600 on 0.81).
+static int choose_one_round(const GemmArgs& g) {
+  if (g.N % 16 || g.K < 5 * BKE) return -1;
   const int64_t cus = cu_count() > 0 ? cu_count() : 256;
-  if (g.M <= 16) {
-    if (choose_gemm_w8a16(g) != 13) return -1;
-    return (g.N + 31) / 32 <= cus ? 22 : (g.N + 63) / 64 <= cus ? 21 : -1;
-  }
   if (g.K < 10 * BKE && tiles32(g.M, g.N).tiles > cus && wavetile_better(g)) return -1;
   int best = -1;
   int64_t time = INT64_MAX;
@@ -1736,6 +1730,15 @@ int choose_one_round_w8a16(const GemmArgs& g) {
     if (t < time) best = c.variant, time = t;
   }
   return best;
+}
+
+// Up to 16 rows on tiles (tiles_better_for_few()): the kernel above in place of the 32 x 32 tiles, whose sums it gives bit for
+// bit: 0.82 of their time where 32 x 32 tiles are one round, 0.96 with 16 x 64 (122 problems, none slower; 16 x 96 and
+// 16 x 128: 1.13 and 1.49).
+static int choose_few(const GemmArgs& g) {
+  const int64_t cus = cu_count() > 0 ? cu_count() : 256;
+  if (g.K < 5 * BKE) return 13;
+  return (g.N + 31) / 32 <= cus ? 22 : (g.N + 63) / 64 <= cus ? 21 : 13;
 }
 
 int launch_gemm_w8a16_fed(const GemmArgs& g, int variant, hipStream_t stream) {
@@ -1752,22 +1755,23 @@ int launch_gemm_w8a16_fed(const GemmArgs& g, int variant, hipStream_t stream) {
   }
 }
 
-// The kernel for a problem that one round does not cover (choose_one_round_w8a16()): 100 for any shape and alignment, 51
-// whole rows (up to four), 50 up to 16 rows, 13 a workgroup
-// per 32 x 32 tile, else a tile of the wide kernel (K remainders: of its instances for them) or of the tiled one.
+// The kernel for a problem: 100 for any shape and alignment, 51 whole rows (up to four), 50 up to 16 rows, 21 to 29 a tile of
+// which one round covers it, 13 a workgroup per 32 x 32 tile, else a tile of the wide kernel (K remainders: of its
+// instances for them) or of the tiled one.
 int choose_gemm_w8a16(const GemmArgs& g) {
   if (!aligned_ok(g)) return 100;
   const bool few_on_tiles = g.M <= 16 && g.N % 16 == 0 && tiles_better_for_few(g);
   if (g.M <= 4 && g.K <= 4096 && whole_rows_better(g) && (g.K % 128 || !few_on_tiles)) return 51;
   if (g.M <= 16 && !few_on_tiles) return 50;
+  if (few_on_tiles) return choose_few(g);
   // what is left of K remainders is for the wide kernel, which stores 16 columns per lane
   if (!tiled_ok(g) && g.N % 16 != 0) return 100;
-  return few_on_tiles || wavetile_better(g) ? 13 : choose_tile(g);
+  if (const int one = choose_one_round(g); one >= 0) return one;
+  return wavetile_better(g) ? 13 : choose_tile(g);
 }
 
 int launch_gemm_w8a16(const GemmArgs& g, int variant, hipStream_t stream) {
   const bool k_tail = !tiled_ok(g);  // K not a whole number of steps
-  if (variant < 0) variant = choose_one_round_w8a16(g);
   if (variant < 0) variant = choose_gemm_w8a16(g);
   auto launch_generic = [&]() {
     dim3 grid((g.N + 15) / 16, (g.M + 15) / 16);

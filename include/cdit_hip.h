@@ -382,9 +382,8 @@ int cdit_debug_set_quant_hints(int hints);
 /*
  * What the automatic choice is for a shape with contiguous, aligned operands, on the current
  * device (without one: 256 compute units). Nothing is launched. -1: no such problem.
- * cdit_debug_gemm_choice: weight_only 0: the variant that cdit_fp8_gemm_rowwise runs where no tile
- * covers the problem in one round, 2: that tile's, which goes before it (0: there is none); 1 and 3:
- * the same for cdit_w8a16_gemm, whose only output type is bf16.
+ * cdit_debug_gemm_choice: the variant that cdit_fp8_gemm_rowwise runs (weight_only != 0:
+ * cdit_w8a16_gemm, whose only output type is bf16).
  * cdit_debug_linear_launches: kernels that cdit_fp8_linear_w8a8 launches, 1 or 2.
  */
 int cdit_debug_gemm_choice(int weight_only, int64_t M, int64_t N, int64_t K, int out_dtype_id);

@@ -46,19 +46,36 @@ def test_launches_of_few_rows(lib, M, N, K, want):
 
 
 @pytest.mark.parametrize("M,N,K,tiles", [
-    (77, 3072, 4096, True), (303, 640, 4736, True), (203, 3392, 4992, True), (300, 3072, 2224, True),
-    # three (K remainders: five and four) tiles per CU and beyond
-    (96, 8192, 3072, True), (97, 8192, 3072, False), (160, 8192, 400, True), (161, 8192, 400, False),
+    (300, 3072, 2224, True),
+    # five and four tiles per CU (K remainders, K of one or two steps) and beyond
+    (160, 8192, 400, True), (161, 8192, 400, False),
     (144, 8032, 1680, False), (128, 8192, 1680, True), (72, 11840, 8992, False), (898, 1088, 11536, False),
     (160, 8192, 256, True), (161, 8192, 256, False),
     # few columns, of which some XCDs get twice as many as others
-    (1579, 352, 12032, False), (1631, 480, 9600, False), (1806, 304, 3840, False), (639, 1168, 3200, True),
-    (1848, 400, 1024, True), (1107, 592, 384, True), (2280, 320, 1408, False), (2416, 288, 896, False),
-    (2048, 320, 1408, True), (2240, 288, 15136, False), (1366, 576, 3920, False), (1366, 576, 784, True), (1199, 704, 4160, True),
+    (2240, 288, 15136, False), (1366, 576, 3920, False), (1366, 576, 784, True), (1199, 704, 4160, True),
     (1199, 704, 6160, False)])
 def test_tiles_of_more_than_16_rows(lib, M, N, K, tiles):
   for dtype in (F16, BF16, F32):
     assert (lib.cdit_debug_gemm_choice(0, M, N, K, dtype) == TILE32) == tiles
+
+
+@pytest.mark.parametrize("M,N,K,want", [
+    # whole steps that one round of a tile covers
+    (77, 3072, 4096, 39), (303, 640, 4736, 38), (203, 3392, 4992, 33), (96, 8192, 3072, 34), (97, 8192, 3072, 34),
+    (1579, 352, 12032, 33), (1631, 480, 9600, 33), (1806, 304, 3840, 33), (639, 1168, 3200, 33), (1848, 400, 1024, 33),
+    (2280, 320, 1408, 33), (2048, 320, 1408, 33)])
+def test_tiles_of_one_round(lib, M, N, K, want):
+  for dtype in (F16, BF16, F32):
+    if dtype != F32 or K > 1024:
+      assert lib.cdit_debug_gemm_choice(0, M, N, K, dtype) == want
+
+
+@pytest.mark.parametrize("M,N,K,want", [
+    # fp32 outputs of short K
+    (1848, 400, 1024, TILE32), (1107, 592, 384, TILE32), (96, 8192, 1024, TILE32), (97, 8192, 1024, 17), (2416, 288, 896, 17),
+    (4608, 3072, 1024, 18)])
+def test_fp32_outputs_of_short_k(lib, M, N, K, want):
+  assert lib.cdit_debug_gemm_choice(0, M, N, K, F32) == want
 
 
 @pytest.mark.parametrize("M,N,K,want", [
@@ -70,13 +87,14 @@ def test_tiles_for_k_remainders(lib, M, N, K, want):
 
 
 @pytest.mark.parametrize("M,N,K,want", [
-    # few columns, of which some XCDs get twice as many as others
-    (2257, 272, 15680, 12), (2346, 288, 3392, 12), (2277, 272, 1408, 12), (1738, 272, 2944, 12), (1524, 288, 256, 13),
-    # two to three tiles per CU on many weights
-    (158, 4800, 14400, 12), (152, 4768, 6320, 12), (146, 3520, 11392, 12), (254, 2896, 7744, 13), (42, 11008, 9536, 13),
-    (245, 2560, 1664, 13), (299, 2368, 3328, 13), (77, 3072, 4096, 13), (154, 5056, 2560, 12),
+    # tiles of which one round covers the problem
+    (2257, 272, 15680, 25), (2346, 288, 3392, 25), (2277, 272, 1408, 25), (1738, 272, 2944, 25),
+    (158, 4800, 14400, 26), (152, 4768, 6320, 26), (146, 3520, 11392, 25), (254, 2896, 7744, 26), (42, 11008, 9536, 25),
+    (245, 2560, 1664, 25), (299, 2368, 3328, 26), (77, 3072, 4096, 21), (154, 5056, 2560, 26),
+    # shorter K
+    (1524, 288, 256, 13), (53, 6016, 320, 13), (127, 5584, 192, 13),
     # up to 16 rows
-    (5, 7952, 2944, 50), (5, 9216, 3072, 13), (6, 7952, 2944, 13), (16, 18432, 5120, 13), (16, 3072, 3072, 50),
+    (5, 7952, 2944, 50), (5, 9216, 3072, 21), (6, 7952, 2944, 22), (16, 18432, 5120, 13), (16, 3072, 3072, 50),
     (2, 18432, 3072, 51), (1, 9216, 3072, 51), (16, 18432, 3136, 13)])
 def test_weight_only(lib, M, N, K, want):
   assert lib.cdit_debug_gemm_choice(1, M, N, K, BF16) == want
