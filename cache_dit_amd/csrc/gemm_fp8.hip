@@ -2374,6 +2374,18 @@ static int choose_one_round(const GemmArgs& g) {
     const int64_t t = launch_ns(kOneLaunch, c, tiles, cus, g.K / BK);
     if (t < time) best = c.variant, time = t;
   }
+  if (best >= 0 && best < 31 && g.out_dtype != CDIT_DT_BF16) {
+    // fp32 and fp16 outputs on a round of 256 x 192 tiles in place of two rounds of smaller ones. Of 64 x 128: only for few
+    // rows on many columns, long K, and where the columns of tiles are no multiple of 8. Of 128 x 128: not where the second round
+    // is one tile for each XCD. us, two rounds / one, M x N x K: 5417 x 736 x 1408 12.3 / 17.7, 1590 x 2560 x 1664 16.6 / 21.1, 1064 x 3744 x 2048 22.6 / 24.1, 277 x 11264 x 6528 44.0 / 52.5 (88
+    // columns), 409 x 9120 x 4736 35.2 / 42.9 (72); 447 x 8880 x 8832 87.4 / 69.6, 1065 x 3744 x 6528 62.8 / 53.4; with 128 x 128 361 x
+    // 11184 x 10752 (264 tiles) 81.7 / 88.0, 374 x 11120 x 3840 (261) 41.8 / 34.8. Over 600 such problems 0.93 of the time of two rounds
+    // (without the rule 0.97, 181 more than 3 % slower, up to 1.44 times the time).
+    const int other = choose_other_out_variant(g, -1, WideOk{g.K});
+    const int64_t columns = (g.N + 127) / 128, tiles128 = (int64_t)((g.M + 127) / 128) * columns;
+    if (other == 17 && (g.M > 1088 || g.K < (g.out_dtype == CDIT_DT_F32 ? 17 : 13) * BK || columns % 8 == 0)) return -1;
+    if (other == 18 && tiles128 == cus + 8) return -1;
+  }
   return best;
 }
 

@@ -79,6 +79,17 @@ def test_fp32_outputs_of_short_k(lib, M, N, K, want):
 
 
 @pytest.mark.parametrize("M,N,K,want", [
+    # a round of 256 x 192 tiles not in place of two of 64 x 128 for many rows, short K or columns in eights
+    (5417, 736, 1408, 17), (1590, 2560, 1664, 17), (1069, 3648, 1152, 17), (277, 11264, 6528, 17), (409, 9120, 4736, 17),
+    (447, 8880, 8832, 15), (1065, 3744, 6528, 15), (282, 12144, 11008, 15),
+    # two of 128 x 128
+    (361, 11184, 10752, 18), (374, 11120, 3840, 15)])
+def test_fp16_and_fp32_outputs_of_two_rounds(lib, M, N, K, want):
+  for dtype in (F16, F32):
+    assert lib.cdit_debug_gemm_choice(0, M, N, K, dtype) == want
+
+
+@pytest.mark.parametrize("M,N,K,want", [
     # 256 x 128 tiles between one round of 128 x 128 and two of 256 x 192, not in their place
     (1357, 4464, 2224, 19), (3261, 7280, 1040, 15), (5499, 3440, 1296, 15), (1678, 12080, 4000, 15), (947, 5216, 3728, 16),
     (2269, 7248, 1344, 16), (4608, 3072, 3056, 14), (256, 12288, 2992, 18)])
