@@ -2345,12 +2345,25 @@ struct WideOk {
   bool operator()(int depth) const { return K >= 128 * (depth > 3 ? depth : 3); }
 };
 
+// The tile of the wide kernel (or of the tiled one) for a K of whole steps.
+int choose_whole(const GemmArgs& g) {
+  // the wide kernels stream K two or more steps ahead: shorter K runs the 128x128 kernel
+  const WideOk wide_ok{g.K};
+  if (g.out_dtype != CDIT_DT_BF16) {
+    // fp16 / fp32 outputs (the op's other two out_dtype ids); what no wide tile can take
+    // runs the generic kernel.
+    const int v = choose_other_out_variant(g, -1, wide_ok);
+    return v >= 0 ? v : 100;
+  }
+  return choose_bf16_variant(
+      [&](int bm, int bn) { return (int64_t)((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn); }, wide_ok, g.K).variant;
+}
+
 // Tiles for problems that one round of them covers, with their measured round times: the kernel above (31 to 39)
 // and the wide kernel's. Fitted to the times of 250 to 400 problems with every tile (M 17 to 4000, K 1024 to 15360,
 // N 1024 to 12288, at most 160 tiles of 256 x 256, weights from HBM; 8.5 % rms): of those that one round covers it takes one
 // that is 1.1 % off the best (geometric mean), 0.87 of the time that the choice among the older tiles gives (0.94 over all
-// problems of M 17 to 6889, K 256 to 15360, N 256 to 12288, bf16 and fp32 outputs), with 6 of 500 more than 4 % slower (11 %
-// the worst, 1028 x 1792 x 6272, M x N x K: 96 x 96 tiles against 128 x 128).
+// problems of M 17 to 6889, K 256 to 15360, N 256 to 12288, bf16 and fp32 outputs).
 constexpr LaunchModel kOneLaunch = {1425, 907, 907};
 constexpr TileTime kOneRound[] = {{15, 256, 192, V15::DEPTH, 5000, 987}, {16, 128, 192, V16::DEPTH, 3710, 676},
                                   {18, 128, 128, V18::DEPTH, 3100, 517}, {17, 64, 128, V17::DEPTH, 2620, 434},
@@ -2359,6 +2372,37 @@ constexpr TileTime kOneRound[] = {{15, 256, 192, V15::DEPTH, 5000, 987}, {16, 12
                                   {33, 80, 48, 3, 2310, 244},            {32, 48, 48, 3, 1910, 198},
                                   {31, 32, 48, 3, 1640, 183},            {39, 48, 32, 3, 1992, 153},
                                   {38, 32, 32, 3, 1509, 147}};
+
+// Whether the older choice is the better one where one round of `tile` is modelled as the shortest. us, older / `tile`, M x N x K:
+// - 32 x 32 (38) for K of three steps, of which the second part of a step is empty: 35 x 320 x 384 2.76 / 2.95; from four steps
+//   on the same time and less.
+// - 80 x 48 (33) in place of 32 x 32: for three and four steps (49 x 7072 x 384 4.0 / 4.5, 1440 x 480 x 512 4.0 / 4.2; 426 x 1616 x
+//   512, 2.8 tiles of 32 x 32 per CU, 4.5 / 4.2), and to K = 3072 where 32 x 32 are two tiles per CU at most: 52 x 6704 x 1408
+//   6.1 / 6.4, 102 x 4096 x 1280 5.4 / 5.7; 57 x 7280 x 3840 12.2 / 12.1.
+// - 128 x 96 (37) up to K = 1024 where rows of the output are whole 64-byte pieces, which 128 x 128 stores best: 1037 x 2304 x 512
+//   6.1 / 6.5, 2209 x 1120 x 768 6.9 / 7.2; 531 x 4368 x 512 7.4 / 6.8, 361 x 7936 x 1280 10.9 / 10.4.
+// - 96 x 96 (36) in place of one round of 64 x 128, as many bytes per CU. The wide kernel gives the XCDs consecutive tiles only
+//   where their number is a multiple of 8: up to 600 rows it is then the faster one if there are 5 % more of them (178 x 9216
+//   x 4480, 216 and 192 of 96 x 96, 19.9 / 20.7; 446 x 4416 x 7424, 245 and 230, 39.0 / 27.8). Of more rows, also with 11 % more
+//   tiles, unless much of the last 96 x 96 tiles' rows is empty and need not be fetched: 838 x 1984 x 14720 (224, 189) 42.7 / 49.3,
+//   1221 x 1408 x 13568 (220, 195) 40.6 / 45.1; 1265 x 1216 x 5888 (200, 182; 17 of 96 rows) 21.6 / 18.1; 5283 x 304 x 2560 10.1 / 11.1.
+// Over 4400 problems for which the choice among the tiles of one round differs from the older one 0.85 of the time of the
+// older one with and without this; 13 are more than 3 % slower than that (6 % the worst), without it 88 (16 %).
+bool older_better(const GemmArgs& g, int tile, int64_t cus) {
+  const int64_t tiles = tiles32(g.M, g.N).tiles;
+  if (tile == 38) return g.K < 4 * BK && tile32_better(g);
+  if (tile == 33) {
+    if (g.K <= 4 * BK ? tiles * 10 > 27 * cus : g.K > 24 * BK || tiles > 2 * cus) return false;
+    return tile32_better(g);
+  }
+  if (tile == 37) return g.K <= 8 * BK && g.N % 32 == 0;
+  if (tile != 36) return false;
+  const int64_t n64 = (int64_t)((g.M + 63) / 64) * ((g.N + 127) / 128), n96 = (int64_t)((g.M + 95) / 96) * ((g.N + 95) / 96);
+  if (n64 > cus) return false;
+  const bool whole_turns = n64 % 8 == 0, full = (g.M - 1) % 96 >= 56 || (g.M > 2400 && g.K < 34 * BK);
+  if (g.M < 600 ? !whole_turns || n96 * 100 >= n64 * 95 : !full || (!whole_turns && n96 * 10 > n64 * 9)) return false;
+  return choose_whole(g) == 17;
+}
 
 // The tile of a problem that one round covers, -1 if there is none. fp32 outputs of short K are bound by their stores: the
 // other rules know them (1116 x 6016 x 512, M x N x K: 13.7 us, 15.4 by this one).
@@ -2386,7 +2430,7 @@ static int choose_one_round(const GemmArgs& g) {
     if (other == 17 && (g.M > 1088 || g.K < (g.out_dtype == CDIT_DT_F32 ? 17 : 13) * BK || columns % 8 == 0)) return -1;
     if (other == 18 && tiles128 == cus + 8) return -1;
   }
-  return best;
+  return best >= 31 && older_better(g, best, cus) ? -1 : best;
 }
 
 int launch_gemm_fp8_fed(const GemmArgs& g, int variant, hipStream_t stream) {
@@ -2412,17 +2456,7 @@ int choose_gemm_fp8(const GemmArgs& g) {
   if (g.M <= 16) return few_on_tiles(g) ? 26 : 50;
   if (const int one = choose_one_round(g); one >= 0) return one;
   if (tile32_better(g)) return 26;
-  if (!tiled_ok(g)) return choose_ktail_variant(g, -1);
-  // the wide kernels stream K two or more steps ahead: shorter K runs the 128x128 kernel
-  const WideOk wide_ok{g.K};
-  if (g.out_dtype != CDIT_DT_BF16) {
-    // fp16 / fp32 outputs (the op's other two out_dtype ids); what no wide tile can take
-    // runs the generic kernel.
-    const int v = choose_other_out_variant(g, -1, wide_ok);
-    return v >= 0 ? v : 100;
-  }
-  return choose_bf16_variant(
-      [&](int bm, int bn) { return (int64_t)((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn); }, wide_ok, g.K).variant;
+  return tiled_ok(g) ? choose_whole(g) : choose_ktail_variant(g, -1);
 }
 
 int linear_fp8_launches(const GemmArgs& g) {

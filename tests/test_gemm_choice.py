@@ -79,6 +79,21 @@ def test_fp32_outputs_of_short_k(lib, M, N, K, want):
 
 
 @pytest.mark.parametrize("M,N,K,want", [
+    # three steps; 80 x 48 tiles for four steps, and where 32 x 32 are two per CU
+    (35, 320, 384, TILE32), (35, 320, 512, 38), (49, 7072, 384, TILE32), (1440, 480, 512, TILE32), (1440, 480, 640, 33),
+    (426, 1616, 512, 33), (52, 6704, 1408, TILE32), (102, 4096, 1280, TILE32), (52, 6704, 3200, 33), (67, 7552, 1152, 33), (49, 12032, 1152, 33),
+    # 128 x 96
+    (1037, 2304, 512, 18), (2209, 1120, 1024, 18), (531, 4368, 512, 37), (361, 7936, 1280, 37),
+    # 96 x 96 in place of one round of 64 x 128
+    (838, 1984, 14720, 17), (178, 9216, 4480, 17), (1221, 1408, 13568, 17), (5283, 304, 2560, 17), (446, 4416, 7424, 36),
+    (316, 5600, 14464, 36), (1163, 1648, 13568, 36), (1265, 1216, 5888, 36), (5283, 304, 5120, 36)])
+def test_where_the_older_tiles_stay(lib, M, N, K, want):
+  for dtype in (F16, BF16, F32):
+    if dtype != F32 or K > 1024:
+      assert lib.cdit_debug_gemm_choice(0, M, N, K, dtype) == want
+
+
+@pytest.mark.parametrize("M,N,K,want", [
     # a round of 256 x 192 tiles not in place of two of 64 x 128 for many rows, short K or columns in eights
     (5417, 736, 1408, 17), (1590, 2560, 1664, 17), (1069, 3648, 1152, 17), (277, 11264, 6528, 17), (409, 9120, 4736, 17),
     (447, 8880, 8832, 15), (1065, 3744, 6528, 15), (282, 12144, 11008, 15),
