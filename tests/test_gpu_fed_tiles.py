@@ -54,7 +54,7 @@ def test_bits_of_the_wide_kernel(variant, dtype):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N,K", [(77, 3072, 4096), (200, 2560, 8192), (512, 3072, 3072), (250, 12288, 1024)])
+@pytest.mark.parametrize("M,N,K", [(77, 3072, 4096), (200, 2560, 8192), (512, 3072, 3072), (250, 12288, 1152)])
 def test_the_choice_and_its_neighbours(M, N, K):
   """By shape, against the wide kernel, on both sides of a round: M rows and as many as need one more."""
   from cache_dit_amd import _native, ops
