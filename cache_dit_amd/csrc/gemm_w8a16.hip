@@ -1729,7 +1729,10 @@ static int choose_one_round(const GemmArgs& g) {
     const int64_t t = launch_ns(kOneLaunch, c, tiles, cus, g.K / BKE);
     if (t < time) best = c.variant, time = t;
   }
-  return best;
+  // One round of 256 x 192 tiles in place of two of 128 x 128: not where the weights' rows are whole lines of 128 bytes. us, two rounds / one, M x N x K: 616 x 12224 x 8064 119 / 132, 1152 x 6624 x
+  // 11392 164 / 179 (36 such problems: 1.06 of the time, none faster); 630 x 12288 x 4800 89 / 82 (0.97 over 38 with K a multiple
+  // of 64, 0.85 over 225 with K remainders).
+  return best < 21 && g.K % 128 == 0 ? -1 : best;
 }
 
 // Up to 16 rows on tiles (tiles_better_for_few()): the kernel above in place of the 32 x 32 tiles, whose sums it gives bit for

@@ -117,6 +117,8 @@ def test_tiles_for_k_remainders(lib, M, N, K, want):
     (2257, 272, 15680, 25), (2346, 288, 3392, 25), (2277, 272, 1408, 25), (1738, 272, 2944, 25),
     (158, 4800, 14400, 26), (152, 4768, 6320, 26), (146, 3520, 11392, 25), (254, 2896, 7744, 26), (42, 11008, 9536, 25),
     (245, 2560, 1664, 25), (299, 2368, 3328, 26), (77, 3072, 4096, 21), (154, 5056, 2560, 26),
+    # a round of 256 x 192 tiles or two of 128 x 128
+    (616, 12224, 8064, 11), (1152, 6624, 11392, 11), (630, 12288, 4800, 8), (878, 6928, 13424, 8),
     # shorter K
     (1524, 288, 256, 13), (53, 6016, 320, 13), (127, 5584, 192, 13),
     # up to 16 rows
