@@ -2346,7 +2346,7 @@ struct WideOk {
 };
 
 // The tile of the wide kernel (or of the tiled one) for a K of whole steps.
-int choose_whole(const GemmArgs& g) {
+static int choose_whole(const GemmArgs& g) {
   // the wide kernels stream K two or more steps ahead: shorter K runs the 128x128 kernel
   const WideOk wide_ok{g.K};
   if (g.out_dtype != CDIT_DT_BF16) {
@@ -2388,7 +2388,7 @@ constexpr TileTime kOneRound[] = {{15, 256, 192, V15::DEPTH, 5000, 987}, {16, 12
 //   1221 x 1408 x 13568 (220, 195) 40.6 / 45.1; 1265 x 1216 x 5888 (200, 182; 17 of 96 rows) 21.6 / 18.1; 5283 x 304 x 2560 10.1 / 11.1.
 // Over 4400 problems for which the choice among the tiles of one round differs from the older one 0.85 of the time of the
 // older one with and without this; 13 are more than 3 % slower than that (6 % the worst), without it 88 (16 %).
-bool older_better(const GemmArgs& g, int tile, int64_t cus) {
+static bool older_better(const GemmArgs& g, int tile, int64_t cus) {
   const int64_t tiles = tiles32(g.M, g.N).tiles;
   if (tile == 38) return g.K < 4 * BK && tile32_better(g);
   if (tile == 33) {

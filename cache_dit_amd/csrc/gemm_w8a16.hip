@@ -1705,14 +1705,54 @@ int choose_tile(const GemmArgs& g) {
 // Tiles for problems that one round of them covers, with their measured round times: the kernel above (21 to 29) and the
 // wide kernel's. Fitted, with a start of 3 us, to the times of 300 problems with every tile (M 17 to 3000, K 1024 to 15360, N 1024
 // to 12288, at most 128 tiles of 256 x 256, weights from HBM; 7 % rms): of those that one round covers it takes one that is
-// 0.7 % off the best (geometric mean), 0.88 of the time that the choice among the older tiles gives, with 9 of 300 more than
-// 4 % slower (14 % the worst, 2004 x 1408 x 1088, M x N x K). With K remainders from K = 320 on 0.86 (113 problems).
+// 0.7 % off the best (geometric mean), 0.88 of the time that the choice among the older tiles gives. With K remainders
+// from K = 320 on 0.86 (113 problems).
 constexpr LaunchModel kOneLaunch = {2960, 852, 852};
 constexpr TileTime kOneRound[] = {{8, 256, 192, W8::DEPTH, 3218, 912}, {10, 128, 192, W10::DEPTH, 3134, 560}, {11, 128, 128, W11::DEPTH, 2395, 424},
                                   {12, 128, 64, W12::DEPTH, 1467, 299},  {29, 96, 128, 0, 2087, 389},  {28, 96, 96, 0, 1366, 332},
                                   {27, 64, 96, 0, 953, 287},    {26, 80, 64, 0, 686, 252},    {25, 48, 64, 0, 1025, 178},
                                   {24, 32, 64, 0, 593, 163},    {23, 48, 32, 0, 362, 142},    {21, 16, 64, 0, 227, 125},
                                   {22, 32, 32, 0, 0, 105}};
+
+// Whether the older choice is the better one where one round of `tile` is modelled as the shortest. us, older / `tile`, M x N x K.
+// In place of up to two 32 x 32 tiles per CU:
+// - 48 x 32 (23) and 32 x 64 (24) where 32 x 32 have an even number of rows, to K = 2176 and 1664 (K remainders 1344): 42 x 7936 x 2128
+//   9.0 / 9.5 (23), 254 x 1152 x 1056 4.8 / 5.2 (23), 103 x 3008 x 672 4.8 / 5.3 (24); 127 x 3072 x 4160 14.7 / 14.0.
+// - 48 x 32 for up to 48 rows to K = 4224 (43 x 6032 x 2064 8.5 / 9.0), and with K remainders where the last tile's rows are full and
+//   few CUs get a second 32 x 32 (284 x 976 x 13104, 279 tiles, 29.4 / 35.8).
+// - 32 x 64 to K = 832 (200 x 1968 x 704 4.3 / 4.8), and to 2432 with up to one and a half 32 x 32 per CU whose last rows are not
+//   full (20 x 8832 x 1600 7.3 / 7.7).
+// And of up to three per CU: 48 x 64 (25) for short K and few columns (492 x 1216 x 1344 6.4 / 7.0), 80 x 64 (26) for up to 128 rows and
+// K = 1408 (57 x 8208 x 1360 9.0 / 10.7).
+// In place of one round of the wide kernel's tiles, whose rows beyond M are all the same row and cost next to nothing:
+// - 64 x 96 (27) where the last tile of either has 33 to 64 rows, 128 x 64 the emptier one, from K = 2048 on: 178 x 8160 x 14896 88 / 105,
+//   177 x 6144 x 13952 60 / 67; 248 x 5376 x 6016 35.5 / 32.1.
+// - 96 x 128 (29) where the last tile of 128 x 128 is the emptier one, K no multiple of 128: 1051 x 2336 x 8304 68 / 82; 1391 x 1888 x
+//   5984 (111 of 128 rows) 58 / 49.
+// Over 3000 problems for which the choice among the tiles of one round differs from the older one 0.85 of the time of the
+// older one with and without this; 54 are more than 3 % slower than that (16 % the worst), without it 128 (23 %).
+static bool older_better(const GemmArgs& g, int tile, int64_t cus) {
+  auto rest = [&](int rows) { return (g.M - 1) % rows + 1; };  // rows of the last tile
+  if (wavetile_better(g)) {
+    const Tiles32 t = tiles32(g.M, g.N);
+    const bool two = t.tiles <= 2 * cus, even = (g.M + 31) / 32 % 2 == 0;
+    switch (tile) {
+      case 23:
+        return two && ((even && g.K <= (g.K % BKE ? 1344 : 2176)) || (g.M <= 48 && g.K <= 4224) ||
+                       (g.K % BKE && t.tiles * 8 <= 9 * cus && rest(48) > 34));
+      case 24:
+        return two && ((even && g.K <= (g.K % BKE ? 1344 : 1664) && rest(32) <= 28) || g.K <= 832 ||
+                       (t.padded * 2 <= 3 * cus && g.K <= 2432 && rest(32) <= 24));
+      case 25: return g.K <= 1472 && g.N <= 1536 && t.padded * 2 <= 5 * cus;
+      case 26: return g.K <= 1408 && g.M <= 128;
+      default: return false;
+    }
+  }
+  if (tile == 27) return rest(128) > 32 && rest(128) <= 64 && g.K > 2048 && choose_tile(g) == 12;
+  if (tile == 29)
+    return rest(128) <= 64 && rest(96) > rest(128) && g.K % 128 && (g.K % BKE == 0 || g.K > 1024) && choose_tile(g) == 11;
+  return false;
+}
 
 // The tile of a problem that one round covers, -1 if there is none. Shorter K than 5 steps stays with the other rules (127 x
 // 5584 x 192, M x N x K, 3.8 us and 5.2 with this one), than 10 where those take two or three 32 x 32 tiles per CU (53 x 6016 x
@@ -1732,7 +1772,8 @@ static int choose_one_round(const GemmArgs& g) {
   // One round of 256 x 192 tiles in place of two of 128 x 128: not where the weights' rows are whole lines of 128 bytes. us, two rounds / one, M x N x K: 616 x 12224 x 8064 119 / 132, 1152 x 6624 x
   // 11392 164 / 179 (36 such problems: 1.06 of the time, none faster); 630 x 12288 x 4800 89 / 82 (0.97 over 38 with K a multiple
   // of 64, 0.85 over 225 with K remainders).
-  return best < 21 && g.K % 128 == 0 ? -1 : best;
+  if (best < 21 && g.K % 128 == 0) return -1;
+  return best >= 21 && older_better(g, best, cus) ? -1 : best;
 }
 
 // Up to 16 rows on tiles (tiles_better_for_few()): the kernel above in place of the 32 x 32 tiles, whose sums it gives bit for

@@ -119,6 +119,11 @@ def test_tiles_for_k_remainders(lib, M, N, K, want):
     (245, 2560, 1664, 25), (299, 2368, 3328, 26), (77, 3072, 4096, 21), (154, 5056, 2560, 26),
     # a round of 256 x 192 tiles or two of 128 x 128
     (616, 12224, 8064, 11), (1152, 6624, 11392, 11), (630, 12288, 4800, 8), (878, 6928, 13424, 8),
+    # where the older tiles stay
+    (94, 2752, 1216, 23), (124, 2752, 1216, 13), (254, 1152, 1056, 13), (103, 3008, 672, 13), (127, 3072, 4160, 24), (43, 6032, 2064, 13), (43, 6032, 4288, 23),
+    (284, 976, 13104, 13), (200, 1968, 704, 13), (20, 8832, 1600, 13), (20, 8832, 2496, 24), (492, 1216, 1344, 13), (57, 8208, 1360, 13),
+    (57, 8208, 1424, 26), (178, 8160, 14896, 12), (177, 6144, 13952, 12), (248, 5376, 6016, 27), (1051, 2336, 8304, 11),
+    (1391, 1888, 5984, 29),
     # shorter K
     (1524, 288, 256, 13), (53, 6016, 320, 13), (127, 5584, 192, 13),
     # up to 16 rows
