@@ -2318,23 +2318,21 @@ int launch_other_out(const GemmArgs& g, int variant, hipStream_t stream) {
 // conversions of two steps cost nothing (36 x 3904 x 256, M x N x K: 7.4 us with the tiled kernel, 4.2).
 bool tile32_tail(const GemmArgs& g) { return g.K % BK != 0 || g.K < 3 * BK; }
 
-// More than 16 rows on the workgroup-per-tile kernel: up to three tiles per CU (figures at the kernel; beyond, it wins with short
-// K and loses with long: 864 tiles 7.1 us with the wide kernel, 6.4 with this one at K = 896, 816 tiles 30.1
-// and 32.9 at K = 10624). With K remainders, where the wide kernel's wavefronts convert, up to five for short
-// K (1209 tiles 9.5 and 8.3), but 144 x 1680 x 8032 (1255 tiles) 15.4 and 17.3, 72 x 8992 x 11840 (1110) 52.9
-// and 65.4; four to K = 6144: 1199 x 4160 x 704 (836) 24.5 and 21.9, 75 x 4528 x 9088 (852) 28.9 and 30.5. From K = 2048 on it counts if some XCDs get so many more columns than others (Tiles32::padded) that
-// theirs are more than three per CU: 1579 x 12032 x 352 (550 tiles, 800 padded) 26.9 and 41.8, 1631 x 9600 x 480
-// (765 and 816) 30.4 and 37.2; but 203 x 4992 x 3392 (742 and 784) 16.1 and 15.3, 1107 x 384 x 592 7.1 and 4.5. (M x K x
-// N.) Four per CU of an XCD are the limit for shorter K too: 2280 x 1408 x 320 (720 and 1152) 7.3 and 9.0, 2416 x
-// 896 x 288 5.8 and 6.4; with K remainders six below K = 1024: 2240 x 15136 x 288 74 and 89, 1366 x 3920 x 576 23.5 and
-// 26.8. Over 1900 shapes it is 0.7 % off the better one (geometric mean), the worst 14 % (1398 x 11392 x 496).
+// More than 16 rows on the workgroup-per-tile kernel. K remainders, where the wide kernel's wavefronts convert: up to five
+// tiles per CU for short K (160 x 8192 x 400, 1280 tiles, is the last that goes there), four from K = 1024 on (144 x 8032 x 1680, 1255
+// tiles, 15.4 us with the wide kernel and 17.3 with this one; 1199 x 704 x 4160, 836, 24.5 and 21.9), three from K = 6144 on (75 x 9088
+// x 4528 28.9 and 30.5, 72 x 11840 x 8992 52.9 and 65.4). K of one or two steps: five. Longer K of whole steps has one round of
+// the tiles below in front (choose_one_round()); what it leaves here, up to three per CU, are fp32 outputs of K to 1024 and what
+// older_better() gives back (M x N x K: 96 x 8192 x 1024, fp32, 768 tiles; 49 x 7072 x 384). If some XCDs get many more columns
+// than others (Tiles32::padded), at most four per CU of an XCD (three from K = 2048 on), six with K remainders to K = 1024: 2416 x 288 x 896 (684 tiles and
+// 1216 padded) 5.8 and 6.4; 2240 x 288 x 15136 74 and 89, 1366 x 576 x 3920 23.5 and 26.8. Over the shapes with K remainders 0.7 %
+// off the better one (geometric mean), the worst 14 % (1398 x 496 x 11392).
 bool tile32_better(const GemmArgs& g) {
   const int64_t cus = cu_count() > 0 ? cu_count() : 256;
   const Tiles32 t = tiles32(g.M, g.N);
   if (t.padded > (g.K % BK != 0 && g.K <= 1024 ? 6 : 4) * cus && g.K >= 3 * BK) return false;
   if (g.K % BK != 0) return t.tiles <= (g.K > 6144 ? 3 : g.K > 1024 ? 4 : 5) * cus;
-  if (g.K < 3 * BK) return t.tiles <= 5 * cus;
-  return t.tiles <= 3 * cus && (g.K <= 2048 || t.padded <= 3 * cus || (g.K <= 6144 && t.padded * 10 <= t.tiles * 11));
+  return t.tiles <= (g.K < 3 * BK ? 5 : 3) * cus && (g.K <= 2048 || t.padded <= 3 * cus);
 }
 
 // at least `depth` K steps to prefetch, and at least 3: the epilogue operands of a tile are

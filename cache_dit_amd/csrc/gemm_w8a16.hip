@@ -1668,24 +1668,16 @@ bool tiles_better_for_few(const GemmArgs& g) {
   return g.M == 2 && g.K > 4096 && g.N > 8000;
 }
 
-// More than 16 rows on the workgroup-per-tile kernel; us, wide kernel / this one, M x N x K. Two tiles per CU and less: always,
-// unless some XCDs get so many more columns than others (Tiles32::padded) that theirs are more than three per CU, from K
-// = 1024 on (1738 x 272 x 2944, 476 tiles and 880 padded, 16.4 / 18.7; up to K = 4096 not for the last tenth, 299 x 2368 x 3328,
-// 740 and 800, 18.1 / 15.1); below, more than four (1524 x 288 x 256 7.1 / 4.0).
-// Beyond four the CUs take a second round: 2257 x 272 x 15680, 639 and 1136, 63 / 133. Up to three per CU on weights of up to
-// 20 MB (486 shapes: 0.73 of the time in the middle, 0.95 at the 95th percentile); on more where there are few of the wide
-// kernel's smallest tiles (254 x 2896 x 7744, 92 of 128 x 64, 43.5 / 32.1) or they are mostly empty (42 x 11008 x 9536 42.9 /
-// 37.4), else a round of those is the faster one: 158 x 4800 x 14400 59.2 / 72.1, 152 x 4768 x 6320 38.7 / 49.3, 146 x 3520 x
-// 11392 46.5 / 55.0. At four per CU it wins or loses with the shape. Over 720 shapes of two to three per CU 1 % off the better one
-// (geometric mean), 7 are more than 4 % slower than the wide kernel (17 % the worst, 1327 x 496 x 15424).
+// More than 16 rows on the workgroup-per-tile kernel, where one round of the tiles below is not in front of it
+// (choose_one_round(), older_better()): up to three tiles per CU, unless some XCDs get many more columns than others
+// (Tiles32::padded), more than four per CU of an XCD (1524 x 288 x 256, M x N x K, 768 padded, 7.1 us with the wide kernel and 4.0 with
+// this one) or, from K = 1024 on, three (up to K = 4096 not for the last tenth).
 bool wavetile_better(const GemmArgs& g) {
   if (g.N % 16) return false;
   const int64_t cus = cu_count() > 0 ? cu_count() : 256;
   const Tiles32 t = tiles32(g.M, g.N);
   if (t.tiles > 3 * cus || t.padded > 4 * cus) return false;
-  if (g.K > 1024 && t.padded > 3 * cus && (g.K > 4096 || t.padded * 10 > t.tiles * 11)) return false;
-  if (t.tiles <= 2 * cus || (int64_t)g.N * g.K <= 20000000 || g.M <= 48) return true;
-  return (int64_t)((g.M + 127) / 128) * ((g.N + 63) / 64) * 11 <= 4 * cus;
+  return g.K <= 1024 || t.padded <= 3 * cus || (g.K <= 4096 && t.padded * 10 <= t.tiles * 11);
 }
 
 // at least `depth` K steps to prefetch, and at least 3: the epilogue operands of a tile are
@@ -1730,28 +1722,25 @@ constexpr TileTime kOneRound[] = {{8, 256, 192, W8::DEPTH, 3218, 912}, {10, 128,
 // - 96 x 128 (29) where the last tile of 128 x 128 is the emptier one, K no multiple of 128: 1051 x 2336 x 8304 68 / 82; 1391 x 1888 x
 //   5984 (111 of 128 rows) 58 / 49.
 // Over 3000 problems for which the choice among the tiles of one round differs from the older one 0.85 of the time of the
-// older one with and without this; 54 are more than 3 % slower than that (16 % the worst), without it 128 (23 %).
+// older one with and without this; 54 are more than 3 % slower than that (16 % the worst), without it 128 (18 %).
 static bool older_better(const GemmArgs& g, int tile, int64_t cus) {
   auto rest = [&](int rows) { return (g.M - 1) % rows + 1; };  // rows of the last tile
-  if (wavetile_better(g)) {
-    const Tiles32 t = tiles32(g.M, g.N);
-    const bool two = t.tiles <= 2 * cus, even = (g.M + 31) / 32 % 2 == 0;
-    switch (tile) {
-      case 23:
-        return two && ((even && g.K <= (g.K % BKE ? 1344 : 2176)) || (g.M <= 48 && g.K <= 4224) ||
-                       (g.K % BKE && t.tiles * 8 <= 9 * cus && rest(48) > 34));
-      case 24:
-        return two && ((even && g.K <= (g.K % BKE ? 1344 : 1664) && rest(32) <= 28) || g.K <= 832 ||
-                       (t.padded * 2 <= 3 * cus && g.K <= 2432 && rest(32) <= 24));
-      case 25: return g.K <= 1472 && g.N <= 1536 && t.padded * 2 <= 5 * cus;
-      case 26: return g.K <= 1408 && g.M <= 128;
-      default: return false;
-    }
+  const Tiles32 t = tiles32(g.M, g.N);
+  const bool two = t.tiles <= 2 * cus, even = (g.M + 31) / 32 % 2 == 0;
+  switch (tile) {
+    case 23:
+      return two && ((even && g.K <= (g.K % BKE ? 1344 : 2176)) || (g.M <= 48 && g.K <= 4224) ||
+                     (g.K % BKE && t.tiles * 8 <= 9 * cus && rest(48) > 34)) && wavetile_better(g);
+    case 24:
+      return two && ((even && g.K <= (g.K % BKE ? 1344 : 1664) && rest(32) <= 28) || g.K <= 832 ||
+                     (t.padded * 2 <= 3 * cus && g.K <= 2432 && rest(32) <= 24)) && wavetile_better(g);
+    case 25: return g.K <= 1472 && g.N <= 1536 && t.padded * 2 <= 5 * cus && wavetile_better(g);
+    case 26: return g.K <= 1408 && g.M <= 128 && wavetile_better(g);
+    case 27: return rest(128) > 32 && rest(128) <= 64 && g.K > 2048 && choose_tile(g) == 12;
+    case 29:
+      return rest(128) <= 64 && rest(96) > rest(128) && g.K % 128 && (g.K % BKE == 0 || g.K > 1024) && choose_tile(g) == 11;
+    default: return false;
   }
-  if (tile == 27) return rest(128) > 32 && rest(128) <= 64 && g.K > 2048 && choose_tile(g) == 12;
-  if (tile == 29)
-    return rest(128) <= 64 && rest(96) > rest(128) && g.K % 128 && (g.K % BKE == 0 || g.K > 1024) && choose_tile(g) == 11;
-  return false;
 }
 
 // The tile of a problem that one round covers, -1 if there is none. Shorter K than 5 steps stays with the other rules (127 x
