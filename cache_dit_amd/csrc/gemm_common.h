@@ -335,19 +335,20 @@ __device__ __forceinline__ void tile_epilogue(v16f (&acc)[C::TM][C::TN], const G
 
 // Epilogue of the kernels with a workgroup per tile and wavefronts that only feed it (FP8 and weight-only). acc[i][j][e] is
 // out[16 i + (lane & 15)][C::col(j, lane >> 4) + e] of the wave tile at out_wave, of which rows x cols exist. Per element: one
-// multiply by a_scale (1 in the weight-only kernel), one FMA with b_scale and bias, optional GELU. 16-bit outputs change
-// lanes before they are stored so that adjacent lanes hold adjacent bytes (the memory pipeline merges only those): C::LP
-// blocks of 64 columns as whole lines, C::NH of 32, and C::ODD fragments of 16. Rows beyond the last are beyond the descriptor,
-// columns beyond the last get an offset that is (N % 8 == 0: the 4 or 8 columns of a lane are all in or all out).
+// multiply by a_scale (1 in the weight-only kernel), one FMA with b_scale and bias, optional GELU. A wave tile has up to three
+// fragments of 16 columns. 16-bit outputs of a pair of them (C::NH) change lanes before they are stored so that four adjacent
+// lanes hold the 64 adjacent bytes of a row (the memory pipeline merges only those); a single fragment (C::ODD) is stored as it
+// is, 8 bytes per lane. Rows beyond the last are beyond the descriptor, columns beyond the last get an offset that is
+// (N % 8 == 0: the 4 or 8 columns of a lane are all in or all out).
 template <class C, int OUT, bool GELU>
 __device__ __forceinline__ void store_fed_tile(const v4f (&acc)[C::TM][C::TN], const float (&as)[C::TM],
                                                const v4f (&bs)[C::TN], const uint2 (&bi)[C::TN], uint8_t* out_wave,
                                                int64_t ldo_elems, int rows_wave, int cols_wave, int lane) {
   constexpr int OB = OUT == CDIT_DT_F32 ? 4 : 2, TM = C::TM, TN = C::TN;
+  static_assert(TN <= 3 && TN == 2 * C::NH + C::ODD, "a pair of fragments and a single one");
   const uint32_t ldo = (uint32_t)ldo_elems * OB;
   const int r16 = lane & 15, kg = lane >> 4;
   auto at = [&](int row, int c) { return (int)(c < cols_wave ? (uint32_t)row * ldo + (uint32_t)(c * OB) : 0x80000000u); };
-  const int bp_line = 4 * (16 * (lane & 3) + 8 * ((lane >> 2) & 1) + (lane >> 3));
   const int bp_half = 4 * (16 * (lane & 3) + (lane >> 2));
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
@@ -376,27 +377,12 @@ __device__ __forceinline__ void store_fed_tile(const v4f (&acc)[C::TM][C::TN], c
       }
     }
     if constexpr (OUT != CDIT_DT_F32) {
-#pragma unroll
-      for (int v = 0; v < C::LP; ++v) {
-        v4u x, y;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          const int w0 = (int)pk[4 * v + (k >> 1)][k & 1], w1 = (int)pk[4 * v + 2 + (k >> 1)][k & 1];
-          const int p = __builtin_amdgcn_update_dpp(w0, w1, 0x128, 0xf, 0xc, false);
-          const int q = __builtin_amdgcn_update_dpp(w1, w0, 0x128, 0xf, 0x3, false);
-          x[k] = (uint32_t)__builtin_amdgcn_ds_bpermute(bp_line, p);
-          y[k] = (uint32_t)__builtin_amdgcn_ds_bpermute(bp_line, q);
-        }
-        const int c = 64 * v + 8 * (lane & 7);
-        __builtin_amdgcn_raw_buffer_store_b128(x, out_row, at(lane >> 3, c), 0, 2);
-        __builtin_amdgcn_raw_buffer_store_b128(y, out_row, at(8 + (lane >> 3), c), 0, 2);
-      }
       if constexpr (C::NH) {
         v4u x;
 #pragma unroll
         for (int k = 0; k < 4; ++k)
-          x[k] = (uint32_t)__builtin_amdgcn_ds_bpermute(bp_half, (int)pk[4 * C::LP + (k >> 1)][k & 1]);
-        __builtin_amdgcn_raw_buffer_store_b128(x, out_row, at(lane >> 2, 64 * C::LP + 8 * (lane & 3)), 0, 0);
+          x[k] = (uint32_t)__builtin_amdgcn_ds_bpermute(bp_half, (int)pk[k >> 1][k & 1]);
+        __builtin_amdgcn_raw_buffer_store_b128(x, out_row, at(lane >> 2, 8 * (lane & 3)), 0, 0);
       }
       if constexpr (C::ODD)
         __builtin_amdgcn_raw_buffer_store_b64(v2u{pk[TN - 1][0], pk[TN - 1][1]}, out_row, at(r16, C::col(TN - 1, kg)),

@@ -1444,7 +1444,7 @@ int launch_tile32(const GemmArgs& g, hipStream_t stream) {
 
 // ---------------------------------------------------------------------------
 // Problems that one round of tiles covers (a prompt's or a few hundred tokens' projections, K a whole number of
-// steps): a workgroup per tile, four (three, five) wavefronts that multiply and two that only feed them.
+// steps): a workgroup per tile, two to five wavefronts that multiply and two that only feed them.
 // What bounds such a problem is what one CU gets through its vector memory path: some 64 KB in flight, whatever
 // the instructions issued ahead and whatever their cache policy, i.e. 58 GB/s of panels that come from HBM, 85 to 100
 // from the last-level cache (loads alone, without the arithmetic, of 256 x 12288 x 3072, M x N x K, on 192 tiles of 128 x
@@ -1471,9 +1471,9 @@ struct CfgFed {
   static constexpr int WM = BM / WGM, WN = BN / WGN, TM = WM / 16, TN = WN / 16;  // wave tile, in fragments of 16 rows
   static constexpr int A_BYTES = BM * 128, PART = (BM + BN) * 128, STAGE = SUB * PART, LDS_BYTES = DEPTH * STAGE;
   static constexpr int NDMA = (BM + BN) / 8 / FEEDERS;  // DMA instructions (8 panel rows) per feeding wavefront and part
-  // Columns of a wave tile: LP blocks of 64 and NH of 32 in pairs of fragments as in the wide kernel, with an odd TN
-  // one fragment of 16 in its natural order behind them (store_fed_tile).
-  static constexpr int LP = TN / 4, NH = TN % 4 / 2, ODD = TN % 2;
+  // Columns of a wave tile: a pair of fragments (NH) in the order of the wide kernel's, and a single one of 16 columns in its
+  // natural order behind it (store_fed_tile).
+  static constexpr int NH = TN / 2, ODD = TN % 2;
   static_assert(BM % (16 * WGM) == 0 && BN % (16 * WGN) == 0 && (BM + BN) / 8 % FEEDERS == 0, "whole fragments, whole instructions");
   static_assert(DEPTH >= 3 && (DEPTH - 1) * NDMA * SUB <= 63 && LDS_BYTES <= 160 * 1024, "vmcnt has 6 bits; LDS");
   // first of the four columns (of the wave tile) that lane group q holds of fragment j
