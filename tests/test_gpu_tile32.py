@@ -70,11 +70,14 @@ def test_bits_of_the_wide_kernel(M, N, K, dtype):
 
 
 @pytest.mark.parametrize("M,N", [(512, 1536), (512, 1568), (640, 2048), (640, 2080)])
-@pytest.mark.parametrize("K", [128, 256, 1040, 1152])
+@pytest.mark.parametrize("K", [128, 256, 1008, 1024, 1040, 1152])
 def test_on_both_sides_of_the_tile_rule(M, N, K):
-  """768 and 784 tiles (whole steps), 1280 and 1300 (remainders and one or two steps, whose sums are
-  in full fp32 there: products of 448 x 448 that cancel next to products of a few units)."""
-  from cache_dit_amd import ops
+  """768 and 784 tiles (fp32 outputs, whole steps to K = 1024), 1280 and 1300 (remainders to K = 1024 and one or two steps,
+  whose sums are in full fp32 there: products of 448 x 448 that cancel next to products of a few units). Longer K
+  has other rules."""
+  from cache_dit_amd import _native, ops
+  choice = _native.load().cdit_debug_gemm_choice
+  assert (choice(0, M, N, 1024, 2) == 26) == (M * N <= 512 * 1536) and (choice(0, M, N, 1008, 2) == 26) == (M * N <= 640 * 2048)
   g = torch.Generator(device=DEV).manual_seed(M + N + K)
   a, w = _codes((M, K), -3, 4, 16, g), _codes((N, K), -3, 4, 16, g)
   one_m, one_n = torch.ones(M, device=DEV), torch.ones(N, device=DEV)
