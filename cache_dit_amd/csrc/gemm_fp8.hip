@@ -2659,12 +2659,12 @@ int launch_gemm_fp8_grouped(const GemmArgs& common, const GemmGroup& grp, int va
       // (FLUX ff.net.0.proj: 4096 rows fill three rounds of 256 x 256 tiles exactly, the
       // 512 text rows add a fourth, nearly empty one; on its own the text GEMM is one round
       // of small tiles: measured 148 us as two launches, 173 as one). Compare with one
-      // launch per activation, each with the tile it would choose; the time of each launch
-      // counts its start. Over 120 joint-block stages (image 1024 to 6889, text 17 to 512
-      // rows, widths 1536 to 3072) the form chosen is 0.3 % slower than the better one
-      // (geometric mean): 1184 + 59 rows, three members, K 2816: 36 us as one launch, 42 as two.
-      // A text stream that alone would run on 32 x 32 tiles is priced as a tile of the wide kernel:
-      // 6 of the 120 are more than 3 % slower as one launch (2889 + 77 rows, K 2944, N 11776 99.6 us, 94.0 as two).
+      // launch per activation, each priced with the wide kernel's tile for it; the time of each
+      // launch counts its start. 1184 + 59 rows, three members, K 2816: 36 us as one launch, 42 as two.
+      // Not priced is that a single member launched apart may take one round of smaller tiles
+      // (choose_one_round()): over 150 joint-block stages (image 1024 to 6889, text 17 to 512 rows,
+      // widths 1536 to 3072) the form chosen is 0.6 % slower than the better one (geometric mean),
+      // and 9 are more than 3 % slower as one launch (1313 + 205 rows, K 2688, N 10752 57.2 us, 51.7 as two).
       int64_t apart = 0;
       for (int s = 0; s < grp.acts; ++s) {
         auto tiles_s = [&](int bm, int bn) {

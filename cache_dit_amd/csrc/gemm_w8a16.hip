@@ -1889,9 +1889,9 @@ int launch_gemm_w8a16_grouped(const GemmArgs& common, const GemmGroup& grp, int 
     if (grp.acts > 1) {
       // one tile stream against one launch per activation, as in the w8a8 launcher: a small
       // activation can push a batch that filled whole rounds into one more, nearly empty one
-      // (over 120 joint-block stages of 17 to 512 text rows 0.3 % slower than the better form; 1104 +
-      // 100 rows, three members, K 2816: 63 us as one launch, 71 as two. A text stream that alone would run on 32 x
-      // 32 tiles is priced as a tile of the wide kernel: 2104 + 81 rows, K = N = 2816 46.8 us, 42.2 as two)
+      // (1104 + 100 rows, three members, K 2816: 63 us as one launch, 71 as two). As there, one round of
+      // smaller tiles is not priced: over 150 joint-block stages of 17 to 512 text rows 0.4 % slower than the better
+      // form, 8 more than 3 % (2254 + 106 rows, K 10240, N 2560 147 us as one launch, 131 as two)
       int64_t apart = 0;
       for (int s = 0; s < grp.acts; ++s) {
         auto tiles_s = [&](int bm, int bn) {
