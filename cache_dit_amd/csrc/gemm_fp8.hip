@@ -1446,23 +1446,24 @@ int launch_tile32(const GemmArgs& g, hipStream_t stream) {
 // Problems that one round of tiles covers (a prompt's or a few hundred tokens' projections, K a whole number of
 // steps): a workgroup per tile, two to five wavefronts that multiply and two that only feed them.
 // What bounds such a problem is what one CU gets through its vector memory path: some 64 KB in flight, whatever
-// the instructions issued ahead and whatever their cache policy, i.e. 58 GB/s of panels that come from HBM, 85 to 100
+// the instructions issued ahead and whatever their cache policy, i.e. 52 to 60 GB/s of panels that come from HBM, some 90
 // from the last-level cache (loads alone, without the arithmetic, of 256 x 12288 x 3072, M x N x K, on 192 tiles of 128 x
-// 128: 18.4 us from HBM of the kernel's 20.4). Lines that the other workgroups of the XCD have in flight or in the L2 count
+// 128: 18.2 us from HBM of the 20.7 of the wide kernel; profiles/one_round_tiles.txt). Lines that the other workgroups of the XCD have in flight or in the L2 count
 // like the rest, and touching them ahead from another wavefront takes as much of the path as it saves. So the time of a round
 // is (BM + BN) K bytes of the fullest CU, and the tile to take is the one with the shortest sides of which every CU gets
 // at most one: 96 x 96, 48 x 48, 32 x 48, 80 x 48 ... next to the wide kernel's and the 32 x 32 one. us, another weight
-// matrix per launch, the best of those -> this kernel, M x N x K: 77 x 3072 x 4096 10.6 -> 8.0 (48 x 32; on 288 tiles of 32 x 32 some
-// CUs get two), 200 x 2560 x 8192 20.7 -> 15.3, 512 x 3072 x 3072 14.8 -> 12.7 (96 x 96, 192 tiles; 64 x 128 as many), 512 x 3072 x
-// 12288 47.0 -> 37.4, 263 x 1216 x 8832 18.8 -> 13.1. With a second round of tiles it loses to the wide kernel, whose
+// matrix per launch, the best of those -> this kernel, M x N x K: 77 x 3072 x 4096 10.5 -> 8.0 (48 x 32; 32 x 48 the same; on 288
+// tiles of 32 x 32 some CUs get two), 200 x 2560 x 8192 20.7 -> 17.2, 512 x 3072 x 3072 14.8 -> 12.5 (96 x 96, 192 tiles; 64 x 128 as
+// many), 512 x 3072 x 12288 47.0 -> 37.1, 263 x 1216 x 8832 18.6 -> 12.4. With a second round of tiles it loses to the wide kernel, whose
 // stream of panels runs on from one tile to the next: chosen only for one (choose_one_round()).
 // The ring, its barrier and the order of K are those of gemm_fp8_tile32, MFMA and epilogue arithmetic the wide kernel's:
 // the same bits. Stages: as many as keep 64 KB in flight; one more or less is within 2 % (32 x 48: 5 stages 4 % slower
 // than 6), and where two workgroups then fit a CU's LDS a partial second round costs less (64 x 64 with 5 stages in place
 // of 6, 96 x 64 with 4: 9 %). A step is SUB times 128 bytes of K between two barriers: with 256 the shortest steps, those of
-// 32 x 32, take 10 % less (62 x 2560 x 4480, M x N x K: 8.9 us with gemm_fp8_tile32, 8.2), those of 32 x 48 and 48 x 48 1 to
-// 2 % more, of 80 x 48 and 64 x 64, with room for three stages then, 4 to 6 %. Feeding wavefronts: with the multiplying ones issuing the DMA themselves the same time where the
-// panels come from HBM, 22 % longer K steps where they are in the L2 (0.25 us against 0.32 with 128 x 128).
+// 32 x 32, take 7 to 10 % less (62 x 2560 x 4480, M x N x K: 8.8 us with gemm_fp8_tile32, 8.2), those of 32 x 48 and 48 x 48 1 to
+// 2 % more, of 80 x 48 and 64 x 64, with room for three stages then, 4 to 6 %. Feeding wavefronts: with the multiplying
+// ones issuing the DMA themselves the same time where the panels come from HBM, 22 % longer K steps where they are
+// in the L2 (0.25 us against 0.32 with 128 x 128).
 template <int BM_, int BN_, int WGM_, int WGN_, int SUB_, int DEPTH_>
 struct CfgFed {
   static constexpr int BM = BM_, BN = BN_, WGM = WGM_, WGN = WGN_, SUB = SUB_, DEPTH = DEPTH_;

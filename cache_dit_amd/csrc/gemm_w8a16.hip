@@ -1111,7 +1111,7 @@ int launch_wavetile(const GemmArgs& g, hipStream_t stream) {
 
 // ---------------------------------------------------------------------------
 // Problems that one round of tiles covers, as gemm_fp8_fed: bound by what one CU gets through its vector memory path (64 KB
-// in flight: 58 GB/s from HBM, 85 to 100 from the last-level cache), here (2 BM + BN) K bytes of the fullest CU. So tiles that
+// in flight: 52 to 60 GB/s from HBM, some 90 from the last-level cache), here (2 BM + BN) K bytes of the fullest CU. So tiles that
 // are wider than they are high, and of as many shapes as it takes for every CU to get at most one. A wavefront multiplies all
 // rows of the tile with its 16 columns, whose weights are then converted once per workgroup (8 conversions per 16
 // columns and 64 elements next to 2 MFMAs per 16 x 16 block); two wavefronts only feed. A step is SUB times 64
@@ -1121,9 +1121,9 @@ int launch_wavetile(const GemmArgs& g, hipStream_t stream) {
 // the accumulator: a chain of them over the pieces in the order in which the wide kernel's 32x32x16 instructions take theirs
 // (in each 32 elements the first, third, second and fourth eight) gives the same bits, which is what the swap of the piece's
 // two low bits in the swizzle is for.
-// us, another weight matrix per launch, the best of the other kernels -> this one, M x N x K: 77 x 3072 x 4096 13.9 -> 10.9 (16 x
-// 64: 240 tiles; of the 288 of 32 x 32 some CUs get two), 200 x 2560 x 8192 31.5 -> 26.1 (48 x 64), 17 x 3072 x 3072 9.2 -> 8.7
-// (32 x 32), 342 x 2752 x 12352 61.1 -> 46.3 (80 x 64).
+// us, another weight matrix per launch, the best of the other kernels -> this one, M x N x K: 77 x 3072 x 4096 14.0 -> 10.8 (16 x
+// 64: 240 tiles; of the 288 of 32 x 32 some CUs get two), 200 x 2560 x 8192 31.1 -> 22.8 (48 x 64), 17 x 3072 x 3072 9.0 -> 7.4
+// (32 x 32), 342 x 2752 x 12352 61.5 -> 46.6 (80 x 64).
 template <int BM_, int BN_, int WAVES_, int SUB_, int DEPTH_>
 struct CfgFedW {
   static constexpr int BM = BM_, BN = BN_, WAVES = WAVES_, SUB = SUB_, DEPTH = DEPTH_;
