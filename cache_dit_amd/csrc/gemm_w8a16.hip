@@ -1655,13 +1655,16 @@ bool tiles_better_for_few(const GemmArgs& g) {
 // More than 16 rows on the workgroup-per-tile kernel, where one round of the tiles below is not in front of it
 // (choose_one_round(), older_better()): up to three tiles per CU, unless some XCDs get many more columns than others
 // (Tiles32::padded), more than four per CU of an XCD (1524 x 288 x 256, M x N x K, 768 padded, 7.1 us with the wide kernel and 4.0 with
-// this one) or, from K = 1024 on, three (up to K = 4096 not for the last tenth).
+// this one) or, from K = 1024 on, three (up to K = 4096 not for the last tenth). More than two per CU on more than 20 MB of
+// weights: only where there are few of the wide kernel's smallest tiles (158 x 4800 x 14400 59.2 / 72.1, 152 x 4768 x 6320 38.7 / 49.3).
 bool wavetile_better(const GemmArgs& g) {
   if (g.N % 16) return false;
   const int64_t cus = cu_count() > 0 ? cu_count() : 256;
   const Tiles32 t = tiles32(g.M, g.N);
   if (t.tiles > 3 * cus || t.padded > 4 * cus) return false;
-  return g.K <= 1024 || t.padded <= 3 * cus || (g.K <= 4096 && t.padded * 10 <= t.tiles * 11);
+  if (g.K > 1024 && t.padded > 3 * cus && (g.K > 4096 || t.padded * 10 > t.tiles * 11)) return false;
+  if (t.tiles <= 2 * cus || (int64_t)g.N * g.K <= 20000000 || g.M <= 48) return true;
+  return (int64_t)((g.M + 127) / 128) * ((g.N + 63) / 64) * 11 <= 4 * cus;
 }
 
 // at least `depth` K steps to prefetch, and at least 3: the epilogue operands of a tile are
@@ -1694,33 +1697,41 @@ constexpr TileTime kOneRound[] = {{8, 256, 192, W8::DEPTH, 3218, 912}, {10, 128,
 // In place of up to two 32 x 32 tiles per CU:
 // - 48 x 32 (23) and 32 x 64 (24) where 32 x 32 have an even number of rows, to K = 2176 and 1664 (K remainders 1344): 42 x 7936 x 2128
 //   9.0 / 9.5 (23), 254 x 1152 x 1056 4.8 / 5.2 (23), 103 x 3008 x 672 4.8 / 5.3 (24); 127 x 3072 x 4160 14.7 / 14.0.
-// - 48 x 32 for up to 48 rows to K = 4224 (43 x 6032 x 2064 8.5 / 9.0), and with K remainders where the last tile's rows are full and
-//   few CUs get a second 32 x 32 (284 x 976 x 13104, 279 tiles, 29.4 / 35.8).
+// - 48 x 32 for up to 48 rows to K = 4224 (43 x 6032 x 2064 8.5 / 9.0) and with K remainders. Also where the last tile's rows are
+//   full and few CUs get a second 32 x 32: three rows of them to 264 tiles (89 x 2768 x 12144, 261, 28 / 34), more rows with K
+//   remainders to 288 (284 x 976 x 13104, 279, 29.4 / 35.8); 91 x 3008 x 10656, 282, 44.4 / 29.5.
 // - 32 x 64 to K = 832 (200 x 1968 x 704 4.3 / 4.8), and to 2432 with up to one and a half 32 x 32 per CU whose last rows are not
-//   full (20 x 8832 x 1600 7.3 / 7.7).
+//   full (20 x 8832 x 1600 7.3 / 7.7); of 97 to 112 rows to K = 7168 (103 x 2880 x 5952 16.2 / 16.8).
 // And of up to three per CU: 48 x 64 (25) for short K and few columns (492 x 1216 x 1344 6.4 / 7.0), 80 x 64 (26) for up to 128 rows and
 // K = 1408 (57 x 8208 x 1360 9.0 / 10.7).
 // In place of one round of the wide kernel's tiles, whose rows beyond M are all the same row and cost next to nothing:
 // - 64 x 96 (27) where the last tile of either has 33 to 64 rows, 128 x 64 the emptier one, from K = 2048 on: 178 x 8160 x 14896 88 / 105,
 //   177 x 6144 x 13952 60 / 67; 248 x 5376 x 6016 35.5 / 32.1.
+// - 80 x 64 (26) with its last tile full and up to 32 rows in 128 x 64's, from K = 4096 on: 159 x 5312 x 14336 62 / 67.
+// - 96 x 96 (28) with K remainders and up to 32 rows in the last tile of 128 x 128, from K = 4096 on: 284 x 6048 x 13088 92 / 104.
 // - 96 x 128 (29) where the last tile of 128 x 128 is the emptier one, K no multiple of 128: 1051 x 2336 x 8304 68 / 82; 1391 x 1888 x
 //   5984 (111 of 128 rows) 58 / 49.
-// Over 3000 problems for which the choice among the tiles of one round differs from the older one 0.85 of the time of the
-// older one with and without this; 54 are more than 3 % slower than that (16 % the worst), without it 128 (18 %).
+// Over 4000 problems for which the choice among the tiles of one round differs from the older one 0.85 of the time of the
+// older one with and without this; 38 are more than 3 % slower than that (17 % the worst), without it 171 (20 %).
 static bool older_better(const GemmArgs& g, int tile, int64_t cus) {
   auto rest = [&](int rows) { return (g.M - 1) % rows + 1; };  // rows of the last tile
   const Tiles32 t = tiles32(g.M, g.N);
   const bool two = t.tiles <= 2 * cus, even = (g.M + 31) / 32 % 2 == 0;
   switch (tile) {
     case 23:
-      return two && ((even && g.K <= (g.K % BKE ? 1344 : 2176)) || (g.M <= 48 && g.K <= 4224) ||
-                     (g.K % BKE && t.tiles * 8 <= 9 * cus && rest(48) > 34)) && wavetile_better(g);
+      return two && ((even && g.K <= (g.K % BKE ? 1344 : 2176)) || (g.M <= 48 && (g.K <= 4224 || g.K % BKE)) ||
+                     (rest(48) > 34 && g.N > 448 &&
+                      (g.M <= 96 ? t.tiles * 32 <= 33 * cus : g.K % BKE && t.tiles * 8 <= 9 * cus))) && wavetile_better(g);
     case 24:
       return two && ((even && g.K <= (g.K % BKE ? 1344 : 1664) && rest(32) <= 28) || g.K <= 832 ||
-                     (t.padded * 2 <= 3 * cus && g.K <= 2432 && rest(32) <= 24)) && wavetile_better(g);
+                     (t.padded * 2 <= 3 * cus && g.K <= 2432 && rest(32) <= 24) ||
+                     (g.M > 96 && g.M <= 112 && g.K <= 7168)) && wavetile_better(g);
     case 25: return g.K <= 1472 && g.N <= 1536 && t.padded * 2 <= 5 * cus && wavetile_better(g);
-    case 26: return g.K <= 1408 && g.M <= 128 && wavetile_better(g);
+    case 26:
+      if (g.K > 4096) return rest(80) > 64 && rest(128) <= 32 && choose_tile(g) == 12;
+      return g.K <= 1408 && g.M <= 128 && wavetile_better(g);
     case 27: return rest(128) > 32 && rest(128) <= 64 && g.K > 2048 && choose_tile(g) == 12;
+    case 28: return rest(96) > 56 && rest(128) <= 32 && g.K % BKE && g.K > 4096 && choose_tile(g) == 11;
     case 29:
       return rest(128) <= 64 && rest(96) > rest(128) && g.K % 128 && (g.K % BKE == 0 || g.K > 1024) && choose_tile(g) == 11;
     default: return false;

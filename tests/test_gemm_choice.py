@@ -115,15 +115,16 @@ def test_tiles_for_k_remainders(lib, M, N, K, want):
 @pytest.mark.parametrize("M,N,K,want", [
     # tiles of which one round covers the problem
     (2257, 272, 15680, 25), (2346, 288, 3392, 25), (2277, 272, 1408, 25), (1738, 272, 2944, 25),
-    (158, 4800, 14400, 26), (152, 4768, 6320, 26), (146, 3520, 11392, 25), (254, 2896, 7744, 26), (42, 11008, 9536, 25),
+    (158, 4800, 14400, 12), (152, 4768, 6320, 12), (89, 2768, 12144, 13), (91, 3008, 10656, 23), (146, 3520, 11392, 25), (254, 2896, 7744, 26), (42, 11008, 9536, 25),
     (245, 2560, 1664, 25), (299, 2368, 3328, 26), (77, 3072, 4096, 21), (154, 5056, 2560, 26),
     # a round of 256 x 192 tiles or two of 128 x 128
     (616, 12224, 8064, 11), (1152, 6624, 11392, 11), (630, 12288, 4800, 8), (878, 6928, 13424, 8),
     # where the older tiles stay
-    (94, 2752, 1216, 23), (124, 2752, 1216, 13), (254, 1152, 1056, 13), (103, 3008, 672, 13), (127, 3072, 4160, 24), (43, 6032, 2064, 13), (43, 6032, 4288, 23),
+    (94, 2752, 1216, 13), (94, 3008, 1216, 23), (124, 2752, 1216, 13), (254, 1152, 1056, 13), (103, 3008, 672, 13), (127, 3072, 4160, 24), (43, 6032, 2064, 13), (43, 6032, 4288, 23),
     (284, 976, 13104, 13), (200, 1968, 704, 13), (20, 8832, 1600, 13), (20, 8832, 2496, 24), (492, 1216, 1344, 13), (57, 8208, 1360, 13),
     (57, 8208, 1424, 26), (178, 8160, 14896, 12), (177, 6144, 13952, 12), (248, 5376, 6016, 27), (1051, 2336, 8304, 11),
-    (1391, 1888, 5984, 29),
+    (1391, 1888, 5984, 29), (41, 5776, 9040, 13), (41, 5776, 9024, 23), (107, 3456, 2752, 13), (115, 3456, 2752, 24), (159, 5312, 14336, 12),
+    (159, 5312, 4096, 26), (284, 6048, 13088, 11), (284, 6048, 13120, 28),
     # shorter K
     (1524, 288, 256, 13), (53, 6016, 320, 13), (127, 5584, 192, 13),
     # up to 16 rows
