@@ -2324,7 +2324,7 @@ bool tile32_tail(const GemmArgs& g) { return g.K % BK != 0 || g.K < 3 * BK; }
 // tiles, 15.4 us with the wide kernel and 17.3 with this one; 1199 x 704 x 4160, 836, 24.5 and 21.9), three from K = 6144 on (75 x 9088
 // x 4528 28.9 and 30.5, 72 x 11840 x 8992 52.9 and 65.4). K of one or two steps: five. Longer K of whole steps has one round of
 // the tiles below in front (choose_one_round()); what it leaves here, up to three per CU, are fp32 outputs of K to 1024 and what
-// older_better() gives back (M x N x K: 96 x 8192 x 1024, fp32, 768 tiles; 49 x 7072 x 384). If some XCDs get many more columns
+// others_better() gives back (M x N x K: 96 x 8192 x 1024, fp32, 768 tiles; 49 x 7072 x 384). If some XCDs get many more columns
 // than others (Tiles32::padded), at most four per CU of an XCD (three from K = 2048 on), six with K remainders to K = 1024: 2416 x 288 x 896 (684 tiles and
 // 1216 padded) 5.8 and 6.4; 2240 x 288 x 15136 74 and 89, 1366 x 576 x 3920 23.5 and 26.8. Over the shapes with K remainders 0.7 %
 // off the better one (geometric mean), the worst 14 % (1398 x 496 x 11392).
@@ -2361,7 +2361,7 @@ static int choose_whole(const GemmArgs& g) {
 // Tiles for problems that one round of them covers, with their measured round times: the kernel above (31 to 39)
 // and the wide kernel's. Fitted to the times of 250 to 400 problems with every tile (M 17 to 4000, K 1024 to 15360,
 // N 1024 to 12288, at most 160 tiles of 256 x 256, weights from HBM; 8.5 % rms): of those that one round covers it takes one
-// that is 1.1 % off the best (geometric mean), 0.87 of the time that the choice among the older tiles gives (0.94 over all
+// that is 1.1 % off the best (geometric mean), 0.87 of the time that the choice among the other tiles gives (0.94 over all
 // problems of M 17 to 6889, K 256 to 15360, N 256 to 12288, bf16 and fp32 outputs).
 constexpr LaunchModel kOneLaunch = {1425, 907, 907};
 constexpr TileTime kOneRound[] = {{15, 256, 192, V15::DEPTH, 5000, 987}, {16, 128, 192, V16::DEPTH, 3710, 676},
@@ -2372,7 +2372,8 @@ constexpr TileTime kOneRound[] = {{15, 256, 192, V15::DEPTH, 5000, 987}, {16, 12
                                   {31, 32, 48, 3, 1640, 183},            {39, 48, 32, 3, 1992, 153},
                                   {38, 32, 32, 3, 1509, 147}};
 
-// Whether the older choice is the better one where one round of `tile` is modelled as the shortest. us, older / `tile`, M x N x K:
+// Whether what the other rules choose (a tile of the wide kernel, or 32 x 32 ones) is the better one where one round of
+// `tile` is modelled as the shortest. us, theirs / `tile`, M x N x K:
 // - 32 x 32 (38) for K of three steps, of which the second part of a step is empty: 35 x 320 x 384 2.76 / 2.95; from four steps
 //   on the same time and less.
 // - 80 x 48 (33) in place of 32 x 32: for three and four steps (49 x 7072 x 384 4.0 / 4.5, 1440 x 480 x 512 4.0 / 4.2; 426 x 1616 x
@@ -2385,9 +2386,9 @@ constexpr TileTime kOneRound[] = {{15, 256, 192, V15::DEPTH, 5000, 987}, {16, 12
 //   x 4480, 216 and 192 of 96 x 96, 19.9 / 20.7; 446 x 4416 x 7424, 245 and 230, 39.0 / 27.8). Of more rows, also with 11 % more
 //   tiles, unless much of the last 96 x 96 tiles' rows is empty and need not be fetched: 838 x 1984 x 14720 (224, 189) 42.7 / 49.3,
 //   1221 x 1408 x 13568 (220, 195) 40.6 / 45.1; 1265 x 1216 x 5888 (200, 182; 17 of 96 rows) 21.6 / 18.1; 5283 x 304 x 2560 10.1 / 11.1.
-// Over 4400 problems for which the choice among the tiles of one round differs from the older one 0.85 of the time of the
-// older one with and without this; 13 are more than 3 % slower than that (6 % the worst), without it 88 (16 %).
-static bool older_better(const GemmArgs& g, int tile, int64_t cus) {
+// Over 4400 problems for which the choice among the tiles of one round differs from the other rules' 0.85 of the time of
+// theirs with and without this; 13 are more than 3 % slower than that (6 % the worst), without it 88 (16 %).
+static bool others_better(const GemmArgs& g, int tile, int64_t cus) {
   const int64_t tiles = tiles32(g.M, g.N).tiles;
   if (tile == 38) return g.K < 4 * BK && tile32_better(g);
   if (tile == 33) {
@@ -2429,7 +2430,7 @@ static int choose_one_round(const GemmArgs& g) {
     if (other == 17 && (g.M > 1088 || g.K < (g.out_dtype == CDIT_DT_F32 ? 17 : 13) * BK || columns % 8 == 0)) return -1;
     if (other == 18 && tiles128 == cus + 8) return -1;
   }
-  return best >= 31 && older_better(g, best, cus) ? -1 : best;
+  return best >= 31 && others_better(g, best, cus) ? -1 : best;
 }
 
 int launch_gemm_fp8_fed(const GemmArgs& g, int variant, hipStream_t stream) {

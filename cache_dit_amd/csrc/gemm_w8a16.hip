@@ -1653,7 +1653,7 @@ bool tiles_better_for_few(const GemmArgs& g) {
 }
 
 // More than 16 rows on the workgroup-per-tile kernel, where one round of the tiles below is not in front of it
-// (choose_one_round(), older_better()): up to three tiles per CU, unless some XCDs get many more columns than others
+// (choose_one_round(), others_better()): up to three tiles per CU, unless some XCDs get many more columns than others
 // (Tiles32::padded), more than four per CU of an XCD (1524 x 288 x 256, M x N x K, 768 padded, 7.1 us with the wide kernel and 4.0 with
 // this one) or, from K = 1024 on, three (up to K = 4096 not for the last tenth). More than two per CU on more than 20 MB of
 // weights: only where there are few of the wide kernel's smallest tiles (158 x 4800 x 14400 59.2 / 72.1, 152 x 4768 x 6320 38.7 / 49.3).
@@ -1684,7 +1684,7 @@ int choose_tile(const GemmArgs& g) {
 // Tiles for problems that one round of them covers, with their measured round times: the kernel above (21 to 29) and the
 // wide kernel's. Fitted, with a start of 3 us, to the times of 300 problems with every tile (M 17 to 3000, K 1024 to 15360, N 1024
 // to 12288, at most 128 tiles of 256 x 256, weights from HBM; 7 % rms): of those that one round covers it takes one that is
-// 0.7 % off the best (geometric mean), 0.88 of the time that the choice among the older tiles gives. With K remainders
+// 0.7 % off the best (geometric mean), 0.88 of the time that the choice among the other tiles gives. With K remainders
 // from K = 320 on 0.86 (113 problems).
 constexpr LaunchModel kOneLaunch = {2960, 852, 852};
 constexpr TileTime kOneRound[] = {{8, 256, 192, W8::DEPTH, 3218, 912}, {10, 128, 192, W10::DEPTH, 3134, 560}, {11, 128, 128, W11::DEPTH, 2395, 424},
@@ -1693,7 +1693,8 @@ constexpr TileTime kOneRound[] = {{8, 256, 192, W8::DEPTH, 3218, 912}, {10, 128,
                                   {24, 32, 64, 0, 593, 163},    {23, 48, 32, 0, 362, 142},    {21, 16, 64, 0, 227, 125},
                                   {22, 32, 32, 0, 0, 105}};
 
-// Whether the older choice is the better one where one round of `tile` is modelled as the shortest. us, older / `tile`, M x N x K.
+// Whether what the other rules choose (a tile of the wide kernel, or 32 x 32 ones) is the better one where one round of
+// `tile` is modelled as the shortest. us, theirs / `tile`, M x N x K.
 // In place of up to two 32 x 32 tiles per CU:
 // - 48 x 32 (23) and 32 x 64 (24) where 32 x 32 have an even number of rows, to K = 2176 and 1664 (K remainders 1344): 42 x 7936 x 2128
 //   9.0 / 9.5 (23), 254 x 1152 x 1056 4.8 / 5.2 (23), 103 x 3008 x 672 4.8 / 5.3 (24); 127 x 3072 x 4160 14.7 / 14.0.
@@ -1711,9 +1712,9 @@ constexpr TileTime kOneRound[] = {{8, 256, 192, W8::DEPTH, 3218, 912}, {10, 128,
 // - 96 x 96 (28) with K remainders and up to 32 rows in the last tile of 128 x 128, from K = 4096 on: 284 x 6048 x 13088 92 / 104.
 // - 96 x 128 (29) where the last tile of 128 x 128 is the emptier one, K no multiple of 128: 1051 x 2336 x 8304 68 / 82; 1391 x 1888 x
 //   5984 (111 of 128 rows) 58 / 49.
-// Over 4000 problems for which the choice among the tiles of one round differs from the older one 0.85 of the time of the
-// older one with and without this; 38 are more than 3 % slower than that (17 % the worst), without it 171 (20 %).
-static bool older_better(const GemmArgs& g, int tile, int64_t cus) {
+// Over 4000 problems for which the choice among the tiles of one round differs from the other rules' 0.85 of the time of
+// theirs with and without this; 38 are more than 3 % slower than that (17 % the worst), without it 171 (20 %).
+static bool others_better(const GemmArgs& g, int tile, int64_t cus) {
   auto rest = [&](int rows) { return (g.M - 1) % rows + 1; };  // rows of the last tile
   const Tiles32 t = tiles32(g.M, g.N);
   const bool two = t.tiles <= 2 * cus, even = (g.M + 31) / 32 % 2 == 0;
@@ -1757,7 +1758,7 @@ static int choose_one_round(const GemmArgs& g) {
   // 11392 164 / 179 (36 such problems: 1.06 of the time, none faster); 630 x 12288 x 4800 89 / 82 (0.97 over 38 with K a multiple
   // of 64, 0.85 over 225 with K remainders).
   if (best < 21 && g.K % 128 == 0) return -1;
-  return best >= 21 && older_better(g, best, cus) ? -1 : best;
+  return best >= 21 && others_better(g, best, cus) ? -1 : best;
 }
 
 // Up to 16 rows on tiles (tiles_better_for_few()): the kernel above in place of the 32 x 32 tiles, whose sums it gives bit for

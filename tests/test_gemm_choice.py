@@ -87,7 +87,7 @@ def test_fp32_outputs_of_short_k(lib, M, N, K, want):
     # 96 x 96 in place of one round of 64 x 128
     (838, 1984, 14720, 17), (178, 9216, 4480, 17), (1221, 1408, 13568, 17), (5283, 304, 2560, 17), (446, 4416, 7424, 36),
     (316, 5600, 14464, 36), (1163, 1648, 13568, 36), (1265, 1216, 5888, 36), (5283, 304, 5120, 36)])
-def test_where_the_older_tiles_stay(lib, M, N, K, want):
+def test_where_other_tiles_are_better(lib, M, N, K, want):
   for dtype in (F16, BF16, F32):
     if dtype != F32 or K > 1024:
       assert lib.cdit_debug_gemm_choice(0, M, N, K, dtype) == want
@@ -119,7 +119,7 @@ def test_tiles_for_k_remainders(lib, M, N, K, want):
     (245, 2560, 1664, 25), (299, 2368, 3328, 26), (77, 3072, 4096, 21), (154, 5056, 2560, 26),
     # a round of 256 x 192 tiles or two of 128 x 128
     (616, 12224, 8064, 11), (1152, 6624, 11392, 11), (630, 12288, 4800, 8), (878, 6928, 13424, 8),
-    # where the older tiles stay
+    # where other tiles are better than one round
     (94, 2752, 1216, 13), (94, 3008, 1216, 23), (124, 2752, 1216, 13), (254, 1152, 1056, 13), (103, 3008, 672, 13), (127, 3072, 4160, 24), (43, 6032, 2064, 13), (43, 6032, 4288, 23),
     (284, 976, 13104, 13), (200, 1968, 704, 13), (20, 8832, 1600, 13), (20, 8832, 2496, 24), (492, 1216, 1344, 13), (57, 8208, 1360, 13),
     (57, 8208, 1424, 26), (178, 8160, 14896, 12), (177, 6144, 13952, 12), (248, 5376, 6016, 27), (1051, 2336, 8304, 11),
