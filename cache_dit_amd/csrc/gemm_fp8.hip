@@ -11,7 +11,9 @@
 // lane&31, K half lane>>5 of a 64-byte step.
 //
 // Kernels in this file: gemm_fp8_wide (persistent, one wave per SIMD, the one every
-// large or medium problem runs; described in front of CfgWide), gemm_fp8_tiled (the
+// large or medium problem runs; described in front of CfgWide), gemm_fp8_fed and
+// gemm_fp8_tile32 (a workgroup per small tile with wavefronts that only feed it: problems of
+// one round of tiles; K remainders and short K), gemm_fp8_tiled (the
 // older kernel described next, kept for very short K), gemm_fp8_skinny and
 // linear_fp8_skinny_fused (M <= 16), linear_fp8_row1 (M = 1, K <= 4096),
 // gemm_fp8_generic (any shape and alignment).
