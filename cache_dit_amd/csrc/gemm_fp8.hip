@@ -2381,8 +2381,10 @@ constexpr TileTime kOneRound[] = {{15, 256, 192, V15::DEPTH, 5000, 987}, {16, 12
 // - 80 x 48 (33) in place of 32 x 32: for three and four steps (49 x 7072 x 384 4.0 / 4.5, 1440 x 480 x 512 4.0 / 4.2; 426 x 1616 x
 //   512, 2.8 tiles of 32 x 32 per CU, 4.5 / 4.2), and to K = 3072 where 32 x 32 are two tiles per CU at most: 52 x 6704 x 1408
 //   6.1 / 6.4, 102 x 4096 x 1280 5.4 / 5.7; 57 x 7280 x 3840 12.2 / 12.1.
-// - 128 x 96 (37) up to K = 1024 where rows of the output are whole 64-byte pieces, which 128 x 128 stores best: 1037 x 2304 x 512
-//   6.1 / 6.5, 2209 x 1120 x 768 6.9 / 7.2; 531 x 4368 x 512 7.4 / 6.8, 361 x 7936 x 1280 10.9 / 10.4.
+// - 128 x 96 (37) in place of 128 x 128 up to K = 1024 where rows of the output are whole 64-byte pieces, which 128 x 128 stores
+//   best: 1037 x 2304 x 512 6.1 / 6.5, 2209 x 1120 x 768 6.9 / 7.2; 531 x 4368 x 512 7.4 / 6.8, 361 x 7936 x 1280 10.9 / 10.4. K of three steps
+//   is too short for the 128 x 128 tile's ring, and the larger tiles that it then has are slower: 494 x 4576 x 384 7.4 / 6.4 (128 x 192),
+//   587 x 3968 x 384, fp16, 8.6 / 6.2 (256 x 192).
 // - 96 x 96 (36) in place of one round of 64 x 128, as many bytes per CU. The wide kernel gives the XCDs consecutive tiles only
 //   where their number is a multiple of 8: up to 600 rows it is then the faster one if there are 5 % more of them (178 x 9216
 //   x 4480, 216 and 192 of 96 x 96, 19.9 / 20.7; 446 x 4416 x 7424, 245 and 230, 39.0 / 27.8). Of more rows, also with 11 % more
@@ -2397,7 +2399,7 @@ static bool others_better(const GemmArgs& g, int tile, int64_t cus) {
     if (g.K <= 4 * BK ? tiles * 10 > 27 * cus : g.K > 24 * BK || tiles > 2 * cus) return false;
     return tile32_better(g);
   }
-  if (tile == 37) return g.K <= 8 * BK && g.N % 32 == 0;
+  if (tile == 37) return g.K <= 8 * BK && g.N % 32 == 0 && choose_whole(g) == 18;
   if (tile != 36) return false;
   const int64_t n64 = (int64_t)((g.M + 63) / 64) * ((g.N + 127) / 128), n96 = (int64_t)((g.M + 95) / 96) * ((g.N + 95) / 96);
   if (n64 > cus) return false;

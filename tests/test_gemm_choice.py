@@ -83,7 +83,7 @@ def test_fp32_outputs_of_short_k(lib, M, N, K, want):
     (35, 320, 384, TILE32), (35, 320, 512, 38), (49, 7072, 384, TILE32), (1440, 480, 512, TILE32), (1440, 480, 640, 33),
     (426, 1616, 512, 33), (52, 6704, 1408, TILE32), (102, 4096, 1280, TILE32), (52, 6704, 3200, 33), (67, 7552, 1152, 33), (49, 12032, 1152, 33),
     # 128 x 96
-    (1037, 2304, 512, 18), (2209, 1120, 1024, 18), (531, 4368, 512, 37), (361, 7936, 1280, 37),
+    (1037, 2304, 512, 18), (2209, 1120, 1024, 18), (531, 4368, 512, 37), (361, 7936, 1280, 37), (494, 4576, 384, 37), (587, 3968, 384, 37),
     # 96 x 96 in place of one round of 64 x 128
     (838, 1984, 14720, 17), (178, 9216, 4480, 17), (1221, 1408, 13568, 17), (5283, 304, 2560, 17), (446, 4416, 7424, 36),
     (316, 5600, 14464, 36), (1163, 1648, 13568, 36), (1265, 1216, 5888, 36), (5283, 304, 5120, 36)])
