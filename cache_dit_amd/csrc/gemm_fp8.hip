@@ -2327,7 +2327,7 @@ bool tile32_tail(const GemmArgs& g) { return g.K % BK != 0 || g.K < 3 * BK; }
 // x 4528 28.9 and 30.5, 72 x 11840 x 8992 52.9 and 65.4). K of one or two steps: five. Longer K of whole steps has one round of
 // the tiles below in front (choose_one_round()); what it leaves here, up to three per CU, are fp32 outputs of K to 1024 and what
 // others_better() gives back (M x N x K: 96 x 8192 x 1024, fp32, 768 tiles; 49 x 7072 x 384). If some XCDs get many more columns
-// than others (Tiles32::padded), at most four per CU of an XCD (three from K = 2048 on), six with K remainders to K = 1024: 2416 x 288 x 896 (684 tiles and
+// than others (Tiles32::padded), at most four per CU of an XCD, six with K remainders to K = 1024: 2416 x 288 x 896 (684 tiles and
 // 1216 padded) 5.8 and 6.4; 2240 x 288 x 15136 74 and 89, 1366 x 576 x 3920 23.5 and 26.8. Over the shapes with K remainders 0.7 %
 // off the better one (geometric mean), the worst 14 % (1398 x 496 x 11392).
 bool tile32_better(const GemmArgs& g) {
@@ -2335,7 +2335,7 @@ bool tile32_better(const GemmArgs& g) {
   const Tiles32 t = tiles32(g.M, g.N);
   if (t.padded > (g.K % BK != 0 && g.K <= 1024 ? 6 : 4) * cus && g.K >= 3 * BK) return false;
   if (g.K % BK != 0) return t.tiles <= (g.K > 6144 ? 3 : g.K > 1024 ? 4 : 5) * cus;
-  return t.tiles <= (g.K < 3 * BK ? 5 : 3) * cus && (g.K <= 2048 || t.padded <= 3 * cus);
+  return t.tiles <= (g.K < 3 * BK ? 5 : 3) * cus;
 }
 
 // at least `depth` K steps to prefetch, and at least 3: the epilogue operands of a tile are
@@ -2376,35 +2376,35 @@ constexpr TileTime kOneRound[] = {{15, 256, 192, V15::DEPTH, 5000, 987}, {16, 12
 
 // Whether what the other rules choose (a tile of the wide kernel, or 32 x 32 ones) is the better one where one round of
 // `tile` is modelled as the shortest. us, theirs / `tile`, M x N x K:
-// - 32 x 32 (38) for K of three steps, of which the second part of a step is empty: 35 x 320 x 384 2.76 / 2.95; from four steps
-//   on the same time and less.
-// - 80 x 48 (33) in place of 32 x 32: for three and four steps (49 x 7072 x 384 4.0 / 4.5, 1440 x 480 x 512 4.0 / 4.2; 426 x 1616 x
-//   512, 2.8 tiles of 32 x 32 per CU, 4.5 / 4.2), and to K = 3072 where 32 x 32 are two tiles per CU at most: 52 x 6704 x 1408
-//   6.1 / 6.4, 102 x 4096 x 1280 5.4 / 5.7; 57 x 7280 x 3840 12.2 / 12.1.
+// - 80 x 48 (33) in place of 32 x 32 to K = 2432 where no CU of an XCD gets more than two of those: 49 x 7072 x 384 4.81 / 5.14, 52 x 6704
+//   x 1408 7.06 / 7.30, 102 x 4096 x 1280 6.23 / 6.47; 57 x 7280 x 3840 13.25 / 13.23, 632 x 1216 x 1280 (760 tiles, 800 padded) 8.31 / 7.03,
+//   2032 x 256 x 2688 9.67 / 8.52. Three, for three and four steps and many rows: 2028 x 256 x 384 4.44 / 4.94.
 // - 128 x 96 (37) in place of 128 x 128 up to K = 1024 where rows of the output are whole 64-byte pieces, which 128 x 128 stores
 //   best: 1037 x 2304 x 512 6.1 / 6.5, 2209 x 1120 x 768 6.9 / 7.2; 531 x 4368 x 512 7.4 / 6.8, 361 x 7936 x 1280 10.9 / 10.4. K of three steps
 //   is too short for the 128 x 128 tile's ring, and the larger tiles that it then has are slower: 494 x 4576 x 384 7.4 / 6.4 (128 x 192),
 //   587 x 3968 x 384, fp16, 8.6 / 6.2 (256 x 192).
-// - 96 x 96 (36) in place of one round of 64 x 128, as many bytes per CU. The wide kernel gives the XCDs consecutive tiles only
-//   where their number is a multiple of 8: up to 600 rows it is then the faster one if there are 5 % more of them (178 x 9216
-//   x 4480, 216 and 192 of 96 x 96, 19.9 / 20.7; 446 x 4416 x 7424, 245 and 230, 39.0 / 27.8). Of more rows, also with 11 % more
-//   tiles, unless much of the last 96 x 96 tiles' rows is empty and need not be fetched: 838 x 1984 x 14720 (224, 189) 42.7 / 49.3,
-//   1221 x 1408 x 13568 (220, 195) 40.6 / 45.1; 1265 x 1216 x 5888 (200, 182; 17 of 96 rows) 21.6 / 18.1; 5283 x 304 x 2560 10.1 / 11.1.
-// Over 4400 problems for which the choice among the tiles of one round differs from the other rules' 0.85 of the time of
-// theirs with and without this; 13 are more than 3 % slower than that (6 % the worst), without it 88 (16 %).
+// - 96 x 96 (36) in place of one round of 64 x 128, as many bytes per CU, unless much of the last 96 x 96 tiles' rows is empty and
+//   need not be fetched (57 of them exist, 46 to K = 3072, 32 to K = 1536 and of more than 2400 rows): 838 x 1984 x 14720 44.2 / 51.2, 1221 x 1408 x 13568 42.1 / 46.3, 2959 x 608 x 3328 13.8 / 15.1; 1265 x 1216 x 5888
+//   (17 of 96 rows) 22.4 / 19.0, 2600 x 656 x 1792 10.2 / 9.3. Few rows have many columns, and the wide kernel gives the XCDs consecutive
+//   tiles only where their number is a multiple of 8: other numbers, up to 960 rows, only with a tenth more of them than of 96 x 96 (638 x 2944 x
+//   6528, 230 and 217, 29.1 / 25.6), up to 600 rows none, and these only where they are 5 % more: 178 x 9216 x 4480, 216 and 192,
+//   20.9 / 21.4; 446 x 4416 x 7424, 245 and 230, 38.6 / 28.6.
+// Drawn problems for which `tile` (33, 36, 37) differs from the other rules' one: what this takes is 0.11, 0.27 and 0.12 % off the
+// better of both (geometric mean; `tile` always: 0.61, 1.80 and 0.61) and slower than theirs by more than 3 % for 15 of 1295,
+// 15 of 1464 and 1 of 1143, 8 % the worst (`tile` always: 129, 376 and 92). 32 x 32 tiles (38) are it for none of 3900.
 static bool others_better(const GemmArgs& g, int tile, int64_t cus) {
-  const int64_t tiles = tiles32(g.M, g.N).tiles;
-  if (tile == 38) return g.K < 4 * BK && tile32_better(g);
-  if (tile == 33) {
-    if (g.K <= 4 * BK ? tiles * 10 > 27 * cus : g.K > 24 * BK || tiles > 2 * cus) return false;
-    return tile32_better(g);
-  }
+  const Tiles32 t = tiles32(g.M, g.N);
+  if (tile == 33)
+    return g.K <= 19 * BK && t.padded <= (g.K <= 4 * BK && g.M > 1824 ? 3 : 2) * cus && tile32_better(g);
   if (tile == 37) return g.K <= 8 * BK && g.N % 32 == 0 && choose_whole(g) == 18;
   if (tile != 36) return false;
   const int64_t n64 = (int64_t)((g.M + 63) / 64) * ((g.N + 127) / 128), n96 = (int64_t)((g.M + 95) / 96) * ((g.N + 95) / 96);
+  const int rest = (g.M - 1) % 96 + 1;  // rows of the last 96 x 96 tile
   if (n64 > cus) return false;
-  const bool whole_turns = n64 % 8 == 0, full = (g.M - 1) % 96 >= 56 || (g.M > 2400 && g.K < 34 * BK);
-  if (g.M < 600 ? !whole_turns || n96 * 100 >= n64 * 95 : !full || (!whole_turns && n96 * 10 > n64 * 9)) return false;
+  const bool turns = n64 % 8 == 0;
+  if (g.M < 600 && (!turns || n96 * 100 >= n64 * 95 || rest <= 45)) return false;
+  if (g.M < 960 && !turns && n96 * 10 > n64 * 9) return false;
+  if (g.M >= 600 && rest <= (g.K <= 24 * BK ? 45 : 56) && (rest <= 31 || g.M <= 2400 || g.K > 12 * BK)) return false;
   return choose_whole(g) == 17;
 }
 

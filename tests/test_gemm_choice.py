@@ -80,13 +80,14 @@ def test_fp32_outputs_of_short_k(lib, M, N, K, want):
 
 @pytest.mark.parametrize("M,N,K,want", [
     # three steps; 80 x 48 tiles for four steps, and where 32 x 32 are two per CU
-    (35, 320, 384, TILE32), (35, 320, 512, 38), (49, 7072, 384, TILE32), (1440, 480, 512, TILE32), (1440, 480, 640, 33),
+    (35, 320, 384, 38), (35, 320, 512, 38), (49, 7072, 384, TILE32), (1440, 480, 512, 33), (1440, 480, 640, 33),
     (426, 1616, 512, 33), (52, 6704, 1408, TILE32), (102, 4096, 1280, TILE32), (52, 6704, 3200, 33), (67, 7552, 1152, 33), (49, 12032, 1152, 33),
+    (773, 320, 384, 38), (632, 1216, 1280, 33), (2032, 256, 2688, 33), (2028, 256, 384, 26),
     # 128 x 96
     (1037, 2304, 512, 18), (2209, 1120, 1024, 18), (531, 4368, 512, 37), (361, 7936, 1280, 37), (494, 4576, 384, 37), (587, 3968, 384, 37),
     # 96 x 96 in place of one round of 64 x 128
-    (838, 1984, 14720, 17), (178, 9216, 4480, 17), (1221, 1408, 13568, 17), (5283, 304, 2560, 17), (446, 4416, 7424, 36),
-    (316, 5600, 14464, 36), (1163, 1648, 13568, 36), (1265, 1216, 5888, 36), (5283, 304, 5120, 36)])
+    (838, 1984, 14720, 17), (178, 9216, 4480, 17), (1221, 1408, 13568, 17), (5283, 304, 2560, 36), (446, 4416, 7424, 36),
+    (316, 5600, 14464, 36), (1163, 1648, 13568, 36), (1265, 1216, 5888, 36), (638, 2944, 6528, 36), (2959, 608, 3328, 17), (2600, 656, 1792, 36), (5283, 304, 5120, 36)])
 def test_where_other_tiles_are_better(lib, M, N, K, want):
   for dtype in (F16, BF16, F32):
     if dtype != F32 or K > 1024:
