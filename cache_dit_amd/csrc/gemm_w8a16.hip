@@ -1655,16 +1655,15 @@ bool tiles_better_for_few(const GemmArgs& g) {
 // More than 16 rows on the workgroup-per-tile kernel, where one round of the tiles below is not in front of it
 // (choose_one_round(), others_better()): up to three tiles per CU, unless some XCDs get many more columns than others
 // (Tiles32::padded), more than four per CU of an XCD (1524 x 288 x 256, M x N x K, 768 padded, 7.1 us with the wide kernel and 4.0 with
-// this one) or, from K = 1024 on, three (up to K = 4096 not for the last tenth). More than two per CU on more than 20 MB of
-// weights: only where there are few of the wide kernel's smallest tiles (158 x 4800 x 14400 59.2 / 72.1, 152 x 4768 x 6320 38.7 / 49.3).
+// this one) or, from K = 1024 on, three; not more than two per CU on more than 20 MB of weights (158 x 4800 x 14400 59.2 / 72.1,
+// 152 x 4768 x 6320 38.7 / 49.3).
 bool wavetile_better(const GemmArgs& g) {
   if (g.N % 16) return false;
   const int64_t cus = cu_count() > 0 ? cu_count() : 256;
   const Tiles32 t = tiles32(g.M, g.N);
   if (t.tiles > 3 * cus || t.padded > 4 * cus) return false;
-  if (g.K > 1024 && t.padded > 3 * cus && (g.K > 4096 || t.padded * 10 > t.tiles * 11)) return false;
-  if (t.tiles <= 2 * cus || (int64_t)g.N * g.K <= 20000000 || g.M <= 48) return true;
-  return (int64_t)((g.M + 127) / 128) * ((g.N + 63) / 64) * 11 <= 4 * cus;
+  if (g.K > 1024 && t.padded > 3 * cus) return false;
+  return t.tiles <= 2 * cus || (int64_t)g.N * g.K <= 20000000;
 }
 
 // at least `depth` K steps to prefetch, and at least 3: the epilogue operands of a tile are
@@ -1695,46 +1694,47 @@ constexpr TileTime kOneRound[] = {{8, 256, 192, W8::DEPTH, 3218, 912}, {10, 128,
 
 // Whether what the other rules choose (a tile of the wide kernel, or 32 x 32 ones) is the better one where one round of
 // `tile` is modelled as the shortest. us, theirs / `tile`, M x N x K.
-// In place of up to two 32 x 32 tiles per CU:
-// - 48 x 32 (23) and 32 x 64 (24) where 32 x 32 have an even number of rows, to K = 2176 and 1664 (K remainders 1344): 42 x 7936 x 2128
-//   9.0 / 9.5 (23), 254 x 1152 x 1056 4.8 / 5.2 (23), 103 x 3008 x 672 4.8 / 5.3 (24); 127 x 3072 x 4160 14.7 / 14.0.
-// - 48 x 32 for up to 48 rows to K = 4224 (43 x 6032 x 2064 8.5 / 9.0) and with K remainders. Also where the last tile's rows are
-//   full and few CUs get a second 32 x 32: three rows of them to 264 tiles (89 x 2768 x 12144, 261, 28 / 34), more rows with K
-//   remainders to 288 (284 x 976 x 13104, 279, 29.4 / 35.8); 91 x 3008 x 10656, 282, 44.4 / 29.5.
-// - 32 x 64 to K = 832 (200 x 1968 x 704 4.3 / 4.8), and to 2432 with up to one and a half 32 x 32 per CU whose last rows are not
-//   full (20 x 8832 x 1600 7.3 / 7.7); of 97 to 112 rows to K = 7168 (103 x 2880 x 5952 16.2 / 16.8).
-// And of up to three per CU: 48 x 64 (25) for short K and few columns (492 x 1216 x 1344 6.4 / 7.0), 80 x 64 (26) for up to 128 rows and
-// K = 1408 (57 x 8208 x 1360 9.0 / 10.7).
+// In place of up to two 32 x 32 tiles per CU of every XCD (Tiles32::padded; where some get three, those win next to never: 2489 x 256 x 1248
+// 12.9 / 8.6, 1626 x 304 x 816 9.1 / 6.4):
+// - 48 x 32 (23) for up to 48 rows to K = 1472 (41 x 5776 x 1104 6.8 / 7.2), 2448 with rows of weights that are no whole lines (42 x
+//   7936 x 2128 10.2 / 10.7), and with K remainders for up to 44 rows (41 x 5776 x 9040 26.0 / 28.8). Also where the last tile's rows are
+//   full and few CUs get a second 32 x 32: to 264 tiles (89 x 2768 x 12144, 261, 29.4 / 35.4; 96 x 2976 x 896, 279, 6.7 / 6.0), with long
+//   K remainders to 288 (282 x 928 x 4272 12.6 / 14.9; 91 x 3008 x 10656, 282, of two rows of 48 x 32, 45.8 / 31.2).
+// - 32 x 64 (24) to K = 1152 of up to 64 rows (20 x 8832 x 1088 6.9 / 7.2), of four 32-row tiles and their multiples on more than 1328
+//   columns (103 x 3008 x 672 5.5 / 5.9), and beyond 730 rows; 200 x 2800 x 1104 11.4 / 10.5, 127 x 3072 x 4160 16.0 / 15.2.
+// And of up to three per CU: 80 x 64 (26) for up to 128 rows and K = 1152 (98 x 5568 x 1136 8.3 / 9.1; 123 x 6112 x 1312 11.1 / 10.2).
 // In place of one round of the wide kernel's tiles, whose rows beyond M are all the same row and cost next to nothing:
-// - 64 x 96 (27) where the last tile of either has 33 to 64 rows, 128 x 64 the emptier one, from K = 2048 on: 178 x 8160 x 14896 88 / 105,
-//   177 x 6144 x 13952 60 / 67; 248 x 5376 x 6016 35.5 / 32.1.
-// - 80 x 64 (26) with its last tile full and up to 32 rows in 128 x 64's, from K = 4096 on: 159 x 5312 x 14336 62 / 67.
-// - 96 x 96 (28) with K remainders and up to 32 rows in the last tile of 128 x 128, from K = 4096 on: 284 x 6048 x 13088 92 / 104.
-// - 96 x 128 (29) where the last tile of 128 x 128 is the emptier one, K no multiple of 128: 1051 x 2336 x 8304 68 / 82; 1391 x 1888 x
-//   5984 (111 of 128 rows) 58 / 49.
-// Over 4000 problems for which the choice among the tiles of one round differs from the other rules' 0.85 of the time of
-// theirs with and without this; 38 are more than 3 % slower than that (17 % the worst), without it 171 (20 %).
+// - 64 x 96 (27) where the last tile of either has 41 to 64 rows, 128 x 64 the emptier one, from K = 2560 on: 178 x 8160 x 14896 91 / 105,
+//   177 x 6144 x 13952 61 / 67; 248 x 5376 x 6016 36.6 / 33.3.
+// - 80 x 64 (26) with its last tile full and up to 32 rows in 128 x 64's, from K = 4096 on, to 3.5 tiles of 32 x 32 per CU: 159 x 5312 x
+//   14336 64 / 66.
+// - 96 x 128 (29) where the last tile of 128 x 128 is the emptier one, K no multiple of 128 and not short: 1051 x 2336 x 8304 70 / 83; 1391 x
+//   1888 x 5984 (111 of 128 rows) 60 / 51, 1331 x 2256 x 576 11.6 / 9.7.
+// Drawn problems for which `tile` (23, 24, 26, 27, 29) differs from the other rules' one: what this takes is 0.49, 0.22, 0.10, 0.21 and
+// 0.51 % off the better of both (geometric mean; `tile` always: 1.35, 1.10, 0.27, 1.01 and 1.51) and slower than theirs by more
+// than 3 % for 76 of 1503, 42 of 1852, 17 of 2380, 9 of 1142 and 50 of 1400, 19 % the worst (`tile` always: 260, 293, 85, 152 and 243). Rules
+// for 48 x 64 (25) and 96 x 96 (28) were measured to lose more than they give.
 static bool others_better(const GemmArgs& g, int tile, int64_t cus) {
   auto rest = [&](int rows) { return (g.M - 1) % rows + 1; };  // rows of the last tile
   const Tiles32 t = tiles32(g.M, g.N);
-  const bool two = t.tiles <= 2 * cus, even = (g.M + 31) / 32 % 2 == 0;
+  const bool two = t.padded <= 2 * cus;
   switch (tile) {
     case 23:
-      return two && ((even && g.K <= (g.K % BKE ? 1344 : 2176)) || (g.M <= 48 && (g.K <= 4224 || g.K % BKE)) ||
-                     (rest(48) > 34 && g.N > 448 &&
-                      (g.M <= 96 ? t.tiles * 32 <= 33 * cus : g.K % BKE && t.tiles * 8 <= 9 * cus))) && wavetile_better(g);
+      if (!two) return false;
+      if (g.M <= 48) {
+        if (g.K > (g.K % 128 ? 2448 : 1472) && (g.K % BKE == 0 || g.M > 44)) return false;
+      } else if (g.N <= 448 || rest(48) <= 34 || (t.tiles * 32 > 33 * cus && (g.K % BKE == 0 || g.K <= 2448 || g.M <= 96 || t.padded * 8 > 9 * cus))) {
+        return false;
+      }
+      return wavetile_better(g);
     case 24:
-      return two && ((even && g.K <= (g.K % BKE ? 1344 : 1664) && rest(32) <= 28) || g.K <= 832 ||
-                     (t.padded * 2 <= 3 * cus && g.K <= 2432 && rest(32) <= 24) ||
-                     (g.M > 96 && g.M <= 112 && g.K <= 7168)) && wavetile_better(g);
-    case 25: return g.K <= 1472 && g.N <= 1536 && t.padded * 2 <= 5 * cus && wavetile_better(g);
+      return two && g.K <= 1152 && (g.M <= 64 || g.M > 730 || ((g.M + 31) / 32 % 4 == 0 && g.N > 1328)) && wavetile_better(g);
     case 26:
-      if (g.K > 4096) return rest(80) > 64 && rest(128) <= 32 && choose_tile(g) == 12;
-      return g.K <= 1408 && g.M <= 128 && wavetile_better(g);
-    case 27: return rest(128) > 32 && rest(128) <= 64 && g.K > 2048 && choose_tile(g) == 12;
-    case 28: return rest(96) > 56 && rest(128) <= 32 && g.K % BKE && g.K > 4096 && choose_tile(g) == 11;
+      if (g.K > 4096) return rest(80) > 64 && rest(128) <= 32 && t.padded * 2 <= 7 * cus && choose_tile(g) == 12;
+      return g.K <= 1152 && g.M <= 128 && wavetile_better(g);
+    case 27: return rest(128) > 40 && rest(128) <= 64 && g.K > 2528 && choose_tile(g) == 12;
     case 29:
-      return rest(128) <= 64 && rest(96) > rest(128) && g.K % 128 && (g.K % BKE == 0 || g.K > 1024) && choose_tile(g) == 11;
+      return rest(128) <= 64 && rest(96) > rest(128) && g.K % 128 && g.K > (g.K % BKE ? 1024 : 832) && choose_tile(g) == 11;
     default: return false;
   }
 }

@@ -121,11 +121,13 @@ def test_tiles_for_k_remainders(lib, M, N, K, want):
     # a round of 256 x 192 tiles or two of 128 x 128
     (616, 12224, 8064, 11), (1152, 6624, 11392, 11), (630, 12288, 4800, 8), (878, 6928, 13424, 8),
     # where other tiles are better than one round
-    (94, 2752, 1216, 13), (94, 3008, 1216, 23), (124, 2752, 1216, 13), (254, 1152, 1056, 13), (103, 3008, 672, 13), (127, 3072, 4160, 24), (43, 6032, 2064, 13), (43, 6032, 4288, 23),
-    (284, 976, 13104, 13), (200, 1968, 704, 13), (20, 8832, 1600, 13), (20, 8832, 2496, 24), (492, 1216, 1344, 13), (57, 8208, 1360, 13),
+    (94, 2752, 1216, 13), (94, 3008, 1216, 23), (124, 2752, 1216, 24), (254, 1152, 1056, 23), (103, 3008, 672, 13), (127, 3072, 4160, 24), (43, 6032, 2064, 13), (43, 6032, 4288, 23),
+    (284, 976, 13104, 13), (200, 1968, 704, 24), (20, 8832, 1088, 13), (20, 8832, 2496, 24), (492, 1216, 1344, 25), (98, 5568, 1136, 13), (123, 6112, 1312, 26),
     (57, 8208, 1424, 26), (178, 8160, 14896, 12), (177, 6144, 13952, 12), (248, 5376, 6016, 27), (1051, 2336, 8304, 11),
-    (1391, 1888, 5984, 29), (41, 5776, 9040, 13), (41, 5776, 9024, 23), (107, 3456, 2752, 13), (115, 3456, 2752, 24), (159, 5312, 14336, 12),
-    (159, 5312, 4096, 26), (284, 6048, 13088, 11), (284, 6048, 13120, 28),
+    (1391, 1888, 5984, 29), (41, 5776, 9040, 13), (41, 5776, 9024, 23), (107, 3456, 2752, 24), (115, 3456, 2752, 24), (159, 5312, 14336, 12),
+    (159, 5312, 4096, 26), (284, 6048, 13088, 28), (284, 6048, 13120, 28),
+    (2489, 256, 1248, 25), (1626, 304, 816, 24), (1151, 256, 12976, 23), (282, 928, 4272, 13), (96, 2976, 896, 23),
+    (1331, 2256, 576, 29),
     # shorter K
     (1524, 288, 256, 13), (53, 6016, 320, 13), (127, 5584, 192, 13),
     # up to 16 rows
