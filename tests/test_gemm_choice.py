@@ -79,7 +79,7 @@ def test_fp32_outputs_of_short_k(lib, M, N, K, want):
 
 
 @pytest.mark.parametrize("M,N,K,want", [
-    # three steps; 80 x 48 tiles for four steps, and where 32 x 32 are two per CU
+    # 32 x 32 tiles, and in place of 80 x 48 where no XCD has more than two of them per CU
     (35, 320, 384, 38), (35, 320, 512, 38), (49, 7072, 384, TILE32), (1440, 480, 512, 33), (1440, 480, 640, 33),
     (426, 1616, 512, 33), (52, 6704, 1408, TILE32), (102, 4096, 1280, TILE32), (52, 6704, 3200, 33), (67, 7552, 1152, 33), (49, 12032, 1152, 33),
     (773, 320, 384, 38), (632, 1216, 1280, 33), (2032, 256, 2688, 33), (2028, 256, 384, 26),
